@@ -81,7 +81,6 @@ __global__ void k_set_f64(double* p, double v) { *p = v; }
 // Candidates of each tuned choice, in order of preference.
 const std::vector<int> kTunePPDepth = {6, 4, 8, kPPBrick8 + 6, kPPBrick8 + 4, kPPBrick8 + 8};
 const std::vector<int> kTuneDepListThreads = {512, 256, 1024};
-const std::vector<int> kTuneFFTShape = {0, 1, 2};
 const std::vector<int> kTuneInterpShape = {0, 1, 2};
 
 // Autotuner picks persisted across runs: when the environment names a file in
@@ -95,7 +94,6 @@ bool tune_pick_valid(const std::string& key, int pick) {
   static const std::pair<const char*, const std::vector<int>*> choices[] = {
       {"pp_depth_l", &kTunePPDepth},
       {"dep_list_threads_l", &kTuneDepListThreads},
-      {"fft_shape_l", &kTuneFFTShape},
       {"interp_shape_l", &kTuneInterpShape}};
   for (const auto& c : choices)
     if (key.compare(0, std::strlen(c.first), c.first) == 0)
@@ -234,7 +232,6 @@ struct cube_p3m_ctx {
   cube_p3m_ctx* nu = nullptr;
   float nu_mass = 0;
   DevBuf<char> work2;  // the second species' level meshes before they are added
-  DevBuf<char> ftune;  // the FFT shape trials' meshes (released after the trials)
   void sig_add(std::initializer_list<uint64_t> v) { gsig_acc.insert(gsig_acc.end(), v.begin(), v.end()); }
   void graph_drop() {
     for (int i = 0; i < 2; ++i) {
@@ -463,25 +460,6 @@ void cube_p3m_ctx::run_level(int level, int slot, const std::vector<PMBox>& bx_i
       } else if (CP)
         pm_deposit<R>((int)g.izipx, L, boxes.p, nb, xpc(), rhocc(), off.p, mesh, in.mass_p_cdm, s);
     }
-    // launch shape of the tile / sub-tile FFT passes, tuned on a fixed
-    // pattern in scratch meshes (every shape gives the same result)
-    int fshape = 0;
-    if (std::is_same<R, float>::value && level >= 2 && fft_plane_tunable((int)n)) {
-      const std::string key = tune_key("fft_shape", level, n);
-      const int64_t nt = std::min<int64_t>(nmesh, 256);
-      const bool trials = !tune_picks.count(key);
-      if (trials) ftune.ensure(sizeof(R) * (size_t)(nt * nreal));
-      const R n3t = (R)((float)n * (float)n * (float)n);
-      fshape = autotune(
-          key, kTuneFFTShape,
-          [&](int sh) {
-            fill_pattern((float*)ftune.p, nt * nreal, s);
-            fft_convolve<R>(fc, (R*)ftune.p, cplx, G, nt, n3t, (R)0, s, nullptr, "", sh);
-          },
-          ftune.p, sizeof(R) * (size_t)(nt * nreal));
-      if (trials) ftune.release();
-      if (SZ) sig_add({(uint64_t)fshape});
-    }
     // the interpolation's block shape so far (its trials need the potential)
     if (SZ) sig_add({(uint64_t)interp_shape<R>(level, (int)n, L, boxes.p, nb, in, (const R*)nullptr, false)});
     if (!CP) continue;
@@ -502,12 +480,12 @@ void cube_p3m_ctx::run_level(int level, int slot, const std::vector<PMBox>& bx_i
       for (int64_t i = 0; i < nreal; ++i) density_host[i] = (float)tmp[i];
     }
     const R n3 = (R)((float)n * (float)n * (float)n);
-    // PM1 (pencil_fft.f90:77) on the generic line passes: under the overlapped
-    // kick a coarse-mesh plane pass (one 1024-thread, 67.5 KB workgroup per
-    // z plane) waits for room on the CUs behind the second stream's list
-    // building, 1.9 ms against 0.34 for the line passes
-    if (level == 1) fft_convolve<R>(fc, mesh, cplx, G, 1, (R)0, (R)(float)n, s, &tm, tag, -1);
-    else fft_convolve<R>(fc, mesh, cplx, G, nmesh, n3, (R)0, s, &tm, tag, fshape);        // kick.f90:846
+    // PM1 (pencil_fft.f90:77) without the larger plane passes: under the
+    // overlapped kick a workgroup that needs half a CU's LDS waits behind the
+    // second stream's list building (128-point planes of 67.5 KB: 1.9 ms
+    // against 0.34 for line passes)
+    if (level == 1) fft_convolve<R>(fc, mesh, cplx, G, 1, (R)0, (R)(float)n, s, &tm, tag, true);
+    else fft_convolve<R>(fc, mesh, cplx, G, nmesh, n3, (R)0, s, &tm, tag);                // kick.f90:846
     const int ishape = interp_shape<R>(level, (int)n, L, boxes.p, nb, in, mesh, kph == 0);
     {
       KScope k(&tm, (t + "interp_kick").c_str(), cells * sizeof(R));

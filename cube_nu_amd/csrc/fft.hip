@@ -477,21 +477,16 @@ void fft_c2r3d(const FFTCube<R>& c, typename Cplx<R>::T* in, R* out, int64_t nbo
   CUBE_HIP(hipGetLastError());
 }
 
-bool fft_plane_tunable(int n) {
-  if (!use_plane_path()) return false;
-  switch (n) {
-    case 64: case 72: case 80: case 96: case 128: case 144: case 160: return true;
-    default: return false;
-  }
-}
-
 template <typename R>
 void fft_convolve(const FFTCube<R>& c, R* rho, typename Cplx<R>::T* work, const float* G, int64_t nbox, R div3,
-                  R div1, hipStream_t s, KTimer* tm, const char* tag, int shape) {
+                  R div1, hipStream_t s, KTimer* tm, const char* tag, bool small_lds) {
   using C = typename Cplx<R>::T;
-  if (use_plane_path() && shape >= 0 &&
-      fft_convolve_plane<R>(c, rho, work, G, nbox, div3, div1, s, tm ? tm : &null_timer(), tag, shape))
-    return;
+  if (use_plane_path()) {
+    KTimer* t = tm ? tm : &null_timer();
+    // a plane of 88 points is the largest below 40 KB
+    if (!(small_lds && c.n > 88) && fft_convolve_plane<R>(c, rho, work, G, nbox, div3, div1, s, t, tag)) return;
+    if (fft_convolve_lines<R>(c, rho, work, G, nbox, div3, div1, s, t, tag)) return;
+  }
   const int n = c.n, h = n / 2;
   const int64_t nrows = nbox * n * n;
   const double Gb = (double)n * n * n * sizeof(R) * nbox;          // real cube bytes
@@ -529,9 +524,9 @@ void fft_convolve(const FFTCube<R>& c, R* rho, typename Cplx<R>::T* work, const 
 template struct FFTCube<float>;
 template struct FFTCube<double>;
 template void fft_convolve<float>(const FFTCube<float>&, float*, float2*, const float*, int64_t, float, float,
-                                  hipStream_t, KTimer*, const char*, int);
+                                  hipStream_t, KTimer*, const char*, bool);
 template void fft_convolve<double>(const FFTCube<double>&, double*, double2*, const float*, int64_t, double, double,
-                                   hipStream_t, KTimer*, const char*, int);
+                                   hipStream_t, KTimer*, const char*, bool);
 template void fft_r2c3d<float>(const FFTCube<float>&, const float*, float2*, int64_t, hipStream_t);
 template void fft_r2c3d<double>(const FFTCube<double>&, const double*, double2*, int64_t, hipStream_t);
 template void fft_c2r3d<float>(const FFTCube<float>&, float2*, float*, int64_t, hipStream_t);

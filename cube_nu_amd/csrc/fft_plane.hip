@@ -1,460 +1,378 @@
-// fft_plane.hip -- size-specialised 3-pass FFT convolution for cubes with
-// n <= 160: (A) per z-plane, r2c along x and forward c2c along y in LDS;
-// (B) per y-slice, forward c2c along z, times G, inverse along z in LDS;
-// (C) per z-plane, inverse along y and c2r along x, with the normalisation.
-// The radix plan, line counts and per-thread butterfly counts are
-// compile-time constants; stages run in place in LDS (each thread loads its
-// butterflies into registers, barrier, writes them back).
+// fft_plane.hip -- size-specialised 3-pass FFT convolution for cubes whose
+// z-plane of half-complex values fits in LDS: (A) per z-plane, r2c along x and
+// forward c2c along y; (B) lines along z: forward, times G, inverse; (C) per
+// z-plane, inverse along y and c2r along x, with the normalisation.
+//
+// Every line length is split in two radices N = R1 R2 (half-length rows: A1
+// A2) held in registers, and the ends of a pass work on registers directly:
+// the first stage reads global memory, the last one writes it, the r2c split
+// and the c2r merge ride on the row stage next to them (a task owns butterflies
+// j and A1-j, whose elements are each other's conjugate partners), and in pass
+// B the inverse starts with the radix the forward transform ended with, on the
+// same registers.  A plane value crosses LDS 3 times per pass (write + read)
+// and a z value twice, instead of 6 and 6 times with each stage, the split and
+// the kernel product as LDS round trips of their own.  The passes move
+// 8 bytes per mesh point and pass, and are bound by HBM and by the barriers
+// between the stages: the more workgroups share a CU, the better.  Measured on
+// MI355X: 4096 boxes of 80^3, 16.9 GB a pass, 3.1 + 3.5 + 4.0 ms (5.5, 4.9 and
+// 4.2 TB/s; 4.1 + 5.5 + 4.3 ms with a stage per LDS round trip; a large copy
+// reaches 4.9 TB/s), 64 boxes of 160^3 0.52 + 0.51 + 0.62 ms (1.01 + 1.20 +
+// 1.07); 4096 boxes of 40^3 1.3 ms in all and of 56^3 3.5 ms, against 9.4 and
+// 18 ms on the generic line passes.
 #include "fft.h"
+#include "fft_zlines.h"
 #include "timing.h"
 
 namespace cube {
 namespace {
 
-struct Fac {
-  int n;
-  int r[16];
+using namespace fftr;
+
+// Work split of one size: planes per workgroup and threads of the plane passes.
+template <typename R, int N>
+struct Plan {
+  static constexpr int H = N / 2, P = H + 1;
+  static constexpr Split row = split2(H), col = split2(N);
+  static constexpr int R1 = col.r1, R2 = col.r2;
+  // rows: the stage that pairs butterflies has half the tasks, so it takes the larger number of
+  // them: forward A1 = RB, A2 = RS (split stage A1/2+1 tasks), inverse A1 = RS, A2 = RB (merge A2/2+1)
+  static constexpr int RB = cmax(row.r1, row.r2), RS = H / RB, TP = RB / 2 + 1;
+  static constexpr int LS = P % 2 ? P : P + 1;  // odd row stride: rows start in different banks
+  static constexpr int tasks = cmax(N * cmax(RS, TP), P * cmax(R1, R2));
+  static constexpr int bytes = N * LS * (int)sizeof(CP<R>);
+  // small planes: several per workgroup, up to about 512 tasks and 32 KB
+  static constexpr int fit(int pb) { return N % pb == 0 && pb * tasks <= 512 && pb * bytes <= 32768 ? pb : 0; }
+  static constexpr int PB = fit(8) ? 8 : (fit(4) ? 4 : (fit(2) ? 2 : 1));
+  static constexpr int NT = round64(PB * tasks) < 1024 ? round64(PB * tasks) : 1024;
 };
-constexpr Fac factor(int n) {
-  Fac f{};
-  int m = n;
-  // the largest in-register radices first: fewer LDS round trips per line
-  while (m % 16 == 0) { f.r[f.n++] = 16; m /= 16; }
-  while (m % 8 == 0) { f.r[f.n++] = 8; m /= 8; }
-  while (m % 4 == 0) { f.r[f.n++] = 4; m /= 4; }
-  while (m % 2 == 0) { f.r[f.n++] = 2; m /= 2; }
-  while (m % 3 == 0) { f.r[f.n++] = 3; m /= 3; }
-  while (m % 5 == 0) { f.r[f.n++] = 5; m /= 5; }
-  return f;  // m == 1 for every specialised size
-}
 
-template <typename C>
-struct CT;
-template <>
-struct CT<float2> {
-  using R = float;
-  __device__ static float2 mk(float a, float b) { return make_float2(a, b); }
-};
-template <>
-struct CT<double2> {
-  using R = double;
-  __device__ static double2 mk(double a, double b) { return make_double2(a, b); }
-};
-template <typename C>
-__device__ inline C add(C a, C b) { return CT<C>::mk(a.x + b.x, a.y + b.y); }
-template <typename C>
-__device__ inline C sub(C a, C b) { return CT<C>::mk(a.x - b.x, a.y - b.y); }
-template <typename C>
-__device__ inline C mul(C a, C b) { return CT<C>::mk(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x); }
-template <typename C>
-__device__ inline C scl(C a, typename CT<C>::R s) { return CT<C>::mk(a.x * s, a.y * s); }
-template <typename C>
-__device__ inline C miu(C a, typename CT<C>::R u) { return CT<C>::mk(-u * a.y, u * a.x); }  // i*u*a
-template <typename C>
-__device__ inline C cj(C a) { return CT<C>::mk(a.x, -a.y); }
-
-template <int SIGN, int R, typename C>
-__device__ inline void bfly(C* v);
-
-// 4-point DFT of (a, b, c, d) in place, e^{SIGN 2 pi i jk/4}
-template <int SIGN, typename C>
-__device__ inline void dft4(C& a, C& b, C& c, C& d) {
-  using RR = typename CT<C>::R;
-  const RR s = (RR)SIGN;
-  const C p = add(a, c), q = sub(a, c), r = add(b, d), t = miu(sub(b, d), s);
-  a = add(p, r);
-  c = sub(p, r);
-  b = add(q, t);
-  d = sub(q, t);
-}
-
-template <int SIGN, int R, typename C>
-__device__ inline void bfly(C* v) {
-  using RR = typename CT<C>::R;
-  const RR s = (RR)SIGN;
-  if constexpr (R == 16) {
-    // four 4-point DFTs over n = r + 4m, twiddles W16^(r k1), then 4-point
-    // DFTs over r: X[k1 + 4 k2]
-    C u[16];
+// Pass A: PB z-planes: rho (N x N reals) -> complex (N rows of N/2+1).
+template <typename R, int N>
+__global__ void __launch_bounds__((Plan<R, N>::NT)) k_plane_fwd(const R* __restrict__ rho, CP<R>* __restrict__ out,
+                                                                const CP<R>* __restrict__ twg) {
+  using C = CP<R>;
+  using L = Plan<R, N>;
+  constexpr int H = L::H, P = L::P, LS = L::LS, A1 = L::RB, A2 = L::RS, R1 = L::R1, R2 = L::R2, PB = L::PB,
+                NT = L::NT;
+  __shared__ C buf[PB * N * LS];
+  __shared__ C tw[N];
+  const int64_t plane0 = (int64_t)blockIdx.x * PB;
+  const C* src = reinterpret_cast<const C*>(rho + plane0 * N * N);
+  for (int i = threadIdx.x; i < N; i += NT) tw[i] = twg[i];
+  // rows, first stage: global -> registers -> LDS
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      C a = v[r], b = v[r + 4], c = v[r + 8], d = v[r + 12];
-      dft4<SIGN>(a, b, c, d);
-      u[4 * r + 0] = a;
-      u[4 * r + 1] = b;
-      u[4 * r + 2] = c;
-      u[4 * r + 3] = d;
+  for (int i0 = 0; i0 < PB * N * A2; i0 += NT) {
+    const int i = i0 + threadIdx.x;
+    if (i < PB * N * A2) {
+      const int row = i / A2, j = i % A2;
+      C v[A1];
+#pragma unroll
+      for (int r = 0; r < A1; ++r) v[r] = src[row * H + j + r * A2];
+      bfly<-1, A1>(v);
+#pragma unroll
+      for (int k = 0; k < A1; ++k) buf[row * LS + j * A1 + k] = v[k];
     }
-    constexpr double kC[10] = {1.0, 0.92387953251128675613, 0.70710678118654752440, 0.38268343236508977173, 0.0,
-                               -0.38268343236508977173, -0.70710678118654752440, -0.92387953251128675613, -1.0,
-                               -0.92387953251128675613};
-    constexpr double kS[10] = {0.0, 0.38268343236508977173, 0.70710678118654752440, 0.92387953251128675613, 1.0,
-                               0.92387953251128675613, 0.70710678118654752440, 0.38268343236508977173, 0.0,
-                               -0.38268343236508977173};
-#pragma unroll
-    for (int k1 = 0; k1 < 4; ++k1) {
-      C t[4];
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int j = r * k1;  // 0..9
-        const C w = CT<C>::mk((RR)kC[j], s * (RR)kS[j]);
-        t[r] = (j == 0) ? u[4 * r + k1] : mul(u[4 * r + k1], w);
-      }
-      dft4<SIGN>(t[0], t[1], t[2], t[3]);
-#pragma unroll
-      for (int k2 = 0; k2 < 4; ++k2) v[k1 + 4 * k2] = t[k2];
-    }
-  } else if constexpr (R == 8) {
-    // even/odd 4-point DFTs, X[k] = E[k] + W8^k O[k], X[k+4] = E[k] - W8^k O[k]
-    C e0 = v[0], e1 = v[2], e2 = v[4], e3 = v[6], o0 = v[1], o1 = v[3], o2 = v[5], o3 = v[7];
-    dft4<SIGN>(e0, e1, e2, e3);
-    dft4<SIGN>(o0, o1, o2, o3);
-    const RR h = (RR)0.70710678118654752440;
-    const C w1 = CT<C>::mk(h, s * h), w3 = CT<C>::mk(-h, s * h);
-    o1 = mul(o1, w1);
-    o2 = miu(o2, s);
-    o3 = mul(o3, w3);
-    v[0] = add(e0, o0);
-    v[4] = sub(e0, o0);
-    v[1] = add(e1, o1);
-    v[5] = sub(e1, o1);
-    v[2] = add(e2, o2);
-    v[6] = sub(e2, o2);
-    v[3] = add(e3, o3);
-    v[7] = sub(e3, o3);
-  } else if constexpr (R == 2) {
-    C a = v[0], b = v[1];
-    v[0] = add(a, b);
-    v[1] = sub(a, b);
-  } else if constexpr (R == 4) {
-    C a = add(v[0], v[2]), b = sub(v[0], v[2]);
-    C c = add(v[1], v[3]), d = miu(sub(v[1], v[3]), s);
-    v[0] = add(a, c);
-    v[2] = sub(a, c);
-    v[1] = add(b, d);
-    v[3] = sub(b, d);
-  } else if constexpr (R == 3) {
-    const RR c = (RR)-0.5, u = s * (RR)0.86602540378443864676;
-    C t1 = add(v[1], v[2]);
-    C m = add(v[0], scl(t1, c));
-    C r = miu(sub(v[1], v[2]), u);
-    v[0] = add(v[0], t1);
-    v[1] = add(m, r);
-    v[2] = sub(m, r);
-  } else {
-    static_assert(R == 5, "radix");
-    const RR c1 = (RR)0.30901699437494742410, c2 = (RR)-0.80901699437494742410;
-    const RR s1 = (RR)0.95105651629515357212, s2 = (RR)0.58778525229247312917;
-    C a1 = add(v[1], v[4]), a2 = add(v[2], v[3]);
-    C b1 = sub(v[1], v[4]), b2 = sub(v[2], v[3]);
-    C p1 = add(v[0], add(scl(a1, c1), scl(a2, c2)));
-    C p2 = add(v[0], add(scl(a1, c2), scl(a2, c1)));
-    C q1 = miu(add(scl(b1, s1), scl(b2, s2)), s);
-    C q2 = miu(sub(scl(b1, s2), scl(b2, s1)), s);
-    v[0] = add(v[0], add(a1, a2));
-    v[1] = add(p1, q1);
-    v[4] = sub(p1, q1);
-    v[2] = add(p2, q2);
-    v[3] = sub(p2, q2);
   }
-}
-
-// In-place Stockham over NL lines of length N held in LDS; element e of line
-// l lives at buf[l*LS + e*ES].  LFAST selects the thread mapping (lines
-// fastest for strided lines, elements fastest for contiguous lines).  tw is
-// the W_{N*TWS} table; twiddles are W_N^e = tw[e*TWS].
-template <int SIGN, int N, int NL, int LS, int ES, bool LFAST, int NT, int S, int NS, int TWS, typename C>
-__device__ inline void stages(C* buf, const C* __restrict__ tw) {
-  constexpr Fac F = factor(N);
-  if constexpr (S < F.n) {
-    constexpr int R = F.r[S];
-    constexpr int NB = N / R;
-    constexpr int TOT = NL * NB;
-    constexpr int MB = (TOT + NT - 1) / NT;
-    constexpr int STEP = N / (NS * R);
-    C v[MB][R];
+  __syncthreads();
+  // rows, second stage, and the split X[q] = (Z[q] + conj Z[H-q])/2 - i/2 W_N^q (Z[q] - conj Z[H-q]):
+  // butterflies j and A1-j hold each other's partners q and H-q
+  {
+    constexpr int T = PB * N * L::TP, MB = (T + NT - 1) / NT;
+    C xa[MB][A2], xb[MB][A2];
 #pragma unroll
     for (int b = 0; b < MB; ++b) {
-      const int idx = threadIdx.x + b * NT;
-      if (idx < TOT) {
-        const int l = LFAST ? idx % NL : idx / NB;
-        const int j = LFAST ? idx / NL : idx % NB;
-        const int jm = j % NS;
-        const C* sp = buf + l * LS + j * ES;
-        v[b][0] = sp[0];
+      const int i = b * NT + threadIdx.x;
+      if (i < T) {
+        const int row = i / L::TP, j = i % L::TP, j2 = j == 0 ? 0 : A1 - j;
+        C v[A2], u[A2];
 #pragma unroll
-        for (int r = 1; r < R; ++r) {
-          C w = tw[(r * jm * STEP) * TWS];
-          if (SIGN > 0) w.y = -w.y;
-          v[b][r] = mul(sp[r * NB * ES], w);
+        for (int r = 0; r < A2; ++r) {
+          v[r] = buf[row * LS + j + r * A1];
+          u[r] = buf[row * LS + j2 + r * A1];
+          if (r > 0) {
+            v[r] = mulw<-1>(v[r], tw[2 * r * j]);
+            u[r] = mulw<-1>(u[r], tw[2 * r * j2]);
+          }
         }
-        bfly<SIGN, R>(v[b]);
+        bfly<-1, A2>(v);
+        bfly<-1, A2>(u);
+        const R half = (R)0.5;
+#pragma unroll
+        for (int k = 0; k < A2; ++k) {
+          const C p = cj(j == 0 ? v[(A2 - k) % A2] : u[A2 - 1 - k]);
+          const C xe = scl(add(v[k], p), half), d = scl(sub(v[k], p), half);
+          const C t = mul(tw[j + k * A1], mi<-1>(d));
+          xa[b][k] = add(xe, t);
+          xb[b][k] = cj(sub(xe, t));
+        }
       }
     }
     __syncthreads();
 #pragma unroll
     for (int b = 0; b < MB; ++b) {
-      const int idx = threadIdx.x + b * NT;
-      if (idx < TOT) {
-        const int l = LFAST ? idx % NL : idx / NB;
-        const int j = LFAST ? idx / NL : idx % NB;
-        const int jm = j % NS;
-        C* dp = buf + l * LS + ((j / NS) * NS * R + jm) * ES;
+      const int i = b * NT + threadIdx.x;
+      if (i < T) {
+        const int row = i / L::TP, j = i % L::TP;
 #pragma unroll
-        for (int k = 0; k < R; ++k) dp[k * NS * ES] = v[b][k];
+        for (int k = 0; k < A2; ++k) {
+          buf[row * LS + j + k * A1] = xa[b][k];
+          // j = 0 holds q and H-q both: only X[H] is written from the partner side
+          if (j != 0 || k == 0) buf[row * LS + H - j - k * A1] = xb[b][k];
+        }
+      }
+    }
+  }
+  __syncthreads();
+  // columns, first stage, in place
+  {
+    constexpr int T = PB * P * R2, MB = (T + NT - 1) / NT;
+    C v[MB][R1];
+#pragma unroll
+    for (int b = 0; b < MB; ++b) {
+      const int i = b * NT + threadIdx.x;
+      if (i < T) {
+        const int x = i % P, j = (i / P) % R2, pl = i / (P * R2);
+#pragma unroll
+        for (int r = 0; r < R1; ++r) v[b][r] = buf[(pl * N + j + r * R2) * LS + x];
+        bfly<-1, R1>(v[b]);
       }
     }
     __syncthreads();
-    stages<SIGN, N, NL, LS, ES, LFAST, NT, S + 1, NS * R, TWS>(buf, tw);
-  }
-}
-
-template <typename R>
-using CP = typename Cplx<R>::T;
-
-// Pass A: one z-plane: rho (N x N reals) -> complex (N rows of N/2+1).
-template <typename R, int N, int NT>
-__global__ void __launch_bounds__(NT) k_plane_fwd(const R* __restrict__ rho, CP<R>* __restrict__ out,
-                                                  const CP<R>* __restrict__ twg) {
-  using C = CP<R>;
-  constexpr int H = N / 2, P = H + 1;
-  __shared__ C buf[N * P];
-  __shared__ C tw[N];  // W_N^e, staged once: the stages read it from LDS
-  const int64_t plane = blockIdx.x;  // box * N + z
-  const R* src = rho + plane * N * N;
-  for (int i = threadIdx.x; i < N * H; i += NT) {
-    const int y = i / H, j = i % H;
-    buf[y * P + j] = CT<C>::mk(src[y * N + 2 * j], src[y * N + 2 * j + 1]);
-  }
-  for (int i = threadIdx.x; i < N; i += NT) tw[i] = twg[i];
-  __syncthreads();
-  stages<-1, H, N, P, 1, false, NT, 0, 1, 2>(buf, tw);  // half-length rows
-  // split: X[k] = (Z[k]+conj Z[H-k])/2 - i/2 W_N^k (Z[k]-conj Z[H-k]), k=0..H
-  const R half = (R)0.5;
-  constexpr int NPAIR = H / 2 + 1;
-  C xa[(N * NPAIR + NT - 1) / NT], xb[(N * NPAIR + NT - 1) / NT];
 #pragma unroll
-  for (int b = 0; b < (N * NPAIR + NT - 1) / NT; ++b) {
-    const int i = threadIdx.x + b * NT;
-    if (i < N * NPAIR) {
-      const int y = i / NPAIR, k = i % NPAIR;
-      const int k2 = H - k;
-      C zk = buf[y * P + (k == H ? 0 : k)], zk2 = buf[y * P + (k2 == H ? 0 : k2)];
-      // X[k]
-      {
-        C zc = cj(zk2);
-        C xe = scl(add(zk, zc), half), d = scl(sub(zk, zc), half);
-        C xo = CT<C>::mk(d.y, -d.x);
-        xa[b] = add(xe, mul(tw[k], xo));
-      }
-      // X[H-k]
-      {
-        C zc = cj(zk);
-        C xe = scl(add(zk2, zc), half), d = scl(sub(zk2, zc), half);
-        C xo = CT<C>::mk(d.y, -d.x);
-        xb[b] = add(xe, mul(tw[k2], xo));
+    for (int b = 0; b < MB; ++b) {
+      const int i = b * NT + threadIdx.x;
+      if (i < T) {
+        const int x = i % P, j = (i / P) % R2, pl = i / (P * R2);
+#pragma unroll
+        for (int k = 0; k < R1; ++k) buf[(pl * N + j * R1 + k) * LS + x] = v[b][k];
       }
     }
   }
   __syncthreads();
+  // columns, second stage: LDS -> registers -> global
+  C* dst = out + plane0 * N * P;
 #pragma unroll
-  for (int b = 0; b < (N * NPAIR + NT - 1) / NT; ++b) {
-    const int i = threadIdx.x + b * NT;
-    if (i < N * NPAIR) {
-      const int y = i / NPAIR, k = i % NPAIR;
-      buf[y * P + k] = xa[b];
-      buf[y * P + (H - k)] = xb[b];
+  for (int i0 = 0; i0 < PB * P * R1; i0 += NT) {
+    const int i = i0 + threadIdx.x;
+    if (i < PB * P * R1) {
+      const int x = i % P, j = (i / P) % R1, pl = i / (P * R1);
+      C v[R2];
+#pragma unroll
+      for (int r = 0; r < R2; ++r) {
+        v[r] = buf[(pl * N + j + r * R1) * LS + x];
+        if (r > 0) v[r] = mulw<-1>(v[r], tw[r * j]);
+      }
+      bfly<-1, R2>(v);
+#pragma unroll
+      for (int k = 0; k < R2; ++k) dst[(pl * N + j + k * R1) * P + x] = v[k];
     }
   }
-  __syncthreads();
-  stages<-1, N, P, 1, P, true, NT, 0, 1, 1>(buf, tw);  // columns along y
-  C* dst = out + plane * N * P;
-  for (int i = threadIdx.x; i < N * P; i += NT) dst[i] = buf[i];
 }
 
-// Pass B: YB consecutive y-slices of one box: lines along z, times G, back.
-// Several slices per block make the reads and writes of each z row longer
-// contiguous runs (YB*(N/2+1) complex values).
-template <typename R, int N, int NT, int YB>
-__global__ void __launch_bounds__(NT) k_zslice(CP<R>* __restrict__ data, const float* __restrict__ G,
-                                               const CP<R>* __restrict__ twg) {
+// Pass C: PB z-planes: inverse along y, c2r along x, normalisation.
+template <typename R, int N>
+__global__ void __launch_bounds__((Plan<R, N>::NT)) k_plane_inv(const CP<R>* __restrict__ in, R* __restrict__ phi,
+                                                                const CP<R>* __restrict__ twg, R div3, R div1) {
   using C = CP<R>;
-  constexpr int P = N / 2 + 1, W = YB * P;
-  __shared__ C buf[N * W];
+  using L = Plan<R, N>;
+  constexpr int H = L::H, P = L::P, LS = L::LS, A1 = L::RS, A2 = L::RB, R1 = L::R1, R2 = L::R2, PB = L::PB,
+                NT = L::NT;
+  __shared__ C buf[PB * N * LS];
   __shared__ C tw[N];
-  const int64_t box = blockIdx.x / (N / YB);
-  const int y0 = (blockIdx.x % (N / YB)) * YB;
-  C* base = data + box * (int64_t)N * N * P + (int64_t)y0 * P;
-  for (int i = threadIdx.x; i < N * W; i += NT) {
-    const int z = i / W, x = i % W;
-    buf[i] = base[(int64_t)z * N * P + x];
-  }
+  const int64_t plane0 = (int64_t)blockIdx.x * PB;
+  const C* src = in + plane0 * N * P;
   for (int i = threadIdx.x; i < N; i += NT) tw[i] = twg[i];
-  __syncthreads();
-  stages<-1, N, W, 1, W, true, NT, 0, 1, 1>(buf, tw);
-  const float* gb = G + (int64_t)y0 * P;
-  for (int i = threadIdx.x; i < N * W; i += NT) {
-    const int z = i / W, x = i % W;
-    const R g = (R)gb[(int64_t)z * N * P + x];
-    buf[i] = CT<C>::mk(buf[i].x * g, buf[i].y * g);  // cxyz*tf (kick.f90:698)
-  }
-  __syncthreads();
-  stages<+1, N, W, 1, W, true, NT, 0, 1, 1>(buf, tw);
-  for (int i = threadIdx.x; i < N * W; i += NT) {
-    const int z = i / W, x = i % W;
-    base[(int64_t)z * N * P + x] = buf[i];
-  }
-}
-
-// Pass C: one z-plane: inverse along y, c2r along x, normalisation.
-template <typename R, int N, int NT>
-__global__ void __launch_bounds__(NT) k_plane_inv(const CP<R>* __restrict__ in, R* __restrict__ phi,
-                                                  const CP<R>* __restrict__ twg, R div3, R div1) {
-  using C = CP<R>;
-  constexpr int H = N / 2, P = H + 1;
-  __shared__ C buf[N * P];
-  __shared__ C tw[N];
-  const int64_t plane = blockIdx.x;
-  const C* src = in + plane * N * P;
-  for (int i = threadIdx.x; i < N * P; i += NT) buf[i] = src[i];
-  for (int i = threadIdx.x; i < N; i += NT) tw[i] = twg[i];
-  __syncthreads();
-  stages<+1, N, P, 1, P, true, NT, 0, 1, 1>(buf, tw);
-  // Z[k] = E + iO with E = X[k] + conj X[H-k], O = (X[k] - conj X[H-k]) W_N^-k
-  constexpr int NPAIR = H / 2 + 1;
-  constexpr int MB = (N * NPAIR + NT - 1) / NT;
-  C za[MB], zb[MB];
+  // columns, first stage: global -> registers -> LDS
 #pragma unroll
-  for (int b = 0; b < MB; ++b) {
-    const int i = threadIdx.x + b * NT;
-    if (i < N * NPAIR) {
-      const int y = i / NPAIR, k = i % NPAIR, k2 = H - k;
-      const C xk = buf[y * P + k], xk2 = buf[y * P + k2];
-      {
-        C xc = cj(xk2), w = tw[k];
-        w.y = -w.y;
-        za[b] = add(add(xk, xc), miu(mul(sub(xk, xc), w), (typename CT<C>::R)1));
+  for (int i0 = 0; i0 < PB * P * R2; i0 += NT) {
+    const int i = i0 + threadIdx.x;
+    if (i < PB * P * R2) {
+      const int x = i % P, j = (i / P) % R2, pl = i / (P * R2);
+      C v[R1];
+#pragma unroll
+      for (int r = 0; r < R1; ++r) v[r] = src[(pl * N + j + r * R2) * P + x];
+      bfly<+1, R1>(v);
+#pragma unroll
+      for (int k = 0; k < R1; ++k) buf[(pl * N + j * R1 + k) * LS + x] = v[k];
+    }
+  }
+  __syncthreads();
+  // columns, second stage, in place
+  {
+    constexpr int T = PB * P * R1, MB = (T + NT - 1) / NT;
+    C v[MB][R2];
+#pragma unroll
+    for (int b = 0; b < MB; ++b) {
+      const int i = b * NT + threadIdx.x;
+      if (i < T) {
+        const int x = i % P, j = (i / P) % R1, pl = i / (P * R1);
+#pragma unroll
+        for (int r = 0; r < R2; ++r) {
+          v[b][r] = buf[(pl * N + j + r * R1) * LS + x];
+          if (r > 0) v[b][r] = mulw<+1>(v[b][r], tw[r * j]);
+        }
+        bfly<+1, R2>(v[b]);
       }
-      {
-        C xc = cj(xk), w = tw[k2];
-        w.y = -w.y;
-        zb[b] = add(add(xk2, xc), miu(mul(sub(xk2, xc), w), (typename CT<C>::R)1));
+    }
+    __syncthreads();
+#pragma unroll
+    for (int b = 0; b < MB; ++b) {
+      const int i = b * NT + threadIdx.x;
+      if (i < T) {
+        const int x = i % P, j = (i / P) % R1, pl = i / (P * R1);
+#pragma unroll
+        for (int k = 0; k < R2; ++k) buf[(pl * N + j + k * R1) * LS + x] = v[b][k];
       }
     }
   }
   __syncthreads();
+  // rows: the merge Z[q] = E + iO, E = X[q] + conj X[H-q], O = (X[q] - conj X[H-q]) W_N^-q, and the
+  // first stage of the half-length inverse (inputs q = j + r A2; partners H-q belong to A2-j)
+  {
+    constexpr int T = PB * N * L::TP, MB = (T + NT - 1) / NT;
+    C za[MB][A1], zb[MB][A1];
 #pragma unroll
-  for (int b = 0; b < MB; ++b) {
-    const int i = threadIdx.x + b * NT;
-    if (i < N * NPAIR) {
-      const int y = i / NPAIR, k = i % NPAIR, k2 = H - k;
-      if (k < H) buf[y * P + k] = za[b];
-      if (k2 < H) buf[y * P + k2] = zb[b];
+    for (int b = 0; b < MB; ++b) {
+      const int i = b * NT + threadIdx.x;
+      if (i < T) {
+        const int row = i / L::TP, j = i % L::TP, j2 = j == 0 ? 0 : A2 - j;
+        const C* rp = buf + row * LS;
+        C v[A1], u[A1];
+#pragma unroll
+        for (int r = 0; r < A1; ++r) {
+          v[r] = rp[j + r * A2];
+          u[r] = rp[j2 + r * A2];
+        }
+        const C xh = rp[H];
+#pragma unroll
+        for (int r = 0; r < A1; ++r) {
+          const C p = cj(j == 0 ? (r == 0 ? xh : v[(A1 - r) % A1]) : u[A1 - 1 - r]);
+          const C e = add(v[r], p), o = mi<+1>(mulw<+1>(sub(v[r], p), tw[j + r * A2]));
+          za[b][r] = add(e, o);
+          zb[b][A1 - 1 - r] = cj(sub(e, o));
+        }
+        bfly<+1, A1>(za[b]);
+        bfly<+1, A1>(zb[b]);
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int b = 0; b < MB; ++b) {
+      const int i = b * NT + threadIdx.x;
+      if (i < T) {
+        const int row = i / L::TP, j = i % L::TP, j2 = j == 0 ? 0 : A2 - j;
+#pragma unroll
+        for (int k = 0; k < A1; ++k) {
+          buf[row * LS + j * A1 + k] = za[b][k];
+          if (j2 != j) buf[row * LS + j2 * A1 + k] = zb[b][k];
+        }
+      }
     }
   }
   __syncthreads();
-  stages<+1, H, N, P, 1, false, NT, 0, 1, 2>(buf, tw);
-  R* dst = phi + plane * N * N;
-  for (int i = threadIdx.x; i < N * H; i += NT) {
-    const int y = i / H, j = i % H;
-    const C z = buf[y * P + j];
-    R a = z.x, b = z.y;
-    if (div3 != (R)0) {
-      a = a / div3;
-      b = b / div3;
-    } else {
-      a = ((a / div1) / div1) / div1;
-      b = ((b / div1) / div1) / div1;
+  // rows, second stage: LDS -> registers -> global, normalised
+  C* dst = reinterpret_cast<C*>(phi + plane0 * N * N);
+#pragma unroll
+  for (int i0 = 0; i0 < PB * N * A1; i0 += NT) {
+    const int i = i0 + threadIdx.x;
+    if (i < PB * N * A1) {
+      const int row = i / A1, j = i % A1;
+      C v[A2];
+#pragma unroll
+      for (int r = 0; r < A2; ++r) {
+        v[r] = buf[row * LS + j + r * A1];
+        if (r > 0) v[r] = mulw<+1>(v[r], tw[2 * r * j]);
+      }
+      bfly<+1, A2>(v);
+#pragma unroll
+      for (int k = 0; k < A2; ++k) {
+        R a = v[k].x, b = v[k].y;
+        if (div3 != (R)0) {
+          a = a / div3;
+          b = b / div3;
+        } else {
+          a = ((a / div1) / div1) / div1;
+          b = ((b / div1) / div1) / div1;
+        }
+        dst[row * H + j + k * A1] = CT<C>::mk(a, b);
+      }
     }
-    dst[y * N + 2 * j] = a;
-    dst[y * N + 2 * j + 1] = b;
   }
 }
 
-template <typename R, int N, int NT, int NTZ, int YB>
-void run_plane_shape(const FFTCube<R>& c, R* rho, CP<R>* work, const float* G, int64_t nbox, R div3, R div1,
-                     hipStream_t s, KTimer* tm, const std::string& t) {
+template <typename R, int N>
+bool run_plane(const FFTCube<R>& c, R* rho, CP<R>* work, const float* G, int64_t nbox, R div3, R div1,
+               hipStream_t s, KTimer* tm, const std::string& t) {
+  using L = Plan<R, N>;
   const double Gb = (double)N * N * N * sizeof(R) * nbox;
-  const double Kb = (double)N * N * (N / 2 + 1) * sizeof(CP<R>) * nbox;
-  const double Gk = (double)N * N * (N / 2 + 1) * sizeof(float);
+  const double Kb = (double)N * N * L::P * sizeof(CP<R>) * nbox;
+  const double Gk = (double)N * N * L::P * sizeof(float);
+  const dim3 planes((unsigned)(nbox * (N / L::PB)));
   {
     KScope k(tm, (t + "fft_xy_fwd").c_str(), Gb + Kb);
-    hipLaunchKernelGGL((k_plane_fwd<R, N, NT>), dim3((unsigned)(nbox * N)), dim3(NT), 0, s, rho, work, c.tw);
+    hipLaunchKernelGGL((k_plane_fwd<R, N>), planes, dim3(L::NT), 0, s, rho, work, c.tw);
     CUBE_HIP(hipGetLastError());
   }
   {
     KScope k(tm, (t + "fft_z_green").c_str(), 2 * Kb + Gk);
-    hipLaunchKernelGGL((k_zslice<R, N, NTZ, YB>), dim3((unsigned)(nbox * (N / YB))), dim3(NTZ), 0, s, work, G, c.tw);
-    CUBE_HIP(hipGetLastError());
+    launch_zlines<R, N>(work, G, c.tw, nbox, s);
   }
   {
     KScope k(tm, (t + "fft_xy_inv").c_str(), Gb + Kb);
-    hipLaunchKernelGGL((k_plane_inv<R, N, NT>), dim3((unsigned)(nbox * N)), dim3(NT), 0, s, work, rho, c.tw, div3,
-                       div1);
+    hipLaunchKernelGGL((k_plane_inv<R, N>), planes, dim3(L::NT), 0, s, work, rho, c.tw, div3, div1);
     CUBE_HIP(hipGetLastError());
   }
-}
-
-// Launch shapes: shape 0 = threads per plane / slice measured best at n = 80 and
-// 160 on MI355X; shape 1 = the other thread count for the plane passes; shape
-// 2 = one z slice per workgroup instead of two (or half the threads where one
-// slice already fills the workgroup's LDS).  Every shape computes each
-// butterfly with the same operations, so all give the same result; the FP64
-// form keeps shape 0.
-template <typename R, int N>
-bool run_plane(const FFTCube<R>& c, R* rho, CP<R>* work, const float* G, int64_t nbox, R div3, R div1,
-               hipStream_t s, KTimer* tm, const std::string& t, int shape) {
-  constexpr int NT = N >= 128 ? 1024 : (N >= 80 ? 512 : 256);
-  constexpr int NTZ = N >= 80 ? 1024 : 256;
-  // two slices per block where their LDS fits in 64 KB
-  constexpr int YB = (N % 2 == 0 && 2 * N * (N / 2 + 1) * (int)sizeof(CP<R>) <= 65536) ? 2 : 1;
-  if constexpr (std::is_same<R, float>::value && N >= 64) {
-    constexpr int NT1 = N >= 128 ? 512 : (N >= 80 ? 256 : 512);
-    constexpr int NTZ2 = YB == 2 ? NTZ : (NTZ >= 512 ? NTZ / 2 : 512);
-    if (shape == 1) {
-      run_plane_shape<R, N, NT1, NTZ, YB>(c, rho, work, G, nbox, div3, div1, s, tm, t);
-      return true;
-    }
-    if (shape == 2) {
-      run_plane_shape<R, N, NT, NTZ2, 1>(c, rho, work, G, nbox, div3, div1, s, tm, t);
-      return true;
-    }
-  }
-  run_plane_shape<R, N, NT, NTZ, YB>(c, rho, work, G, nbox, div3, div1, s, tm, t);
   return true;
 }
 
 }  // namespace
 
 // Returns false when n has no specialised kernel (the caller then uses the
-// generic line passes).
+// generic line passes).  The sizes are the multiples of 8 that tile and
+// sub-tile meshes take (16k + 32 and 8k + 16, and their finer levels) whose
+// plane fits in LDS.
 template <typename R>
 bool fft_convolve_plane(const FFTCube<R>& c, R* rho, typename Cplx<R>::T* work, const float* G, int64_t nbox,
-                        R div3, R div1, hipStream_t s, KTimer* tm, const char* tag, int shape) {
-  std::string t(tag);
+                        R div3, R div1, hipStream_t s, KTimer* tm, const char* tag) {
+  const std::string t(tag);
   switch (c.n) {
-    case 16: return run_plane<R, 16>(c, rho, work, G, nbox, div3, div1, s, tm, t, shape);
-    case 24: return run_plane<R, 24>(c, rho, work, G, nbox, div3, div1, s, tm, t, shape);
-    case 32: return run_plane<R, 32>(c, rho, work, G, nbox, div3, div1, s, tm, t, shape);
-    case 48: return run_plane<R, 48>(c, rho, work, G, nbox, div3, div1, s, tm, t, shape);
-    case 64: return run_plane<R, 64>(c, rho, work, G, nbox, div3, div1, s, tm, t, shape);
-    case 72: return run_plane<R, 72>(c, rho, work, G, nbox, div3, div1, s, tm, t, shape);
-    case 80: return run_plane<R, 80>(c, rho, work, G, nbox, div3, div1, s, tm, t, shape);
-    case 96: return run_plane<R, 96>(c, rho, work, G, nbox, div3, div1, s, tm, t, shape);
+#define CUBE_FFT_SIZE(n) \
+  case n: return run_plane<R, n>(c, rho, work, G, nbox, div3, div1, s, tm, t);
+    CUBE_FFT_SIZE(16)
+    CUBE_FFT_SIZE(24)
+    CUBE_FFT_SIZE(32)
+    CUBE_FFT_SIZE(40)
+    CUBE_FFT_SIZE(48)
+    CUBE_FFT_SIZE(56)
+    CUBE_FFT_SIZE(64)
+    CUBE_FFT_SIZE(72)
+    CUBE_FFT_SIZE(80)
+    CUBE_FFT_SIZE(88)
+    CUBE_FFT_SIZE(96)
+    CUBE_FFT_SIZE(104)
+    CUBE_FFT_SIZE(112)
+    CUBE_FFT_SIZE(120)
+    CUBE_FFT_SIZE(128)
     default: break;
   }
-  // n^2 (n/2+1) planes of FP64 beyond 96 do not fit in LDS
+  // FP64 planes beyond 128 points do not fit in LDS
   if constexpr (std::is_same<R, float>::value) {
-    if (c.n == 128) return run_plane<R, 128>(c, rho, work, G, nbox, div3, div1, s, tm, t, shape);
-    if (c.n == 144) return run_plane<R, 144>(c, rho, work, G, nbox, div3, div1, s, tm, t, shape);  // PM3 at 1024^3
-    if (c.n == 160) return run_plane<R, 160>(c, rho, work, G, nbox, div3, div1, s, tm, t, shape);
+    switch (c.n) {
+      CUBE_FFT_SIZE(144)
+      CUBE_FFT_SIZE(160)
+      CUBE_FFT_SIZE(168)
+      CUBE_FFT_SIZE(176)
+      CUBE_FFT_SIZE(192)
+      default: break;
+    }
   }
+#undef CUBE_FFT_SIZE
   return false;
 }
 
 template bool fft_convolve_plane<float>(const FFTCube<float>&, float*, float2*, const float*, int64_t, float, float,
-                                        hipStream_t, KTimer*, const char*, int);
+                                        hipStream_t, KTimer*, const char*);
 template bool fft_convolve_plane<double>(const FFTCube<double>&, double*, double2*, const float*, int64_t, double,
-                                         double, hipStream_t, KTimer*, const char*, int);
+                                         double, hipStream_t, KTimer*, const char*);
 
 }  // namespace cube
