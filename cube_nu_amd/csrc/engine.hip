@@ -20,6 +20,7 @@
 #include "fft.h"
 #include "ic.h"
 #include "pm.h"
+#include "pm_mesh.h"
 #include "pp.h"
 #include "timing.h"
 
@@ -162,6 +163,12 @@ struct cube_p3m_ctx {
   // scratch
   DevBuf<char> scan_tmp;
   DevBuf<char> work;
+  DevBuf<float> gmesh, gfaces;  // whole-image mesh and window faces (pm_mesh.h)
+  // buffer cells as periodic images of the physical ones: 1 by construction
+  // (the buffer step), 0 not looked at yet (uploaded state), -1 they are not
+  int images = 0;
+  bool image_meshes = false;  // this kick's densities may be cut from whole-image meshes
+  DevBuf<int32_t> dbad;
   DevBuf<char> stencil;  // coarse-level deposit: 27 tap sums per coarse cell
   // per-slot box lists and binned lists (slot 0 PM1, 1 PM2, 2..5 PM3 at
   // iapm 2..5; PP by iapm 2..5): a captured kick reads each level's lists
@@ -324,6 +331,26 @@ struct cube_p3m_ctx {
     return std::string(what) + "_l" + std::to_string(level) + "_n" + std::to_string(size) + "_fp" +
            std::to_string(prec);
   }
+  PMLevel level_pm2() const {
+    PMLevel L{};
+    L.n = (int)g.ngt; L.m0 = 1 - (int)g.ngb; L.periodic = 0; L.win_lo = 1 - (int)g.ngb;
+    L.win_hi = (int)(g.ngp + g.ngb); L.nloop = (int)g.ncb; L.w = (int)g.rcs; L.rcs = (int)g.rcs; L.gridsize = 1.0;
+    L.nforce = (int)g.ngp; L.nte = (int)g.nte; L.ncb = (int)g.ncb; L.nt = (int)g.nt;
+    pm_level_scale(L);
+    return L;
+  }
+  PMLevel level_pm3(int iapm) const {
+    PMLevel L{};
+    L.n = (int)g.nft[iapm]; L.m0 = 1 - (int)g.nfb[iapm]; L.periodic = 0; L.win_lo = 1 - (int)g.nfb[iapm];
+    L.win_hi = (int)(g.nfp[iapm] + g.nfb[iapm]); L.nloop = 1; L.w = (int)(g.rcs * g.sf[iapm]);
+    L.rcs = (int)g.rcs; L.gridsize = (double)(1.0f / (float)g.sf[iapm]); L.nforce = (int)g.nfp[iapm];
+    L.nte = (int)g.nte; L.ncb = (int)g.ncb; L.nt = (int)g.nt;
+    pm_level_scale(L);
+    return L;
+  }
+  void check_images();
+  template <typename R>
+  bool image_mesh_level(int level, const PMLevel& L, int64_t nbox, int64_t batch) const;
   void drift(const cube_drift_in& in, cube_drift_out& out);
   void buffer(int64_t* np_ext);
   void buffer_vel();
@@ -384,6 +411,30 @@ void cube_p3m_ctx::set_tf_default() {
   CUBE_HIP(hipStreamSynchronize(s));
 }
 
+// Whether a level's windows are cut from the whole image's mesh: the FP32
+// form, a level that most of the image takes (the tile level, and the
+// sub-tile level of at least half the sub-tiles: below that the boxes' own
+// particles are fewer than the image's), state whose buffer cells are the
+// periodic images they stand for, and meshes within half the workspace
+// budget.  Either form gives the same densities bit for bit.
+template <typename R>
+bool cube_p3m_ctx::image_mesh_level(int level, const PMLevel& L, int64_t nbox, int64_t batch) const {
+  if (!std::is_same<R, float>::value || level < 2 || !image_meshes || !pm_mesh_applies(g, L)) return false;
+  if (level >= 3 && 2 * nbox < g.ns3) return false;
+  const int64_t n = g.nc * L.w, bytes = 4 * (n * n * n + batch * 6 * (int64_t)L.n * L.n);
+  return bytes <= ws_budget() / 2;
+}
+
+// One look at uploaded state (a read-back); state of the buffer step needs none.
+void cube_p3m_ctx::check_images() {
+  if (images != 0) return;
+  int32_t bad = 0;
+  mesh_check_images((int)g.izipx, g, xpc(), rhocc(), off.p, dbad.ensure(1), s);
+  CUBE_HIP(hipMemcpyAsync(&bad, dbad.p, sizeof(bad), hipMemcpyDeviceToHost, s));
+  CUBE_HIP(hipStreamSynchronize(s));
+  images = bad ? -1 : 1;
+}
+
 template <typename R>
 void cube_p3m_ctx::run_level(int level, int slot, const std::vector<PMBox>& bx_in, const float* G,
                              const FFTCube<R>& fc, const PMLevel& L0, const cube_kick_in& in, PMOut* o,
@@ -404,6 +455,12 @@ void cube_p3m_ctx::run_level(int level, int slot, const std::vector<PMBox>& bx_i
   C* cplx = (C*)(work.p + batch * nreal * sizeof(R));
   const size_t bchunk = (level == 1) ? bx_in.size() : (size_t)batch;
   if (kph == 1 && bchunk < bx_in.size()) graph_ok = false;  // a captured kick holds one batch per level
+  const bool image = image_mesh_level<R>(level, L0, nmesh_total, batch);
+  const MeshGeo M = mesh_geo(g, L0.w, (int)g.B);
+  if (image) {
+    gmesh.ensure((size_t)M.n * M.n * M.n);
+    gfaces.ensure((size_t)batch * 6 * n * n);
+  }
   DevBuf<PMBox>& boxes = lboxes[slot];
   boxes.ensure(std::max<size_t>(boxes.n, bchunk));
   for (size_t b0 = 0; b0 < bx_in.size(); b0 += bchunk) {
@@ -429,6 +486,21 @@ void cube_p3m_ctx::run_level(int level, int slot, const std::vector<PMBox>& bx_i
         if (SZ) sig_add({(uint64_t)(uintptr_t)st});
         if (CP)
           pm1_deposit<R>((int)g.izipx, L, xpc(), rhocc(), off.p, st, mesh, in.mass_p_cdm, o, s);
+      } else if (image) {
+        if (SZ) sig_add({(uint64_t)(uintptr_t)gmesh.p, (uint64_t)(uintptr_t)gfaces.p});
+        if constexpr (std::is_same<R, float>::value) {
+          auto window = [&](cube_p3m_ctx* c, float m, float* out) {
+            // the image's mesh holds every box of the level: once per level and species
+            if (b0 == 0 || nu) pm_mesh_deposit((int)g.izipx, M, c->xpc(), c->rhocc(), c->off.p, gmesh.p, m, s);
+            pm_mesh_faces((int)g.izipx, M, L, boxes.p, nb, c->xpc(), c->rhocc(), c->off.p, gfaces.p, m, s);
+            pm_mesh_window(M, L, boxes.p, nb, gmesh.p, gfaces.p, out, s);
+          };
+          if (CP) window(this, in.mass_p_cdm, mesh);
+          if (CP && nu && level <= 2) {
+            window(nu, nu_mass, (float*)work2.ensure(sizeof(R) * (size_t)(nreal * nmesh)));
+            mesh_add<R>(mesh, (R*)work2.p, nreal * nmesh, s);
+          }
+        }
       } else if (level >= 3 && pm_deposit_binned_applies(L)) {
         const int64_t nblk = nb * pm_dep_blocks(L);
         DepBins S;
@@ -463,7 +535,7 @@ void cube_p3m_ctx::run_level(int level, int slot, const std::vector<PMBox>& bx_i
     // the interpolation's block shape so far (its trials need the potential)
     if (SZ) sig_add({(uint64_t)interp_shape<R>(level, (int)n, L, boxes.p, nb, in, (const R*)nullptr, false)});
     if (!CP) continue;
-    if (nu && level <= 2) {
+    if (nu && level <= 2 && !image) {
       KScope k(&tm, (t + "deposit_nu").c_str(), cells * sizeof(R));
       R* mesh2 = (R*)work2.ensure(sizeof(R) * (size_t)(nreal * nmesh));
       if (level == 1)
@@ -743,10 +815,7 @@ void cube_p3m_ctx::kick_pass(const cube_kick_in& in, cube_kick_out& out, float* 
   }
   // PM2 (kick.f90:47-69)
   if (mask & 2) {
-    PMLevel L{};
-    L.n = (int)g.ngt; L.m0 = 1 - (int)g.ngb; L.periodic = 0; L.win_lo = 1 - (int)g.ngb;
-    L.win_hi = (int)(g.ngp + g.ngb); L.nloop = (int)g.ncb; L.w = (int)g.rcs; L.rcs = (int)g.rcs; L.gridsize = 1.0;
-    L.nforce = (int)g.ngp; L.nte = (int)g.nte; L.ncb = (int)g.ncb; L.nt = (int)g.nt;
+    const PMLevel L = level_pm2();
     std::vector<PMBox> bx;
     for (int64_t T = 0; T < g.ntiles; ++T) {
       PMBox b{};
@@ -769,11 +838,7 @@ void cube_p3m_ctx::kick_pass(const cube_kick_in& in, cube_kick_out& out, float* 
   if ((mask & 4) && cfg.pm3) {
     const int64_t nns = g.nns;
     for (int iapm = 2; iapm <= 5; ++iapm) {
-      PMLevel L{};
-      L.n = (int)g.nft[iapm]; L.m0 = 1 - (int)g.nfb[iapm]; L.periodic = 0; L.win_lo = 1 - (int)g.nfb[iapm];
-      L.win_hi = (int)(g.nfp[iapm] + g.nfb[iapm]); L.nloop = 1; L.w = (int)(g.rcs * g.sf[iapm]);
-      L.rcs = (int)g.rcs; L.gridsize = (double)(1.0f / (float)g.sf[iapm]); L.nforce = (int)g.nfp[iapm];
-      L.nte = (int)g.nte; L.ncb = (int)g.ncb; L.nt = (int)g.nt;
+      const PMLevel L = level_pm3(iapm);
       std::vector<PMBox> bx;
       for (int64_t it = 0; it < g.ns3; ++it) {
         if (ires_h[it] != iapm) continue;
@@ -835,6 +900,26 @@ bool cube_p3m_ctx::classify_and_reserve(cube_kick_out& out, std::vector<int32_t>
       if (nb > 0 && std::max<int64_t>(1, ws_budget() / 4 / (m3 * 12)) < nb) multi = true;
     }
     work.ensure((size_t)need);
+    // the whole-image meshes of the levels that take them
+    int64_t cells = 0, faces = 0;
+    auto image_ws = [&](int level, const PMLevel& L, int64_t nmesh) {
+      if (nmesh <= 0) return;
+      const int64_t n = L.n;
+      const int64_t per = n * n * n * (int64_t)sizeof(R) + n * n * (n / 2 + 1) * (int64_t)sizeof(C);
+      const int64_t batch = std::max<int64_t>(1, std::min<int64_t>(nmesh, ws_budget() / per));
+      if (!image_mesh_level<R>(level, L, nmesh, batch)) return;
+      const int64_t m = g.nc * L.w;
+      cells = std::max(cells, m * m * m);
+      faces = std::max(faces, batch * 6 * n * n);
+    };
+    image_ws(2, level_pm2(), g.ntiles);
+    if (cfg.pm3)
+      for (int iapm = 2; iapm <= 5; ++iapm)
+        image_ws(3, level_pm3(iapm), (int64_t)std::count(ires_h.begin(), ires_h.end(), iapm));
+    if (cells > 0) {
+      gmesh.ensure((size_t)cells);
+      gfaces.ensure((size_t)faces);
+    }
   }
   return multi;
 }
@@ -1009,6 +1094,14 @@ void cube_p3m_ctx::kick(const cube_kick_in& in, cube_kick_out& out, float* densi
   } hold{wsb};
   wsb = -1;
   wsb = ws_budget();
+  image_meshes = false;
+  if (std::is_same<R, float>::value && (mask & 6)) {
+    check_images();
+    if (nu && nu->images == 0) {
+      nu->check_images();
+    }
+    image_meshes = images == 1 && (!nu || nu->images == 1);
+  }
   const bool use_graph = graph_on && mask == 15 && !density_host && !nu;
   const bool overlap =
       !use_graph && overlap_on && mask == 15 && !density_host && !nu && cfg.pm3 && cfg.pp && kicks_done > 0;
@@ -1235,6 +1328,7 @@ void cube_p3m_ctx::buffer(int64_t* np_ext) {
   }
   cur = other;
   layout = 1;
+  images = 1;
   np = n;
   off_valid = true;
   if (np_ext) *np_ext = n;
@@ -1326,6 +1420,7 @@ static void upload_ext(cube_p3m_ctx* c, const void* xp, const float* vp, const i
   c->np = n;
   c->off_valid = false;
   c->vmax_valid = false;
+  c->images = 0;
 }
 
 // The second species' outputs of a coupled kick: its PM1/PM2 maxima (its

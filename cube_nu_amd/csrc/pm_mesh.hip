@@ -1,0 +1,365 @@
+// pm_mesh.hip -- tile and sub-tile densities from one deposit per mesh
+// resolution.
+//
+// The windows of the tile (PM2) and sub-tile (PM3) meshes overlap by their
+// buffers: depositing per window repeats every particle 1.95 times at 512^3,
+// 8 at 128^3 and 27 at 64^3.  The buffer cells are periodic images of the
+// physical ones, and the deposit sums integers, so a window's density is, bit
+// for bit, a cut from the periodic mesh of the whole image at that resolution
+// -- but for the window's outermost layer of cells, which lacks the taps of
+// the particles outside the window.  So every physical particle is deposited
+// once into the image's mesh (k_mesh_deposit), the six faces of every window
+// are summed on their own from the window's boundary coarse cells
+// (k_mesh_faces: a quarter of their particles at w = 8, nine taps each), and
+// k_mesh_window cuts the windows out.
+#include <algorithm>
+
+#include "pm_dev.h"
+#include "pm_mesh.h"
+
+namespace cube {
+namespace {
+
+// Mesh of the whole image: cell a covers [a, a+1) mesh units; a particle with
+// floor f deposits into f-1, f, f+1 with the weights of particle_mesh.f90:56-62.
+//
+// Workgroup = BD^3 cells [BD b - 1, BD b + BD - 2] per axis: with this offset
+// the contributors are the block's own coarse cells and one lower layer,
+// (BD/w + 1)^3 cells.  Their particles form one list (LDS prefix sum of the
+// counts) that the wavefronts share in 8 segments each; lane l reads particle
+// l/8, l/8 + 8, ... of segment l%8, so that the 64 lanes of a deposit come
+// from 8 places of the block: particles of one coarse cell share few mesh
+// cells, and their atomics would serialise (a microbenchmark of 64-bit LDS
+// adds: 18.5 CU cycles per wavefront from one 4^3-cell coarse cell, 13.2 from
+// several).  Hits (1.42 per particle at BD = 16) queue per wavefront and are
+// deposited 64 at a time into 2^-32 fixed-point sums.
+template <int IZ, int BD>
+__global__ void __launch_bounds__(256) k_mesh_deposit(MeshGeo M, const XT<IZ>* __restrict__ xp,
+                                                      const int32_t* __restrict__ rhoc,
+                                                      const int64_t* __restrict__ off, float* __restrict__ mesh,
+                                                      float mass) {
+  constexpr int MAXC = (BD / 4 + 1) * (BD / 4 + 1) * (BD / 4 + 1);
+  constexpr int NS = 32;  // list segments of a workgroup
+  __shared__ unsigned long long acc[BD * BD * BD];
+  __shared__ unsigned long long queue[4][128];
+  __shared__ int cnt[MAXC], pre[MAXC + 1], wsum[4];
+  __shared__ int64_t gof[MAXC];
+  const int nb = M.n / BD, g = BD / M.w, gc = g + 1;
+  int64_t b = xcd_block(blockIdx.x, gridDim.x);
+  const int bi[3] = {(int)(b % nb), (int)((b / nb) % nb), (int)(b / ((int64_t)nb * nb))};
+  const int nC = gc * gc * gc;
+  for (int t = threadIdx.x; t < nC; t += 256) {
+    const int l[3] = {t % gc, (t / gc) % gc, t / (gc * gc)};
+    int T = 0, c[3];
+    for (int d = 2; d >= 0; --d) {
+      int cc = bi[d] * g - 1 + l[d];
+      cc = cc < 0 ? cc + M.nc : cc;
+      const int it = cc / M.nt;
+      c[d] = cc - it * M.nt + 1;
+      T = T * M.nnt + it;
+    }
+    const int64_t cell = rc_index(c[0], c[1], c[2], T, M.nte, M.ncb);
+    cnt[t] = rhoc[cell];
+    gof[t] = off[cell];
+  }
+  for (int t = threadIdx.x; t < BD * BD * BD; t += 256) acc[t] = 0;
+  __syncthreads();
+  block_scan(cnt, pre, nC, wsum);
+  const int total = pre[nC];
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int sh = M.sh;
+  const float rsh = 1.0f / (float)(1u << sh);
+  const uint32_t fmask = (1u << sh) - 1u;
+  unsigned long long* q = queue[wave];
+  // entry: block-local floor + 8 of each axis (5 bits, floors -w..BD-1) above the coordinates
+  auto process = [&](int nq) {
+    wave_sync_lds();
+    if (lane < nq) {
+      const unsigned long long e = q[lane];
+      int f[3];
+      float w[3][3];
+      for (int d = 0; d < 3; ++d) {
+        f[d] = (int)((e >> (48 + 5 * d)) & 31) - 8;
+        tsc_weights_frac<float>(((float)((uint32_t)(e >> (16 * d)) & fmask) + 0.5f) * rsh, w[d]);
+      }
+      for (int i = 0; i < 3; ++i) w[2][i] *= kFixF;  // exact: a power of two
+#pragma unroll
+      for (int i3 = 0; i3 < 3; ++i3) {
+        const int z = f[2] + i3;
+        if ((unsigned)z >= (unsigned)BD) continue;
+#pragma unroll
+        for (int i2 = 0; i2 < 3; ++i2) {
+          const int y = f[1] + i2;
+          if ((unsigned)y >= (unsigned)BD) continue;
+          const int row = (z * BD + y) * BD, sw = (5 * y + 9 * z) & (BD - 1);
+#pragma unroll
+          for (int i1 = 0; i1 < 3; ++i1) {
+            const int x = f[0] + i1;
+            if ((unsigned)x < (unsigned)BD)
+              atomicAdd(&acc[row + (x ^ sw)],
+                        (unsigned long long)__float2uint_rn((w[0][i1] * w[1][i2]) * w[2][i3]));
+          }
+        }
+      }
+    }
+    wave_sync_lds();
+  };
+  const int seg = wave * 8 + (lane & 7);
+  const int i1 = (int)((int64_t)total * (seg + 1) / NS);
+  int i = (int)((int64_t)total * seg / NS) + (lane >> 3);
+  int c = i < i1 ? find_cell(pre, nC, i) : 0;
+  int qn = 0;
+  constexpr int U = 4;
+  while (__any(i < i1)) {
+    uint32_t u[U][3];
+    int cl[U];
+    bool val[U];
+#pragma unroll
+    for (int k = 0; k < U; ++k) {
+      val[k] = i < i1;
+      while (val[k] && i >= pre[c + 1]) ++c;
+      cl[k] = c;
+      const int64_t ip = val[k] ? gof[c] + (i - pre[c]) : 0;
+      for (int d = 0; d < 3; ++d) u[k][d] = val[k] ? XP<IZ>::raw(xp, ip, d) : 0u;
+      i += 8;
+    }
+#pragma unroll
+    for (int k = 0; k < U; ++k) {
+      const int l[3] = {cl[k] % gc, (cl[k] / gc) % gc, cl[k] / (gc * gc)};
+      bool hit = val[k];
+      unsigned long long e = 0;
+      for (int d = 0; d < 3; ++d) {
+        const int f = M.w * (l[d] - 1) + (int)(u[k][d] >> sh);  // floor relative to BD b
+        hit = hit && f >= -2;
+        e |= ((unsigned long long)u[k][d] << (16 * d)) | ((unsigned long long)((f + 8) & 31) << (48 + 5 * d));
+      }
+      const unsigned long long m = __ballot(hit);
+      if (hit) q[qn + (int)__popcll(m & ((1ull << lane) - 1ull))] = e;
+      qn += (int)__popcll(m);
+      if (qn >= 64) {
+        process(64);
+        const unsigned long long mv = (lane < qn - 64) ? q[64 + lane] : 0ull;
+        wave_sync_lds();
+        if (lane < qn - 64) q[lane] = mv;
+        qn -= 64;
+      }
+    }
+  }
+  if (qn > 0) process(qn);
+  __syncthreads();
+  for (int t = threadIdx.x; t < BD * BD * BD; t += 256) {
+    const int lx = t % BD, ly = (t / BD) % BD, lz = t / (BD * BD);
+    const unsigned long long v = acc[(lz * BD + ly) * BD + (lx ^ ((5 * ly + 9 * lz) & (BD - 1)))];
+    const int l[3] = {lx, ly, lz};
+    int a[3];
+    for (int d = 0; d < 3; ++d) {
+      a[d] = bi[d] * BD - 1 + l[d];
+      a[d] = a[d] < 0 ? a[d] + M.n : a[d];
+    }
+    mesh[((int64_t)a[2] * M.n + a[1]) * M.n + a[0]] = (float)((double)v * (1.0 / (double)kFixF)) * mass;
+  }
+}
+
+// Faces of the windows: face 2 axis + side of box b at faces[(6 b + face) n^2],
+// [v][u] with u, v the lower and the higher of the other two axes.  One
+// workgroup per strip of `rows` v-rows of a face sums the taps of the
+// particles of the boundary layer of coarse cells whose floor is the face's
+// layer (middle tap) or the next one inside (outer tap).
+template <int IZ>
+__global__ void __launch_bounds__(256) k_mesh_faces(MeshGeo M, PMLevel L, const PMBox* __restrict__ boxes, int rows,
+                                                    const XT<IZ>* __restrict__ xp, const int32_t* __restrict__ rhoc,
+                                                    const int64_t* __restrict__ off, float* __restrict__ faces,
+                                                    float mass) {
+  extern __shared__ unsigned long long facc[];  // [rows][n]
+  const int n = L.n, nr = n / M.w, nstrip = (n + rows - 1) / rows;
+  const int strip = (int)(blockIdx.x % nstrip), face = (int)((blockIdx.x / nstrip) % 6);
+  const int64_t box = blockIdx.x / ((int64_t)nstrip * 6);
+  const int ax = face >> 1, side = face & 1, au = ax == 0 ? 1 : 0, av = ax == 2 ? 1 : 2;
+  const PMBox B = boxes[box];
+  const int v0 = strip * rows, v1 = min(n, v0 + rows);  // rows [v0, v1)
+  for (int t = threadIdx.x; t < (v1 - v0) * n; t += 256) facc[t] = 0;
+  __syncthreads();
+  const int sh = M.sh, wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const float rsh = 1.0f / (float)(1u << sh);
+  const uint32_t fmask = (1u << sh) - 1u;
+  // coarse cells (window-local 0..nr-1) that reach the strip: floors v0-1 .. v1
+  const int cv0 = max(0, v0 - 1) / M.w, cv1 = min(n - 1, v1) / M.w;
+  const int ncell = nr * (cv1 - cv0 + 1);
+  const int cax = side ? nr - 1 : 0;
+  for (int t = wave; t < ncell; t += 4) {
+    const int cl[2] = {t % nr, cv0 + t / nr};  // along u, v
+    const int c0 = ax == 0 ? cax : cl[0], c1 = ax == 1 ? cax : (ax == 0 ? cl[0] : cl[1]), c2 = ax == 2 ? cax : cl[1];
+    const int64_t cell = rc_index(B.nc1[0] - L.nloop + c0, B.nc1[1] - L.nloop + c1, B.nc1[2] - L.nloop + c2, B.T,
+                                  M.nte, M.ncb);
+    const int cnt = rhoc[cell];
+    const int64_t base = off[cell];
+    for (int l = lane; l < cnt; l += 64) {
+      const uint32_t ua = XP<IZ>::raw(xp, base + l, ax);
+      const int fa = M.w * cax + (int)(ua >> sh);
+      const int in = side ? n - 1 - fa : fa;  // layers inside the face
+      if (in > 1) continue;
+      const uint32_t uu = XP<IZ>::raw(xp, base + l, au), uv = XP<IZ>::raw(xp, base + l, av);
+      const int fu = M.w * cl[0] + (int)(uu >> sh), fv = M.w * cl[1] + (int)(uv >> sh);
+      float wa[3], wu[3], wv[3];
+      tsc_weights_frac<float>(((float)(ua & fmask) + 0.5f) * rsh, wa);
+      tsc_weights_frac<float>(((float)(uu & fmask) + 0.5f) * rsh, wu);
+      tsc_weights_frac<float>(((float)(uv & fmask) + 0.5f) * rsh, wv);
+      // the tap that falls on the face, with the 2^32 of the fixed point (exact)
+      const float w1 = (in == 0 ? wa[1] : (side ? wa[2] : wa[0])) * kFixF;
+#pragma unroll
+      for (int jv = 0; jv < 3; ++jv) {
+        const int mv = fv - 1 + jv;
+        if (mv < v0 || mv >= v1) continue;
+#pragma unroll
+        for (int ju = 0; ju < 3; ++ju) {
+          const int mu = fu - 1 + ju;
+          if (mu < 0 || mu >= n) continue;
+          // (wx wy) wz, as every deposit forms it
+          const float cw = ax == 2 ? (wu[ju] * wv[jv]) * w1 : (w1 * wu[ju]) * wv[jv];
+          atomicAdd(&facc[(mv - v0) * n + mu], (unsigned long long)__float2uint_rn(cw));
+        }
+      }
+    }
+  }
+  __syncthreads();
+  float* out = faces + ((6 * box + face) * n + v0) * n;
+  for (int t = threadIdx.x; t < (v1 - v0) * n; t += 256)
+    out[t] = (float)((double)facc[t] * (1.0 / (double)kFixF)) * mass;
+}
+
+// The windows: one thread per four cells of a row (n is a multiple of w >= 4;
+// a row starts at a multiple of w of the image mesh, so four cells never
+// straddle its end).
+__global__ void __launch_bounds__(256) k_mesh_window(MeshGeo M, PMLevel L, const PMBox* __restrict__ boxes, int nbox,
+                                                     const float* __restrict__ mesh, const float* __restrict__ faces,
+                                                     float* __restrict__ out) {
+  const int n = L.n, nq = n / 4;
+  const int64_t row = ((int64_t)blockIdx.x * 256 + threadIdx.x) / nq;  // box, z, y
+  const int x = (int)(((int64_t)blockIdx.x * 256 + threadIdx.x) % nq) * 4;
+  if (row >= (int64_t)nbox * n * n) return;
+  const int64_t box = row / ((int64_t)n * n);
+  const int y = (int)(row % n), z = (int)((row / n) % n);
+  const PMBox B = boxes[box];
+  const float* fb = faces + 6 * box * n * n;
+  float4 v;
+  if (z == 0 || z == n - 1) v = *(const float4*)(fb + ((int64_t)(z == 0 ? 4 : 5) * n + y) * n + x);
+  else if (y == 0 || y == n - 1) v = *(const float4*)(fb + ((int64_t)(y == 0 ? 2 : 3) * n + z) * n + x);
+  else {
+    const int p[3] = {x, y, z};
+    int a[3];
+    for (int d = 0; d < 3; ++d) {
+      const int T = d == 0 ? B.T % M.nnt : (d == 1 ? (B.T / M.nnt) % M.nnt : B.T / (M.nnt * M.nnt));
+      a[d] = (T * M.nt + B.nc1[d] - 1 - L.nloop) * M.w + p[d];
+      a[d] = a[d] < 0 ? a[d] + M.n : (a[d] >= M.n ? a[d] - M.n : a[d]);
+    }
+    v = *(const float4*)(mesh + ((int64_t)a[2] * M.n + a[1]) * M.n + a[0]);
+    if (x == 0) v.x = fb[(int64_t)z * n + y];
+    if (x == n - 4) v.w = fb[((int64_t)n + z) * n + y];
+  }
+  *(float4*)(out + B.moff + ((int64_t)z * n + y) * n + x) = v;
+}
+
+// Buffer cells as periodic images of the physical ones (counts and encoded
+// coordinates, particle by particle): one wavefront per extended cell.
+template <int IZ>
+__global__ void __launch_bounds__(256) k_mesh_images(Geo g, const XT<IZ>* __restrict__ xp,
+                                                     const int32_t* __restrict__ rhoc,
+                                                     const int64_t* __restrict__ off, int32_t* __restrict__ bad) {
+  const int64_t c = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
+  const int lane = threadIdx.x & 63;
+  if (c >= g.ncells_ext) return;
+  const int64_t T = c / g.ncell_tile, e = c % g.ncell_tile;
+  const int64_t it[3] = {T % g.nnt, (T / g.nnt) % g.nnt, T / (g.nnt * g.nnt)};
+  const int64_t ijk[3] = {e % g.nte + 1 - g.ncb, (e / g.nte) % g.nte + 1 - g.ncb, e / (g.nte * g.nte) + 1 - g.ncb};
+  int64_t st[3], sc[3];
+  bool phys = true;
+  for (int d = 0; d < 3; ++d) {
+    phys = phys && ijk[d] >= 1 && ijk[d] <= g.nt;
+    int64_t gc = (it[d] * g.nt + ijk[d] - 1) % g.nc;
+    gc = gc < 0 ? gc + g.nc : gc;
+    st[d] = gc / g.nt;
+    sc[d] = gc % g.nt + 1;
+  }
+  if (phys) return;
+  const int64_t src = rc_index(sc[0], sc[1], sc[2], (st[2] * g.nnt + st[1]) * g.nnt + st[0], g.nte, g.ncb);
+  const int n = rhoc[c];
+  bool diff = n != rhoc[src];
+  if (!diff)
+    for (int l = lane; l < 3 * n; l += 64) diff = diff || xp[3 * off[c] + l] != xp[3 * off[src] + l];
+  if (__any(diff) && lane == 0) *bad = 1;
+}
+
+}  // namespace
+
+MeshGeo mesh_geo(const Geo& g, int w, int bits) {
+  MeshGeo M;
+  M.w = w;
+  M.n = (int)g.nc * w;
+  M.sh = bits - (31 - __builtin_clz((unsigned)w));
+  M.nc = (int)g.nc;
+  M.nt = (int)g.nt;
+  M.nnt = (int)g.nnt;
+  M.nte = (int)g.nte;
+  M.ncb = (int)g.ncb;
+  return M;
+}
+
+bool pm_mesh_applies(const Geo& g, const PMLevel& L) {
+  return !L.periodic && !L.xdiv && (L.w == 4 || L.w == 8) && L.nforce % L.w == 0 && L.win_lo == 1 - L.nloop * L.w &&
+         L.win_hi == L.nforce + L.nloop * L.w && L.n == L.nforce + 2 * L.nloop * L.w && (g.nc * L.w) % 8 == 0 && L.nloop <= g.nc &&
+         L.nloop <= g.ncb;
+}
+
+void pm_mesh_deposit(int izipx, const MeshGeo& M, const void* xp, const int32_t* rhoc, const int64_t* off,
+                     float* mesh, float mass, hipStream_t s) {
+  // 16^3 blocks have half the repeated contributors of 8^3 ones, but fill the chip only from 2048 of them
+  const int bd = M.n % 16 == 0 && (int64_t)M.n * M.n * M.n / 4096 >= 2048 ? 16 : 8;
+  const int64_t nb = M.n / bd;
+  const dim3 grid((unsigned)(nb * nb * nb));
+  if (izipx == 2 && bd == 16)
+    hipLaunchKernelGGL((k_mesh_deposit<2, 16>), grid, dim3(256), 0, s, M, (const int16_t*)xp, rhoc, off, mesh, mass);
+  else if (izipx == 2)
+    hipLaunchKernelGGL((k_mesh_deposit<2, 8>), grid, dim3(256), 0, s, M, (const int16_t*)xp, rhoc, off, mesh, mass);
+  else if (bd == 16)
+    hipLaunchKernelGGL((k_mesh_deposit<1, 16>), grid, dim3(256), 0, s, M, (const int8_t*)xp, rhoc, off, mesh, mass);
+  else
+    hipLaunchKernelGGL((k_mesh_deposit<1, 8>), grid, dim3(256), 0, s, M, (const int8_t*)xp, rhoc, off, mesh, mass);
+  CUBE_HIP(hipGetLastError());
+}
+
+void pm_mesh_faces(int izipx, const MeshGeo& M, const PMLevel& L, const PMBox* boxes, int nbox, const void* xp,
+                   const int32_t* rhoc, const int64_t* off, float* faces, float mass, hipStream_t s) {
+  // strips of at most 32 KB
+  const int rows = std::min(L.n, std::max(1, 32768 / (8 * L.n)));
+  const int nstrip = (L.n + rows - 1) / rows;
+  const size_t lds = (size_t)rows * L.n * 8;
+  const dim3 grid((unsigned)((int64_t)nbox * 6 * nstrip));
+  if (izipx == 2)
+    hipLaunchKernelGGL(k_mesh_faces<2>, grid, dim3(256), lds, s, M, L, boxes, rows, (const int16_t*)xp, rhoc, off,
+                       faces, mass);
+  else
+    hipLaunchKernelGGL(k_mesh_faces<1>, grid, dim3(256), lds, s, M, L, boxes, rows, (const int8_t*)xp, rhoc, off,
+                       faces, mass);
+  CUBE_HIP(hipGetLastError());
+}
+
+void pm_mesh_window(const MeshGeo& M, const PMLevel& L, const PMBox* boxes, int nbox, const float* mesh,
+                    const float* faces, float* out, hipStream_t s) {
+  const int64_t nthr = (int64_t)nbox * L.n * L.n * (L.n / 4);
+  hipLaunchKernelGGL(k_mesh_window, dim3((unsigned)ceil_div(nthr, 256)), dim3(256), 0, s, M, L, boxes, nbox, mesh,
+                     faces, out);
+  CUBE_HIP(hipGetLastError());
+}
+
+void mesh_check_images(int izipx, const Geo& g, const void* xp, const int32_t* rhoc, const int64_t* off, int32_t* bad,
+                       hipStream_t s) {
+  zero_async(bad, sizeof(int32_t), s);
+  const dim3 grid((unsigned)ceil_div(g.ncells_ext * 64, 256));
+  if (izipx == 2)
+    hipLaunchKernelGGL(k_mesh_images<2>, grid, dim3(256), 0, s, g, (const int16_t*)xp, rhoc, off, bad);
+  else
+    hipLaunchKernelGGL(k_mesh_images<1>, grid, dim3(256), 0, s, g, (const int8_t*)xp, rhoc, off, bad);
+  CUBE_HIP(hipGetLastError());
+}
+
+}  // namespace cube
