@@ -123,13 +123,13 @@ __global__ void __launch_bounds__(256) k_deposit(PMLevel L, const PMBox* __restr
   // neighbours only.  Otherwise blocks tile the window from win_lo.
   const int gcell = BD / L.w;
   const int nblk = CA ? 1 + (L.nforce / L.w - 1 + 2 * L.nloop + gcell - 1) / gcell : (L.win_hi - L.win_lo + BD) / BD;
-  int64_t b = blockIdx.x;
-  const int bx = (int)(b % nblk);
-  b /= nblk;
-  const int by = (int)(b % nblk);
-  b /= nblk;
-  const int bz = (int)(b % nblk);
-  const int ibox = (int)(b / nblk);
+  uint32_t b = blockIdx.x;
+  const int bx = (int)(b % (uint32_t)nblk);
+  b /= (uint32_t)nblk;
+  const int by = (int)(b % (uint32_t)nblk);
+  b /= (uint32_t)nblk;
+  const int bz = (int)(b % (uint32_t)nblk);
+  const int ibox = (int)(b / (uint32_t)nblk);
   const PMBox B = boxes[ibox];
   const int bidx[3] = {bx, by, bz};
   int mlo[3], mhi[3], clo[3], chi[3];
@@ -258,9 +258,9 @@ __global__ void __launch_bounds__(256) k_dep_bin(PMLevel L, const PMBox* __restr
                                                  unsigned long long* __restrict__ ents) {
   const int nr = L.nforce / L.w + 2 * L.nloop;
   const int lane = threadIdx.x & 63;
-  const int64_t wv = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
-  if (wv >= (int64_t)nbox * nr * nr * nr) return;
-  const int ib = (int)(wv / (nr * nr * nr)), qc = (int)(wv % (nr * nr * nr));
+  const uint32_t wv = blockIdx.x * 4u + (threadIdx.x >> 6);
+  if (wv >= (uint32_t)nbox * nr * nr * nr) return;
+  const int ib = (int)(wv / (uint32_t)(nr * nr * nr)), qc = (int)(wv % (uint32_t)(nr * nr * nr));
   const PMBox B = boxes[ib];
   const int cl[3] = {qc % nr, (qc / nr) % nr, qc / (nr * nr)};
   int c[3], lo0[3], b0[3];
@@ -375,13 +375,13 @@ __global__ void __launch_bounds__(NT) k_deposit_lists(PMLevel L, const PMBox* __
   __shared__ Acc acc[BD * BD * BD];
   const int nb = dep_nblk(L);
   const int64_t blk = blockIdx.x;
-  int64_t b = blk;
-  const int bx = (int)(b % nb);
-  b /= nb;
-  const int by = (int)(b % nb);
-  b /= nb;
-  const int bz = (int)(b % nb);
-  const int ibox = (int)(b / nb);
+  uint32_t b = blockIdx.x;
+  const int bx = (int)(b % (uint32_t)nb);
+  b /= (uint32_t)nb;
+  const int by = (int)(b % (uint32_t)nb);
+  b /= (uint32_t)nb;
+  const int bz = (int)(b % (uint32_t)nb);
+  const int ibox = (int)(b / (uint32_t)nb);
   const PMBox B = boxes[ibox];
   const int bidx[3] = {bx, by, bz};
   int mlo[3], mhi[3];
@@ -441,10 +441,11 @@ __global__ void __launch_bounds__(128) k_pm1_stencil(PMLevel L, const XT<IZ>* __
   __shared__ Acc red[2][kRound][65];
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int64_t ncell = (int64_t)L.n * L.n * L.n;
-  const int64_t g = (int64_t)blockIdx.x * 2 + wave;
+  const uint32_t g = blockIdx.x * 2u + (uint32_t)wave;
   if (g >= ncell) return;
   const int nt = L.nt, nnt = L.n / L.nt;
-  const int gx = (int)(g % L.n), gy = (int)((g / L.n) % L.n), gz = (int)(g / ((int64_t)L.n * L.n));
+  const uint32_t gyz = g / (uint32_t)L.n;
+  const int gx = (int)(g - gyz * L.n), gy = (int)(gyz % (uint32_t)L.n), gz = (int)(gyz / (uint32_t)L.n);
   const int T = ((gz / nt) * nnt + gy / nt) * nnt + gx / nt;
   const int ijk[3] = {gx % nt + 1, gy % nt + 1, gz % nt + 1};
   const int64_t cell = rc_index(ijk[0], ijk[1], ijk[2], T, L.nte, L.ncb);
@@ -504,10 +505,11 @@ __global__ void __launch_bounds__(256) k_pm1_gather(PMLevel L, const void* __res
   __shared__ Acc red[4];
   const int n = L.n;
   const int64_t ncell = (int64_t)n * n * n;
-  const int64_t M = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const uint32_t M = blockIdx.x * blockDim.x + threadIdx.x;
   Acc v = 0;
   if (M < ncell) {
-    const int mx = (int)(M % n), my = (int)((M / n) % n), mz = (int)(M / ((int64_t)n * n));
+    const uint32_t myz = M / (uint32_t)n;
+    const int mx = (int)(M - myz * n), my = (int)(myz % (uint32_t)n), mz = (int)(myz / (uint32_t)n);
     const Acc* st = (const Acc*)stencil;
 #pragma unroll
     for (int q = 0; q < 27; ++q) {
@@ -534,15 +536,55 @@ __global__ void __launch_bounds__(256) k_pm1_gather(PMLevel L, const void* __res
   }
 }
 
+// Raises the level's maxima to this wavefront's.  A running maximum saturates
+// after a few workgroups, so nearly every wavefront compares and is done; the
+// others reduce across lanes first (one atomic per wavefront).
 template <typename R>
-__device__ inline R block_max(R v, R* red) {
-  for (int o = 32; o > 0; o >>= 1) v = max(v, __shfl_down(v, o, 64));
-  __syncthreads();
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
-  __syncthreads();
-  R m = 0;
-  for (int q = 0; q < (int)(blockDim.x >> 6); ++q) m = max(m, red[q]);
-  return m;
+__device__ inline void raise_maxima(R f2, const R vm[3], PMOut* __restrict__ out) {
+  R* at[4];
+  if constexpr (std::is_same<R, float>::value) {
+    at[0] = &out->f2max;
+    for (int d = 0; d < 3; ++d) at[1 + d] = &out->vmax[d];
+  } else {
+    at[0] = &out->f2max_d;
+    for (int d = 0; d < 3; ++d) at[1 + d] = &out->vmax_d[d];
+  }
+  const R v[4] = {f2, vm[0], vm[1], vm[2]};
+  R now[4];
+  for (int k = 0; k < 4; ++k) now[k] = *(volatile R*)at[k];
+  for (int k = 0; k < 4; ++k) {
+    if (!__any(v[k] > now[k])) continue;
+    R m = v[k];
+    for (int o = 32; o > 0; o >>= 1) m = max(m, __shfl_xor(m, o, 64));
+    if ((threadIdx.x & 63) == 0) atomic_max_nonneg(at[k], m);
+  }
+}
+
+// PM1 at 512^3: 2.3 -> 1.35 ms with this gather.
+//
+// The 27-point gather of the three force arrays (FN values each, rows of FX,
+// planes of FX FY) at base cell li: sums along x, then y, then z with fused
+// multiply-adds, 39 operations per component instead of 108 for the 27
+// products of three weights (and fewer roundings).
+template <typename R>
+__device__ inline void tsc_gather(const R* __restrict__ F, int FN, int FX, int FXY, int li, const R w[3][3], R dv[3]) {
+#pragma unroll
+  for (int d = 0; d < 3; ++d) {
+    const R* f = F + d * FN + li;
+    R sz = 0;
+#pragma unroll
+    for (int i3 = 0; i3 < 3; ++i3) {
+      R sy = 0;
+#pragma unroll
+      for (int i2 = 0; i2 < 3; ++i2) {
+        const R* r = f + i3 * FXY + i2 * FX;
+        const R sx = fma(r[2], w[0][2], fma(r[1], w[0][1], r[0] * w[0][0]));
+        sy = fma(sx, w[1][i2], sy);
+      }
+      sz = fma(sy, w[2][i3], sz);
+    }
+    dv[d] = sz;
+  }
 }
 
 template <typename R, int IZ, int BD, int MAXC>
@@ -555,18 +597,17 @@ __global__ void __launch_bounds__(256) k_interp(PMLevel L, const PMBox* __restri
   constexpr int NF = (FS * FS * FS + 255) / 256;
   constexpr int LDSN = (PS * PS * PS > 3 * FS * FS * FS) ? PS * PS * PS : 3 * FS * FS * FS;
   __shared__ R lds[LDSN];
-  __shared__ R red[4];
   __shared__ int cnt[MAXC], pre[MAXC + 1], wsum[4];
   __shared__ int64_t gof[MAXC];
   if (L.kdev) kc = *L.kdev;
   const int nblk = (L.nforce + BD - 1) / BD;
-  int64_t b = blockIdx.x;
-  const int bx = (int)(b % nblk);
-  b /= nblk;
-  const int by = (int)(b % nblk);
-  b /= nblk;
-  const int bz = (int)(b % nblk);
-  const int ibox = (int)(b / nblk);
+  uint32_t b = blockIdx.x;
+  const int bx = (int)(b % (uint32_t)nblk);
+  b /= (uint32_t)nblk;
+  const int by = (int)(b % (uint32_t)nblk);
+  b /= (uint32_t)nblk;
+  const int bz = (int)(b % (uint32_t)nblk);
+  const int ibox = (int)(b / (uint32_t)nblk);
   const PMBox B = boxes[ibox];
   const int f0[3] = {bx * BD, by * BD, bz * BD};
   // coarse cells whose particles can have floor(xpos) in this block; a cell i
@@ -721,14 +762,8 @@ __global__ void __launch_bounds__(256) k_interp(PMLevel L, const PMBox* __restri
         mine = mine && f[d] >= 0 && f[d] < BD;
       }
       if (!mine) continue;
-      R dv[3] = {0, 0, 0};
-      for (int i3 = 0; i3 < 3; ++i3)
-        for (int i2 = 0; i2 < 3; ++i2)
-          for (int i1 = 0; i1 < 3; ++i1) {
-            const int li = ((f[2] + i3) * FS + (f[1] + i2)) * FS + (f[0] + i1);
-            for (int d = 0; d < 3; ++d)
-              dv[d] = dv[d] + ((lds[d * FS * FS * FS + li] * w[0][i1]) * w[1][i2]) * w[2][i3];
-          }
+      R dv[3];
+      tsc_gather<R>(lds, FS * FS * FS, FS, FS * FS, (f[2] * FS + f[1]) * FS + f[0], w, dv);
       for (int d = 0; d < 3; ++d) {
         const float v = (float)kick_update((R)v0[d], dv[d], kc);
         vp[3 * ip + d] = v;
@@ -736,18 +771,7 @@ __global__ void __launch_bounds__(256) k_interp(PMLevel L, const PMBox* __restri
       }
     }
   }
-  R bm = block_max(f2, red);
-  if (threadIdx.x == 0 && bm > 0) {
-    if constexpr (std::is_same<R, float>::value) atomic_max_nonneg(&out->f2max, bm);
-    else atomic_max_nonneg(&out->f2max_d, bm);
-  }
-  for (int d = 0; d < 3; ++d) {
-    R m = block_max(vm[d], red);
-    if (threadIdx.x == 0 && m > 0) {
-      if constexpr (std::is_same<R, float>::value) atomic_max_nonneg(&out->vmax[d], m);
-      else atomic_max_nonneg(&out->vmax_d[d], m);
-    }
-  }
+  raise_maxima<R>(f2, vm, out);
 }
 
 // Interpolation for the tile and sub-tile levels with w = 4 or 8 mesh cells per
@@ -763,6 +787,11 @@ __global__ void __launch_bounds__(256) k_interp(PMLevel L, const PMBox* __restri
 // autotuner (every shape gives the same result): a larger block stages a
 // smaller share of halo (phi halo 4.2 -> 3.3 values per cell, FD force on 1.76
 // -> 1.58 cells per cell) with twice the threads.
+// Bound by LDS (85% busy at 512^3 PM3, half of it the bank conflicts of the
+// 81 random reads per particle) and VALU (85%) alike.  4096 boxes of 64^3
+// cells, 1.34e8 particles: 9.9 -> 8.6 ms with quad loads of phi and the
+// separable gather, 6.6 with the FD reads free of bank conflicts (x along the
+// lanes, pairs along z) and the maxima compared before any reduction.
 template <typename R, int IZ, int BX, int BY, int BZ, int NT>
 __global__ void __launch_bounds__(NT) k_interp_cells(PMLevel L, const PMBox* __restrict__ boxes,
                                                       const XT<IZ>* __restrict__ xp, float* __restrict__ vp,
@@ -771,13 +800,18 @@ __global__ void __launch_bounds__(NT) k_interp_cells(PMLevel L, const PMBox* __r
                                                       double kc, PMOut* __restrict__ out) {
   if (L.kdev) kc = *L.kdev;
   constexpr int FX = BX + 2, FY = BY + 2, FZ = BZ + 2, FN = FX * FY * FZ;
-  constexpr int PX = BX + 6, PY = BY + 6, PZ = BZ + 6, PN = PX * PY * PZ;
-  constexpr int NF = (FN + NT - 1) / NT, NPH = (PN + NT - 1) / NT;
+  // phi rows: x = f0-3 .. f0+BX+4, whole 16-byte quads (f0-3 is at a multiple
+  // of 4 of the mesh row)
+  constexpr int PY = BY + 6, PZ = BZ + 6, PQ = (BX + 8) / 4, PS = 4 * PQ, PN = PY * PZ * PS;
+  constexpr int NQ = PY * PZ * PQ, NPH = (NQ + NT - 1) / NT;
+  constexpr int NPR = FN / 2, NF = (NPR + NT - 1) / NT;  // FD tasks: pairs of cells along z
   constexpr int LDSN = PN > 3 * FN ? PN : 3 * FN;
+  struct alignas(16) Quad {
+    R v[4];
+  };
   constexpr int MAXC = (BX / 4) * (BY / 4) * (BZ / 4);  // coarse cells of a block at w >= 4
   constexpr int NW = NT / 64;
-  __shared__ R lds[LDSN];
-  __shared__ R red[NW];
+  __shared__ __align__(16) R lds[LDSN];
   __shared__ int cnt[MAXC], pre[MAXC + 1], wsum[NW], cxyz[MAXC];
   __shared__ int64_t gof[MAXC];
   const int w = L.w;
@@ -785,13 +819,13 @@ __global__ void __launch_bounds__(NT) k_interp_cells(PMLevel L, const PMBox* __r
   const int ncell = L.nforce / w;                // physical coarse cells of a box per axis
   const int nb[3] = {(ncell + g[0] - 1) / g[0], (ncell + g[1] - 1) / g[1], (ncell + g[2] - 1) / g[2]};
   // neighbouring blocks share phi halos: keep them on one XCD's L2
-  int64_t b = xcd_block(blockIdx.x, gridDim.x);
-  const int bx = (int)(b % nb[0]);
-  b /= nb[0];
-  const int by = (int)(b % nb[1]);
-  b /= nb[1];
-  const int bz = (int)(b % nb[2]);
-  const int ibox = (int)(b / nb[2]);
+  uint32_t b = (uint32_t)xcd_block(blockIdx.x, gridDim.x);  // 32-bit: a 64-bit division is ~100 instructions
+  const int bx = (int)(b % (uint32_t)nb[0]);
+  b /= (uint32_t)nb[0];
+  const int by = (int)(b % (uint32_t)nb[1]);
+  b /= (uint32_t)nb[1];
+  const int bz = (int)(b % (uint32_t)nb[2]);
+  const int ibox = (int)(b / (uint32_t)nb[2]);
   const PMBox B = boxes[ibox];
   const int bi[3] = {bx, by, bz};
   int clo[3], chi[3], f0[3], fend[3];
@@ -801,22 +835,24 @@ __global__ void __launch_bounds__(NT) k_interp_cells(PMLevel L, const PMBox* __r
     f0[d] = w * (clo[d] - 1) - B.ushift[d];
     fend[d] = f0[d] + w * (chi[d] - clo[d] + 1);  // last force cell this block counts for f2max
   }
-  // 1. phi(f0-2 .. f0+IB+3) and the cell metadata, all loads before the
+  // 1. phi(f0-2 .. f0+B+3) and the cell metadata, all loads before the
   //    first LDS store
-  R ph[NPH];
+  const int a0[3] = {f0[0] - 3 + B.org[0] - L.m0, f0[1] - 2 + B.org[1] - L.m0, f0[2] - 2 + B.org[2] - L.m0};
+  const R* pb = phi + B.moff;
+  R ph[NPH][4];
 #pragma unroll
   for (int q = 0; q < NPH; ++q) {
     const int t = threadIdx.x + q * NT;
-    ph[q] = (R)0;
-    if (t < PN) {
-      const int l[3] = {t % PX, (t / PX) % PY, t / (PX * PY)};
-      int a[3];
-      bool ok = true;
-      for (int d = 0; d < 3; ++d) {
-        a[d] = f0[d] - 2 + l[d] + B.org[d] - L.m0;
-        ok = ok && a[d] >= 0 && a[d] < L.n;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) ph[q][k] = (R)0;
+    if (t < NQ) {
+      const int row = t / PQ, ax = a0[0] + 4 * (t % PQ), ay = a0[1] + row % PY, az = a0[2] + row / PY;
+      if ((unsigned)ax < (unsigned)L.n && (unsigned)ay < (unsigned)L.n && (unsigned)az < (unsigned)L.n)
+      {
+        const Quad* src = reinterpret_cast<const Quad*>(pb + ((int64_t)(az * L.n + ay) * L.n + ax));
+#pragma unroll
+        for (int k = 0; k < 4; ++k) ph[q][k] = src->v[k];
       }
-      if (ok) ph[q] = phi[B.moff + ((int64_t)a[2] * L.n + a[1]) * L.n + a[0]];
     }
   }
   const int ncx = chi[0] - clo[0] + 1, ncy = chi[1] - clo[1] + 1, ncz = chi[2] - clo[2] + 1;
@@ -831,55 +867,61 @@ __global__ void __launch_bounds__(NT) k_interp_cells(PMLevel L, const PMBox* __r
 #pragma unroll
   for (int q = 0; q < NPH; ++q) {
     const int t = threadIdx.x + q * NT;
-    if (t < PN) lds[t] = ph[q];
+    if (t < NQ) {
+      Quad* dst = reinterpret_cast<Quad*>(lds + (t / PQ) * PS + 4 * (t % PQ));
+#pragma unroll
+      for (int k = 0; k < 4; ++k) dst->v[k] = ph[q][k];
+    }
   }
   __syncthreads();
   block_scan(cnt, pre, nC, wsum);
   const int total = pre[nC];
-  // 2. force(d, f0 .. f0+IB+1) = sum(phi(m + [-2,-1,1,2]) * weight), fused
-  //    multiply-adds (one rounding per term; the kick tolerance is 1e-5)
+  // 2. force(d, f0 .. f0+B+1) = sum(phi(m + [-2,-1,1,2]) * weight), fused
+  //    multiply-adds (one rounding per term; the kick tolerance is 1e-5), two
+  //    cells along z per thread (they share their z neighbours) and x along
+  //    the lanes, so that the LDS reads are free of bank conflicts
   const FDWeights<R> W;
-  R fr[NF][3];
+  R fr[NF][6];
   R f2 = 0;
 #pragma unroll
   for (int q = 0; q < NF; ++q) {
     const int t = threadIdx.x + q * NT;
-    if (t < FN) {
-      const int lx = t % FX, ly = (t / FX) % FY, lz = t / (FX * FY);
-      const int px = lx + 2, py = ly + 2, pz = lz + 2;
-      auto P = [&](int x, int y, int z) { return lds[(z * PY + y) * PX + x]; };
-      R sx = 0, sy = 0, sz = 0;
-      sx = fma(P(px - 2, py, pz), W.w0, sx);
-      sx = fma(P(px - 1, py, pz), W.w1, sx);
-      sx = fma(P(px + 1, py, pz), W.w2, sx);
-      sx = fma(P(px + 2, py, pz), W.w3, sx);
-      sy = fma(P(px, py - 2, pz), W.w0, sy);
-      sy = fma(P(px, py - 1, pz), W.w1, sy);
-      sy = fma(P(px, py + 1, pz), W.w2, sy);
-      sy = fma(P(px, py + 2, pz), W.w3, sy);
-      sz = fma(P(px, py, pz - 2), W.w0, sz);
-      sz = fma(P(px, py, pz - 1), W.w1, sz);
-      sz = fma(P(px, py, pz + 1), W.w2, sz);
-      sz = fma(P(px, py, pz + 2), W.w3, sz);
-      fr[q][0] = sx;
-      fr[q][1] = sy;
-      fr[q][2] = sz;
-      // f2max over force cells 1..nforce (kick.f90:717); neighbouring blocks
-      // share their boundary cell, which is harmless for a maximum
-      const int m[3] = {f0[0] + lx, f0[1] + ly, f0[2] + lz};
-      bool in = true;
-      for (int d = 0; d < 3; ++d) in = in && (m[d] >= 1 && m[d] <= L.nforce && m[d] <= fend[d]);
-      if (in) f2 = max(f2, (sx * sx + sy * sy) + sz * sz);
+    if (t < NPR) {
+      const int lx = t % FX, ly = (t / FX) % FY, lz = 2 * (t / (FX * FY));
+      constexpr int SZ = PY * PS;
+      const R* p = lds + ((lz + 2) * PY + ly + 2) * PS + lx + 3;
+      R z[6];
+#pragma unroll
+      for (int i = 0; i < 6; ++i) z[i] = p[(i - 2) * SZ];
+      const int mx = f0[0] + lx, my = f0[1] + ly;
+      const bool inxy = mx >= 1 && mx <= min(L.nforce, fend[0]) && my >= 1 && my <= min(L.nforce, fend[1]);
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const R* c = p + i * SZ;
+        const R sx = fma(c[2], W.w3, fma(c[1], W.w2, fma(c[-1], W.w1, c[-2] * W.w0)));
+        const R sy = fma(c[2 * PS], W.w3, fma(c[PS], W.w2, fma(c[-PS], W.w1, c[-2 * PS] * W.w0)));
+        const R sz = fma(z[i + 4], W.w3, fma(z[i + 3], W.w2, fma(z[i + 1], W.w1, z[i] * W.w0)));
+        fr[q][i] = sx;
+        fr[q][2 + i] = sy;
+        fr[q][4 + i] = sz;
+        // f2max over force cells 1..nforce (kick.f90:717); neighbouring blocks
+        // share their boundary cell, which is harmless for a maximum
+        const int mz = f0[2] + lz + i;
+        if (inxy && mz >= 1 && mz <= min(L.nforce, fend[2])) f2 = max(f2, (sx * sx + sy * sy) + sz * sz);
+      }
     }
   }
   __syncthreads();
 #pragma unroll
   for (int q = 0; q < NF; ++q) {
     const int t = threadIdx.x + q * NT;
-    if (t < FN) {
-      lds[t] = fr[q][0];
-      lds[FN + t] = fr[q][1];
-      lds[2 * FN + t] = fr[q][2];
+    if (t < NPR) {
+      const int c = t + t / (FX * FY) * (FX * FY);  // cell index of the pair's lower cell
+#pragma unroll
+      for (int d = 0; d < 3; ++d) {
+        lds[d * FN + c] = fr[q][2 * d];
+        lds[d * FN + c + FX * FY] = fr[q][2 * d + 1];
+      }
     }
   }
   __syncthreads();
@@ -908,32 +950,15 @@ __global__ void __launch_bounds__(NT) k_interp_cells(PMLevel L, const PMBox* __r
       ok = ok && f[d] >= 0 && f[d] < (d == 0 ? BX : (d == 1 ? BY : BZ));
     }
     if (!ok) continue;  // unreachable for a power-of-two xmul; guards the LDS reads
-    R dv[3] = {0, 0, 0};
-    for (int i3 = 0; i3 < 3; ++i3)
-      for (int i2 = 0; i2 < 3; ++i2)
-        for (int i1 = 0; i1 < 3; ++i1) {
-          const int li = ((f[2] + i3) * FY + (f[1] + i2)) * FX + (f[0] + i1);
-          for (int d = 0; d < 3; ++d)
-            dv[d] = dv[d] + ((lds[d * FN + li] * wt[0][i1]) * wt[1][i2]) * wt[2][i3];
-        }
+    R dv[3];
+    tsc_gather<R>(lds, FN, FX, FX * FY, (f[2] * FY + f[1]) * FX + f[0], wt, dv);
     for (int d = 0; d < 3; ++d) {
       const float v = (float)kick_update((R)v0[d], dv[d], kc);
       vp[3 * ip + d] = v;
       vm[d] = max(vm[d], (R)fabsf(v));
     }
   }
-  R bm = block_max(f2, red);
-  if (threadIdx.x == 0 && bm > 0) {
-    if constexpr (std::is_same<R, float>::value) atomic_max_nonneg(&out->f2max, bm);
-    else atomic_max_nonneg(&out->f2max_d, bm);
-  }
-  for (int d = 0; d < 3; ++d) {
-    R m = block_max(vm[d], red);
-    if (threadIdx.x == 0 && m > 0) {
-      if constexpr (std::is_same<R, float>::value) atomic_max_nonneg(&out->vmax[d], m);
-      else atomic_max_nonneg(&out->vmax_d[d], m);
-    }
-  }
+  raise_maxima<R>(f2, vm, out);
 }
 
 // Green_3D, Green/Green.f90:22-71 at nn=1.
@@ -990,14 +1015,14 @@ __global__ void k_green(int n, float apm_soft, float apm_range, float gridsize, 
 __global__ void k_classify(Geo g, int ires_fixed, const int32_t* __restrict__ rhoc, int32_t* __restrict__ ires,
                            int32_t* __restrict__ napm, int32_t* __restrict__ cmax) {
   __shared__ int32_t red[256];
-  const int64_t it = blockIdx.x;
-  const int64_t nns = g.nns;
-  const int64_t ifs[3] = {it % nns, (it / nns) % nns, (it / (nns * nns)) % nns};
-  const int64_t T = it / (nns * nns * nns);
-  const int64_t ntt = g.ntt;
+  const uint32_t it = blockIdx.x;
+  const uint32_t nns = (uint32_t)g.nns;
+  const uint32_t ifs[3] = {it % nns, (it / nns) % nns, (it / (nns * nns)) % nns};
+  const uint32_t T = it / (nns * nns * nns);
+  const uint32_t ntt = (uint32_t)g.ntt;
   int32_t mx = 0;
-  for (int64_t q = threadIdx.x; q < ntt * ntt * ntt; q += blockDim.x) {
-    int64_t i = ifs[0] * ntt + q % ntt + 1, j = ifs[1] * ntt + (q / ntt) % ntt + 1, k = ifs[2] * ntt + q / (ntt * ntt) + 1;
+  for (uint32_t q = threadIdx.x; q < ntt * ntt * ntt; q += blockDim.x) {
+    uint32_t i = ifs[0] * ntt + q % ntt + 1, j = ifs[1] * ntt + (q / ntt) % ntt + 1, k = ifs[2] * ntt + q / (ntt * ntt) + 1;
     mx = max(mx, rhoc[rc_index(i, j, k, T, g.nte, g.ncb)]);
   }
   red[threadIdx.x] = mx;
@@ -1285,7 +1310,9 @@ void pm_interp(int izipx, const PMLevel& L, const PMBox* boxes, int nbox, const 
 }
 
 bool pm_interp_cells_form(const PMLevel& L) {
-  return !L.periodic && !L.xdiv && (L.w == 4 || L.w == 8) && L.nforce % L.w == 0;
+  // force cell 1 at a multiple of 4 of rows of a multiple of 4: quad loads
+  return !L.periodic && !L.xdiv && (L.w == 4 || L.w == 8) && L.nforce % L.w == 0 && (1 - L.m0) % 4 == 0 &&
+         L.n % 4 == 0;
 }
 
 template void pm_deposit<float>(int, const PMLevel&, const PMBox*, int, const void*, const int32_t*, const int64_t*,
