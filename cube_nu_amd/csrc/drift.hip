@@ -416,8 +416,8 @@ __global__ void __launch_bounds__(256) k_buffer_rows(Geo g, const int64_t* __res
                                                      XT<IZ>* __restrict__ xo, float* __restrict__ vo,
                                                      int64_t* __restrict__ po) {
   const int nte = (int)g.nte, nt = (int)g.nt, nc = (int)g.nc, nnt = (int)g.nnt, ncb = (int)g.ncb;
-  const int64_t r = blockIdx.x;  // (T, ze, ye) with ye fastest
-  const int ye = (int)(r % nte), ze = (int)((r / nte) % nte), T = (int)(r / ((int64_t)nte * nte));
+  const uint32_t r = blockIdx.x, rz = r / (uint32_t)nte;  // (T, ze, ye) with ye fastest
+  const int ye = (int)(r - rz * nte), ze = (int)(rz % (uint32_t)nte), T = (int)(rz / (uint32_t)nte);
   const int it[3] = {T % nnt, (T / nnt) % nnt, T / (nnt * nnt)};
   // source tile and cell of the row's y and z (periodic)
   int sy, sz, ty, tz;
@@ -465,8 +465,8 @@ template <bool PID>
 __global__ void __launch_bounds__(256) k_buffer_v_rows(Geo g, const int64_t* __restrict__ eoff, float* vp,
                                                        int64_t* pid) {
   const int nte = (int)g.nte, nt = (int)g.nt, nc = (int)g.nc, nnt = (int)g.nnt, ncb = (int)g.ncb;
-  const int64_t r = blockIdx.x;  // (T, ze, ye) with ye fastest
-  const int ye = (int)(r % nte), ze = (int)((r / nte) % nte), T = (int)(r / ((int64_t)nte * nte));
+  const uint32_t r = blockIdx.x, rz = r / (uint32_t)nte;  // (T, ze, ye) with ye fastest
+  const int ye = (int)(r - rz * nte), ze = (int)(rz % (uint32_t)nte), T = (int)(rz / (uint32_t)nte);
   const int it[3] = {T % nnt, (T / nnt) % nnt, T / (nnt * nnt)};
   const bool yz_phys = ye >= ncb && ye < ncb + nt && ze >= ncb && ze < ncb + nt;
   int sy, sz, ty, tz;

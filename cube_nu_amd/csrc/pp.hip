@@ -61,10 +61,11 @@ __global__ void __launch_bounds__(256) k_pp_bin(PPLevel L, const PPBox* __restri
   extern __shared__ int lcnt[];
   const int nr = L.ntt + 2;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int64_t wv = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
-  if (wv >= (int64_t)nbox * nr * nr * nr) return;
-  const int ib = (int)(wv / (nr * nr * nr));
-  const int qc = (int)(wv % (nr * nr * nr));
+  // 32-bit: a 64-bit division is ~100 instructions, and an image has far fewer than 2^32 coarse cells
+  const uint32_t wv = blockIdx.x * 4u + (uint32_t)wave;
+  if (wv >= (uint32_t)nbox * nr * nr * nr) return;
+  const int ib = (int)(wv / (uint32_t)(nr * nr * nr));
+  const int qc = (int)(wv % (uint32_t)(nr * nr * nr));
   const PPBox B = boxes[ib];
   const int c[3] = {B.ifs[0] * L.ntt + (qc % nr), B.ifs[1] * L.ntt + (qc / nr) % nr,
                     B.ifs[2] * L.ntt + qc / (nr * nr)};  // nc1-1 + offset (Fortran nc1 = ifs*ntt+1)
