@@ -164,6 +164,7 @@ struct cube_p3m_ctx {
   DevBuf<char> scan_tmp;
   DevBuf<char> work;
   DevBuf<float> gmesh, gfaces;  // whole-image mesh and window faces (pm_mesh.h)
+  DevBuf<int4> lorg[6];         // and the windows' origins, per slot as lboxes
   // buffer cells as periodic images of the physical ones: 1 by construction
   // (the buffer step), 0 not looked at yet (uploaded state), -1 they are not
   int images = 0;
@@ -420,6 +421,7 @@ void cube_p3m_ctx::set_tf_default() {
 template <typename R>
 bool cube_p3m_ctx::image_mesh_level(int level, const PMLevel& L, int64_t nbox, int64_t batch) const {
   if (!std::is_same<R, float>::value || level < 2 || !image_meshes || !pm_mesh_applies(g, L)) return false;
+  if (np > (int64_t)UINT32_MAX || (nu && nu->np > (int64_t)UINT32_MAX)) return false;  // 32-bit particle offsets
   if (level >= 3 && 2 * nbox < g.ns3) return false;
   const int64_t n = g.nc * L.w, bytes = 4 * (n * n * n + batch * 6 * (int64_t)L.n * L.n);
   return bytes <= ws_budget() / 2;
@@ -471,6 +473,10 @@ void cube_p3m_ctx::run_level(int level, int slot, const std::vector<PMBox>& bx_i
     if (kph == 2) L.kdev = kcoef.p;
     const int nmesh = (level == 1) ? 1 : nb;
     const double cells = (double)nreal * nmesh;
+    // windows of the image's mesh go straight into the transform where it can
+    // read them (one species: the densities of two are added as cubes)
+    const bool direct = image && !(nu && level <= 2) && fft_reads_windows<R>((int)n);
+    FFTWindow win;
     if (SZ) {
       std::vector<PMBox> bx(bx_in.begin() + b0, bx_in.begin() + b0 + nb);
       if (level != 1)
@@ -478,6 +484,12 @@ void cube_p3m_ctx::run_level(int level, int slot, const std::vector<PMBox>& bx_i
       CUBE_HIP(hipMemcpyAsync(boxes.p, bx.data(), sizeof(PMBox) * nb, hipMemcpyHostToDevice, s));
       sig_add({(uint64_t)level, (uint64_t)slot, (uint64_t)nb, (uint64_t)n, (uint64_t)(uintptr_t)boxes.p,
                (uint64_t)(uintptr_t)work.p});
+      if (image) {
+        lorg[slot].ensure(std::max<size_t>(lorg[slot].n, bchunk));
+        std::vector<int4> org(nb);
+        for (int i = 0; i < nb; ++i) org[i] = mesh_origin(M, L, bx[i]);
+        CUBE_HIP(hipMemcpyAsync(lorg[slot].p, org.data(), sizeof(int4) * nb, hipMemcpyHostToDevice, s));
+      }
     }
     {
       KScope k(&tm, (t + "deposit").c_str(), cells * sizeof(R));
@@ -487,13 +499,16 @@ void cube_p3m_ctx::run_level(int level, int slot, const std::vector<PMBox>& bx_i
         if (CP)
           pm1_deposit<R>((int)g.izipx, L, xpc(), rhocc(), off.p, st, mesh, in.mass_p_cdm, o, s);
       } else if (image) {
-        if (SZ) sig_add({(uint64_t)(uintptr_t)gmesh.p, (uint64_t)(uintptr_t)gfaces.p});
+        if (SZ)
+          sig_add({(uint64_t)(uintptr_t)gmesh.p, (uint64_t)(uintptr_t)gfaces.p, (uint64_t)(uintptr_t)lorg[slot].p,
+                   (uint64_t)direct});
         if constexpr (std::is_same<R, float>::value) {
           auto window = [&](cube_p3m_ctx* c, float m, float* out) {
             // the image's mesh holds every box of the level: once per level and species
             if (b0 == 0 || nu) pm_mesh_deposit((int)g.izipx, M, c->xpc(), c->rhocc(), c->off.p, gmesh.p, m, s);
             pm_mesh_faces((int)g.izipx, M, L, boxes.p, nb, c->xpc(), c->rhocc(), c->off.p, gfaces.p, m, s);
-            pm_mesh_window(M, L, boxes.p, nb, gmesh.p, gfaces.p, out, s);
+            if (direct) win = FFTWindow{gmesh.p, gfaces.p, lorg[slot].p, M.n};
+            else pm_mesh_window(M, (int)n, lorg[slot].p, nb, gmesh.p, gfaces.p, out, s);
           };
           if (CP) window(this, in.mass_p_cdm, mesh);
           if (CP && nu && level <= 2) {
@@ -557,7 +572,7 @@ void cube_p3m_ctx::run_level(int level, int slot, const std::vector<PMBox>& bx_i
     // second stream's list building (128-point planes of 67.5 KB: 1.9 ms
     // against 0.34 for line passes)
     if (level == 1) fft_convolve<R>(fc, mesh, cplx, G, 1, (R)0, (R)(float)n, s, &tm, tag, true);
-    else fft_convolve<R>(fc, mesh, cplx, G, nmesh, n3, (R)0, s, &tm, tag);                // kick.f90:846
+    else fft_convolve<R>(fc, mesh, cplx, G, nmesh, n3, (R)0, s, &tm, tag, false, direct ? &win : nullptr);  // kick.f90:846
     const int ishape = interp_shape<R>(level, (int)n, L, boxes.p, nb, in, mesh, kph == 0);
     {
       KScope k(&tm, (t + "interp_kick").c_str(), cells * sizeof(R));

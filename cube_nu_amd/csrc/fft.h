@@ -32,18 +32,36 @@ struct FFTCube {
 // rho/phi: [box][z][y][x] real (n^3 per box); work: complex scratch of
 // nbox * n*n*(n/2+1) elements.  The division follows the reference: one FP
 // division by div3 when div3 != 0, else three divisions by div1.
+// A convolution's input cut from one larger periodic mesh instead of cubes of
+// its own: box b's point (x, y, z) is mesh[(org[b] + (x, y, z)) mod n], except
+// on the window's faces, which are given: face 2 axis + side of box b at
+// faces[(6 b + face) c^2] (c the cube size), rows along the lower of the other
+// two axes.  org.x and n are even.
+struct FFTWindow {
+  const float* mesh = nullptr;
+  const float* faces = nullptr;
+  const int4* org = nullptr;
+  int n = 0;
+};
+// True when cubes of n points take the plane passes (the only ones that read
+// windows).
+template <typename R>
+bool fft_reads_windows(int n);
+
 // Sizes with a specialised form take it: plane passes (fft_plane.hip) where a
 // z-plane fits in LDS, line passes (fft_line.hip) for larger ones; the others
 // take the generic line passes.  small_lds: no pass that needs more than about
 // 40 KB of LDS per workgroup (a launch beside another stream's kernels).
 template <typename R>
 void fft_convolve(const FFTCube<R>& c, R* rho, typename Cplx<R>::T* work, const float* G, int64_t nbox, R div3,
-                  R div1, hipStream_t s, KTimer* tm = nullptr, const char* tag = "", bool small_lds = false);
+                  R div1, hipStream_t s, KTimer* tm = nullptr, const char* tag = "", bool small_lds = false,
+                  const FFTWindow* win = nullptr);
 
 // The specialised forms; false when n has none.
 template <typename R>
 bool fft_convolve_plane(const FFTCube<R>& c, R* rho, typename Cplx<R>::T* work, const float* G, int64_t nbox,
-                        R div3, R div1, hipStream_t s, KTimer* tm, const char* tag);
+                        R div3, R div1, hipStream_t s, KTimer* tm, const char* tag, const FFTWindow* win);
+bool fft_plane_size(int n);  // FP32
 template <typename R>
 bool fft_convolve_lines(const FFTCube<R>& c, R* rho, typename Cplx<R>::T* work, const float* G, int64_t nbox,
                         R div3, R div1, hipStream_t s, KTimer* tm, const char* tag);

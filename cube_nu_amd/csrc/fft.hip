@@ -478,13 +478,21 @@ void fft_c2r3d(const FFTCube<R>& c, typename Cplx<R>::T* in, R* out, int64_t nbo
 }
 
 template <typename R>
+bool fft_reads_windows(int n) {
+  return std::is_same<R, float>::value && use_plane_path() && fft_plane_size(n);
+}
+template bool fft_reads_windows<float>(int);
+template bool fft_reads_windows<double>(int);
+
+template <typename R>
 void fft_convolve(const FFTCube<R>& c, R* rho, typename Cplx<R>::T* work, const float* G, int64_t nbox, R div3,
-                  R div1, hipStream_t s, KTimer* tm, const char* tag, bool small_lds) {
+                  R div1, hipStream_t s, KTimer* tm, const char* tag, bool small_lds, const FFTWindow* win) {
   using C = typename Cplx<R>::T;
   if (use_plane_path()) {
     KTimer* t = tm ? tm : &null_timer();
     // a plane of 88 points is the largest below 40 KB
-    if (!(small_lds && c.n > 88) && fft_convolve_plane<R>(c, rho, work, G, nbox, div3, div1, s, t, tag)) return;
+    if (!(small_lds && c.n > 88) && fft_convolve_plane<R>(c, rho, work, G, nbox, div3, div1, s, t, tag, win)) return;
+    if (win) throw Error(1, "FFT of " + std::to_string(c.n) + " points does not read windows");
     if (fft_convolve_lines<R>(c, rho, work, G, nbox, div3, div1, s, t, tag)) return;
   }
   const int n = c.n, h = n / 2;
@@ -524,9 +532,9 @@ void fft_convolve(const FFTCube<R>& c, R* rho, typename Cplx<R>::T* work, const 
 template struct FFTCube<float>;
 template struct FFTCube<double>;
 template void fft_convolve<float>(const FFTCube<float>&, float*, float2*, const float*, int64_t, float, float,
-                                  hipStream_t, KTimer*, const char*, bool);
+                                  hipStream_t, KTimer*, const char*, bool, const FFTWindow*);
 template void fft_convolve<double>(const FFTCube<double>&, double*, double2*, const float*, int64_t, double, double,
-                                   hipStream_t, KTimer*, const char*, bool);
+                                   hipStream_t, KTimer*, const char*, bool, const FFTWindow*);
 template void fft_r2c3d<float>(const FFTCube<float>&, const float*, float2*, int64_t, hipStream_t);
 template void fft_r2c3d<double>(const FFTCube<double>&, const double*, double2*, int64_t, hipStream_t);
 template void fft_c2r3d<float>(const FFTCube<float>&, float2*, float*, int64_t, hipStream_t);

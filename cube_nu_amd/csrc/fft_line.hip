@@ -128,15 +128,16 @@ __global__ void __launch_bounds__((LPlan<R, N>::NT)) k_line_c2r(const CP<R>* __r
   }
   bfly<+1, A2>(v);
   C* dst = reinterpret_cast<C*>(out + row * N);
+  const R inv = (R)1 / (div3 != (R)0 ? div3 : div1);
 #pragma unroll
   for (int k = 0; k < A2; ++k) {
     R a = v[k].x, b = v[k].y;
     if (div3 != (R)0) {
-      a = a / div3;
-      b = b / div3;
+      a = div_by(a, div3, inv);
+      b = div_by(b, div3, inv);
     } else {
-      a = ((a / div1) / div1) / div1;
-      b = ((b / div1) / div1) / div1;
+      a = div_by(div_by(div_by(a, div1, inv), div1, inv), div1, inv);
+      b = div_by(div_by(div_by(b, div1, inv), div1, inv), div1, inv);
     }
     dst[j + k * A1] = CT<C>::mk(a, b);
   }

@@ -46,6 +46,14 @@ __device__ inline C mi(C a) { return SIGN > 0 ? CT<C>::mk(-a.y, a.x) : CT<C>::mk
 template <int SIGN, typename C>
 __device__ inline C mulw(C a, C w) { return mul(a, SIGN > 0 ? cj(w) : w); }
 
+// a / d from inv = 1 / d: the product and one correction by the remainder, the
+// rounding of the division (3 operations instead of the 10 of an exact one).
+__device__ inline float div_by(float a, float d, float inv) {
+  const float q = a * inv;
+  return __builtin_fmaf(__builtin_fmaf(-q, d, a), inv, q);
+}
+__device__ inline double div_by(double a, double d, double) { return a / d; }
+
 // e^{2 pi i k/n} as compile-time values: the angle reduced to [0, pi/4] by
 // the octant symmetries, then the Taylor series.
 struct CS {

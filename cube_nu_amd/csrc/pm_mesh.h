@@ -20,9 +20,11 @@ void pm_mesh_deposit(int izipx, const MeshGeo& M, const void* xp, const int32_t*
 // The outermost layers of the windows: faces, 6 n^2 floats per box.
 void pm_mesh_faces(int izipx, const MeshGeo& M, const PMLevel& L, const PMBox* boxes_dev, int nbox, const void* xp,
                    const int32_t* rhoc, const int64_t* cell_off, float* faces, float mass, hipStream_t s);
-// The windows' densities, each at its box's moff of `out`.
-void pm_mesh_window(const MeshGeo& M, const PMLevel& L, const PMBox* boxes_dev, int nbox, const float* mesh,
-                    const float* faces, float* out, hipStream_t s);
+// A box's window in the image's mesh: its first point per axis, in [0, n).
+int4 mesh_origin(const MeshGeo& M, const PMLevel& L, const PMBox& B);
+// The windows (n points per dim, origins on the device) written out as cubes.
+void pm_mesh_window(const MeshGeo& M, int n, const int4* org_dev, int nbox, const float* mesh, const float* faces,
+                    float* out, hipStream_t s);
 // *bad = 1 unless every buffer cell holds the coordinates of the physical
 // cell it is the periodic image of, in the same order.
 void mesh_check_images(int izipx, const Geo& g, const void* xp, const int32_t* rhoc, const int64_t* cell_off,

@@ -20,19 +20,43 @@
 namespace cube {
 namespace {
 
+// The three encoded coordinates of particle ip, in two loads.
+template <int IZ>
+__device__ inline void load_xp(const XT<IZ>* __restrict__ xp, int64_t ip, uint32_t u[3]) {
+  const XT<IZ>* p = xp + 3 * ip;
+  if constexpr (IZ == 2) {
+    uint32_t xy;
+    __builtin_memcpy(&xy, p, 4);
+    u[0] = xy & 0xffffu;
+    u[1] = xy >> 16;
+    u[2] = (uint16_t)p[2];
+  } else {
+    uint16_t xy;
+    __builtin_memcpy(&xy, p, 2);
+    u[0] = xy & 0xffu;
+    u[1] = xy >> 8;
+    u[2] = (uint8_t)p[2];
+  }
+}
+
 // Mesh of the whole image: cell a covers [a, a+1) mesh units; a particle with
 // floor f deposits into f-1, f, f+1 with the weights of particle_mesh.f90:56-62.
 //
 // Workgroup = BD^3 cells [BD b - 1, BD b + BD - 2] per axis: with this offset
 // the contributors are the block's own coarse cells and one lower layer,
-// (BD/w + 1)^3 cells.  Their particles form one list (LDS prefix sum of the
-// counts) that the wavefronts share in 8 segments each; lane l reads particle
-// l/8, l/8 + 8, ... of segment l%8, so that the 64 lanes of a deposit come
-// from 8 places of the block: particles of one coarse cell share few mesh
-// cells, and their atomics would serialise (a microbenchmark of 64-bit LDS
-// adds: 18.5 CU cycles per wavefront from one 4^3-cell coarse cell, 13.2 from
-// several).  Hits (1.42 per particle at BD = 16) queue per wavefront and are
-// deposited 64 at a time into 2^-32 fixed-point sums.
+// (BD/w + 1)^3 cells; of a lower cell's particles those in the last two mesh
+// layers along each lower axis reach the block.  The cells' particles form one
+// list (LDS prefix sum of the counts) that the wavefronts share in 8 segments
+// each; lane l reads particle l/8, l/8 + 8, ... of segment l%8, so that the 64
+// lanes of a deposit come from 8 places of the block: particles of one coarse
+// cell share few mesh cells, and their atomics would serialise (a
+// microbenchmark of 64-bit LDS adds: 18.5 CU cycles per wavefront from one
+// 4^3-cell coarse cell, 13.2 from several).  Hits (1.42 per particle at BD =
+// 16) queue per wavefront and are deposited 64 at a time into 2^-32
+// fixed-point sums; rows are padded to BD + 1 cells, so that the 27 addresses
+// are one base and constant offsets and neighbouring rows start in other banks.
+// 512^3 particles: 2.6 ms at w = 4 (512^3 mesh), 4.5 at w = 8 (1024^3 mesh, 4.3
+// GB written); the deposit per window took 8.9 and 6.4 + 5.8 for its lists.
 template <int IZ, int BD>
 __global__ void __launch_bounds__(256) k_mesh_deposit(MeshGeo M, const XT<IZ>* __restrict__ xp,
                                                       const int32_t* __restrict__ rhoc,
@@ -40,67 +64,66 @@ __global__ void __launch_bounds__(256) k_mesh_deposit(MeshGeo M, const XT<IZ>* _
                                                       float mass) {
   constexpr int MAXC = (BD / 4 + 1) * (BD / 4 + 1) * (BD / 4 + 1);
   constexpr int NS = 32;  // list segments of a workgroup
-  __shared__ unsigned long long acc[BD * BD * BD];
+  constexpr int SY = BD + 1, SZ = BD * SY;
+  __shared__ unsigned long long acc[BD * SZ];
   __shared__ unsigned long long queue[4][128];
   __shared__ int cnt[MAXC], pre[MAXC + 1], wsum[4];
-  __shared__ int64_t gof[MAXC];
+  __shared__ uint32_t gof[MAXC];        // first particle of a cell (the caller holds np < 2^32)
+  __shared__ unsigned short key[MAXC];  // cell coordinates l (3 bits each), bit 9 + d: l_d == 0
   const int nb = M.n / BD, g = BD / M.w, gc = g + 1;
-  int64_t b = xcd_block(blockIdx.x, gridDim.x);
-  const int bi[3] = {(int)(b % nb), (int)((b / nb) % nb), (int)(b / ((int64_t)nb * nb))};
+  const int b = (int)xcd_block(blockIdx.x, gridDim.x);
+  const int bi[3] = {b % nb, (b / nb) % nb, b / (nb * nb)};
   const int nC = gc * gc * gc;
   for (int t = threadIdx.x; t < nC; t += 256) {
     const int l[3] = {t % gc, (t / gc) % gc, t / (gc * gc)};
-    int T = 0, c[3];
+    int T = 0, c[3], k = 0;
     for (int d = 2; d >= 0; --d) {
       int cc = bi[d] * g - 1 + l[d];
       cc = cc < 0 ? cc + M.nc : cc;
       const int it = cc / M.nt;
       c[d] = cc - it * M.nt + 1;
       T = T * M.nnt + it;
+      k |= (l[d] << (3 * d)) | (l[d] == 0 ? 512 << d : 0);
     }
     const int64_t cell = rc_index(c[0], c[1], c[2], T, M.nte, M.ncb);
     cnt[t] = rhoc[cell];
-    gof[t] = off[cell];
+    gof[t] = (uint32_t)off[cell];
+    key[t] = (unsigned short)k;
   }
-  for (int t = threadIdx.x; t < BD * BD * BD; t += 256) acc[t] = 0;
+  for (int t = threadIdx.x; t < BD * SZ; t += 256) acc[t] = 0;
   __syncthreads();
   block_scan(cnt, pre, nC, wsum);
   const int total = pre[nC];
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int sh = M.sh;
+  const int sh = M.sh, w = M.w;
   const float rsh = 1.0f / (float)(1u << sh);
-  const uint32_t fmask = (1u << sh) - 1u;
+  const uint32_t fmask = (1u << sh) - 1u, low = (uint32_t)(w - 2) << sh;  // a lower cell's last two layers
   unsigned long long* q = queue[wave];
-  // entry: block-local floor + 8 of each axis (5 bits, floors -w..BD-1) above the coordinates
   auto process = [&](int nq) {
     wave_sync_lds();
     if (lane < nq) {
       const unsigned long long e = q[lane];
+      const int k = (int)(e >> 48);
       int f[3];
-      float w[3][3];
+      float wt[3][3];
+      bool ok[3][3];
       for (int d = 0; d < 3; ++d) {
-        f[d] = (int)((e >> (48 + 5 * d)) & 31) - 8;
-        tsc_weights_frac<float>(((float)((uint32_t)(e >> (16 * d)) & fmask) + 0.5f) * rsh, w[d]);
+        const uint32_t u = (uint32_t)(e >> (16 * d)) & 0xffffu;
+        f[d] = w * (((k >> (3 * d)) & 7) - 1) + (int)(u >> sh);  // floor relative to BD b
+        tsc_weights_frac<float>(((float)(u & fmask) + 0.5f) * rsh, wt[d]);
+        for (int i = 0; i < 3; ++i) ok[d][i] = (unsigned)(f[d] + i) < (unsigned)BD;
       }
-      for (int i = 0; i < 3; ++i) w[2][i] *= kFixF;  // exact: a power of two
+      for (int i = 0; i < 3; ++i) wt[2][i] *= kFixF;  // exact: a power of two
+      unsigned long long* a = acc + (f[2] * SZ + f[1] * SY + f[0]);
 #pragma unroll
-      for (int i3 = 0; i3 < 3; ++i3) {
-        const int z = f[2] + i3;
-        if ((unsigned)z >= (unsigned)BD) continue;
+      for (int i3 = 0; i3 < 3; ++i3)
 #pragma unroll
-        for (int i2 = 0; i2 < 3; ++i2) {
-          const int y = f[1] + i2;
-          if ((unsigned)y >= (unsigned)BD) continue;
-          const int row = (z * BD + y) * BD, sw = (5 * y + 9 * z) & (BD - 1);
+        for (int i2 = 0; i2 < 3; ++i2)
 #pragma unroll
-          for (int i1 = 0; i1 < 3; ++i1) {
-            const int x = f[0] + i1;
-            if ((unsigned)x < (unsigned)BD)
-              atomicAdd(&acc[row + (x ^ sw)],
-                        (unsigned long long)__float2uint_rn((w[0][i1] * w[1][i2]) * w[2][i3]));
-          }
-        }
-      }
+          for (int i1 = 0; i1 < 3; ++i1)
+            if (ok[2][i3] && ok[1][i2] && ok[0][i1])
+              atomicAdd(&a[i3 * SZ + i2 * SY + i1],
+                        (unsigned long long)__float2uint_rn((wt[0][i1] * wt[1][i2]) * wt[2][i3]));
     }
     wave_sync_lds();
   };
@@ -112,29 +135,29 @@ __global__ void __launch_bounds__(256) k_mesh_deposit(MeshGeo M, const XT<IZ>* _
   constexpr int U = 4;
   while (__any(i < i1)) {
     uint32_t u[U][3];
-    int cl[U];
+    int kc[U];
     bool val[U];
 #pragma unroll
     for (int k = 0; k < U; ++k) {
       val[k] = i < i1;
-      while (val[k] && i >= pre[c + 1]) ++c;
-      cl[k] = c;
-      const int64_t ip = val[k] ? gof[c] + (i - pre[c]) : 0;
-      for (int d = 0; d < 3; ++d) u[k][d] = val[k] ? XP<IZ>::raw(xp, ip, d) : 0u;
+      kc[k] = 0;
+      u[k][0] = u[k][1] = u[k][2] = 0;
+      if (val[k]) {
+        while (i >= pre[c + 1]) ++c;
+        kc[k] = key[c];
+        load_xp<IZ>(xp, (int64_t)gof[c] + (i - pre[c]), u[k]);
+      }
       i += 8;
     }
 #pragma unroll
     for (int k = 0; k < U; ++k) {
-      const int l[3] = {cl[k] % gc, (cl[k] / gc) % gc, cl[k] / (gc * gc)};
-      bool hit = val[k];
-      unsigned long long e = 0;
-      for (int d = 0; d < 3; ++d) {
-        const int f = M.w * (l[d] - 1) + (int)(u[k][d] >> sh);  // floor relative to BD b
-        hit = hit && f >= -2;
-        e |= ((unsigned long long)u[k][d] << (16 * d)) | ((unsigned long long)((f + 8) & 31) << (48 + 5 * d));
-      }
+      const bool hit = val[k] && u[k][0] >= ((kc[k] & 512) ? low : 0u) && u[k][1] >= ((kc[k] & 1024) ? low : 0u) &&
+                       u[k][2] >= ((kc[k] & 2048) ? low : 0u);
       const unsigned long long m = __ballot(hit);
-      if (hit) q[qn + (int)__popcll(m & ((1ull << lane) - 1ull))] = e;
+      if (hit)
+        q[qn + (int)__popcll(m & ((1ull << lane) - 1ull))] =
+            ((unsigned long long)kc[k] << 48) | ((unsigned long long)u[k][2] << 32) |
+            (unsigned long long)((u[k][1] << 16) | u[k][0]);
       qn += (int)__popcll(m);
       if (qn >= 64) {
         process(64);
@@ -148,9 +171,8 @@ __global__ void __launch_bounds__(256) k_mesh_deposit(MeshGeo M, const XT<IZ>* _
   if (qn > 0) process(qn);
   __syncthreads();
   for (int t = threadIdx.x; t < BD * BD * BD; t += 256) {
-    const int lx = t % BD, ly = (t / BD) % BD, lz = t / (BD * BD);
-    const unsigned long long v = acc[(lz * BD + ly) * BD + (lx ^ ((5 * ly + 9 * lz) & (BD - 1)))];
-    const int l[3] = {lx, ly, lz};
+    const int l[3] = {t % BD, (t / BD) % BD, t / (BD * BD)};
+    const unsigned long long v = acc[l[2] * SZ + l[1] * SY + l[0]];
     int a[3];
     for (int d = 0; d < 3; ++d) {
       a[d] = bi[d] * BD - 1 + l[d];
@@ -172,8 +194,8 @@ __global__ void __launch_bounds__(256) k_mesh_faces(MeshGeo M, PMLevel L, const 
                                                     float mass) {
   extern __shared__ unsigned long long facc[];  // [rows][n]
   const int n = L.n, nr = n / M.w, nstrip = (n + rows - 1) / rows;
-  const int strip = (int)(blockIdx.x % nstrip), face = (int)((blockIdx.x / nstrip) % 6);
-  const int64_t box = blockIdx.x / ((int64_t)nstrip * 6);
+  const int strip = (int)(blockIdx.x % (unsigned)nstrip), face = (int)((blockIdx.x / (unsigned)nstrip) % 6);
+  const int64_t box = blockIdx.x / ((unsigned)nstrip * 6);
   const int ax = face >> 1, side = face & 1, au = ax == 0 ? 1 : 0, av = ax == 2 ? 1 : 2;
   const PMBox B = boxes[box];
   const int v0 = strip * rows, v1 = min(n, v0 + rows);  // rows [v0, v1)
@@ -227,36 +249,31 @@ __global__ void __launch_bounds__(256) k_mesh_faces(MeshGeo M, PMLevel L, const 
     out[t] = (float)((double)facc[t] * (1.0 / (double)kFixF)) * mass;
 }
 
-// The windows: one thread per four cells of a row (n is a multiple of w >= 4;
-// a row starts at a multiple of w of the image mesh, so four cells never
-// straddle its end).
-__global__ void __launch_bounds__(256) k_mesh_window(MeshGeo M, PMLevel L, const PMBox* __restrict__ boxes, int nbox,
+// The windows as cubes: one thread per four cells of a row (n is a multiple of
+// w >= 4; a row starts at a multiple of w of the image mesh, so four cells
+// never straddle its end), one workgroup row of the grid per z-plane.
+__global__ void __launch_bounds__(256) k_mesh_window(MeshGeo M, int n, const int4* __restrict__ org,
                                                      const float* __restrict__ mesh, const float* __restrict__ faces,
                                                      float* __restrict__ out) {
-  const int n = L.n, nq = n / 4;
-  const int64_t row = ((int64_t)blockIdx.x * 256 + threadIdx.x) / nq;  // box, z, y
-  const int x = (int)(((int64_t)blockIdx.x * 256 + threadIdx.x) % nq) * 4;
-  if (row >= (int64_t)nbox * n * n) return;
-  const int64_t box = row / ((int64_t)n * n);
-  const int y = (int)(row % n), z = (int)((row / n) % n);
-  const PMBox B = boxes[box];
+  const int nq = n / 4, t = blockIdx.y * 256 + threadIdx.x;
+  const int y = t / nq, x = (t - y * nq) * 4;
+  if (y >= n) return;
+  const int64_t box = blockIdx.x / (unsigned)n;
+  const int z = (int)(blockIdx.x % (unsigned)n);
   const float* fb = faces + 6 * box * n * n;
   float4 v;
   if (z == 0 || z == n - 1) v = *(const float4*)(fb + ((int64_t)(z == 0 ? 4 : 5) * n + y) * n + x);
   else if (y == 0 || y == n - 1) v = *(const float4*)(fb + ((int64_t)(y == 0 ? 2 : 3) * n + z) * n + x);
   else {
-    const int p[3] = {x, y, z};
+    const int4 o = org[box];
+    const int p[3] = {o.x + x, o.y + y, o.z + z};
     int a[3];
-    for (int d = 0; d < 3; ++d) {
-      const int T = d == 0 ? B.T % M.nnt : (d == 1 ? (B.T / M.nnt) % M.nnt : B.T / (M.nnt * M.nnt));
-      a[d] = (T * M.nt + B.nc1[d] - 1 - L.nloop) * M.w + p[d];
-      a[d] = a[d] < 0 ? a[d] + M.n : (a[d] >= M.n ? a[d] - M.n : a[d]);
-    }
+    for (int d = 0; d < 3; ++d) a[d] = p[d] >= M.n ? p[d] - M.n : p[d];
     v = *(const float4*)(mesh + ((int64_t)a[2] * M.n + a[1]) * M.n + a[0]);
     if (x == 0) v.x = fb[(int64_t)z * n + y];
     if (x == n - 4) v.w = fb[((int64_t)n + z) * n + y];
   }
-  *(float4*)(out + B.moff + ((int64_t)z * n + y) * n + x) = v;
+  *(float4*)(out + ((box * n + z) * n + y) * n + x) = v;
 }
 
 // Buffer cells as periodic images of the physical ones (counts and encoded
@@ -306,7 +323,7 @@ MeshGeo mesh_geo(const Geo& g, int w, int bits) {
 
 bool pm_mesh_applies(const Geo& g, const PMLevel& L) {
   return !L.periodic && !L.xdiv && (L.w == 4 || L.w == 8) && L.nforce % L.w == 0 && L.win_lo == 1 - L.nloop * L.w &&
-         L.win_hi == L.nforce + L.nloop * L.w && L.n == L.nforce + 2 * L.nloop * L.w && (g.nc * L.w) % 8 == 0 && L.nloop <= g.nc &&
+         L.win_hi == L.nforce + L.nloop * L.w && L.n == L.nforce + 2 * L.nloop * L.w && (g.nc * L.w) % 8 == 0 && L.n <= g.nc * L.w &&
          L.nloop <= g.ncb;
 }
 
@@ -343,11 +360,17 @@ void pm_mesh_faces(int izipx, const MeshGeo& M, const PMLevel& L, const PMBox* b
   CUBE_HIP(hipGetLastError());
 }
 
-void pm_mesh_window(const MeshGeo& M, const PMLevel& L, const PMBox* boxes, int nbox, const float* mesh,
-                    const float* faces, float* out, hipStream_t s) {
-  const int64_t nthr = (int64_t)nbox * L.n * L.n * (L.n / 4);
-  hipLaunchKernelGGL(k_mesh_window, dim3((unsigned)ceil_div(nthr, 256)), dim3(256), 0, s, M, L, boxes, nbox, mesh,
-                     faces, out);
+int4 mesh_origin(const MeshGeo& M, const PMLevel& L, const PMBox& B) {
+  const int it[3] = {B.T % M.nnt, (B.T / M.nnt) % M.nnt, B.T / (M.nnt * M.nnt)};
+  int a[3];
+  for (int d = 0; d < 3; ++d) a[d] = (((it[d] * M.nt + B.nc1[d] - 1 - L.nloop) * M.w) % M.n + M.n) % M.n;
+  return make_int4(a[0], a[1], a[2], 0);
+}
+
+void pm_mesh_window(const MeshGeo& M, int n, const int4* org, int nbox, const float* mesh, const float* faces,
+                    float* out, hipStream_t s) {
+  hipLaunchKernelGGL(k_mesh_window, dim3((unsigned)(nbox * n), (unsigned)ceil_div(n * (n / 4), 256)), dim3(256), 0, s,
+                     M, n, org, mesh, faces, out);
   CUBE_HIP(hipGetLastError());
 }
 
