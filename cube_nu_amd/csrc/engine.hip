@@ -80,7 +80,7 @@ inline uint64_t fbits(float f) {
 __global__ void k_set_f64(double* p, double v) { *p = v; }
 
 // Candidates of each tuned choice, in order of preference.
-const std::vector<int> kTunePPDepth = {6, 4, 8, kPPBrick8 + 6, kPPBrick8 + 4, kPPBrick8 + 8};
+const std::vector<int> kTunePPDepth = {3, 2, 4};
 const std::vector<int> kTuneDepListThreads = {512, 256, 1024};
 const std::vector<int> kTuneInterpShape = {0, 1, 2};
 
@@ -656,7 +656,7 @@ void cube_p3m_ctx::pp_phase(const std::vector<int32_t>& ires_h, const std::vecto
       S.start = lppstart[iapm].ensure((size_t)(nb * m3 + 1));
       S.scan_tmp = scan_scratch(nb * m3);
       S.scan_tmp_bytes = scan_tmp.n;
-      S.claim = ppclaim.ensure(8);  // the force kernel's work-queue counters
+      S.claim = ppclaim.ensure(kPPClaimCounters * kPPClaimStride);  // the force kernel's work-queue counters
       int64_t total = 0;
       if (SZ) {
         CUBE_HIP(hipMemcpyAsync(boxes.p, bx.data() + b0, sizeof(PPBox) * nb, hipMemcpyHostToDevice, s));
@@ -676,14 +676,14 @@ void cube_p3m_ctx::pp_phase(const std::vector<int32_t>& ires_h, const std::vecto
         }
       }
       S.entries = lppent[iapm].p;
-      const int unroll = prec == 32 ? tune_pp(iapm, L, boxes.p, nb, S) : 6;
+      const int unroll = prec == 32 ? tune_pp(iapm, L, boxes.p, nb, S) : 3;
       if (SZ)
         sig_add({(uint64_t)iapm, (uint64_t)nb, (uint64_t)(uintptr_t)boxes.p, (uint64_t)(uintptr_t)S.start,
                  (uint64_t)(uintptr_t)S.entries, (uint64_t)(uintptr_t)S.claim, (uint64_t)unroll,
                  fbits(mass_scale)});
       if (CP) {
         KScope k(&tm, "pp_force", (double)total * 16);
-        pp_force(L, prec, boxes.p, nb, vpc(), S, o, s, unroll);
+        pp_force(L, prec, boxes.p, nb, off.p, vpc(), S, o, s, unroll);
       }
     }
   }
@@ -778,10 +778,10 @@ int cube_p3m_ctx::interp_shape(int level, int n, const PMLevel& L, const PMBox* 
 
 // PP load depth (candidates in flight per lane), tuned per PP level on the
 // level's first batch.  The trials run on a scratch copy of the velocities and
-// of the outputs.  The preference order 6, 4, 8 keeps the middle depth unless
-// another is more than 1% faster (a deeper one holds more registers, which the
-// kernel's 64-VGPR bound turns into spill traffic).  All depths sum the pairs
-// in the same order, so the choice changes the time of the step only.
+// of the outputs.  The preference order 3, 2, 4 keeps the middle depth unless
+// another is more than 1% faster (a deeper one wastes more reads past the ends
+// of runs, a shallower one walks more often).  All depths sum the pairs in the
+// same order, so the choice changes the time of the step only.
 int cube_p3m_ctx::tune_pp(int iapm, const PPLevel& L, const PPBox* boxes, int nb, PPScratch& S) {
   vtune.ensure((size_t)std::max<int64_t>(np, 1) * 3);
   otune.ensure(1);
@@ -790,7 +790,7 @@ int cube_p3m_ctx::tune_pp(int iapm, const PPLevel& L, const PPBox* boxes, int nb
       [&](int u) {
         CUBE_HIP(hipMemcpyAsync(vtune.p, vpc(), sizeof(float) * 3 * (size_t)np, hipMemcpyDeviceToDevice, s));
         zero_async(otune.p, sizeof(PPOut), s);
-        pp_force(L, 32, boxes, nb, vtune.p, S, otune.p, s, u);
+        pp_force(L, 32, boxes, nb, off.p, vtune.p, S, otune.p, s, u);
       },
       vtune.p, sizeof(float) * 3 * (size_t)np);
 }
@@ -1135,19 +1135,13 @@ void cube_p3m_ctx::kick(const cube_kick_in& in, cube_kick_out& out, float* densi
   CUBE_HIP(hipMemcpyAsync(po, pmout.p, sizeof(PMOut) * 4, hipMemcpyDeviceToHost, s));
   CUBE_HIP(hipMemcpyAsync(&pq, ppout.p, sizeof(PPOut), hipMemcpyDeviceToHost, s));
   CUBE_HIP(hipStreamSynchronize(s));
-  auto f2 = [&](const PMOut& p) { return std::is_same<R, float>::value ? p.f2max : (float)p.f2max_d; };
-  auto vm = [&](const PMOut& p, int d) { return std::is_same<R, float>::value ? p.vmax[d] : (float)p.vmax_d[d]; };
+  auto f2 = [&](const PMOut& p) { return p.template f2max<R>(); };
+  auto vm = [&](const PMOut& p, int d) { return p.template vmax<R>(d); };
   float vmax[3] = {0, 0, 0};
   if (mask & 1) {
     out.f2max_pm1 = f2(po[0]);
     out.dt_pm1 = dt_from_f2(0.5f, out.f2max_pm1, (float)in.a_mid);
-    unsigned long long tfx = 0;
-    double td = 0;
-    for (int q = 0; q < kSumSlots; ++q) {
-      tfx += po[0].testrho_fx[q];
-      td += po[0].testrho_d[q];
-    }
-    out.testrho = std::is_same<R, float>::value ? (double)tfx / 4294967296.0 : td;
+    out.testrho = po[0].template testrho<R>();
     for (int d = 0; d < 3; ++d) vmax[d] = vm(po[0], d);
   }
   if (mask & 2) {
@@ -1161,14 +1155,15 @@ void cube_p3m_ctx::kick(const cube_kick_in& in, cube_kick_out& out, float* densi
     for (int d = 0; d < 3; ++d) vmax[d] = vm(po[2], d);
   }
   if ((mask & 8) && cfg.pp) {
-    out.f2max_pp = pq.f2max;
-    out.dt_pp = dt_from_f2(0.05f, pq.f2max, (float)in.a_mid);
-    for (int d = 0; d < 3; ++d) vmax[d] = pq.vmax[d];
     unsigned long long npp = 0, npg = 0;
-    for (int q = 0; q < kSumSlots; ++q) {
-      npp += pq.pairs_pp[q];
-      npg += pq.pairs_pg[q];
+    for (int d = 0; d < 3; ++d) vmax[d] = 0;
+    for (const PPOut::Slot& q : pq.slot) {
+      out.f2max_pp = std::max(out.f2max_pp, q.f2max);
+      for (int d = 0; d < 3; ++d) vmax[d] = std::max(vmax[d], q.vmax[d]);
+      npp += q.pairs_pp;
+      npg += q.pairs_pg;
     }
+    out.dt_pp = dt_from_f2(0.05f, out.f2max_pp, (float)in.a_mid);
     last_pairs = (int64_t)(npp / 2 + npg);
   }
   for (int d = 0; d < 3; ++d) out.vmax[d] = vmax[d];
@@ -1447,28 +1442,20 @@ static void nu_outputs(cube_p3m_ctx* ctx, cube_p3m_ctx* nu, const cube_kick_in& 
   PMOut pn[4];
   CUBE_HIP(hipMemcpyAsync(pn, nu->pmout.p, sizeof(PMOut) * 4, hipMemcpyDeviceToHost, ctx->s));
   CUBE_HIP(hipStreamSynchronize(ctx->s));
-  const bool f = std::is_same<R, float>::value;
-  auto f2 = [&](const PMOut& p) { return f ? p.f2max : (float)p.f2max_d; };
   float vmax[3] = {0, 0, 0};
   for (int lv = 0; lv < 2; ++lv) {
     if (!(mask & (1 << lv))) continue;
     const PMOut& p = pn[lv];
-    const float q = f2(p);
+    const float q = p.template f2max<R>();
     if (lv == 0) {
       o.f2max_pm1 = q;
       o.dt_pm1 = dt_from_f2(0.5f, q, (float)in.a_mid);
-      unsigned long long tfx = 0;
-      double td = 0;
-      for (int k = 0; k < kSumSlots; ++k) {
-        tfx += p.testrho_fx[k];
-        td += p.testrho_d[k];
-      }
-      o.testrho = f ? (double)tfx / 4294967296.0 : td;
+      o.testrho = p.template testrho<R>();
     } else {
       o.f2max_pm2 = q;
       o.dt_pm2 = dt_from_f2(0.5f, q, (float)in.a_mid);
     }
-    for (int d = 0; d < 3; ++d) vmax[d] = f ? p.vmax[d] : (float)p.vmax_d[d];
+    for (int d = 0; d < 3; ++d) vmax[d] = p.template vmax<R>(d);
   }
   for (int d = 0; d < 3; ++d) o.vmax[d] = vmax[d];
   o.dt_vmax = (0.9f * 14.0f) / std::max({vmax[0], vmax[1], vmax[2]});

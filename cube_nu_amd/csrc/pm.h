@@ -2,6 +2,9 @@
 // (sub-tile) levels: TSC deposit, fused gradient + interpolation + kick,
 // Green's function generation and sub-tile classification.
 #pragma once
+#include <algorithm>
+#include <type_traits>
+
 #include "common.h"
 
 namespace cube {
@@ -36,13 +39,41 @@ struct PMBox {
   int64_t moff;      // element offset of this box's mesh array
 };
 
-struct PMOut {  // device-side reductions of one level
-  float f2max;
-  float vmax[3];
-  double f2max_d;
-  double vmax_d[3];
-  unsigned long long testrho_fx[kSumSlots];  // PM1 density sum in 2^-32 fixed point
-  double testrho_d[kSumSlots];
+// Reductions of one level: maxima and the PM1 density sum, spread over slots
+// (by workgroup) on cache lines of their own, so that the workgroups of a short
+// launch, which all end at once, do not queue on one address; the host reduces
+// the slots.  Only the fields of the form in use are written.
+struct PMOut {
+  struct alignas(128) Slot {
+    float f2max, vmax[3];
+    double f2max_d, vmax_d[3];
+    unsigned long long testrho_fx;  // PM1 density sum in 2^-32 fixed point
+    double testrho_d;
+  } slot[kSumSlots];
+
+  // the maxima of the FP32 (R = float) or FP64 form
+  template <typename R>
+  float f2max() const {
+    R m = 0;
+    for (const Slot& q : slot) m = std::max(m, std::is_same<R, float>::value ? (R)q.f2max : (R)q.f2max_d);
+    return (float)m;
+  }
+  template <typename R>
+  float vmax(int d) const {
+    R m = 0;
+    for (const Slot& q : slot) m = std::max(m, std::is_same<R, float>::value ? (R)q.vmax[d] : (R)q.vmax_d[d]);
+    return (float)m;
+  }
+  template <typename R>
+  double testrho() const {
+    unsigned long long fx = 0;
+    double sum = 0;
+    for (const Slot& q : slot) {
+      fx += q.testrho_fx;
+      sum += q.testrho_d;
+    }
+    return std::is_same<R, float>::value ? (double)fx / 4294967296.0 : sum;
+  }
 };
 
 // Tile/sub-tile (fine) level deposit into each box's mesh.

@@ -531,23 +531,25 @@ __global__ void __launch_bounds__(256) k_pm1_gather(PMLevel L, const void* __res
   if (threadIdx.x == 0) {
     Acc s = 0;
     for (int q = 0; q < (int)(blockDim.x >> 6); ++q) s += red[q];
-    if constexpr (std::is_same<R, float>::value) atomicAdd(&out->testrho_fx[blockIdx.x % kSumSlots], s);
-    else atomicAdd(&out->testrho_d[blockIdx.x % kSumSlots], s);
+    if constexpr (std::is_same<R, float>::value) atomicAdd(&out->slot[blockIdx.x % kSumSlots].testrho_fx, s);
+    else atomicAdd(&out->slot[blockIdx.x % kSumSlots].testrho_d, s);
   }
 }
 
-// Raises the level's maxima to this wavefront's.  A running maximum saturates
+// Raises the workgroup's slot of the level's maxima to this wavefront's.  A
+// running maximum saturates
 // after a few workgroups, so nearly every wavefront compares and is done; the
 // others reduce across lanes first (one atomic per wavefront).
 template <typename R>
 __device__ inline void raise_maxima(R f2, const R vm[3], PMOut* __restrict__ out) {
+  PMOut::Slot& sl = out->slot[blockIdx.x % kSumSlots];
   R* at[4];
   if constexpr (std::is_same<R, float>::value) {
-    at[0] = &out->f2max;
-    for (int d = 0; d < 3; ++d) at[1 + d] = &out->vmax[d];
+    at[0] = &sl.f2max;
+    for (int d = 0; d < 3; ++d) at[1 + d] = &sl.vmax[d];
   } else {
-    at[0] = &out->f2max_d;
-    for (int d = 0; d < 3; ++d) at[1 + d] = &out->vmax_d[d];
+    at[0] = &sl.f2max_d;
+    for (int d = 0; d < 3; ++d) at[1 + d] = &sl.vmax_d[d];
   }
   const R v[4] = {f2, vm[0], vm[1], vm[2]};
   R now[4];
@@ -560,12 +562,10 @@ __device__ inline void raise_maxima(R f2, const R vm[3], PMOut* __restrict__ out
   }
 }
 
-// PM1 at 512^3: 2.3 -> 1.35 ms with this gather.
-//
 // The 27-point gather of the three force arrays (FN values each, rows of FX,
 // planes of FX FY) at base cell li: sums along x, then y, then z with fused
 // multiply-adds, 39 operations per component instead of 108 for the 27
-// products of three weights (and fewer roundings).
+// products of three weights (and fewer roundings); PM1 at 512^3: 2.3 -> 1.35 ms.
 template <typename R>
 __device__ inline void tsc_gather(const R* __restrict__ F, int FN, int FX, int FXY, int li, const R w[3][3], R dv[3]) {
 #pragma unroll

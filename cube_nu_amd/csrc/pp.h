@@ -31,12 +31,17 @@ struct PPBox {
   int ifs[3];      // 0-based sub-tile coordinates within the tile
 };
 
+// Reductions of the pair forces, in slots as PMOut's.
 struct PPOut {
-  float f2max;
-  float vmax[3];
-  unsigned long long pairs_pp[kSumSlots];  // directed physical-physical pair count
-  unsigned long long pairs_pg[kSumSlots];  // physical-ghost pair count
+  struct alignas(128) Slot {
+    float f2max, vmax[3];
+    unsigned long long pairs_pp;  // directed physical-physical pair count
+    unsigned long long pairs_pg;  // physical-ghost pair count
+  } slot[kSumSlots];
 };
+
+// Work-queue counters of the force kernels, a cache line (32 words) apart.
+constexpr int kPPClaimCounters = 8, kPPClaimStride = 32;
 
 // Scratch the caller provides for one level batch.
 struct PPScratch {
@@ -44,7 +49,7 @@ struct PPScratch {
   int64_t* start = nullptr;   // nbox * m^3 * kSX + 1
   float4* entries = nullptr;  // capacity entries + kPPPad readable padding
   int64_t capacity = 0;
-  unsigned* claim = nullptr;  // 8 work-queue counters of the force kernel
+  unsigned* claim = nullptr;  // kPPClaimCounters * kPPClaimStride words
   void* scan_tmp = nullptr;
   size_t scan_tmp_bytes = 0;
 };
@@ -55,12 +60,11 @@ int64_t pp_bin_count(int izipx, const PPLevel& L, const PPBox* boxes_dev, int nb
                      const int32_t* rhoc, const int64_t* cell_off, PPScratch& S, hipStream_t s);
 void pp_bin_fill(int izipx, const PPLevel& L, const PPBox* boxes_dev, int nbox, const void* xp, const int32_t* rhoc,
                  const int64_t* cell_off, PPScratch& S, hipStream_t s);
-// unroll: candidate loads in flight per lane in the FP32 kernel (4, 6 or 8),
-// plus kPPBrick8 for bricks of 8^3 PP cells instead of 4^3; every value gives
-// the same result.
-constexpr int kPPBrick8 = 100;
-void pp_force(const PPLevel& L, int precision, const PPBox* boxes_dev, int nbox, float* vp, PPScratch& S, PPOut* out,
-              hipStream_t s, int unroll = 6);
+// cell_off: the extended cells' offsets (entries hold the particle's index
+// within its tile).  unroll: candidate loads in flight per lane in the FP32
+// kernel, 2, 3 or 4; the partial sums' order depends on it.
+void pp_force(const PPLevel& L, int precision, const PPBox* boxes_dev, int nbox, const int64_t* cell_off, float* vp,
+              PPScratch& S, PPOut* out, hipStream_t s, int unroll = 3);
 
 // Entries past the last one that the force kernel may read (and ignore).
 constexpr int kPPPad = 16;

@@ -6,9 +6,9 @@
 // atomics, and the in-cell order is the reference's (coarse-cell particle
 // order).
 //
-// Force: a persistent kernel whose workgroups claim bricks of PB^3 physical
-// PP cells from a work queue; each thread owns target particles and sums the
-// pair force from the 27 neighbouring PP cells in a fixed order.  Both
+// Force: a persistent kernel whose workgroups claim bricks of 4^3 physical PP
+// cells from a work queue; each pair of lanes owns a target particle and sums
+// the pair force from the 27 neighbouring PP cells in a fixed order.  Both
 // members of a physical pair evaluate the pair, so no cross-thread
 // accumulation is needed and the result is deterministic.
 // The in-range test uses the reference's FP32 operations on exact FP32
@@ -71,7 +71,7 @@ __global__ void __launch_bounds__(256) k_pp_bin(PPLevel L, const PPBox* __restri
                     B.ifs[2] * L.ntt + qc / (nr * nr)};  // nc1-1 + offset (Fortran nc1 = ifs*ntt+1)
   const int64_t cell = rc_index(c[0], c[1], c[2], B.T, L.nte, L.ncb);
   const int cnt = rhoc[cell];
-  const int64_t base = off[cell];
+  const int64_t base = off[cell], tile = off[(int64_t)B.T * L.nte * L.nte * L.nte];
   const int m = L.npgrid + 2;
   const int sf = L.sf, nsb = sf * sf * sf * kSX;
   const int kbits = 32 - __clz(nsb - 1);  // bits of a sub-bin key
@@ -102,8 +102,12 @@ __global__ void __launch_bounds__(256) k_pp_bin(PPLevel L, const PPBox* __restri
       const int rank = (int)__popcll(eq & lt);
       if (FILL) {
         const int64_t pc = cbase + ((int64_t)idx[2] * m + idx[1]) * m + idx[0];
-        ent[start[pc * kSX + q] + prev + rank] =
-            make_float4(xf[0], xf[1], xf[2], __uint_as_float((unsigned)(base + l)));
+        bool ghost = false;
+        for (int d = 0; d < 3; ++d) ghost = ghost || idx[d] == 0 || idx[d] == L.npgrid + 1;
+        // particle index within its tile, ghosts of the sub-tile marked by the sign
+        ent[start[pc * kSX + q] + prev + rank] = make_float4(
+            xf[0], xf[1], xf[2],
+            __uint_as_float((unsigned)(base + l - tile) | (ghost ? 0x80000000u : 0u)));
       }
     }
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -125,107 +129,71 @@ __global__ void __launch_bounds__(256) k_pp_bin(PPLevel L, const PPBox* __restri
   }
 }
 
-// Physical PP cells per brick per dim: PB = 4 or 8, chosen with the load
-// depth by the engine's autotuner (a target's sums do not depend on the
-// brick it is in, so neither choice changes a result).
+// Physical PP cells per brick per dim.
+constexpr int kPB = 4;
 // Lanes per target in the FP32 force kernel: a target's candidates are dealt
-// to kPPGroup lanes in turn and their partial sums combined at the end (26.1
-// ms at 512^3 against 27.3 with one lane per target, 27.2 with four, 31.5
-// with eight: pairs of lanes read consecutive entries and wait less on the
-// longest column of the wavefront).
+// to kPPGroup lanes in turn and their partial sums combined at the end (pairs
+// of lanes read consecutive entries).
 constexpr int kPPGroup = 2;
-// Candidate loads in flight per lane: U in {4, 6, 8}, chosen per PP level at
-// run time by the engine's autotuner (every U sums the pairs in the same
-// order, so the choice never changes a result).
 
+// FP32 pair law.  F(r, app) - F(r, r_pp) along the pair, divided by r: for r >
+// app it is 1/r^3 - c Q(ep)/r with ep = 2r/r_pp < 2 and Q the two polynomials of
+// F_ra (kick.f90:360-374; Q = 12/ep^2 + po(ep) above ep = 1).  Q(ep)/ep comes
+// from a cubic Hermite table over kQSeg segments of s = ep^2 in [0, 4], kept in
+// LDS: in r^2 it needs neither r nor a square root of its own.  ep = 1 is a
+// segment edge and the function is C^1 there.  Interpolation error: below 2e-6
+// of values up to 224 beyond the first segments (h^4 max|y^(4)|/384, h = 1/32);
+// in the first, where s^(3/2) is not smooth, 0.012, which is below 5e-7 of the
+// pair's force (1/r^3 dominates there): the level of FP32 rounding.
+constexpr int kQSeg = 128;
 
-// F(r, r_pp) = c Q(ep), ep = 2r/r_pp < 2, with Q(ep) = pi(ep) for ep <= 1 and
-// 12/ep^2 + po(ep) above (the two polynomials of F_ra, kick.f90:360-374).
-// The FP32 force takes Q from a cubic Hermite table over kQSeg segments of
-// [0, 2] kept in LDS: ep = 1 is a segment edge and Q is C^1 there, so every
-// segment interpolates one smooth branch; the table's error is below 2e-5 on
-// |Q| <= 104 (h^4 max|Q^(4)| / 384 with h = 1/32), i.e. below 1e-6 of
-// 1/r_pp^2 in the pair force, at the level of FP32 rounding.
-constexpr int kQSeg = 64;
-
-__device__ inline void q_branch(double e, bool outer, double& q, double& dq) {
+__device__ inline void q_over_ep(double s, bool outer, double& y, double& dy) {
+  const double e = sqrt(s);
   if (outer) {
-    q = 12.0 / (e * e) + (((((7.0 * e - 48.0) * e + 70.0) * e + 224.0) * e - 840.0) * e + 896.0) * e - 224.0;
-    dq = -24.0 / (e * e * e) + ((((42.0 * e - 240.0) * e + 280.0) * e + 672.0) * e - 1680.0) * e + 896.0;
+    y = 12.0 / (e * e * e) - 224.0 / e + ((((7.0 * e - 48.0) * e + 70.0) * e + 224.0) * e - 840.0) * e + 896.0;
+    dy = (-36.0 / (e * e * e * e) + 224.0 / (e * e) + (((35.0 * e - 192.0) * e + 210.0) * e + 448.0) * e - 840.0) /
+         (2.0 * e);
   } else {
-    q = e * (224.0 + e * e * (-224.0 + e * (70.0 + e * (48.0 - 21.0 * e))));
-    dq = 224.0 + e * e * (-672.0 + e * (280.0 + e * (240.0 - 126.0 * e)));
+    y = 224.0 + s * (-224.0 + e * (70.0 + e * (48.0 - 21.0 * e)));
+    dy = -224.0 + e * (105.0 + e * (96.0 - 52.5 * e));
   }
 }
 
-// Segment s of the table: Q(s h + f h) = ((c.w f + c.z) f + c.y) f + c.x.
-__device__ inline void fill_qtab(float4* tab) {
-  for (int sg = threadIdx.x; sg < kQSeg; sg += blockDim.x) {
-    const double h = 2.0 / kQSeg;
-    const bool outer = sg >= kQSeg / 2;
+// Segment i of the table: scale * y(i h + f h) = ((c.w f + c.z) f + c.y) f + c.x;
+// entry kQSeg holds the end value (an r^2 just below the range may round to it).
+__device__ inline void fill_qtab(float4* tab, double scale) {
+  for (int i = threadIdx.x; i <= kQSeg; i += blockDim.x) {
+    const double h = 4.0 / kQSeg;
+    const bool outer = i >= kQSeg / 4;
     double y0, d0, y1, d1;
-    q_branch(sg * h, outer, y0, d0);
-    q_branch((sg + 1) * h, outer, y1, d1);
-    d0 *= h;
-    d1 *= h;
-    tab[sg] = make_float4((float)y0, (float)d0, (float)(3.0 * (y1 - y0) - 2.0 * d0 - d1),
-                          (float)(2.0 * (y0 - y1) + d0 + d1));
+    q_over_ep(i * h, outer, y0, d0);
+    q_over_ep((i + 1) * h, outer, y1, d1);
+    y0 *= scale;
+    y1 *= scale;
+    d0 *= h * scale;
+    d1 *= h * scale;
+    tab[i] = i == kQSeg ? make_float4((float)y0, 0.0f, 0.0f, 0.0f)
+                        : make_float4((float)y0, (float)d0, (float)(3.0 * (y1 - y0) - 2.0 * d0 - d1),
+                                      (float)(2.0 * (y0 - y1) + d0 + d1));
   }
 }
 
-// FP32 pair law from the table: F(r, app) - F(r, r_pp) = 1/r^2 - c Q(ep) for
-// r > app; the rare r <= app pair takes F(r, app) in full.
-__device__ inline float pair_law_tab(const PPLevel& L, const float4* qtab, float r2, float& rinv_out) {
-  const float rinv = __builtin_amdgcn_rsqf(r2);
-  const float r = r2 * rinv;
-  const float t = r * (L.two_inv_range * (0.5f * kQSeg));
-  const int i = min((int)t, kQSeg - 1);
-  const float f = t - (float)i;
-  const float4 c = qtab[i];
-  const float q = fmaf(fmaf(fmaf(c.w, f, c.z), f, c.y), f, c.x);
-  float s = fmaf(-L.c_range, q, rinv * rinv);
-  if (r2 <= L.app2) {  // ep(r, app) <= 2
-    const float ea = (2.0f * r) * L.inv_app;
-    const float a2 = ea * ea;
-    const float fa =
-        ea > 1.0f
-            ? L.c_app * (12.0f * __builtin_amdgcn_rcpf(a2) +
-                         fmaf(ea, fmaf(ea, fmaf(ea, fmaf(ea, fmaf(ea, fmaf(ea, 7.0f, -48.0f), 70.0f), 224.0f),
-                                                -840.0f),
-                                       896.0f),
-                              -224.0f))
-            : L.c_app * ea * fmaf(a2, fmaf(ea, fmaf(ea, fmaf(ea, -21.0f, 48.0f), 70.0f), -224.0f), 224.0f);
-    s = fmaf(-L.c_range, q, fa);
-  }
-  rinv_out = rinv;
-  return s;
+// F(r, app) in full for the rare r <= app (ep <= 2), times c.
+__device__ inline float f_app(const PPLevel& L, float r) {
+  const float ea = (2.0f * r) * L.inv_app;
+  const float a2 = ea * ea;
+  return ea > 1.0f
+             ? L.c_app * (12.0f * __builtin_amdgcn_rcpf(a2) +
+                          fmaf(ea, fmaf(ea, fmaf(ea, fmaf(ea, fmaf(ea, fmaf(ea, 7.0f, -48.0f), 70.0f), 224.0f),
+                                                 -840.0f),
+                                        896.0f),
+                               -224.0f))
+             : L.c_app * ea * fmaf(a2, fmaf(ea, fmaf(ea, fmaf(ea, -21.0f, 48.0f), 70.0f), -224.0f), 224.0f);
 }
 
-// Pair force of candidate o on target me (kick.f90:523-530, 554-560):
+// FP64 form: the reference's operations (kick.f90:523-530, 554-560) in FP64:
 // f1 += (x2-x1)/r * (F(r,app) - F(r,r_pp)).
-// FP32 form: r^-1 from the hardware reciprocal square root, F(r, app) = 1/r^2
-// (r > app) and F(r, r_pp) from the LDS table (pair_law_tab); the error of a
-// pair term stays at the level of FP32 rounding.  FP64 form: the reference's
-// operations in FP64.
-template <typename R>
-__device__ inline void pair_force(const PPLevel& L, const float4* qtab, const float4 me, const float4 o, R f1[3]);
-
-template <>
-__device__ inline void pair_force<float>(const PPLevel& L, const float4* qtab, const float4 me, const float4 o,
-                                         float f1[3]) {
-  const float rv0 = o.x - me.x, rv1 = o.y - me.y, rv2 = o.z - me.z;
-  const float r2 = (rv0 * rv0 + rv1 * rv1) + rv2 * rv2;
-  float rinv;
-  const float s = pair_law_tab(L, qtab, r2, rinv);
-  const float sc = rinv * s;
-  f1[0] = fmaf(rv0, sc, f1[0]);
-  f1[1] = fmaf(rv1, sc, f1[1]);
-  f1[2] = fmaf(rv2, sc, f1[2]);
-}
-
-template <>
-__device__ inline void pair_force<double>(const PPLevel& L, const float4*, const float4 me, const float4 o,
-                                          double f1[3]) {
+__device__ inline void pair_force64(const PPLevel& L, const float4 me, const float4 o, double f1[3]) {
   const double rv0 = (double)o.x - me.x, rv1 = (double)o.y - me.y, rv2 = (double)o.z - me.z;
   const double r2 = (rv0 * rv0 + rv1 * rv1) + rv2 * rv2;
   const double r = sqrt(r2);
@@ -236,250 +204,350 @@ __device__ inline void pair_force<double>(const PPLevel& L, const float4*, const
   f1[2] = f1[2] + (rv2 / r) * fr;
 }
 
-// Persistent: each workgroup claims bricks of PB^3 physical PP cells from one
-// of kPPClaimCounters counters (workgroup i uses counter i % 8, which hands
-// out the bricks of sub-tiles i % 8, i % 8 + 8, ..., one sub-tile at a time,
-// so that a sub-tile's bricks run on one XCD and share its L2; with fewer
-// than 64 sub-tiles in a launch, bricks 8c + i % 8, so that every counter has
-// work) until they run out.  The host orders the boxes
-// densest sub-tile first (kick.f90:132-138 sorts by npc_max for
-// schedule(dynamic,1), kick.f90:285), so every counter drains the heaviest
-// bricks first and the launch does not end on a few heavy workgroups.  In a
-// brick each group of G lanes owns a target particle and sums the pair forces
-// of the 27 neighbouring PP cells in the fixed (dz, dy, x) order, lane j of
-// the group taking candidates j, j + G, ... of each run; the G partial sums
-// are added by a fixed butterfly, so the result is deterministic.  PP cells
-// are split into kSX sub-bins along x and
-// the CSR is x-ordered along each (y, z) row, so the part of a (dy, dz)
-// column that can hold partners, x within x_t +- sqrt(r_pp^2 - e^2) for the
-// column's nearest y/z distance e from the target, is one contiguous run
-// found from two sub-bin starts; columns with e > r_pp are skipped.  Both windows carry a margin far
-// above FP32 rounding, so every pair the reference tests in range is tested
-// here with the reference's FP32 operations and the interacting set is the
-// reference's.  The sub-bin starts of the (PB+2)^3 neighbourhood are staged
-// in LDS; candidates are read U at a time from L1/L2 (the entry array is
-// padded by kPPPad > (U-1) G entries so the reads need no clamp).
-// Measured at 512^3 (texture address and data units ~90-100% busy, VALU ~65%
-// busy in the chosen form), slower variants: a two-pass form
-// (in-range tests of 32 candidates into a bit mask, then the pair law over
-// the set bits only, each partner read again) measured 37.9 against 27.2 ms
-// at 512^3: the second pass's reads come from L2, one per pair.  Staging
-// each brick's neighbourhood (up to 2560 entries) in LDS and reading the
-// candidates from there measured 50.3 ms: 50 KB of LDS per workgroup leaves
-// three wavefronts per SIMD, and the lanes' scattered 16-byte LDS reads
-// conflict.  8-byte entries (positions as exact integers in units of 2^-15
-// fine cells, differences formed exactly through 2^23 + n in FP32) halved the
-// load instructions but added ~30% VALU work: 30.3 ms.  Deferring the pair
-// law until some lane holds two pairs (so it runs on most lanes at once)
-// cut the VALU count but its branches and spills gave 32.4 ms.  Splitting PP
-// cells also along y (fewer candidates, twice the columns) gave 30.2 ms.
-// FP32 form: eight 256-thread workgroups per CU (the launch bound's second
-// value), i.e. at most 64 VGPRs and eight wavefronts per SIMD to cover the
-// candidate loads' latency (28.5 vs 30.2 ms at 512^3 with 71 VGPRs and seven
-// wavefronts, a few values spilled); the FP64 form keeps its registers.  The
-// 8^3-brick variants' staged starts (35.5 KB of LDS per workgroup) leave room
-// for four workgroups only, so there the target is unmet (the compiler says
-// so) and they take 88 VGPRs without spills; they are autotune candidates
-// that lose at 512^3.
-template <typename R>
-constexpr int pp_min_blocks_per_cu() {
-  return sizeof(R) == 4 ? 8 : 1;
-}
-constexpr int kPPClaimCounters = 8;
-
-template <typename R, int U, int G, int PB>
-__global__ void __launch_bounds__(256, pp_min_blocks_per_cu<R>()) k_pp_force(PPLevel L, const PPBox* __restrict__ boxes,
-                                                  int64_t nbricks, const int64_t* __restrict__ start,
-                                                  const float4* __restrict__ ent, float* __restrict__ vp,
-                                                  PPOut* __restrict__ out, unsigned* __restrict__ claim,
-                                                  bool xcd_local) {
-  constexpr int NB = PB + 2, RW = kSX * NB + 1;  // staged sub-bin starts per (y, z) row
-  __shared__ int pre[PB * PB * PB + 1];
-  __shared__ int rs[NB * NB * RW];  // entry indices (a batch holds < 2^31 entries)
-  __shared__ float red[4];
-  __shared__ unsigned long long cnt_red[2];
-  __shared__ float4 qtab[kQSeg];
-  __shared__ int64_t s_brick;
-  if (sizeof(R) == 4) fill_qtab(qtab);
-  const double vsc = L.vdev ? *L.vdev : L.v_scale;
-  const int nbr = (L.npgrid + PB - 1) / PB;
+// Bricks of kPB^3 physical PP cells are claimed by persistent workgroups from
+// kPPClaimCounters counters (workgroup i uses counter i % 8) until none remain.
+// With at least 64 sub-tiles a counter hands out the bricks of sub-tiles ctr,
+// ctr + 8, ... (the host's densest-first order, kick.f90:132-138), one sub-tile's
+// bricks in turn, so that they run on one XCD and share its L2; with fewer, it
+// hands out bricks 8 k + ctr, so that every counter has work.  A claim is one of
+// `parts` shares of a brick's targets: with few bricks a launch would end on
+// the densest one's workgroup (64^3 particles, 4096 bricks: 365 us with whole
+// bricks, 309 in shares, 202 with the counters and the output slots on cache
+// lines of their own; 128^3, 32768 bricks: 0.48 ms against 1.25 at the start).
+// A workgroup's first claim is its own place in the queue; the counters, each
+// on a cache line of its own, hand out the rest.
+__device__ inline int64_t claim_brick(unsigned* claim, bool first, int64_t nbricks, int64_t nbps, bool xcd_local) {
   const int ctr = blockIdx.x % kPPClaimCounters;
-  if (threadIdx.x == 0) {
-    cnt_red[0] = 0;
-    cnt_red[1] = 0;
+  const int64_t k = first ? (int64_t)(blockIdx.x / kPPClaimCounters)
+                          : (int64_t)atomicAdd(&claim[ctr * kPPClaimStride], 1u) +
+                                (gridDim.x - ctr + kPPClaimCounters - 1) / kPPClaimCounters;
+  if (!xcd_local) return min(k * kPPClaimCounters + ctr, nbricks);
+  const int64_t box = (k / nbps) * kPPClaimCounters + ctr;
+  return box < nbricks / nbps ? box * nbps + k % nbps : nbricks;
+}
+
+// A brick's tables: rs, the starts of the x sub-bins of its (kPB+2)^2 rows
+// (cells c0-1 .. c0+kPB along x; rows outside the PP grid are empty, sub-bins
+// past a row's end read the end), and pre, the prefix sums of its cells' counts.
+constexpr int kNB = kPB + 2, kRW = kSX * kNB + 1;
+struct Brick {
+  int ib, c0[3];
+};
+__device__ inline Brick brick_tables(const PPLevel& L, int64_t brick, int nbr, const int64_t* __restrict__ start,
+                                     int* rs, int* pre) {
+  Brick K;
+  const uint32_t b = (uint32_t)brick, n = (uint32_t)nbr;  // nbox nbr^3 < 2^32
+  K.c0[0] = 1 + (int)(b % n) * kPB;
+  K.c0[1] = 1 + (int)((b / n) % n) * kPB;
+  K.c0[2] = 1 + (int)((b / (n * n)) % n) * kPB;
+  K.ib = (int)(b / (n * n * n));
+  const int m = L.npgrid + 2, mS = m * kSX;
+  const int64_t cbase = (int64_t)K.ib * m * m * m;
+  for (int q = threadIdx.x; q < kNB * kNB * kRW; q += blockDim.x) {
+    const int row = q / kRW, xs = q - row * kRW, y = K.c0[1] - 1 + row % kNB, z = K.c0[2] - 1 + row / kNB;
+    int st = 0;
+    if (y <= L.npgrid + 1 && z <= L.npgrid + 1)
+      st = (int)start[(cbase + ((int64_t)z * m + y) * m) * kSX + min(kSX * (K.c0[0] - 1) + xs, mS)];
+    rs[q] = st;
   }
+  __syncthreads();
+  if (threadIdx.x < kPB * kPB * kPB) {  // one wavefront: cell counts and their prefix sums
+    const int q = threadIdx.x, lx = q % kPB, ly = (q / kPB) % kPB, lz = q / (kPB * kPB);
+    const int row = ((lz + 1) * kNB + ly + 1) * kRW;
+    const bool in = K.c0[0] + lx <= L.npgrid && K.c0[1] + ly <= L.npgrid && K.c0[2] + lz <= L.npgrid;
+    int s = in ? rs[row + kSX * (lx + 2)] - rs[row + kSX * (lx + 1)] : 0;
+    for (int o = 1; o < 64; o <<= 1) {
+      const int v = __shfl_up(s, o, 64);
+      if (q >= o) s += v;
+    }
+    pre[q + 1] = s;
+    if (q == 0) pre[0] = 0;
+  }
+  __syncthreads();
+  return K;
+}
+static_assert(kPB * kPB * kPB == 64, "a brick's cells are one wavefront");
+
+// Cell of a brick's target t: the largest c with pre[c] <= t.
+__device__ inline int target_cell(const int* pre, int t) {
+  int lo = 0;
+#pragma unroll
+  for (int s = kPB * kPB * kPB / 2; s > 0; s >>= 1)
+    if (pre[lo + s] <= t) lo += s;
+  return lo;
+}
+
+// The x window of the (dy, dz) column of PP cells around a target: a partner
+// at y/z distance >= (ey, ez) is in range only within x +- sqrt(r_pp^2 - ey^2 -
+// ez^2), a contiguous run of the x-ordered row, found from two sub-bin starts.
+// fr: the target's offset in its PP cell; u: its x in sub-bins of the staged
+// rows; lx: its cell.  The cut carries a margin of 1e-3 cell, far above the
+// rounding here, so every pair the reference tests in range is in a window.
+__device__ inline void column_run(const PPLevel& L, const int* rs, int rowt, int lx, float u, const float fr[3],
+                                  int dy, int dz, int& beg, int& n) {
+  const float ey = dy < 0 ? fr[1] : (dy > 0 ? 1.0f - fr[1] : 0.0f);
+  const float ez = dz < 0 ? fr[2] : (dz > 0 ? 1.0f - fr[2] : 0.0f);
+  const float e2 = ey * ey + ez * ez;
+  const float hw = (float)kSX * __builtin_amdgcn_sqrtf(fmaxf(L.rcut2 - e2, 0.0f));
+  const int wlo = max((int)floorf(u - hw), kSX * lx);
+  const int whi = min((int)floorf(u + hw), kSX * (lx + 3) - 1);
+  const int row = rowt + (dz * kNB + dy) * kRW;
+  beg = rs[row + wlo];
+  n = e2 < L.rcut2 ? rs[row + whi + 1] - beg : 0;
+}
+
+// Maxima and pair counts of a workgroup into its slot (one wavefront's atomics).
+// Counts are per lane, or (wave_counts) held by every lane of a wavefront.
+__device__ inline void pp_reduce(PPOut* __restrict__ out, float f2, const float vm[3], unsigned long long npp,
+                                 unsigned long long npg, bool wave_counts) {
+  __shared__ float rm[4][4];
+  __shared__ unsigned long long rc[4][2];
+  float v[4] = {f2, vm[0], vm[1], vm[2]};
+  for (int o = 32; o > 0; o >>= 1)
+    for (int k = 0; k < 4; ++k) v[k] = fmaxf(v[k], __shfl_xor(v[k], o, 64));
+  if (!wave_counts)
+    for (int o = 32; o > 0; o >>= 1) {
+      npp += __shfl_xor(npp, o, 64);
+      npg += __shfl_xor(npg, o, 64);
+    }
+  if ((threadIdx.x & 63) == 0) {
+    const int w = threadIdx.x >> 6;
+    for (int k = 0; k < 4; ++k) rm[w][k] = v[k];
+    rc[w][0] = npp;
+    rc[w][1] = npg;
+  }
+  __syncthreads();
+  PPOut::Slot& sl = out->slot[blockIdx.x % kSumSlots];
+  if (threadIdx.x < 4) {
+    const int k = threadIdx.x;
+    const float m = fmaxf(fmaxf(rm[0][k], rm[1][k]), fmaxf(rm[2][k], rm[3][k]));
+    atomic_max_nonneg(k == 0 ? &sl.f2max : &sl.vmax[k - 1], m);
+  } else if (threadIdx.x < 6) {
+    const int k = threadIdx.x - 4;
+    const unsigned long long c = rc[0][k] + rc[1][k] + rc[2][k] + rc[3][k];
+    if (c) atomicAdd(k == 0 ? &sl.pairs_pp : &sl.pairs_pg, c);
+  }
+}
+
+// v += f mass_scale a_mid dt/6/pi (kick.f90:576-582): g = fl32(f mass_scale) as
+// the reference forms it, times the FP64 coefficient, added in FP64.
+__device__ inline void pp_kick(const PPLevel& L, double vsc, const float f[3], float* __restrict__ vp, int64_t ip,
+                               float& f2, float vm[3]) {
+  float g[3];
+  for (int d = 0; d < 3; ++d) g[d] = f[d] * L.mass_scale;
+  f2 = fmaxf(f2, (g[0] * g[0] + g[1] * g[1]) + g[2] * g[2]);
+  for (int d = 0; d < 3; ++d) {
+    const float v = (float)((double)vp[3 * ip + d] + (double)g[d] * vsc);
+    vp[3 * ip + d] = v;
+    vm[d] = fmaxf(vm[d], fabsf(v));
+  }
+}
+
+// FP32 force.  Two lanes per target particle; a wavefront's 32 targets first
+// write their windows in the nine (dy, dz) columns to LDS (each lane every
+// other column; empty ones dropped), then each pair of lanes walks its own
+// list of runs, 2 U entries at a time, lane j taking entries j, j + 2, ... .  So a
+// wavefront runs as long as its longest target, not the sum over columns of
+// its longest column.  Entries are read U at a time straight from L1/L2 (the
+// array is padded, so the reads need no clamp) and tested with the reference's
+// FP32 operations on exact positions: the interacting set is the reference's.
+// Both members of a physical pair evaluate it, and a target's partial sums are
+// added in a fixed order, so the result is deterministic.  Pairs are counted
+// from the wavefront's in-range masks by scalar instructions.
+//
+// 512^3 at z = 2 (2.85e9 pairs): 22.0 ms, 5.2 TFLOP/s at 40 flops a pair, against
+// 25.4 with the columns walked in step; TA busy 80% and VALU 68% of its cycles.
+// Slower when measured on the column form: candidates staged in LDS (50 KB a
+// workgroup leave three wavefronts per SIMD), 8-byte exact-integer entries (half
+// the load traffic, 30% more VALU), a two-pass form with in-range masks, PP
+// cells split along y as well, one or four lanes per target.
+template <int U>
+__global__ void __launch_bounds__(256, 8) k_pp_force(PPLevel L, const PPBox* __restrict__ boxes, int64_t nbricks,
+                                                     const int64_t* __restrict__ start,
+                                                     const float4* __restrict__ ent, const int64_t* __restrict__ off,
+                                                     float* __restrict__ vp, PPOut* __restrict__ out,
+                                                     unsigned* __restrict__ claim, bool xcd_local, int parts) {
+  constexpr int G = kPPGroup;
+  static_assert(G == 2, "two lanes per target");
+  __shared__ int rs[kNB * kNB * kRW];
+  __shared__ int pre[kPB * kPB * kPB + 1];
+  __shared__ float4 qtab[kQSeg + 1];
+  __shared__ int2 cols[4][32][9];
+  __shared__ int64_t s_brick;
+  fill_qtab(qtab, (double)L.c_range * (double)L.two_inv_range);
+  const float tscale = (float)kQSeg / L.pp_range2;
+  const double vsc = L.vdev ? *L.vdev : L.v_scale;
+  const int nbr = (L.npgrid + kPB - 1) / kPB;
+  const int lane = threadIdx.x & 63, gj = lane & 1;
+  int2* run = cols[threadIdx.x >> 6][lane >> 1];
   float f2 = 0, vm[3] = {0, 0, 0};
-  unsigned long long npp = 0, npg = 0;
-  for (;;) {
+  unsigned long long nall = 0, npg = 0;  // per wavefront
+  for (bool first = true;; first = false) {
     __syncthreads();  // the previous brick's tables are no longer read
-    if (threadIdx.x == 0) {
-      const int64_t k = (int64_t)atomicAdd(&claim[ctr], 1u), nbps = (int64_t)nbr * nbr * nbr;
-      if (xcd_local) {
-        // counter ctr hands out the bricks of sub-tiles ctr, ctr + 8, ...
-        // (in the host's densest-first order), one sub-tile's bricks in
-        // turn: its workgroups (blockIdx % 8 == ctr) share an XCD, whose L2
-        // then holds the neighbourhoods that a sub-tile's bricks read in
-        // common
-        const int64_t box = (k / nbps) * kPPClaimCounters + ctr;
-        s_brick = box < nbricks / nbps ? box * nbps + k % nbps : nbricks;
-      } else {
-        s_brick = k * kPPClaimCounters + ctr;  // few sub-tiles: bricks 8k + ctr, every counter busy
-      }
-    }
+    if (threadIdx.x == 0)
+      s_brick = claim_brick(claim, first, nbricks * parts, (int64_t)nbr * nbr * nbr * parts,
+                            xcd_local);
     __syncthreads();
-    int64_t b = s_brick;
-    if (b >= nbricks) break;
-    const int bx = (int)(b % nbr);
-    b /= nbr;
-    const int by = (int)(b % nbr);
-    b /= nbr;
-    const int bz = (int)(b % nbr);
-    const int ib = (int)(b / nbr);
-    const int m = L.npgrid + 2;
-    const int64_t mS = (int64_t)m * kSX;
-    const int64_t cbase = (int64_t)ib * m * m * m;
-    const int c0[3] = {1 + bx * PB, 1 + by * PB, 1 + bz * PB};
-    // rows (y, z) = c0-1 .. c0+PB, sub-bins kSX*(c0x-1) .. kSX*(c0x+PB+1); rows
-    // outside the PP grid are empty, sub-bins past the row end read the row end
-    for (int q = threadIdx.x; q < NB * NB * RW; q += blockDim.x) {
-      const int xs = q % RW, y = c0[1] - 1 + (q / RW) % NB, z = c0[2] - 1 + q / (RW * NB);
-      int st = 0;
-      if (y <= L.npgrid + 1 && z <= L.npgrid + 1) {
-        const int64_t row = (cbase + ((int64_t)z * m + y) * m) * kSX;
-        st = (int)start[row + min((int64_t)kSX * (c0[0] - 1) + xs, mS)];
+    if (s_brick >= nbricks * parts) break;
+    const int part = (int)(s_brick % parts);
+    const Brick K = brick_tables(L, s_brick / parts, nbr, start, rs, pre);
+    const PPBox B = boxes[K.ib];
+    const int64_t tile = off[(int64_t)B.T * L.nte * L.nte * L.nte];
+    const int nall_t = pre[kPB * kPB * kPB], ntg = (int)((int64_t)nall_t * (part + 1) / parts);
+    for (int t0 = (int)((int64_t)nall_t * part / parts) + (threadIdx.x >> 6) * 32; t0 < ntg; t0 += 128) {
+      const int t = t0 + (lane >> 1);
+      const bool ok = t < ntg;
+      float4 me = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+      int ncol = 0;
+      if (ok) {
+        const int c = target_cell(pre, t);
+        const int lc[3] = {c % kPB, (c / kPB) % kPB, c / (kPB * kPB)};
+        const int rowt = ((lc[2] + 1) * kNB + lc[1] + 1) * kRW;
+        me = ent[rs[rowt + kSX * (lc[0] + 1)] + (t - pre[c])];
+        // PP coordinates of the target, the binning's xv = sf (xvec - ifs ntt)
+        // (xvec = xf / rcs exactly for a power-of-two rcs)
+        const float xme[3] = {me.x, me.y, me.z};
+        float fr[3];
+        for (int d = 0; d < 3; ++d) {
+          const float xv = (float)L.sf * (xme[d] * L.inv_rcs - (float)(B.ifs[d] * L.ntt));
+          fr[d] = xv - (float)(K.c0[d] - 1 + lc[d]);
+        }
+        const float u = (fr[0] + (float)(lc[0] + 1)) * (float)kSX;
+        int beg[5], n[5], mine = 0;
+#pragma unroll
+        for (int i = 0; i < 5; ++i) {
+          const int q = 2 * i + gj;  // column (dy, dz) = (q % 3 - 1, q / 3 - 1)
+          n[i] = 0;
+          beg[i] = 0;
+          if (q < 9) column_run(L, rs, rowt, lc[0], u, fr, q % 3 - 1, q / 3 - 1, beg[i], n[i]);
+          mine += n[i] > 0;
+        }
+        const int other = __shfl_xor(mine, 1, 64);
+        int w = gj ? other : 0;
+        ncol = mine + other;
+#pragma unroll
+        for (int i = 0; i < 5; ++i)
+          if (n[i] > 0) run[w++] = make_int2(beg[i], n[i]);
       }
-      rs[q] = st;
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-      int s = 0;
-      for (int q = 0; q < PB * PB * PB; ++q) {
-        pre[q] = s;
-        const int lx = q % PB, ly = (q / PB) % PB, lz = q / (PB * PB);
-        if (c0[0] + lx <= L.npgrid && c0[1] + ly <= L.npgrid && c0[2] + lz <= L.npgrid) {
-          const int row = ((lz + 1) * NB + ly + 1) * RW;
-          s += (int)(rs[row + kSX * (lx + 2)] - rs[row + kSX * (lx + 1)]);
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      float f1[3] = {0, 0, 0};
+      int k = 0, p = gj;
+      int2 e = ncol > 0 ? run[0] : make_int2(0, 0);
+      // every lane stays until the last is done (finished ones hold an empty
+      // run), so that the pair counts are the wavefront's
+      while (__any(k < ncol)) {
+        const float4* src = ent + (e.x + p);
+        const int rem = e.y - p;
+        float4 o[U];
+#pragma unroll
+        for (int i = 0; i < U; ++i) o[i] = src[i * G];
+        p += U * G;
+        if (p >= e.y) {  // the next run (its first entry is read behind this one's arithmetic)
+          ++k;
+          p = gj;
+          e = k < ncol ? run[k] : make_int2(0, 0);
+        }
+#pragma unroll
+        for (int i = 0; i < U; ++i) {
+          const float rv0 = o[i].x - me.x, rv1 = o[i].y - me.y, rv2 = o[i].z - me.z;
+          const float r2 = (rv0 * rv0 + rv1 * rv1) + rv2 * rv2;  // exact-input FP32 test (kick.f90:525, 556)
+          const bool in = i * G < rem && 0.0f < r2 && r2 < L.pp_range2;
+          nall += __popcll(__ballot(in));
+          npg += __popcll(__ballot(in && __float_as_int(o[i].w) < 0));
+          if (in) {
+            const float rinv = __builtin_amdgcn_rsqf(r2);
+            const float ts = r2 * tscale;
+            const float4 c = qtab[(int)ts];
+            const float f = __builtin_amdgcn_fractf(ts);
+            const float q = fmaf(fmaf(fmaf(c.w, f, c.z), f, c.y), f, c.x);
+            float sc = fmaf(rinv * rinv, rinv, -q);
+            if (r2 <= L.app2) sc = fmaf(f_app(L, r2 * rinv), rinv, -q);  // ep(r, app) <= 2
+            f1[0] = fmaf(rv0, sc, f1[0]);
+            f1[1] = fmaf(rv1, sc, f1[1]);
+            f1[2] = fmaf(rv2, sc, f1[2]);
+          }
         }
       }
-      pre[PB * PB * PB] = s;
+      // the two lanes' sums: each step adds the same two operands on both
+      for (int d = 0; d < 3; ++d) f1[d] += __shfl_xor(f1[d], 1, 64);
+      if (ok && gj == 0) pp_kick(L, vsc, f1, vp, tile + (int64_t)(__float_as_uint(me.w) & 0x7fffffffu), f2, vm);
     }
+  }  // claimed bricks
+  pp_reduce(out, f2, vm, nall - npg, npg, true);
+}
+
+// FP64 form: one lane per target, the pair law in FP64 with the reference's
+// operations, the same bricks, windows and in-range test.
+__global__ void __launch_bounds__(256) k_pp_force64(PPLevel L, const PPBox* __restrict__ boxes, int64_t nbricks,
+                                                    const int64_t* __restrict__ start,
+                                                    const float4* __restrict__ ent, const int64_t* __restrict__ off,
+                                                    float* __restrict__ vp, PPOut* __restrict__ out,
+                                                    unsigned* __restrict__ claim, bool xcd_local, int parts) {
+  constexpr int U = 6;
+  static_assert(U <= kPPPad, "reads past a run stay inside the entry padding");
+  __shared__ int rs[kNB * kNB * kRW];
+  __shared__ int pre[kPB * kPB * kPB + 1];
+  __shared__ int64_t s_brick;
+  const double vsc = L.vdev ? *L.vdev : L.v_scale;
+  const int nbr = (L.npgrid + kPB - 1) / kPB;
+  float f2 = 0, vm[3] = {0, 0, 0};
+  unsigned long long npp = 0, npg = 0;
+  for (bool first = true;; first = false) {
     __syncthreads();
-    const PPBox B = boxes[ib];
-    const float xoff[3] = {(float)(B.ifs[0] * L.ntt), (float)(B.ifs[1] * L.ntt), (float)(B.ifs[2] * L.ntt)};
-    const int ntg = pre[PB * PB * PB];
-    const int gj = (int)threadIdx.x % G;  // lane within the target's group
-    for (int t = (int)threadIdx.x / G; t < ntg; t += (int)blockDim.x / G) {
-      int lo = 0, hi = PB * PB * PB - 1;
-      while (lo < hi) {
-        const int mid = (lo + hi + 1) >> 1;
-        if (pre[mid] <= t) lo = mid;
-        else hi = mid - 1;
-      }
-      const int lx = lo % PB, ly = (lo / PB) % PB, lz = lo / (PB * PB);
-      const int rowt = ((lz + 1) * NB + ly + 1) * RW;
-      const float4 me = ent[rs[rowt + kSX * (lx + 1)] + (t - pre[lo])];
-      // PP coordinates of the target, the binning's xv = sf (xvec - ifs ntt)
-      // (xvec = xf / rcs exactly for a power-of-two rcs)
+    if (threadIdx.x == 0)
+      s_brick = claim_brick(claim, first, nbricks * parts, (int64_t)nbr * nbr * nbr * parts,
+                            xcd_local);
+    __syncthreads();
+    if (s_brick >= nbricks * parts) break;
+    const int part = (int)(s_brick % parts);
+    const Brick K = brick_tables(L, s_brick / parts, nbr, start, rs, pre);
+    const PPBox B = boxes[K.ib];
+    const int64_t tile = off[(int64_t)B.T * L.nte * L.nte * L.nte];
+    const int nall_t = pre[kPB * kPB * kPB], ntg = (int)((int64_t)nall_t * (part + 1) / parts);
+    for (int t = (int)((int64_t)nall_t * part / parts) + threadIdx.x; t < ntg; t += 256) {
+      const int c = target_cell(pre, t);
+      const int lc[3] = {c % kPB, (c / kPB) % kPB, c / (kPB * kPB)};
+      const int rowt = ((lc[2] + 1) * kNB + lc[1] + 1) * kRW;
+      const float4 me = ent[rs[rowt + kSX * (lc[0] + 1)] + (t - pre[c])];
       const float xme[3] = {me.x, me.y, me.z};
       float fr[3];
       for (int d = 0; d < 3; ++d) {
-        const float xv = (float)L.sf * (xme[d] * L.inv_rcs - xoff[d]);
-        fr[d] = xv - (float)(c0[d] - 1 + (d == 0 ? lx : (d == 1 ? ly : lz)));  // offset in its PP cell
+        const float xv = (float)L.sf * (xme[d] * L.inv_rcs - (float)(B.ifs[d] * L.ntt));
+        fr[d] = xv - (float)(K.c0[d] - 1 + lc[d]);
       }
-      // the target's x in local sub-bins (cells lx .. lx+2 of the staged rows)
-      const float u = (fr[0] + (float)(lx + 1)) * (float)kSX;
-      R f1[3] = {0, 0, 0};
-      // pairs in range of this target, and those with a ghost partner (32-bit)
+      const float u = (fr[0] + (float)(lc[0] + 1)) * (float)kSX;
+      double f1[3] = {0, 0, 0};
       int npair = 0, nghost = 0;
-      const bool gx0 = c0[0] + lx - 1 == 0, gx1 = c0[0] + lx + 1 == L.npgrid + 1;
       for (int dz = -1; dz <= 1; ++dz)
         for (int dy = -1; dy <= 1; ++dy) {
-          const float ey = dy < 0 ? fr[1] : (dy > 0 ? 1.0f - fr[1] : 0.0f);
-          const float ez = dz < 0 ? fr[2] : (dz > 0 ? 1.0f - fr[2] : 0.0f);
-          const float e2 = ey * ey + ez * ez;
-          if (e2 >= L.rcut2) continue;
-          // x window of the column: a partner at y/z distance >= (ey, ez)
-          // is in range only within x +- sqrt(r_pp^2 - ey^2 - ez^2)
-          const float hw = (float)kSX * sqrtf(L.rcut2 - e2);
-          const int wlo = max((int)floorf(u - hw), kSX * lx);
-          const int whi = min((int)floorf(u + hw), kSX * (lx + 3) - 1);
-          const int ny = c0[1] + ly + dy, nz = c0[2] + lz + dz;
-          const bool gyz = ny == 0 || nz == 0 || ny == L.npgrid + 1 || nz == L.npgrid + 1;
-          const int row = rowt + (dz * NB + dy) * RW;
-          const int beg = rs[row + wlo];
-          const int nn = (int)(rs[row + whi + 1] - beg);
-          // candidates [ph0, ph1) of the window are physical: the ghost cells
-          // x-1 / x+1 lie before / after them, a ghost row holds none
-          int ph0 = gx0 ? max((int)(rs[row + kSX * (lx + 1)] - beg), 0) : 0;
-          int ph1 = gx1 ? min((int)(rs[row + kSX * (lx + 2)] - beg), nn) : nn;
-          if (gyz) ph0 = ph1 = 0;
-          const unsigned phn = (unsigned)(ph1 - ph0);
+          int beg, nn;
+          column_run(L, rs, rowt, lc[0], u, fr, dy, dz, beg, nn);
           const float4* run = ent + beg;
-          for (int p = gj; p < nn; p += U * G) {
+          for (int p = 0; p < nn; p += U) {
             float4 o[U];
-  #pragma unroll
-            for (int k = 0; k < U; ++k) o[k] = run[p + k * G];
-  #pragma unroll
+#pragma unroll
+            for (int k = 0; k < U; ++k) o[k] = run[p + k];
+#pragma unroll
             for (int k = 0; k < U; ++k) {
               const float rv0 = o[k].x - me.x, rv1 = o[k].y - me.y, rv2 = o[k].z - me.z;
-              const float r2 = (rv0 * rv0 + rv1 * rv1) + rv2 * rv2;  // exact-input FP32 test (kick.f90:525, 556)
-              if (p + k * G < nn && 0.0f < r2 && r2 < L.pp_range2) {
-                pair_force<R>(L, qtab, me, o[k], f1);
+              const float r2 = (rv0 * rv0 + rv1 * rv1) + rv2 * rv2;
+              if (p + k < nn && 0.0f < r2 && r2 < L.pp_range2) {
+                pair_force64(L, me, o[k], f1);
                 ++npair;
-                nghost += (unsigned)(p + k * G - ph0) >= phn;
+                nghost += __float_as_int(o[k].w) < 0;
               }
             }
           }
         }
       npg += (unsigned)nghost;
       npp += (unsigned)(npair - nghost);
-      // the group's partial sums, combined by a butterfly: every lane ends
-      // with the same value (each step adds the same two operands)
-      for (int o = G / 2; o > 0; o >>= 1)
-        for (int d = 0; d < 3; ++d) f1[d] += __shfl_xor(f1[d], o, 64);
-      if (gj == 0) {
-        // update v (kick.f90:576-582): g = fl32(f mass_scale) as the
-        // reference forms it, times the FP64 coefficient, added in FP64
-        const unsigned ip = __float_as_uint(me.w);
-        float g[3];
-        for (int d = 0; d < 3; ++d) g[d] = (float)f1[d] * L.mass_scale;
-        f2 = fmaxf(f2, (g[0] * g[0] + g[1] * g[1]) + g[2] * g[2]);
-        for (int d = 0; d < 3; ++d) {
-          const float v = (float)((double)vp[3 * (int64_t)ip + d] + (double)g[d] * vsc);
-          vp[3 * (int64_t)ip + d] = v;
-          vm[d] = fmaxf(vm[d], fabsf(v));
-        }
-      }
+      const float f[3] = {(float)f1[0], (float)f1[1], (float)f1[2]};
+      pp_kick(L, vsc, f, vp, tile + (int64_t)(__float_as_uint(me.w) & 0x7fffffffu), f2, vm);
     }
-  }  // claimed bricks
-  auto bmax = [&](float v) {
-    for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_down(v, o, 64));
-    __syncthreads();
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
-    __syncthreads();
-    float r = 0;
-    for (int w = 0; w < (int)(blockDim.x >> 6); ++w) r = fmaxf(r, red[w]);
-    return r;
-  };
-  float r = bmax(f2);
-  if (threadIdx.x == 0 && r > 0) atomic_max_nonneg(&out->f2max, r);
-  for (int d = 0; d < 3; ++d) {
-    r = bmax(vm[d]);
-    if (threadIdx.x == 0 && r > 0) atomic_max_nonneg(&out->vmax[d], r);
   }
-  for (int o = 32; o > 0; o >>= 1) {
-    npp += __shfl_down(npp, o, 64);
-    npg += __shfl_down(npg, o, 64);
-  }
-  if ((threadIdx.x & 63) == 0) {
-    atomicAdd(&cnt_red[0], npp);
-    atomicAdd(&cnt_red[1], npg);
-  }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    atomicAdd(&out->pairs_pp[blockIdx.x % kSumSlots], cnt_red[0]);
-    atomicAdd(&out->pairs_pg[blockIdx.x % kSumSlots], cnt_red[1]);
-  }
+  pp_reduce(out, f2, vm, npp, npg, false);
 }
 
 }  // namespace
@@ -520,33 +588,17 @@ void pp_bin_fill(int izipx, const PPLevel& L, const PPBox* boxes, int nbox, cons
   CUBE_HIP(hipGetLastError());
 }
 
-template <int U, int G, int PB>
+template <int U>
 static void launch_pp_f32(dim3 grid, hipStream_t s, const PPLevel& L, const PPBox* boxes, int64_t nbricks,
-                          PPScratch& S, float* vp, PPOut* out) {
-  static_assert((U - 1) * G < kPPPad, "reads past a run stay inside the entry padding");
-  // whole sub-tiles per counter only when there are enough of them to keep
-  // the eight counters evenly busy
-  const bool xcd_local = nbricks / ((int64_t)((L.npgrid + PB - 1) / PB) * ((L.npgrid + PB - 1) / PB) *
-                                    ((L.npgrid + PB - 1) / PB)) >= 64;
-  hipLaunchKernelGGL((k_pp_force<float, U, G, PB>), grid, dim3(256), 0, s, L, boxes, nbricks, S.start, S.entries,
-                     vp, out, S.claim, xcd_local);
+                          PPScratch& S, const int64_t* off, float* vp, PPOut* out, bool xcd_local, int parts) {
+  static_assert(U * kPPGroup <= kPPPad, "reads past a run stay inside the entry padding");
+  hipLaunchKernelGGL((k_pp_force<U>), grid, dim3(256), 0, s, L, boxes, nbricks, S.start, S.entries, off, vp, out,
+                     S.claim, xcd_local, parts);
 }
 
-template <int G, int PB>
-static void launch_pp_f32_u(int depth, dim3 grid, hipStream_t s, const PPLevel& L, const PPBox* boxes,
-                            int64_t nbricks, PPScratch& S, float* vp, PPOut* out) {
-  switch (depth) {
-    case 4: launch_pp_f32<4, G, PB>(grid, s, L, boxes, nbricks, S, vp, out); break;
-    case 8: launch_pp_f32<8, G, PB>(grid, s, L, boxes, nbricks, S, vp, out); break;
-    default: launch_pp_f32<6, G, PB>(grid, s, L, boxes, nbricks, S, vp, out); break;
-  }
-}
-
-void pp_force(const PPLevel& L, int precision, const PPBox* boxes, int nbox, float* vp, PPScratch& S, PPOut* out,
-              hipStream_t s, int unroll) {
-  const int pb = precision == 32 && unroll >= kPPBrick8 ? 8 : 4;
-  const int depth = unroll % kPPBrick8;
-  const int64_t nbr = (L.npgrid + pb - 1) / pb;
+void pp_force(const PPLevel& L, int precision, const PPBox* boxes, int nbox, const int64_t* off, float* vp,
+              PPScratch& S, PPOut* out, hipStream_t s, int unroll) {
+  const int64_t nbr = (L.npgrid + kPB - 1) / kPB;
   const int64_t nbricks = nbr * nbr * nbr * nbox;
   static int n_cu = 0;
   if (n_cu == 0) {
@@ -554,20 +606,25 @@ void pp_force(const PPLevel& L, int precision, const PPBox* boxes, int nbox, flo
     CUBE_HIP(hipGetDevice(&dev));
     CUBE_HIP(hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, dev));
   }
-  zero_async(S.claim, sizeof(unsigned) * kPPClaimCounters, s);
+  zero_async(S.claim, sizeof(unsigned) * kPPClaimCounters * kPPClaimStride, s);
   // as many workgroups as fit on the chip at once (eight per CU in the FP32
-  // form, the launch bound's occupancy; four in the FP64 form, whose 117
-  // VGPRs allow four wavefronts per SIMD), each then claims bricks until
-  // none remain
-  const int per_cu = precision == 64 ? 4 : pp_min_blocks_per_cu<float>();
-  const dim3 grid((unsigned)std::min<int64_t>(nbricks, (int64_t)n_cu * per_cu));
+  // form, the launch bound's occupancy; four in the FP64 form), each then
+  // claims bricks until none remain
+  const int per_cu = precision == 64 ? 4 : 8;
+  const int64_t resident = (int64_t)n_cu * per_cu;
+  // shares of a brick: enough claims that the last ones are short
+  const int parts = (int)std::max<int64_t>(1, std::min<int64_t>(8, ceil_div(8 * resident, std::max<int64_t>(nbricks, 1))));
+  const dim3 grid((unsigned)std::min<int64_t>(nbricks * parts, resident));
+  const bool xcd_local = nbox >= 64;  // whole sub-tiles per counter only when there are enough of them
   if (precision == 64)
-    hipLaunchKernelGGL((k_pp_force<double, 6, 1, 4>), grid, dim3(256), 0, s, L, boxes, nbricks, S.start,
-                       S.entries, vp, out, S.claim, nbox >= 64);
-  else if (pb == 8)
-    launch_pp_f32_u<kPPGroup, 8>(depth, grid, s, L, boxes, nbricks, S, vp, out);
+    hipLaunchKernelGGL(k_pp_force64, grid, dim3(256), 0, s, L, boxes, nbricks, S.start, S.entries, off, vp, out,
+                       S.claim, xcd_local, parts);
+  else if (unroll == 2)
+    launch_pp_f32<2>(grid, s, L, boxes, nbricks, S, off, vp, out, xcd_local, parts);
+  else if (unroll == 4)
+    launch_pp_f32<4>(grid, s, L, boxes, nbricks, S, off, vp, out, xcd_local, parts);
   else
-    launch_pp_f32_u<kPPGroup, 4>(depth, grid, s, L, boxes, nbricks, S, vp, out);
+    launch_pp_f32<3>(grid, s, L, boxes, nbricks, S, off, vp, out, xcd_local, parts);
   CUBE_HIP(hipGetLastError());
 }
 
