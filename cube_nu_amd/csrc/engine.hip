@@ -80,7 +80,7 @@ inline uint64_t fbits(float f) {
 __global__ void k_set_f64(double* p, double v) { *p = v; }
 
 // Candidates of each tuned choice, in order of preference.
-const std::vector<int> kTunePPDepth = {3, 2, 4};
+const std::vector<int> kTunePPDepth = {3, 4, 6};
 const std::vector<int> kTuneDepListThreads = {512, 256, 1024};
 const std::vector<int> kTuneInterpShape = {0, 1, 2};
 
@@ -778,10 +778,9 @@ int cube_p3m_ctx::interp_shape(int level, int n, const PMLevel& L, const PMBox* 
 
 // PP load depth (candidates in flight per lane), tuned per PP level on the
 // level's first batch.  The trials run on a scratch copy of the velocities and
-// of the outputs.  The preference order 3, 2, 4 keeps the middle depth unless
-// another is more than 1% faster (a deeper one wastes more reads past the ends
-// of runs, a shallower one walks more often).  All depths sum the pairs in the
-// same order, so the choice changes the time of the step only.
+// of the outputs, in the order of preference 3, 4, 6 (1% apart or less, the
+// first wins).  All depths sum the pairs in the same order, so the choice
+// changes the time of the step only.
 int cube_p3m_ctx::tune_pp(int iapm, const PPLevel& L, const PPBox* boxes, int nb, PPScratch& S) {
   vtune.ensure((size_t)std::max<int64_t>(np, 1) * 3);
   otune.ensure(1);

@@ -62,7 +62,7 @@ void pp_bin_fill(int izipx, const PPLevel& L, const PPBox* boxes_dev, int nbox, 
                  const int64_t* cell_off, PPScratch& S, hipStream_t s);
 // cell_off: the extended cells' offsets (entries hold the particle's index
 // within its tile).  unroll: candidate loads in flight per lane in the FP32
-// kernel, 2, 3 or 4; the partial sums' order depends on it.
+// kernel, 3, 4 or 6; every value gives the same result.
 void pp_force(const PPLevel& L, int precision, const PPBox* boxes_dev, int nbox, const int64_t* cell_off, float* vp,
               PPScratch& S, PPOut* out, hipStream_t s, int unroll = 3);
 

@@ -61,6 +61,11 @@ __global__ void __launch_bounds__(256) k_pp_bin(PPLevel L, const PPBox* __restri
   extern __shared__ int lcnt[];
   const int nr = L.ntt + 2;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  if (FILL && blockIdx.x == 0 && threadIdx.x < kPPPad) {
+    // the padding behind the last entry is read (and weighted with zero): finite
+    const int64_t m1 = L.npgrid + 2;
+    ent[start[nbox * m1 * m1 * m1 * kSX] + threadIdx.x] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  }
   // 32-bit: a 64-bit division is ~100 instructions, and an image has far fewer than 2^32 coarse cells
   const uint32_t wv = blockIdx.x * 4u + (uint32_t)wave;
   if (wv >= (uint32_t)nbox * nr * nr * nr) return;
@@ -178,7 +183,15 @@ __device__ inline void fill_qtab(float4* tab, double scale) {
   }
 }
 
-// F(r, app) in full for the rare r <= app (ep <= 2), times c.
+// F(r, r_pp)/r at ts = r^2 kQSeg / r_pp^2 (beyond the range: its end value).
+__device__ inline float f_range(const float4* tab, float ts) {
+  ts = fminf(ts, (float)kQSeg);
+  const float4 c = tab[(int)ts];
+  const float f = __builtin_amdgcn_fractf(ts);
+  return fmaf(fmaf(fmaf(c.w, f, c.z), f, c.y), f, c.x);
+}
+
+// F(r, app) in full for the rare r <= app (ep <= 2).
 __device__ inline float f_app(const PPLevel& L, float r) {
   const float ea = (2.0f * r) * L.inv_app;
   const float a2 = ea * ea;
@@ -297,19 +310,17 @@ __device__ inline void column_run(const PPLevel& L, const int* rs, int rowt, int
 }
 
 // Maxima and pair counts of a workgroup into its slot (one wavefront's atomics).
-// Counts are per lane, or (wave_counts) held by every lane of a wavefront.
 __device__ inline void pp_reduce(PPOut* __restrict__ out, float f2, const float vm[3], unsigned long long npp,
-                                 unsigned long long npg, bool wave_counts) {
+                                 unsigned long long npg) {
   __shared__ float rm[4][4];
   __shared__ unsigned long long rc[4][2];
   float v[4] = {f2, vm[0], vm[1], vm[2]};
   for (int o = 32; o > 0; o >>= 1)
     for (int k = 0; k < 4; ++k) v[k] = fmaxf(v[k], __shfl_xor(v[k], o, 64));
-  if (!wave_counts)
-    for (int o = 32; o > 0; o >>= 1) {
-      npp += __shfl_xor(npp, o, 64);
-      npg += __shfl_xor(npg, o, 64);
-    }
+  for (int o = 32; o > 0; o >>= 1) {
+    npp += __shfl_xor(npp, o, 64);
+    npg += __shfl_xor(npg, o, 64);
+  }
   if ((threadIdx.x & 63) == 0) {
     const int w = threadIdx.x >> 6;
     for (int k = 0; k < 4; ++k) rm[w][k] = v[k];
@@ -352,17 +363,22 @@ __device__ inline void pp_kick(const PPLevel& L, double vsc, const float f[3], f
 // array is padded, so the reads need no clamp) and tested with the reference's
 // FP32 operations on exact positions: the interacting set is the reference's.
 // Both members of a physical pair evaluate it, and a target's partial sums are
-// added in a fixed order, so the result is deterministic.  Pairs are counted
-// from the wavefront's in-range masks by scalar instructions.
+// added in a fixed order, so the result is deterministic.
 //
-// 512^3 at z = 2 (2.85e9 pairs): 22.0 ms, 5.2 TFLOP/s at 40 flops a pair, against
-// 25.4 with the columns walked in step; TA busy 80% and VALU 68% of its cycles.
-// Slower when measured on the column form: candidates staged in LDS (50 KB a
-// workgroup leave three wavefronts per SIMD), 8-byte exact-integer entries (half
-// the load traffic, 30% more VALU), a two-pass form with in-range masks, PP
-// cells split along y as well, one or four lanes per target.
+// U reads in flight per lane against wavefronts per SIMD: 3 with eight (64
+// VGPRs) is the fastest on long lists of short runs, whose reads miss L1 (512^3
+// at z = 2: 21.7 ms; 4 with eight 22.6, 6 with five 25.8), 6 with five (96
+// VGPRs) on the long runs of clustered input (192^3 at z = 0.5: 2.8 ms against
+// 3.2), 4 with seven between them (64^3); the engine's autotuner picks.  At 512^3
+// (2.85e9 pairs) 21.7 ms are 5.3 TFLOP/s at 40 flops a pair (25.4 ms with the
+// columns walked in step and a branch per pair); TA is busy 80% and VALU 68% of
+// the cycles.  Slower, on the form with columns in step: candidates staged in
+// LDS (50 KB a workgroup leave three wavefronts per SIMD), 8-byte exact-integer
+// entries (half the load traffic, 30% more VALU), a two-pass form with in-range
+// masks, PP cells split along y as well, one or four lanes per target.
+constexpr int pp_workgroups(int u) { return u == 3 ? 8 : (u == 4 ? 7 : 5); }
 template <int U>
-__global__ void __launch_bounds__(256, 8) k_pp_force(PPLevel L, const PPBox* __restrict__ boxes, int64_t nbricks,
+__global__ void __launch_bounds__(256, pp_workgroups(U)) k_pp_force(PPLevel L, const PPBox* __restrict__ boxes, int64_t nbricks,
                                                      const int64_t* __restrict__ start,
                                                      const float4* __restrict__ ent, const int64_t* __restrict__ off,
                                                      float* __restrict__ vp, PPOut* __restrict__ out,
@@ -381,7 +397,7 @@ __global__ void __launch_bounds__(256, 8) k_pp_force(PPLevel L, const PPBox* __r
   const int lane = threadIdx.x & 63, gj = lane & 1;
   int2* run = cols[threadIdx.x >> 6][lane >> 1];
   float f2 = 0, vm[3] = {0, 0, 0};
-  unsigned long long nall = 0, npg = 0;  // per wavefront
+  unsigned long long npp = 0, npg = 0;
   for (bool first = true;; first = false) {
     __syncthreads();  // the previous brick's tables are no longer read
     if (threadIdx.x == 0)
@@ -394,7 +410,8 @@ __global__ void __launch_bounds__(256, 8) k_pp_force(PPLevel L, const PPBox* __r
     const PPBox B = boxes[K.ib];
     const int64_t tile = off[(int64_t)B.T * L.nte * L.nte * L.nte];
     const int nall_t = pre[kPB * kPB * kPB], ntg = (int)((int64_t)nall_t * (part + 1) / parts);
-    for (int t0 = (int)((int64_t)nall_t * part / parts) + (threadIdx.x >> 6) * 32; t0 < ntg; t0 += 128) {
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    for (int t0 = (int)((int64_t)nall_t * part / parts) + wave * 32; t0 < ntg; t0 += 128) {
       const int t = t0 + (lane >> 1);
       const bool ok = t < ntg;
       float4 me = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
@@ -435,47 +452,60 @@ __global__ void __launch_bounds__(256, 8) k_pp_force(PPLevel L, const PPBox* __r
       float f1[3] = {0, 0, 0};
       int k = 0, p = gj;
       int2 e = ncol > 0 ? run[0] : make_int2(0, 0);
-      // every lane stays until the last is done (finished ones hold an empty
-      // run), so that the pair counts are the wavefront's
-      while (__any(k < ncol)) {
+      int npair = 0, nghost = 0;
+      while (k < ncol) {
         const float4* src = ent + (e.x + p);
         const int rem = e.y - p;
         float4 o[U];
 #pragma unroll
         for (int i = 0; i < U; ++i) o[i] = src[i * G];
         p += U * G;
-        if (p >= e.y) {  // the next run (its first entry is read behind this one's arithmetic)
+        if (p >= e.y) {  // the next run
           ++k;
           p = gj;
           e = k < ncol ? run[k] : make_int2(0, 0);
         }
+        // U pairs side by side, without a branch: of 64 lanes one is nearly
+        // always in range
+        float rv[U][3], r2[U], sc[U];
+        bool in[U], near = false;
 #pragma unroll
         for (int i = 0; i < U; ++i) {
-          const float rv0 = o[i].x - me.x, rv1 = o[i].y - me.y, rv2 = o[i].z - me.z;
-          const float r2 = (rv0 * rv0 + rv1 * rv1) + rv2 * rv2;  // exact-input FP32 test (kick.f90:525, 556)
-          const bool in = i * G < rem && 0.0f < r2 && r2 < L.pp_range2;
-          nall += __popcll(__ballot(in));
-          npg += __popcll(__ballot(in && __float_as_int(o[i].w) < 0));
-          if (in) {
-            const float rinv = __builtin_amdgcn_rsqf(r2);
-            const float ts = r2 * tscale;
-            const float4 c = qtab[(int)ts];
-            const float f = __builtin_amdgcn_fractf(ts);
-            const float q = fmaf(fmaf(fmaf(c.w, f, c.z), f, c.y), f, c.x);
-            float sc = fmaf(rinv * rinv, rinv, -q);
-            if (r2 <= L.app2) sc = fmaf(f_app(L, r2 * rinv), rinv, -q);  // ep(r, app) <= 2
-            f1[0] = fmaf(rv0, sc, f1[0]);
-            f1[1] = fmaf(rv1, sc, f1[1]);
-            f1[2] = fmaf(rv2, sc, f1[2]);
+          rv[i][0] = o[i].x - me.x;
+          rv[i][1] = o[i].y - me.y;
+          rv[i][2] = o[i].z - me.z;
+          r2[i] = (rv[i][0] * rv[i][0] + rv[i][1] * rv[i][1]) + rv[i][2] * rv[i][2];
+          in[i] = i * G < rem && 0.0f < r2[i] && r2[i] < L.pp_range2;  // exact-input FP32 test (kick.f90:525, 556)
+          near = near || (in[i] && r2[i] <= L.app2);
+          const float rinv = __builtin_amdgcn_rsqf(r2[i]);
+          sc[i] = fmaf(rinv * rinv, rinv, -f_range(qtab, r2[i] * tscale));
+        }
+        if (__any(near)) {  // ep(r, app) <= 2: F(r, app) in full
+#pragma unroll
+          for (int i = 0; i < U; ++i) {
+            const float rinv = __builtin_amdgcn_rsqf(r2[i]);
+            if (in[i] && r2[i] <= L.app2)
+              sc[i] = fmaf(f_app(L, r2[i] * rinv), rinv, -f_range(qtab, r2[i] * tscale));
           }
+        }
+#pragma unroll
+        for (int i = 0; i < U; ++i) {
+          const float g = in[i] ? sc[i] : 0.0f;
+          f1[0] = fmaf(rv[i][0], g, f1[0]);
+          f1[1] = fmaf(rv[i][1], g, f1[1]);
+          f1[2] = fmaf(rv[i][2], g, f1[2]);
+          npair += in[i];
+          nghost += in[i] && __float_as_int(o[i].w) < 0;
         }
       }
       // the two lanes' sums: each step adds the same two operands on both
       for (int d = 0; d < 3; ++d) f1[d] += __shfl_xor(f1[d], 1, 64);
+      npp += (unsigned)(npair - nghost);
+      npg += (unsigned)nghost;
       if (ok && gj == 0) pp_kick(L, vsc, f1, vp, tile + (int64_t)(__float_as_uint(me.w) & 0x7fffffffu), f2, vm);
     }
   }  // claimed bricks
-  pp_reduce(out, f2, vm, nall - npg, npg, true);
+  pp_reduce(out, f2, vm, npp, npg);
 }
 
 // FP64 form: one lane per target, the pair law in FP64 with the reference's
@@ -547,7 +577,7 @@ __global__ void __launch_bounds__(256) k_pp_force64(PPLevel L, const PPBox* __re
       pp_kick(L, vsc, f, vp, tile + (int64_t)(__float_as_uint(me.w) & 0x7fffffffu), f2, vm);
     }
   }
-  pp_reduce(out, f2, vm, npp, npg, false);
+  pp_reduce(out, f2, vm, npp, npg);
 }
 
 }  // namespace
@@ -607,10 +637,10 @@ void pp_force(const PPLevel& L, int precision, const PPBox* boxes, int nbox, con
     CUBE_HIP(hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, dev));
   }
   zero_async(S.claim, sizeof(unsigned) * kPPClaimCounters * kPPClaimStride, s);
-  // as many workgroups as fit on the chip at once (eight per CU in the FP32
-  // form, the launch bound's occupancy; four in the FP64 form), each then
-  // claims bricks until none remain
-  const int per_cu = precision == 64 ? 4 : 8;
+  // as many workgroups as fit on the chip at once (the launch bound's
+  // occupancy in the FP32 form, four in the FP64 form), each then claims bricks
+  // until none remain
+  const int per_cu = precision == 64 ? 4 : pp_workgroups(unroll);
   const int64_t resident = (int64_t)n_cu * per_cu;
   // shares of a brick: enough claims that the last ones are short
   const int parts = (int)std::max<int64_t>(1, std::min<int64_t>(8, ceil_div(8 * resident, std::max<int64_t>(nbricks, 1))));
@@ -619,10 +649,10 @@ void pp_force(const PPLevel& L, int precision, const PPBox* boxes, int nbox, con
   if (precision == 64)
     hipLaunchKernelGGL(k_pp_force64, grid, dim3(256), 0, s, L, boxes, nbricks, S.start, S.entries, off, vp, out,
                        S.claim, xcd_local, parts);
-  else if (unroll == 2)
-    launch_pp_f32<2>(grid, s, L, boxes, nbricks, S, off, vp, out, xcd_local, parts);
   else if (unroll == 4)
     launch_pp_f32<4>(grid, s, L, boxes, nbricks, S, off, vp, out, xcd_local, parts);
+  else if (unroll == 6)
+    launch_pp_f32<6>(grid, s, L, boxes, nbricks, S, off, vp, out, xcd_local, parts);
   else
     launch_pp_f32<3>(grid, s, L, boxes, nbricks, S, off, vp, out, xcd_local, parts);
   CUBE_HIP(hipGetLastError());
