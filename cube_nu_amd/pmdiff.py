@@ -37,7 +37,7 @@ from .p3m import CubeError, load_library
 
 PM_ABI_FUNCTIONS = (
     "cube_pm_create", "cube_pm_destroy", "cube_pm_last_error", "cube_pm_green", "cube_pm_force",
-    "cube_pm_force_vjp", "cube_pm_cic", "cube_pm_cic_vjp", "cube_pm_cic_noalloc",
+    "cube_pm_force_vjp", "cube_pm_force_phi", "cube_pm_force_vjp_phi", "cube_pm_cic", "cube_pm_cic_vjp", "cube_pm_cic_noalloc",
 )
 
 
@@ -57,6 +57,8 @@ def _lib():
     lib.cube_pm_green.argtypes = [P, vp]
     lib.cube_pm_force.argtypes = [P, vp, i64, vp, vp, vp]
     lib.cube_pm_force_vjp.argtypes = [P, vp, i64, vp, vp, vp, vp]
+    lib.cube_pm_force_phi.argtypes = [P, vp, i64, vp, vp, vp]
+    lib.cube_pm_force_vjp_phi.argtypes = [P, vp, i64, vp, vp, vp, vp]
     lib.cube_pm_cic.argtypes = [P, vp, i64, C.c_int32, C.c_float, vp, vp]
     lib.cube_pm_cic_vjp.argtypes = [P, vp, i64, C.c_int32, C.c_float, vp, vp, vp]
     lib.cube_pm_cic_noalloc.argtypes = [P, vp, i64, C.c_int32, C.c_float, vp, vp]
@@ -137,6 +139,20 @@ class PMForce:
                                                _ptr(g.contiguous()), _ptr(gx), _stream()))
         return gx
 
+    def force_phi(self, x: torch.Tensor, phi: torch.Tensor | None) -> torch.Tensor:
+        """acc alone; the potential (batch, n, n, n) it came from goes to phi if given."""
+        acc = torch.empty_like(x)
+        self._check(self.lib.cube_pm_force_phi(self.ctx, _ptr(x), self._np(x), None if phi is None else _ptr(phi),
+                                               _ptr(acc), _stream()))
+        return acc
+
+    def force_vjp_phi(self, x: torch.Tensor, phi: torch.Tensor, g: torch.Tensor) -> torch.Tensor:
+        """force_vjp from the potential of x."""
+        gx = torch.empty_like(x)
+        self._check(self.lib.cube_pm_force_vjp_phi(self.ctx, _ptr(x), self._np(x), _ptr(phi), _ptr(g.contiguous()),
+                                                   _ptr(gx), _stream()))
+        return gx
+
     def sites(self, dtype=torch.float64, device="cpu") -> torch.Tensor:
         """Lattice site positions (np, 3) in mesh units, x fastest (lattice mode)."""
         L = self.lattice
@@ -162,15 +178,16 @@ class _ForceFn(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, pm):
         x = x.contiguous()
-        acc, F = pm.force(x)
+        phi = torch.empty((pm.batch, pm.n, pm.n, pm.n), dtype=torch.float32, device=x.device)
+        acc = pm.force_phi(x, phi)
         ctx.pm = pm
-        ctx.save_for_backward(x, F)
+        ctx.save_for_backward(x, phi)
         return acc
 
     @staticmethod
     def backward(ctx, g):
-        x, F = ctx.saved_tensors
-        return ctx.pm.force_vjp(x, F, g), None
+        x, phi = ctx.saved_tensors
+        return ctx.pm.force_vjp_phi(x, phi, g), None
 
 
 class _CICFn(torch.autograd.Function):
@@ -197,6 +214,11 @@ def cic_density(x: torch.Tensor, pm: PMForce, nw: int, scale: float) -> torch.Te
     return _CICFn.apply(x, pm, nw, scale)
 
 
+def _axpy(y, c, x):
+    """y + c x, in one kernel for an ordinary number."""
+    return torch.add(y, x, alpha=c) if isinstance(c, float) else y + c * x
+
+
 class _KDKFn(torch.autograd.Function):
     """Kick-drift-kick steps with per-step checkpoints of the positions.
 
@@ -214,13 +236,13 @@ class _KDKFn(torch.autograd.Function):
     def forward(ctx, x, v, pm, kick1, drift, kick2):
         x = x.contiguous()
         keep = [x]
-        a, _ = pm.force(x)
+        a = pm.force_phi(x, None)
         for k1, d, k2 in zip(kick1, drift, kick2):
-            v = v + k1 * a
-            x = (x + d * v).contiguous()
+            v = _axpy(v, k1, a)
+            x = _axpy(x, d, v).contiguous()
             keep.append(x)
-            a, _ = pm.force(x)
-            v = v + k2 * a
+            a = pm.force_phi(x, None)
+            v = _axpy(v, k2, a)
         ctx.pm, ctx.coef = pm, (list(kick1), list(drift), list(kick2))
         ctx.save_for_backward(*keep)
         return x, v
@@ -234,9 +256,9 @@ class _KDKFn(torch.autograd.Function):
         V = torch.zeros_like(xs[-1]) if gv is None else gv.clone()
         A = None
         for s in range(len(drift) - 1, -1, -1):
-            A = kick2[s] * V if A is None else A + kick2[s] * V
+            A = kick2[s] * V if A is None else _axpy(A, kick2[s], V)
             X = X + pm.force_vjp(xs[s + 1], None, A)
-            V = V + drift[s] * X
+            V = _axpy(V, drift[s], X)
             A = kick1[s] * V
         if A is not None:
             X = X + pm.force_vjp(xs[0], None, A)

@@ -75,6 +75,14 @@ int cube_pm_force(cube_pm_ctx* ctx, const float* x, int64_t np, float* F, float*
 int cube_pm_force_vjp(cube_pm_ctx* ctx, const float* x, int64_t np, const float* F, const float* g_acc, float* g_x,
                       void* stream);
 
+/* The same two with the potential phi (B*n^3 floats, [b][z][y][x]; a third of F)
+ * in the place of F: cube_pm_force_phi writes it (phi may be NULL: context
+ * scratch), cube_pm_force_vjp_phi reads it (or recomputes it: NULL).  The force
+ * is formed from phi where it is interpolated. */
+int cube_pm_force_phi(cube_pm_ctx* ctx, const float* x, int64_t np, float* phi, float* acc, void* stream);
+int cube_pm_force_vjp_phi(cube_pm_ctx* ctx, const float* x, int64_t np, const float* phi, const float* g_acc,
+                          float* g_x, void* stream);
+
 /* CIC density on B meshes of nw^3 points of the positions x*scale
  * (cell i covers [i, i+1), weights 1-d, d): rho (B*nw^3). */
 int cube_pm_cic(cube_pm_ctx* ctx, const float* x, int64_t np, int32_t nw, float scale, float* rho, void* stream);
