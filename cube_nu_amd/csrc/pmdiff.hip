@@ -157,9 +157,10 @@ __device__ inline void tsc_dw(float d, float dw[3]) {
   dw[2] = 0.5f + d;
 }
 
-// CIC weights on points i, i+1 (cell i covers [i, i+1)).
+// CIC: cell i = floor(x scale) in [0, nw) and f = x scale - i; weights 1 - f, f on
+// points i, i+1.
 __device__ inline void cic_point(const float* __restrict__ x, uint32_t p, uint32_t np, int nw, float scale,
-                                 const Lattice& lt, uint32_t& b, int i[3], float w[3][2]) {
+                                 const Lattice& lt, uint32_t& b, int i[3], float f[3]) {
   uint32_t c[3];
   b = site_of(p, np, lt, c);
   for (int d = 0; d < 3; ++d) {
@@ -167,10 +168,20 @@ __device__ inline void cic_point(const float* __restrict__ x, uint32_t p, uint32
     const float y = coord(x, p, d, c, lt, (double)scale, ip);
     const float fi = floorf(y);
     i[d] = wrapi((int)fi + ip, nw);
-    const float f = y - fi;
-    w[d][0] = 1.0f - f;
-    w[d][1] = f;
+    f[d] = y - fi;
   }
+}
+__device__ inline void cic_w(float f, float w[2]) {
+  w[0] = 1.0f - f;
+  w[1] = f;
+}
+
+// The point of either kind (scale is of CIC alone).
+template <bool CIC>
+__device__ inline void point(const float* __restrict__ x, uint32_t p, uint32_t np, int n, float scale,
+                             const Lattice& lt, uint32_t& b, int i[3], float d[3]) {
+  if (CIC) cic_point(x, p, np, n, scale, lt, b, i, d);
+  else tsc_point(x, p, np, n, lt, b, i, d);
 }
 
 __global__ void k_zero_u32(unsigned int* a, int64_t n) {
@@ -301,8 +312,9 @@ __device__ inline uint32_t bin_of(uint32_t b, const int i[3], int n) {
   return ((b * n + i[2]) * n + i[1]) * ((n + TX - 1) / TX * kBins) + seg * kBins + (c == 0 ? 0 : (c == w - 1 ? 2 : 1));
 }
 
+template <bool CIC>
 __global__ void __launch_bounds__(256) k_pm_count(const float* __restrict__ x, uint32_t np, uint32_t ntot, int n,
-                                                  Lattice lt, unsigned int* __restrict__ count,
+                                                  float scale, Lattice lt, unsigned int* __restrict__ count,
                                                   unsigned int* __restrict__ rank) {
   const uint32_t p = blockIdx.x * 256u + threadIdx.x;
   const int lane = threadIdx.x & 63;
@@ -311,7 +323,7 @@ __global__ void __launch_bounds__(256) k_pm_count(const float* __restrict__ x, u
     uint32_t b;
     int i[3];
     float d[3];
-    tsc_point(x, p, np, n, lt, b, i, d);
+    point<CIC>(x, p, np, n, scale, lt, b, i, d);
     bin = bin_of(b, i, n);
   }
   // the first lane of each run of equal bins adds the run's length
@@ -412,10 +424,12 @@ __global__ void __launch_bounds__(NT) k_pm_scan(unsigned int* __restrict__ count
   }
 }
 
-// The records in order.  G: with the particle's cotangent, and the slots of max |g|.
-template <bool G>
+// The records in order, with the particles, or with them and their cotangents (and
+// the slots of max |g|), or alone (CIC).
+enum class Sort { kPart, kCotangent, kCIC };
+template <Sort M>
 __global__ void __launch_bounds__(256) k_pm_sort(const float* __restrict__ x, const float* __restrict__ g, uint32_t np,
-                                                 uint32_t ntot, int n, Lattice lt,
+                                                 uint32_t ntot, int n, float scale, Lattice lt,
                                                  const unsigned int* __restrict__ start,
                                                  const unsigned int* __restrict__ rank, float4* __restrict__ rec,
                                                  unsigned int* __restrict__ part, float4* __restrict__ grec,
@@ -426,19 +440,19 @@ __global__ void __launch_bounds__(256) k_pm_sort(const float* __restrict__ x, co
     uint32_t b;
     int i[3];
     float d[3];
-    tsc_point(x, p, np, n, lt, b, i, d);
+    point<M == Sort::kCIC>(x, p, np, n, scale, lt, b, i, d);
     const uint32_t at = start[bin_of(b, i, n)] + rank[p];
     rec[at] =
         make_float4(d[0], d[1], d[2], __uint_as_float((uint32_t)i[0] | ((uint32_t)i[1] << 10) | ((uint32_t)i[2] << 20)));
-    if constexpr (G) {
+    if constexpr (M == Sort::kCotangent) {
       const float* gp = g + 3 * (int64_t)p;
       grec[at] = make_float4(gp[0], gp[1], gp[2], __uint_as_float(p));
       m = fmaxf(fabsf(gp[0]), fmaxf(fabsf(gp[1]), fabsf(gp[2])));
-    } else {
+    } else if constexpr (M == Sort::kPart) {
       part[at] = p;
     }
   }
-  if constexpr (G) {
+  if constexpr (M == Sort::kCotangent) {
     m = block_max<256>(m);
     unsigned int* slot = gmax + (blockIdx.x % kSlots) * kSlotStride;
     if (threadIdx.x == 0 && __float_as_uint(m) > *(volatile unsigned int*)slot) atomicMax(slot, __float_as_uint(m));
@@ -519,17 +533,21 @@ __device__ inline int row_of(const unsigned* pre, int rows, unsigned k) {
 // 1.8 times their particles, 8^3 by 2.0 times.  Four meshes of 256^3 with 128^3
 // particles each: 0.24 ms, NC = 3 0.53 ms (lists by tile of 8^3: 0.46 and 1.12);
 // three of 90^3, 750 000 particles: 0.065 and 0.15 ms (global atomics with their
-// pass to floats: 0.5 and 1.4).
-template <int NC>
+// pass to floats: 0.5 and 1.4).  CIC: the density of cube_pm_cic (contribution
+// u32(W 2^31)); four meshes of 128^3 with as many particles: 0.07 ms, with the sort
+// 0.18 (global atomics 0.65).
+template <int NC, bool CIC>
 __global__ void __launch_bounds__(256) k_pm_deposit(const float4* __restrict__ rec, const float4* __restrict__ grec,
                                                     int n, Tiles ts, const unsigned int* __restrict__ start,
                                                     const unsigned int* __restrict__ gmax, float* __restrict__ out) {
   constexpr int NT = 256, SY = TX + 1, SZ = TY * SY, NR = (TY + 2) * (TZ + 2);
+  constexpr int K = CIC ? 2 : 3, LO = K - 2;  // taps per axis; those below the point (CIC: only cells before reach in)
+  constexpr double kUnit = CIC ? 2147483648.0 : kFix;
   __shared__ __align__(16) unsigned long long acc[NC][TZ * SZ];
   __shared__ unsigned beg[3][NR], len[2][NR], pre[NR], wsum[NT / 64];
   const Tile t = tile_of(ts, n);
   if (t.b < 0) return;
-  const int ry = t.w[1] + 2, rows = ry * (t.w[2] + 2), nseg = (n + TX - 1) / TX;
+  const int ry = t.w[1] + 1 + LO, rows = ry * (t.w[2] + 1 + LO), nseg = (n + TX - 1) / TX;
   static_assert(NC * TZ * SZ % 2 == 0, "cleared in pairs");
   for (int q = threadIdx.x; q < NC * TZ * SZ / 2; q += NT) reinterpret_cast<ulonglong2*>(&acc[0][0])[q] = ulonglong2{};
   unsigned l[3] = {0, 0, 0};
@@ -543,8 +561,10 @@ __global__ void __launch_bounds__(256) k_pm_deposit(const float4* __restrict__ r
     l[0] = s[bb + 1] - s[bb];
     beg[1][r] = s[t.tx * kBins];
     l[1] = s[(t.tx + 1) * kBins] - s[t.tx * kBins];
-    beg[2][r] = s[sa * kBins];
-    l[2] = s[sa * kBins + 1] - s[sa * kBins];
+    if (!CIC) {
+      beg[2][r] = s[sa * kBins];
+      l[2] = s[sa * kBins + 1] - s[sa * kBins];
+    }
     len[0][r] = l[0];
     len[1][r] = l[1];
   }
@@ -575,10 +595,12 @@ __global__ void __launch_bounds__(256) k_pm_deposit(const float4* __restrict__ r
   for (unsigned k = threadIdx.x; k < total; k += NT) {
     const int lz = row / ry, cy = row - lz * ry - 1, cz = lz - 1;
     const int cx = m == 1 ? (int)(__float_as_uint(v.w) & 1023u) - t.o[0] : (m == 0 ? -1 : t.w[0]);
-    float w[3][3], gs[3] = {0, 0, 0};
-    tsc_w(v.x, w[0]);
-    tsc_w(v.y, w[1]);
-    tsc_w(v.z, w[2]);
+    float w[3][K], gs[3] = {0, 0, 0};
+    const float d[3] = {v.x, v.y, v.z};
+    for (int c = 0; c < 3; ++c) {
+      if constexpr (CIC) cic_w(d[c], w[c]);
+      else tsc_w(d[c], w[c]);
+    }
     if (NC == 3) {
       gs[0] = (float)(g.x * S);
       gs[1] = (float)(g.y * S);
@@ -586,20 +608,23 @@ __global__ void __launch_bounds__(256) k_pm_deposit(const float4* __restrict__ r
     }
     if (k + NT < total) fetch(k + NT, row, m, v, g);
 #pragma unroll
-    for (int k3 = 0; k3 < 3; ++k3) {
-      const int z = cz - 1 + k3;
+    for (int k3 = 0; k3 < K; ++k3) {
+      const int z = cz - LO + k3;
       if ((unsigned)z >= (unsigned)t.w[2]) continue;
 #pragma unroll
-      for (int k2 = 0; k2 < 3; ++k2) {
-        const int y = cy - 1 + k2;
+      for (int k2 = 0; k2 < K; ++k2) {
+        const int y = cy - LO + k2;
         if ((unsigned)y >= (unsigned)t.w[1]) continue;
         const float wyz = w[1][k2] * w[2][k3];
 #pragma unroll
-        for (int k1 = 0; k1 < 3; ++k1) {
-          const int xx = cx - 1 + k1;
+        for (int k1 = 0; k1 < K; ++k1) {
+          const int xx = cx - LO + k1;
           if ((unsigned)xx >= (unsigned)t.w[0]) continue;
           const int c = z * SZ + y * SY + xx;
-          if (NC == 1) {
+          if constexpr (CIC) {
+            const float wt = w[0][k1] * w[1][k2] * w[2][k3];
+            atomicAdd(&acc[0][c], (unsigned long long)__float2uint_rn(wt * 2147483648.0f));
+          } else if constexpr (NC == 1) {
             atomicAdd(&acc[0][c], (unsigned long long)__float2uint_rn(w[0][k1] * (wyz * 4294967296.0f)));
           } else {
             const float wt = w[0][k1] * wyz;
@@ -612,7 +637,7 @@ __global__ void __launch_bounds__(256) k_pm_deposit(const float4* __restrict__ r
   }
   __syncthreads();
   // unit is a power of two: the product is the quotient by S
-  const double unit = NC == 1 ? 1.0 / kFix : 1.0 / S;
+  const double unit = NC == 1 ? 1.0 / kUnit : 1.0 / S;
   const int64_t n3 = (int64_t)n * n * n;
   const int lx = threadIdx.x % TX, ly = (threadIdx.x / TX) % TY, lz0 = threadIdx.x / (TX * TY);
   if (lx >= t.w[0] || ly >= t.w[1]) return;
@@ -1013,8 +1038,9 @@ __global__ void k_cic_deposit(const float* __restrict__ x, uint32_t np, uint32_t
   if (p >= ntot) return;
   uint32_t b;
   int i[3];
-  float w[3][2];
-  cic_point(x, p, np, nw, scale, lt, b, i, w);
+  float f[3], w[3][2];
+  cic_point(x, p, np, nw, scale, lt, b, i, f);
+  for (int k = 0; k < 3; ++k) cic_w(f[k], w[k]);
   const int64_t n3 = (int64_t)nw * nw * nw;
   unsigned long long* a = acc + (int64_t)b * n3;
   const int xi[2] = {i[0], up1(i[0], nw)}, yi[2] = {i[1], up1(i[1], nw)}, zi[2] = {i[2], up1(i[2], nw)};
@@ -1033,8 +1059,9 @@ __global__ void k_cic_vjp(const float* __restrict__ x, uint32_t np, uint32_t nto
   if (p >= ntot) return;
   uint32_t b;
   int i[3];
-  float w[3][2];
-  cic_point(x, p, np, nw, scale, lt, b, i, w);
+  float f[3], w[3][2];
+  cic_point(x, p, np, nw, scale, lt, b, i, f);
+  for (int k = 0; k < 3; ++k) cic_w(f[k], w[k]);
   const int64_t n3 = (int64_t)nw * nw * nw;
   const float dw[2] = {-1.0f, 1.0f};
   const float* gr = grho + (int64_t)b * n3;
@@ -1076,7 +1103,17 @@ struct cube_pm_ctx {
   Lattice lat;
   std::string err;
 
-  int64_t nbins() const { return (int64_t)cfg.batch * cfg.n * cfg.n * ((cfg.n + TX - 1) / TX) * kBins; }
+  int64_t nbins(int64_t m) const { return cfg.batch * m * m * ceil_div(m, TX) * kBins; }
+  static bool capturing(hipStream_t s) {
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    return hipStreamIsCapturing(s, &st) != hipSuccess || st != hipStreamCaptureStatusNone;
+  }
+  // the buffers of an order of ntot particles on meshes of m^3 are there, or can be made
+  bool can_sort(int64_t ntot, int64_t m, size_t have, hipStream_t s) const {
+    if (m > 1024 || nbins(m) >= ((int64_t)1 << 31)) return false;
+    return ((size_t)nbins(m) <= bcount.n && (size_t)ntot <= rank.n && (size_t)ntot <= rec.n && (size_t)ntot <= have) ||
+           !capturing(s);
+  }
   // Many particles are sorted first; below these numbers the launches of that form
   // cost more than the global atomics of the other (which also serves meshes
   // beyond 1024 points, and a stream under capture whose order buffers would have
@@ -1085,27 +1122,28 @@ struct cube_pm_ctx {
   // at 64^3 58 / 52 (4096), 58 / 69 (8192), 59 / 102 (16384), at 128^3 104 / 92, 105
   // / 110, 105 / 147.
   static constexpr int64_t kSortFrom = 16384, kSortFromG = 8192;
+  // CIC densities, eight atomics a particle (sorted / not, us): on 64^3 20 / 13
+  // (16384), 20 / 28 (65536), 34 / 94 (262144), on 256^3 54 / 50, 59 / 68, 72 / 137;
+  // meshes below 8 points are all halo.
+  static constexpr int64_t kCICSortFrom = 65536;
   bool sorted(int64_t ntot, bool with_g, hipStream_t s) const {
-    if (ntot < (with_g ? kSortFromG : kSortFrom) || cfg.n > 1024 || nbins() >= ((int64_t)1 << 31)) return false;
-    if (bcount.p && (size_t)ntot <= rec.n && (size_t)ntot <= (with_g ? grec.n : part.n)) return true;
-    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-    return hipStreamIsCapturing(s, &st) == hipSuccess && st == hipStreamCaptureStatusNone;
+    return ntot >= (with_g ? kSortFromG : kSortFrom) && can_sort(ntot, cfg.n, with_g ? grec.n : part.n, s);
   }
-  // the order of x, with the cotangents g and the slots of their maximum (g may be null)
-  void sort(const float* x, const float* g, int64_t np, hipStream_t s) {
-    const int n = cfg.n;
-    const int64_t ntot = np * cfg.batch, nb = nbins();
+  // bin counts, starts and places of x on meshes of m^3 (and gmax cleared)
+  template <bool CIC>
+  void bin(const float* x, int64_t np, int m, float scale, hipStream_t s) {
+    const int64_t ntot = np * cfg.batch, nb = nbins(m);
     const bool few = nb <= 1 << 20;
     const unsigned nch = (unsigned)ceil_div(nb, few ? 1024 : 8192);
-    if (!bcount.p) {
-      bstart.ensure((size_t)nb + 1);
-      bsums.ensure(nch);
-      hipLaunchKernelGGL(k_zero_u32, dim3(nblk(nb)), dim3(256), 0, s, bcount.ensure((size_t)nb), nb);
-    }
+    bsums.ensure((size_t)ceil_div(nb, 1024));
+    bstart.ensure((size_t)nb + 1);
     rank.ensure((size_t)ntot);
     rec.ensure((size_t)ntot);
-    const uint32_t unp = (uint32_t)np, untot = (uint32_t)ntot;
-    hipLaunchKernelGGL(k_pm_count, dim3(nblk(ntot)), dim3(256), 0, s, x, unp, untot, n, lat, bcount.p, rank.p);
+    if ((size_t)nb > bcount.n)
+      hipLaunchKernelGGL(k_zero_u32, dim3(nblk(nb)), dim3(256), 0, s, bcount.ensure((size_t)nb), nb);
+    const uint32_t untot = (uint32_t)ntot;
+    hipLaunchKernelGGL(k_pm_count<CIC>, dim3(nblk(ntot)), dim3(256), 0, s, x, (uint32_t)np, untot, m, scale, lat,
+                       bcount.p, rank.p);
     if (few) {
       hipLaunchKernelGGL(k_pm_sums<128>, dim3(nch), dim3(128), 0, s, bcount.p, nb, bsums.p);
       hipLaunchKernelGGL(k_pm_scan<128>, dim3(nch), dim3(128), 0, s, bcount.p, nb, bsums.p, bstart.p, untot, gmax.p);
@@ -1113,13 +1151,24 @@ struct cube_pm_ctx {
       hipLaunchKernelGGL(k_pm_sums<1024>, dim3(nch), dim3(1024), 0, s, bcount.p, nb, bsums.p);
       hipLaunchKernelGGL(k_pm_scan<1024>, dim3(nch), dim3(1024), 0, s, bcount.p, nb, bsums.p, bstart.p, untot, gmax.p);
     }
-    if (g)
-      hipLaunchKernelGGL((k_pm_sort<true>), dim3(nblk(ntot)), dim3(256), 0, s, x, g, unp, untot, n, lat, bstart.p,
-                         rank.p, rec.p, nullptr, grec.ensure((size_t)ntot), gmax.p);
-    else
-      hipLaunchKernelGGL((k_pm_sort<false>), dim3(nblk(ntot)), dim3(256), 0, s, x, nullptr, unp, untot, n, lat,
-                         bstart.p, rank.p, rec.p, part.ensure((size_t)ntot), nullptr, nullptr);
+  }
+  template <Sort M>
+  void place(const float* x, const float* g, int64_t np, int m, float scale, hipStream_t s) {
+    const int64_t ntot = np * cfg.batch;
+    hipLaunchKernelGGL(k_pm_sort<M>, dim3(nblk(ntot)), dim3(256), 0, s, x, g, (uint32_t)np, (uint32_t)ntot, m, scale,
+                       lat, bstart.p, rank.p, rec.p, part.p, grec.p, gmax.p);
     CUBE_HIP(hipGetLastError());
+  }
+  // the order of x, with the cotangents g and the slots of their maximum (g may be null)
+  void sort(const float* x, const float* g, int64_t np, hipStream_t s) {
+    bin<false>(x, np, cfg.n, 1.0f, s);
+    if (g) {
+      grec.ensure((size_t)(np * cfg.batch));
+      place<Sort::kCotangent>(x, g, np, cfg.n, 1.0f, s);
+    } else {
+      part.ensure((size_t)(np * cfg.batch));
+      place<Sort::kPart>(x, g, np, cfg.n, 1.0f, s);
+    }
   }
   static unsigned few_blocks(int64_t ntot) { return (unsigned)ceil_div(ntot, kFew / 3); }
 
@@ -1150,7 +1199,7 @@ struct cube_pm_ctx {
     const Tiles tiles(n, B);
     if (srt) {
       sort(x, g, np, s);
-      hipLaunchKernelGGL((k_pm_deposit<1>), dim3(tiles.blocks()), dim3(256), 0, s, rec.p, nullptr, n, tiles,
+      hipLaunchKernelGGL((k_pm_deposit<1, false>), dim3(tiles.blocks()), dim3(256), 0, s, rec.p, nullptr, n, tiles,
                          bstart.p, nullptr, phi);
     } else {
       hipLaunchKernelGGL(k_tsc_deposit<1>, dim3(few_blocks(ntot)), dim3(64), 0, s, x, nullptr, (uint32_t)np,
@@ -1194,7 +1243,7 @@ struct cube_pm_ctx {
       sort(x, g, np, s);
     }
     if (srt) {
-      hipLaunchKernelGGL((k_pm_deposit<3>), dim3(tiles.blocks()), dim3(256), 0, s, rec.p, grec.p, n, tiles, bstart.p, gmax.p,
+      hipLaunchKernelGGL((k_pm_deposit<3, false>), dim3(tiles.blocks()), dim3(256), 0, s, rec.p, grec.p, n, tiles, bstart.p, gmax.p,
                          Fbar.p);
     } else {
       if (!F) {
@@ -1341,6 +1390,15 @@ int cube_pm_cic(cube_pm_ctx* ctx, const float* x, int64_t np, int32_t nw, float 
     const hipStream_t s = (hipStream_t)stream;
     const int B = ctx->cfg.batch;
     const int64_t ntot = np * B, nw3 = (int64_t)nw * nw * nw;
+    if (nw >= 8 && ntot >= cube_pm_ctx::kCICSortFrom && ctx->can_sort(ntot, nw, SIZE_MAX, s)) {
+      const Tiles tiles(nw, B);
+      ctx->bin<true>(x, np, nw, scale, s);
+      ctx->place<Sort::kCIC>(x, nullptr, np, nw, scale, s);
+      hipLaunchKernelGGL((k_pm_deposit<1, true>), dim3(tiles.blocks()), dim3(256), 0, s, ctx->rec.p, nullptr, nw, tiles,
+                         ctx->bstart.p, nullptr, rho);
+      CUBE_HIP(hipGetLastError());
+      return;
+    }
     if (ctx->nw_alloc != nw) {
       ctx->accw.release();
       ctx->accw.ensure((size_t)(B * nw3));

@@ -6,7 +6,9 @@ multiple of four points (quads); half of the particles crowded into one cell, so
 that a tile's list is far longer than its workgroup.  Both forms add the same
 integers, so their potentials are equal bit for bit; forces and adjoints agree
 with the FP64 model within the bounds of test_pmdiff.py (rms 1e-5 and 1e-4), in
-each form and with F, phi or neither given.
+each form and with F, phi or neither given.  CIC densities take the sorted form
+from 65536 particles on; cube_pm_cic_noalloc keeps the atomics, and the two are
+equal bit for bit (17 and 33 points end in a tile of one cell).
 """
 import pytest
 import torch
@@ -62,3 +64,18 @@ def test_sorted_and_unsorted_forms_agree(n, batch, lattice):
         assert _rel(v, gx_ref) <= 1e-4, k
     pm.close()
     few.close()
+
+
+@pytest.mark.parametrize("nw,batch,lattice", [(8, 2, 0), (17, 1, 0), (24, 2, 0), (33, 1, 0), (50, 2, 32), (2, 1, 0)])
+def test_sorted_cic_is_the_atomics_cic(nw, batch, lattice):
+    n, m = 32, lattice ** 3 if lattice else 65536 // batch
+    gen = torch.Generator().manual_seed(nw)
+    x = (torch.rand((batch * m, 3), generator=gen) - 0.25) * 2 * n  # beyond the box on both sides
+    x[::2] = torch.tensor([n - 0.2, 0.0, 0.5 * n]) + 0.3 * torch.rand((len(x[::2]), 3), generator=gen)
+    x = x.cuda()
+    pm = pmdiff.PMForce(n, batch, 1.0, lattice=lattice)
+    rho, want = pm.cic(x, nw, nw / n), torch.empty((batch, nw, nw, nw), device="cuda")
+    rc = pm.lib.cube_pm_cic_noalloc(pm.ctx, pmdiff._ptr(x), m, nw, nw / n, pmdiff._ptr(want), pmdiff._stream())
+    assert rc == 0 and torch.equal(rho, want)
+    assert torch.equal(pm.cic(x, nw, nw / n), want)  # counts and starts of a second call
+    pm.close()
