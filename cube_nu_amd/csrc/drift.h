@@ -14,12 +14,14 @@ struct DriftParams {
   double inv_rcs;  // 1/rcs, exact (rcs is a power of two), so x * inv_rcs == x / rcs
   int M[3];       // maximum |cell shift| per axis
   int D[3];       // 2M+1
+  int ring;       // buffer cells around the tile whose particles are sources (ncb, or max M)
+  bool images;    // buffers are images of physical particles, velocities included
 };
 
 struct DriftScratch {
   int32_t* flags = nullptr;     // [0] error bits, [1..3] max shift per axis
   int32_t* rank = nullptr;      // per source particle
-  int32_t* table = nullptr;     // per source cell per direction (count -> offset)
+  int32_t* table = nullptr;     // per source cell (nt + 2 ring a side) per direction (count -> offset)
   int64_t table_cap = 0;        // int32 elements
   int32_t* newcount = nullptr;  // ntiles * nt^3 physical destination counts
   int64_t* base = nullptr;      // ntiles * nt^3 + 1 (scan of newcount)
@@ -39,16 +41,15 @@ void drift_tile_check(const int64_t* off, int64_t ncell_tile, int ntiles, int64_
 // Pass 1: destination range check and maximum shift.
 void drift_shift(const DriftParams& P, const void* xp, const float* vp, const int32_t* rhoc, const int64_t* off,
                  int64_t ncells, DriftScratch& S, hipStream_t s);
-// Passes 2-5 for tiles [t0, t1): rank, offsets, scatter (base scan done by caller).
-// count = true folds pass 1 into the rank pass for all tiles at once, with
-// P.M an upper bound of the cell shift given by the caller (flags as pass 1,
-// plus DRIFT_SHIFT_BOUND when a shift exceeds P.M).
-void drift_rank(const DriftParams& P, const void* xp, const float* vp, const int32_t* rhoc, const int64_t* off,
-                int t0, int t1, DriftScratch& S, hipStream_t s, bool count = false);
-void drift_offsets(const DriftParams& P, int t0, int t1, DriftScratch& S, hipStream_t s);
-void drift_scatter(const DriftParams& P, const void* xp, const float* vp, const int64_t* pid, const int32_t* rhoc,
-                   const int64_t* off, int t0, int t1, DriftScratch& S, void* xp_out, float* vp_out,
-                   int64_t* pid_out, hipStream_t s);
+// Passes 2-5 for tiles [t0, t1): rank, offsets, scatter (base scan done by caller
+// before the scatter).  count = true folds pass 1 into the rank pass (all tiles
+// at once; flags as pass 1, plus DRIFT_SHIFT_BOUND when a shift exceeds P.M, then an
+// upper bound given by the caller) and the destination counts into the offsets.
+void drift_rank(const DriftParams& P, const void* xp, const float* vp, const int64_t* off, int t0, int t1,
+                DriftScratch& S, hipStream_t s, bool count = false);
+void drift_offsets(const DriftParams& P, int t0, int t1, DriftScratch& S, hipStream_t s, bool count = false);
+void drift_scatter(const DriftParams& P, const void* xp, const float* vp, const int64_t* pid, const int64_t* off,
+                   int t0, int t1, DriftScratch& S, void* xp_out, float* vp_out, int64_t* pid_out, hipStream_t s);
 // rhoc with zero buffers and physical counts from newcount.
 void drift_write_rhoc(const DriftParams& P, const DriftScratch& S, int32_t* rhoc_out, hipStream_t s);
 

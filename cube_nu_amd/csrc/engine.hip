@@ -168,6 +168,7 @@ struct cube_p3m_ctx {
   // buffer cells as periodic images of the physical ones: 1 by construction
   // (the buffer step), 0 not looked at yet (uploaded state), -1 they are not
   int images = 0;
+  bool vimages = false;       // buffer velocities, too, are those of the physical particles
   bool image_meshes = false;  // this kick's densities may be cut from whole-image meshes
   DevBuf<int32_t> dbad;
   DevBuf<char> stencil;  // coarse-level deposit: 27 tap sums per coarse cell
@@ -1101,6 +1102,8 @@ void cube_p3m_ctx::kick(const cube_kick_in& in, cube_kick_out& out, float* densi
   std::memset(&out, 0, sizeof(out));
   ensure_offsets();
   const int mask = in.phase_mask ? in.phase_mask : 15;
+  vimages = false;  // physical velocities change; buffer_v follows them
+  if (nu) nu->vimages = false;
   std::vector<int32_t> ires_h(g.ns3, 2), cmax_h(g.ns3, 0);
   struct Hold {  // the workspace budget is read once per kick, so both passes batch alike
     int64_t& w;
@@ -1169,6 +1172,7 @@ void cube_p3m_ctx::kick(const cube_kick_in& in, cube_kick_out& out, float* densi
   out.dt_vmax = (0.9f * 14.0f) / std::max({vmax[0], vmax[1], vmax[2]});  // kick.f90:314
   // every physical particle took the last phase's kick, whose vmax covers it
   vmax_valid = mask == 15;
+  vimages = with_buffer_v && images == 1;
   for (int d = 0; d < 3; ++d) last_vmax[d] = vmax[d];
   out.vz_max = vmax[2];                                                     // kick.f90:315
 }
@@ -1198,11 +1202,15 @@ void cube_p3m_ctx::drift(const cube_drift_in& in, cube_drift_out& out) {
   // passes before the read write scratch arrays only)
   auto start_pass = [&]() {
     zero_async(S.flags, sizeof(int32_t) * 8, s);
-    zero_async(S.newcount, sizeof(int32_t) * nphys_cells, s);
     drift_tile_check(off.p, g.ncell_tile, (int)g.ntiles, g.np_tile_max, S.flags, s);
   };
+  P.ring = (int)g.ncb;
+  auto table_cells = [&]() {  // source cells of a tile
+    const int64_t na = g.nt + 2 * P.ring;
+    return na * na * na;
+  };
   auto table_tiles = [&](int64_t Dt) {  // tiles per rank/offset batch within a 2 GiB table
-    const int64_t per_tile = g.ncell_tile * Dt;
+    const int64_t per_tile = table_cells() * Dt;
     const int64_t tbudget = std::max<int64_t>(per_tile, ((int64_t)2 << 30) / 4);
     return (int)std::max<int64_t>(1, std::min<int64_t>(g.ntiles, tbudget / per_tile));
   };
@@ -1221,14 +1229,14 @@ void cube_p3m_ctx::drift(const cube_drift_in& in, cube_drift_out& out) {
     if (fl[0] & DRIFT_OUT_OF_RANGE)
       throw Error(CUBE_ERR_OUT_OF_RANGE, "error: particle out of range (drift beyond 2*ncb coarse cells)");
   };
-  auto offsets_scatter = [&](int t0, int t1) {
-    {
-      KScope k(&tm, "drift_offsets", (double)(t1 - t0) * nt3 * P.D[0] * P.D[1] * P.D[2] * 8);
-      drift_offsets(P, t0, t1, S, s);
-    }
+  auto offsets = [&](int t0, int t1, bool count) {
+    KScope k(&tm, "drift_offsets", (double)(t1 - t0) * nt3 * P.D[0] * P.D[1] * P.D[2] * 8);
+    drift_offsets(P, t0, t1, S, s, count);
+  };
+  auto scatter = [&](int t0, int t1) {
     {
       KScope k(&tm, "drift_scatter", (double)np * 2 * (3 * esz() + 20) * (t1 - t0) / g.ntiles);
-      drift_scatter(P, xpc(), vpc(), pidc(), rhocc(), off.p, t0, t1, S, xp[other].p, vp[other].p,
+      drift_scatter(P, xpc(), vpc(), pidc(), off.p, t0, t1, S, xp[other].p, vp[other].p,
                     has_pid ? pid[other].p : nullptr, s);
     }
   };
@@ -1246,6 +1254,13 @@ void cube_p3m_ctx::drift(const cube_drift_in& in, cube_drift_out& out) {
     if (!(dm <= (double)kMaxShift)) fused = false;
     else Mb[d] = (int)std::ceil(dm);
   }
+  // Sources beyond the bound send nothing if every buffer particle moves as the
+  // physical one it is an image of.
+  const int far = std::max({Mb[0], Mb[1], Mb[2]});
+  if (fused && vimages && images == 1 && far <= (int)g.ncb) {
+    P.images = true;
+    P.ring = far;
+  }
   if (fused) fused = table_tiles((int64_t)(2 * Mb[0] + 1) * (2 * Mb[1] + 1) * (2 * Mb[2] + 1)) == (int)g.ntiles;
   if (fused) {
     for (int d = 0; d < 3; ++d) {
@@ -1253,22 +1268,25 @@ void cube_p3m_ctx::drift(const cube_drift_in& in, cube_drift_out& out) {
       P.D[d] = 2 * Mb[d] + 1;
     }
     const int64_t Dt = (int64_t)P.D[0] * P.D[1] * P.D[2];
-    S.table = dtable.ensure((size_t)(g.ntiles * g.ncell_tile * Dt));
+    S.table = dtable.ensure((size_t)(g.ntiles * table_cells() * Dt));
     start_pass();
-    zero_async(S.table, sizeof(int32_t) * (size_t)(g.ntiles * g.ncell_tile * Dt), s);
     {
       KScope k(&tm, "drift_rank", (double)np * (3 * esz() + 16));
-      drift_rank(P, xpc(), vpc(), rhocc(), off.p, 0, (int)g.ntiles, S, s, true);
+      drift_rank(P, xpc(), vpc(), off.p, 0, (int)g.ntiles, S, s, true);
     }
+    offsets(0, (int)g.ntiles, true);
     count_scan();
     if (fl[0] & DRIFT_SHIFT_BOUND) fused = false;
     else {
       ensure_set(other, nplocal);
-      offsets_scatter(0, (int)g.ntiles);
+      scatter(0, (int)g.ntiles);
     }
   }
   if (!fused) {
+    P.images = false;
+    P.ring = (int)g.ncb;
     start_pass();
+    zero_async(S.newcount, sizeof(int32_t) * nphys_cells, s);
     {
       KScope k(&tm, "drift_shift", (double)np * (3 * esz() + 12));
       drift_shift(P, xpc(), vpc(), rhocc(), off.p, g.ncells_ext, S, s);
@@ -1282,15 +1300,15 @@ void cube_p3m_ctx::drift(const cube_drift_in& in, cube_drift_out& out) {
     ensure_set(other, nplocal);
     const int64_t Dt = (int64_t)P.D[0] * P.D[1] * P.D[2];
     const int tg = table_tiles(Dt);
-    S.table = dtable.ensure((size_t)(tg * g.ncell_tile * Dt));
+    S.table = dtable.ensure((size_t)(tg * table_cells() * Dt));
     for (int t0 = 0; t0 < (int)g.ntiles; t0 += tg) {
       const int t1 = std::min<int>((int)g.ntiles, t0 + tg);
-      zero_async(S.table, sizeof(int32_t) * (size_t)(t1 - t0) * g.ncell_tile * Dt, s);
       {
         KScope k(&tm, "drift_rank", (double)np * (3 * esz() + 16) * (t1 - t0) / g.ntiles);
-        drift_rank(P, xpc(), vpc(), rhocc(), off.p, t0, t1, S, s);
+        drift_rank(P, xpc(), vpc(), off.p, t0, t1, S, s);
       }
-      offsets_scatter(t0, t1);
+      offsets(t0, t1, false);
+      scatter(t0, t1);
     }
   }
   int32_t* rnew = rhoc[1 - rcur].p;
@@ -1338,6 +1356,7 @@ void cube_p3m_ctx::buffer(int64_t* np_ext) {
   cur = other;
   layout = 1;
   images = 1;
+  vimages = true;
   np = n;
   off_valid = true;
   if (np_ext) *np_ext = n;
@@ -1349,6 +1368,7 @@ void cube_p3m_ctx::buffer_vel() {
   ensure_offsets();
   KScope k(&tm, "buffer_v", (double)np * 12);
   buffer_v(g, off.p, vpc(), nullptr, s);
+  vimages = images == 1;
 }
 
 // ---------------------------------------------------------------------------
@@ -1430,6 +1450,7 @@ static void upload_ext(cube_p3m_ctx* c, const void* xp, const float* vp, const i
   c->off_valid = false;
   c->vmax_valid = false;
   c->images = 0;
+  c->vimages = false;
 }
 
 // The second species' outputs of a coupled kick: its PM1/PM2 maxima (its
@@ -1734,6 +1755,7 @@ int cube_p3m_add_thermal_velocities(cube_p3m_ctx* ctx, double v_scale, uint64_t 
     if (ctx->layout == 0) throw Error(CUBE_ERR_STATE, "no resident particles");
     if (!ctx->has_pid) throw Error(CUBE_ERR_STATE, "thermal velocities are keyed by particle ID: no resident IDs");
     if (!(v_scale >= 0.0)) throw Error(CUBE_ERR_ARG, "v_scale must be >= 0");
+    ctx->vimages = false;
     const float vz = add_thermal_velocities(ctx->vpc(), ctx->pidc(), ctx->np, v_scale, seed, ctx->s);
     ctx->vmax_valid = false;
     if (vz_max) *vz_max = vz;
