@@ -141,53 +141,49 @@ constexpr int kPB = 4;
 // of lanes read consecutive entries).
 constexpr int kPPGroup = 2;
 
-// FP32 pair law.  F(r, app) - F(r, r_pp) along the pair, divided by r: for r >
-// app it is 1/r^3 - c Q(ep)/r with ep = 2r/r_pp < 2 and Q the two polynomials of
-// F_ra (kick.f90:360-374; Q = 12/ep^2 + po(ep) above ep = 1).  Q(ep)/ep comes
-// from a cubic Hermite table over kQSeg segments of s = ep^2 in [0, 4], kept in
-// LDS: in r^2 it needs neither r nor a square root of its own.  ep = 1 is a
-// segment edge and the function is C^1 there.  Interpolation error: below 2e-6
-// of values up to 224 beyond the first segments (h^4 max|y^(4)|/384, h = 1/32);
-// in the first, where s^(3/2) is not smooth, 0.012, which is below 5e-7 of the
-// pair's force (1/r^3 dominates there): the level of FP32 rounding.
-constexpr int kQSeg = 128;
+// FP32 pair law.  F(r, app) - F(r, r_pp) = 1/r^2 - c Q(ep) for r > app, with
+// ep = 2r/r_pp < 2 and Q the two polynomials of F_ra (kick.f90:360-374; Q =
+// 12/ep^2 + po(ep) above ep = 1).  Q comes from a cubic Hermite table over kQSeg
+// segments of [0, 2] kept in LDS: ep = 1 is a segment edge and Q is C^1 there; its
+// error is below 2e-5 on |Q| <= 104 (h^4 max|Q^(4)| / 384 with h = 1/32), below
+// 1e-6 of 1/r_pp^2 in the pair force, at the level of FP32 rounding.  (A table in
+// r^2 saves two operations of a pair and 6 % of the time, but its rounding moves
+// the largest force, and with it the time step and the coordinates' last bits.)
+constexpr int kQSeg = 64;
 
-__device__ inline void q_over_ep(double s, bool outer, double& y, double& dy) {
-  const double e = sqrt(s);
+__device__ inline void q_branch(double e, bool outer, double& q, double& dq) {
   if (outer) {
-    y = 12.0 / (e * e * e) - 224.0 / e + ((((7.0 * e - 48.0) * e + 70.0) * e + 224.0) * e - 840.0) * e + 896.0;
-    dy = (-36.0 / (e * e * e * e) + 224.0 / (e * e) + (((35.0 * e - 192.0) * e + 210.0) * e + 448.0) * e - 840.0) /
-         (2.0 * e);
+    q = 12.0 / (e * e) + (((((7.0 * e - 48.0) * e + 70.0) * e + 224.0) * e - 840.0) * e + 896.0) * e - 224.0;
+    dq = -24.0 / (e * e * e) + ((((42.0 * e - 240.0) * e + 280.0) * e + 672.0) * e - 1680.0) * e + 896.0;
   } else {
-    y = 224.0 + s * (-224.0 + e * (70.0 + e * (48.0 - 21.0 * e)));
-    dy = -224.0 + e * (105.0 + e * (96.0 - 52.5 * e));
+    q = e * (224.0 + e * e * (-224.0 + e * (70.0 + e * (48.0 - 21.0 * e))));
+    dq = 224.0 + e * e * (-672.0 + e * (280.0 + e * (240.0 - 126.0 * e)));
   }
 }
 
-// Segment i of the table: scale * y(i h + f h) = ((c.w f + c.z) f + c.y) f + c.x;
-// entry kQSeg holds the end value (an r^2 just below the range may round to it).
-__device__ inline void fill_qtab(float4* tab, double scale) {
-  for (int i = threadIdx.x; i <= kQSeg; i += blockDim.x) {
-    const double h = 4.0 / kQSeg;
-    const bool outer = i >= kQSeg / 4;
+// Segment s of the table: Q(s h + f h) = ((c.w f + c.z) f + c.y) f + c.x; entry
+// kQSeg holds the last one's value at f = 1 (an r just below r_pp may round to it).
+__device__ inline void fill_qtab(float4* tab) {
+  for (int sg = threadIdx.x; sg <= kQSeg; sg += blockDim.x) {
+    const double h = 2.0 / kQSeg;
+    const int i = min(sg, kQSeg - 1);
+    const bool outer = i >= kQSeg / 2;
     double y0, d0, y1, d1;
-    q_over_ep(i * h, outer, y0, d0);
-    q_over_ep((i + 1) * h, outer, y1, d1);
-    y0 *= scale;
-    y1 *= scale;
-    d0 *= h * scale;
-    d1 *= h * scale;
-    tab[i] = i == kQSeg ? make_float4((float)y0, 0.0f, 0.0f, 0.0f)
-                        : make_float4((float)y0, (float)d0, (float)(3.0 * (y1 - y0) - 2.0 * d0 - d1),
-                                      (float)(2.0 * (y0 - y1) + d0 + d1));
+    q_branch(i * h, outer, y0, d0);
+    q_branch((i + 1) * h, outer, y1, d1);
+    d0 *= h;
+    d1 *= h;
+    const float4 c = make_float4((float)y0, (float)d0, (float)(3.0 * (y1 - y0) - 2.0 * d0 - d1),
+                                 (float)(2.0 * (y0 - y1) + d0 + d1));
+    tab[sg] = sg < kQSeg ? c : make_float4(((c.w + c.z) + c.y) + c.x, 0.0f, 0.0f, 0.0f);
   }
 }
 
-// F(r, r_pp)/r at ts = r^2 kQSeg / r_pp^2 (beyond the range: its end value).
-__device__ inline float f_range(const float4* tab, float ts) {
-  ts = fminf(ts, (float)kQSeg);
-  const float4 c = tab[(int)ts];
-  const float f = __builtin_amdgcn_fractf(ts);
+// Q(2r/r_pp) at t = r kQSeg / r_pp (beyond the range: its end value).
+__device__ inline float q_range(const float4* tab, float t) {
+  t = fminf(t, (float)kQSeg);
+  const float4 c = tab[(int)t];
+  const float f = __builtin_amdgcn_fractf(t);
   return fmaf(fmaf(fmaf(c.w, f, c.z), f, c.y), f, c.x);
 }
 
@@ -363,14 +359,15 @@ __device__ inline void pp_kick(const PPLevel& L, double vsc, const float f[3], f
 // array is padded, so the reads need no clamp) and tested with the reference's
 // FP32 operations on exact positions: the interacting set is the reference's.
 // Both members of a physical pair evaluate it, and a target's partial sums are
-// added in a fixed order, so the result is deterministic.
+// added in a fixed order (its columns in turn, each dealt to the two lanes), so the
+// result is deterministic.
 //
 // U reads in flight per lane against wavefronts per SIMD: 3 with eight (64
 // VGPRs) is the fastest on long lists of short runs, whose reads miss L1 (512^3
-// at z = 2: 21.7 ms; 4 with eight 22.6, 6 with five 25.8), 6 with five (96
-// VGPRs) on the long runs of clustered input (192^3 at z = 0.5: 2.8 ms against
-// 3.2), 4 with seven between them (64^3); the engine's autotuner picks.  At 512^3
-// (2.85e9 pairs) 21.7 ms are 5.3 TFLOP/s at 40 flops a pair (25.4 ms with the
+// at z = 2: 23.2 ms; 4 with eight 23.6, 6 with five 27), 6 with five (96
+// VGPRs) on the long runs of clustered input (192^3 at z = 0.5: 3.0 ms against
+// 3.5), 4 with seven between them (64^3); the engine's autotuner picks.  At 512^3
+// (2.85e9 pairs) 23.2 ms are 4.9 TFLOP/s at 40 flops a pair (25.4 ms with the
 // columns walked in step and a branch per pair); TA is busy 80% and VALU 68% of
 // the cycles.  Slower, on the form with columns in step: candidates staged in
 // LDS (50 KB a workgroup leave three wavefronts per SIMD), 8-byte exact-integer
@@ -390,8 +387,8 @@ __global__ void __launch_bounds__(256, pp_workgroups(U)) k_pp_force(PPLevel L, c
   __shared__ float4 qtab[kQSeg + 1];
   __shared__ int2 cols[4][32][9];
   __shared__ int64_t s_brick;
-  fill_qtab(qtab, (double)L.c_range * (double)L.two_inv_range);
-  const float tscale = (float)kQSeg / L.pp_range2;
+  fill_qtab(qtab);
+  const float tscale = L.two_inv_range * (0.5f * kQSeg);
   const double vsc = L.vdev ? *L.vdev : L.v_scale;
   const int nbr = (L.npgrid + kPB - 1) / kPB;
   const int lane = threadIdx.x & 63, gj = lane & 1;
@@ -430,21 +427,22 @@ __global__ void __launch_bounds__(256, pp_workgroups(U)) k_pp_force(PPLevel L, c
           fr[d] = xv - (float)(K.c0[d] - 1 + lc[d]);
         }
         const float u = (fr[0] + (float)(lc[0] + 1)) * (float)kSX;
-        int beg[5], n[5], mine = 0;
+        int beg[5], n[5], mine = 0;  // columns that hold any, as bits
 #pragma unroll
         for (int i = 0; i < 5; ++i) {
           const int q = 2 * i + gj;  // column (dy, dz) = (q % 3 - 1, q / 3 - 1)
           n[i] = 0;
           beg[i] = 0;
           if (q < 9) column_run(L, rs, rowt, lc[0], u, fr, q % 3 - 1, q / 3 - 1, beg[i], n[i]);
-          mine += n[i] > 0;
+          mine |= (n[i] > 0) << q;
         }
-        const int other = __shfl_xor(mine, 1, 64);
-        int w = gj ? other : 0;
-        ncol = mine + other;
+        const int all = mine | __shfl_xor(mine, 1, 64);
+        ncol = __popc(all);
 #pragma unroll
-        for (int i = 0; i < 5; ++i)
-          if (n[i] > 0) run[w++] = make_int2(beg[i], n[i]);
+        for (int i = 0; i < 5; ++i) {
+          const int q = 2 * i + gj;
+          if (n[i] > 0) run[__popc(all & ((1 << q) - 1))] = make_int2(beg[i], n[i]);
+        }
       }
       __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
       __builtin_amdgcn_wave_barrier();
@@ -478,14 +476,15 @@ __global__ void __launch_bounds__(256, pp_workgroups(U)) k_pp_force(PPLevel L, c
           in[i] = i * G < rem && 0.0f < r2[i] && r2[i] < L.pp_range2;  // exact-input FP32 test (kick.f90:525, 556)
           near = near || (in[i] && r2[i] <= L.app2);
           const float rinv = __builtin_amdgcn_rsqf(r2[i]);
-          sc[i] = fmaf(rinv * rinv, rinv, -f_range(qtab, r2[i] * tscale));
+          sc[i] = rinv * fmaf(-L.c_range, q_range(qtab, (r2[i] * rinv) * tscale), rinv * rinv);
         }
         if (__any(near)) {  // ep(r, app) <= 2: F(r, app) in full
 #pragma unroll
           for (int i = 0; i < U; ++i) {
             const float rinv = __builtin_amdgcn_rsqf(r2[i]);
+            const float r = r2[i] * rinv;
             if (in[i] && r2[i] <= L.app2)
-              sc[i] = fmaf(f_app(L, r2[i] * rinv), rinv, -f_range(qtab, r2[i] * tscale));
+              sc[i] = rinv * fmaf(-L.c_range, q_range(qtab, r * tscale), f_app(L, r));
           }
         }
 #pragma unroll
