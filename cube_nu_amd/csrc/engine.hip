@@ -162,6 +162,8 @@ struct cube_p3m_ctx {
 
   // scratch
   DevBuf<char> scan_tmp;
+  PinnedPage page;      // small read-backs
+  Transfers transfers;  // host programs' arrays
   DevBuf<char> work;
   DevBuf<float> gmesh, gfaces;  // whole-image mesh and window faces (pm_mesh.h)
   DevBuf<int4> lorg[6];         // and the windows' origins, per slot as lboxes
@@ -433,8 +435,9 @@ void cube_p3m_ctx::check_images() {
   if (images != 0) return;
   int32_t bad = 0;
   mesh_check_images((int)g.izipx, g, xpc(), rhocc(), off.p, dbad.ensure(1), s);
-  CUBE_HIP(hipMemcpyAsync(&bad, dbad.p, sizeof(bad), hipMemcpyDeviceToHost, s));
-  CUBE_HIP(hipStreamSynchronize(s));
+  ReadBack rb(page);
+  rb.get(&bad, dbad.p, sizeof(bad), s);
+  rb.wait();
   images = bad ? -1 : 1;
 }
 
@@ -520,6 +523,7 @@ void cube_p3m_ctx::run_level(int level, int slot, const std::vector<PMBox>& bx_i
       } else if (level >= 3 && pm_deposit_binned_applies(L)) {
         const int64_t nblk = nb * pm_dep_blocks(L);
         DepBins S;
+        S.page = &page;
         S.count = ldepcount[slot].ensure((size_t)nblk);
         S.start = ldepstart[slot].ensure((size_t)nblk + 1);
         S.scan_tmp = scan_scratch(nblk);
@@ -657,6 +661,7 @@ void cube_p3m_ctx::pp_phase(const std::vector<int32_t>& ires_h, const std::vecto
       S.start = lppstart[iapm].ensure((size_t)(nb * m3 + 1));
       S.scan_tmp = scan_scratch(nb * m3);
       S.scan_tmp_bytes = scan_tmp.n;
+      S.page = &page;
       S.claim = ppclaim.ensure(kPPClaimCounters * kPPClaimStride);  // the force kernel's work-queue counters
       int64_t total = 0;
       if (SZ) {
@@ -844,10 +849,11 @@ void cube_p3m_ctx::kick_pass(const cube_kick_in& in, cube_kick_out& out, float* 
   // pass's classes
   if ((mask & 12) && SZ && !classified) {
     classify_subtiles(g, cfg.ires_fixed, rhocc(), ires.p, napm.p, cmax.p, s);
-    CUBE_HIP(hipMemcpyAsync(ires_h.data(), ires.p, sizeof(int32_t) * g.ns3, hipMemcpyDeviceToHost, s));
-    CUBE_HIP(hipMemcpyAsync(cmax_h.data(), cmax.p, sizeof(int32_t) * g.ns3, hipMemcpyDeviceToHost, s));
-    CUBE_HIP(hipMemcpyAsync(out.napm, napm.p, sizeof(int32_t) * 7, hipMemcpyDeviceToHost, s));
-    CUBE_HIP(hipStreamSynchronize(s));
+    ReadBack rb(page);
+    rb.get(ires_h.data(), ires.p, sizeof(int32_t) * g.ns3, s);
+    rb.get(cmax_h.data(), cmax.p, sizeof(int32_t) * g.ns3, s);
+    rb.get(out.napm, napm.p, sizeof(int32_t) * 7, s);
+    rb.wait();
   }
   // PM3 (kick.f90:203-239)
   if ((mask & 4) && cfg.pm3) {
@@ -890,10 +896,11 @@ bool cube_p3m_ctx::classify_and_reserve(cube_kick_out& out, std::vector<int32_t>
                                         std::vector<int32_t>& cmax_h) {
   using C = typename Cplx<R>::T;
   classify_subtiles(g, cfg.ires_fixed, rhocc(), ires.p, napm.p, cmax.p, s);
-  CUBE_HIP(hipMemcpyAsync(ires_h.data(), ires.p, sizeof(int32_t) * g.ns3, hipMemcpyDeviceToHost, s));
-  CUBE_HIP(hipMemcpyAsync(cmax_h.data(), cmax.p, sizeof(int32_t) * g.ns3, hipMemcpyDeviceToHost, s));
-  CUBE_HIP(hipMemcpyAsync(out.napm, napm.p, sizeof(int32_t) * 7, hipMemcpyDeviceToHost, s));
-  CUBE_HIP(hipStreamSynchronize(s));
+  ReadBack rb(page);
+  rb.get(ires_h.data(), ires.p, sizeof(int32_t) * g.ns3, s);
+  rb.get(cmax_h.data(), cmax.p, sizeof(int32_t) * g.ns3, s);
+  rb.get(out.napm, napm.p, sizeof(int32_t) * 7, s);
+  rb.wait();
   classified = true;
   bool multi = false;  // a PM3 or PP level in several workspace batches
   {
@@ -1134,9 +1141,10 @@ void cube_p3m_ctx::kick(const cube_kick_in& in, cube_kick_out& out, float* densi
   // collect reductions
   PMOut po[4];
   PPOut pq;
-  CUBE_HIP(hipMemcpyAsync(po, pmout.p, sizeof(PMOut) * 4, hipMemcpyDeviceToHost, s));
-  CUBE_HIP(hipMemcpyAsync(&pq, ppout.p, sizeof(PPOut), hipMemcpyDeviceToHost, s));
-  CUBE_HIP(hipStreamSynchronize(s));
+  ReadBack rb(page);
+  rb.get(po, pmout.p, sizeof(PMOut) * 4, s);
+  rb.get(&pq, ppout.p, sizeof(PPOut), s);
+  rb.wait();
   auto f2 = [&](const PMOut& p) { return p.template f2max<R>(); };
   auto vm = [&](const PMOut& p, int d) { return p.template vmax<R>(d); };
   float vmax[3] = {0, 0, 0};
@@ -1215,13 +1223,14 @@ void cube_p3m_ctx::drift(const cube_drift_in& in, cube_drift_out& out) {
     return (int)std::max<int64_t>(1, std::min<int64_t>(g.ntiles, tbudget / per_tile));
   };
   auto count_scan = [&]() {  // flags and the scan of the destination counts
-    CUBE_HIP(hipMemcpyAsync(fl, S.flags, sizeof(fl), hipMemcpyDeviceToHost, s));
     {
       KScope k(&tm, "drift_scan", (double)nphys_cells * 12);
       scan(S.newcount, S.base, nphys_cells);
     }
-    CUBE_HIP(hipMemcpyAsync(&nplocal, S.base + nphys_cells, sizeof(int64_t), hipMemcpyDeviceToHost, s));
-    CUBE_HIP(hipStreamSynchronize(s));
+    ReadBack rb(page);
+    rb.get(fl, S.flags, sizeof(fl), s);
+    rb.get(&nplocal, S.base + nphys_cells, sizeof(nplocal), s);
+    rb.wait();
     if (fl[0] & DRIFT_TILE_OVERFLOW)
       throw Error(CUBE_ERR_TILE_OVERFLOW, "too many particles in this tile+buffer: " + std::to_string(fl[4]) + " > " +
                                               std::to_string(g.np_tile_max) + "; please set tile_buffer larger");
@@ -1313,8 +1322,9 @@ void cube_p3m_ctx::drift(const cube_drift_in& in, cube_drift_out& out) {
   }
   int32_t* rnew = rhoc[1 - rcur].p;
   drift_write_rhoc(P, S, rnew, s);
-  CUBE_HIP(hipMemcpyAsync(fl, S.flags, sizeof(fl), hipMemcpyDeviceToHost, s));
-  CUBE_HIP(hipStreamSynchronize(s));
+  ReadBack rb(page);
+  rb.get(fl, S.flags, sizeof(fl), s);
+  rb.wait();
   if (fl[0] & 4) throw Error(CUBE_ERR_COUNT_MISMATCH, "warning: density different (rholocal /= rhoce)");
   if (fl[0] & DRIFT_PID_ZERO) throw Error(CUBE_ERR_PID, "found pid=0");
   cur = other;
@@ -1341,8 +1351,9 @@ void cube_p3m_ctx::buffer(int64_t* np_ext) {
   scan(re, off.p, g.ncells_ext);
   scan(physcount.p, physoff.p, nphys_cells);
   int64_t n = 0;
-  CUBE_HIP(hipMemcpyAsync(&n, off.p + g.ncells_ext, sizeof(int64_t), hipMemcpyDeviceToHost, s));
-  CUBE_HIP(hipStreamSynchronize(s));
+  ReadBack rb(page);
+  rb.get(&n, off.p + g.ncells_ext, sizeof(n), s);
+  rb.wait();
   if (n > g.np_image_max)
     throw Error(CUBE_ERR_IMAGE_OVERFLOW, "too many particles in this image+buffer: " + std::to_string(n) + " > " +
                                              std::to_string(g.np_image_max) + "; please set image_buffer larger");
@@ -1440,11 +1451,11 @@ static void upload_ext(cube_p3m_ctx* c, const void* xp, const float* vp, const i
   c->ensure_set(0, std::max<int64_t>(n, 1));
   c->cur = 0;
   c->rcur = 0;
-  CUBE_HIP(hipMemcpyAsync(c->rhoc[0].p, rhoc, sizeof(int32_t) * c->g.ncells_ext, hipMemcpyHostToDevice, c->s));
-  CUBE_HIP(hipMemcpyAsync(c->xp[0].p, xp, (size_t)n * 3 * c->esz(), hipMemcpyHostToDevice, c->s));
-  CUBE_HIP(hipMemcpyAsync(c->vp[0].p, vp, sizeof(float) * 3 * n, hipMemcpyHostToDevice, c->s));
+  c->transfers.in(c->rhoc[0].p, rhoc, sizeof(int32_t) * c->g.ncells_ext, c->s);
+  c->transfers.in(c->xp[0].p, xp, (size_t)n * 3 * c->esz(), c->s);
+  c->transfers.in(c->vp[0].p, vp, sizeof(float) * 3 * n, c->s);
   c->has_pid = pid != nullptr;
-  if (pid) CUBE_HIP(hipMemcpyAsync(c->pid[0].p, pid, sizeof(int64_t) * n, hipMemcpyHostToDevice, c->s));
+  if (pid) c->transfers.in(c->pid[0].p, pid, sizeof(int64_t) * n, c->s);
   c->layout = 1;
   c->np = n;
   c->off_valid = false;
@@ -1460,8 +1471,9 @@ template <typename R>
 static void nu_outputs(cube_p3m_ctx* ctx, cube_p3m_ctx* nu, const cube_kick_in& in, int mask, cube_kick_out& o) {
   std::memset(&o, 0, sizeof(o));
   PMOut pn[4];
-  CUBE_HIP(hipMemcpyAsync(pn, nu->pmout.p, sizeof(PMOut) * 4, hipMemcpyDeviceToHost, ctx->s));
-  CUBE_HIP(hipStreamSynchronize(ctx->s));
+  ReadBack rb(ctx->page);
+  rb.get(pn, nu->pmout.p, sizeof(PMOut) * 4, ctx->s);
+  rb.wait();
   float vmax[3] = {0, 0, 0};
   for (int lv = 0; lv < 2; ++lv) {
     if (!(mask & (1 << lv))) continue;
@@ -1560,7 +1572,7 @@ int cube_p3m_particle_mesh(cube_p3m_ctx* ctx, const void* xp, float* vp, const i
     cube_kick_out o;
     if (ctx->prec == 32) ctx->kick<float>(k, o, density);
     else ctx->kick<double>(k, o, density);
-    CUBE_HIP(hipMemcpyAsync(vp, ctx->vpc(), sizeof(float) * 3 * ctx->np, hipMemcpyDeviceToHost, ctx->s));
+    ctx->transfers.out(vp, ctx->vpc(), sizeof(float) * 3 * ctx->np, ctx->s);
     CUBE_HIP(hipStreamSynchronize(ctx->s));
     if (out) *out = o;
   });
@@ -1575,7 +1587,7 @@ int cube_p3m_kick(cube_p3m_ctx* ctx, const void* xp, float* vp, const int32_t* r
     cube_kick_out o;
     if (ctx->prec == 32) ctx->kick<float>(*in, o, nullptr);
     else ctx->kick<double>(*in, o, nullptr);
-    CUBE_HIP(hipMemcpyAsync(vp, ctx->vpc(), sizeof(float) * 3 * ctx->np, hipMemcpyDeviceToHost, ctx->s));
+    ctx->transfers.out(vp, ctx->vpc(), sizeof(float) * 3 * ctx->np, ctx->s);
     CUBE_HIP(hipStreamSynchronize(ctx->s));
     if (out) *out = o;
   });
@@ -1591,10 +1603,10 @@ int cube_p3m_drift(cube_p3m_ctx* ctx, void* xp, float* vp, int64_t* pid, int32_t
     ctx->drift(*in, o);
     const int64_t n = o.nplocal;
     if (n > np) throw Error(CUBE_ERR_IMAGE_OVERFLOW, "output arrays too short for nplocal");
-    CUBE_HIP(hipMemcpyAsync(xp, ctx->xpc(), (size_t)n * 3 * ctx->esz(), hipMemcpyDeviceToHost, ctx->s));
-    CUBE_HIP(hipMemcpyAsync(vp, ctx->vpc(), sizeof(float) * 3 * n, hipMemcpyDeviceToHost, ctx->s));
-    if (pid) CUBE_HIP(hipMemcpyAsync(pid, ctx->pidc(), sizeof(int64_t) * n, hipMemcpyDeviceToHost, ctx->s));
-    CUBE_HIP(hipMemcpyAsync(rhoc, ctx->rhocc(), sizeof(int32_t) * ctx->g.ncells_ext, hipMemcpyDeviceToHost, ctx->s));
+    ctx->transfers.out(xp, ctx->xpc(), (size_t)n * 3 * ctx->esz(), ctx->s);
+    ctx->transfers.out(vp, ctx->vpc(), sizeof(float) * 3 * n, ctx->s);
+    if (pid) ctx->transfers.out(pid, ctx->pidc(), sizeof(int64_t) * n, ctx->s);
+    ctx->transfers.out(rhoc, ctx->rhocc(), sizeof(int32_t) * ctx->g.ncells_ext, ctx->s);
     CUBE_HIP(hipStreamSynchronize(ctx->s));
     // xp(:,nplocal+1:)=0 etc. (drift.f90:183-186)
     std::memset((char*)xp + (size_t)n * 3 * ctx->esz(), 0, (size_t)(np - n) * 3 * ctx->esz());
@@ -1626,21 +1638,21 @@ int cube_p3m_buffer(cube_p3m_ctx* ctx, void* xp, float* vp, int64_t* pid, int32_
     ctx->ensure_set(0, std::max<int64_t>(nplocal, 1));
     ctx->cur = 0;
     ctx->rcur = 0;
-    CUBE_HIP(hipMemcpyAsync(ctx->rhoc[0].p, rp.data(), sizeof(int32_t) * g.ncells_ext, hipMemcpyHostToDevice, ctx->s));
-    CUBE_HIP(hipMemcpyAsync(ctx->xp[0].p, xp, (size_t)nplocal * 3 * ctx->esz(), hipMemcpyHostToDevice, ctx->s));
-    CUBE_HIP(hipMemcpyAsync(ctx->vp[0].p, vp, sizeof(float) * 3 * nplocal, hipMemcpyHostToDevice, ctx->s));
+    ctx->transfers.in(ctx->rhoc[0].p, rp.data(), sizeof(int32_t) * g.ncells_ext, ctx->s);
+    ctx->transfers.in(ctx->xp[0].p, xp, (size_t)nplocal * 3 * ctx->esz(), ctx->s);
+    ctx->transfers.in(ctx->vp[0].p, vp, sizeof(float) * 3 * nplocal, ctx->s);
     ctx->has_pid = pid != nullptr;
-    if (pid) CUBE_HIP(hipMemcpyAsync(ctx->pid[0].p, pid, sizeof(int64_t) * nplocal, hipMemcpyHostToDevice, ctx->s));
+    if (pid) ctx->transfers.in(ctx->pid[0].p, pid, sizeof(int64_t) * nplocal, ctx->s);
     ctx->vmax_valid = false;
     ctx->layout = 2;
     ctx->np = nplocal;
     int64_t n = 0;
     ctx->buffer(&n);
     if (n > np_cap) throw Error(CUBE_ERR_IMAGE_OVERFLOW, "output arrays too short for the buffered layout");
-    CUBE_HIP(hipMemcpyAsync(xp, ctx->xpc(), (size_t)n * 3 * ctx->esz(), hipMemcpyDeviceToHost, ctx->s));
-    CUBE_HIP(hipMemcpyAsync(vp, ctx->vpc(), sizeof(float) * 3 * n, hipMemcpyDeviceToHost, ctx->s));
-    if (pid) CUBE_HIP(hipMemcpyAsync(pid, ctx->pidc(), sizeof(int64_t) * n, hipMemcpyDeviceToHost, ctx->s));
-    CUBE_HIP(hipMemcpyAsync(rhoc, ctx->rhocc(), sizeof(int32_t) * g.ncells_ext, hipMemcpyDeviceToHost, ctx->s));
+    ctx->transfers.out(xp, ctx->xpc(), (size_t)n * 3 * ctx->esz(), ctx->s);
+    ctx->transfers.out(vp, ctx->vpc(), sizeof(float) * 3 * n, ctx->s);
+    if (pid) ctx->transfers.out(pid, ctx->pidc(), sizeof(int64_t) * n, ctx->s);
+    ctx->transfers.out(rhoc, ctx->rhocc(), sizeof(int32_t) * g.ncells_ext, ctx->s);
     CUBE_HIP(hipStreamSynchronize(ctx->s));
     host_spine(g, rhoc, idx_b_l, idx_b_r, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr);
     if (np_ext) *np_ext = n;
@@ -1656,9 +1668,9 @@ int cube_p3m_buffer_v(cube_p3m_ctx* ctx, float* vp, int64_t* pid, const int32_t*
     ctx->ensure_set(0, std::max<int64_t>(n, 1));
     ctx->cur = 0;
     ctx->rcur = 0;
-    CUBE_HIP(hipMemcpyAsync(ctx->rhoc[0].p, rhoc, sizeof(int32_t) * g.ncells_ext, hipMemcpyHostToDevice, ctx->s));
-    CUBE_HIP(hipMemcpyAsync(ctx->vp[0].p, vp, sizeof(float) * 3 * n, hipMemcpyHostToDevice, ctx->s));
-    if (pid) CUBE_HIP(hipMemcpyAsync(ctx->pid[0].p, pid, sizeof(int64_t) * n, hipMemcpyHostToDevice, ctx->s));
+    ctx->transfers.in(ctx->rhoc[0].p, rhoc, sizeof(int32_t) * g.ncells_ext, ctx->s);
+    ctx->transfers.in(ctx->vp[0].p, vp, sizeof(float) * 3 * n, ctx->s);
+    if (pid) ctx->transfers.in(ctx->pid[0].p, pid, sizeof(int64_t) * n, ctx->s);
     ctx->layout = 1;
     ctx->np = n;
     ctx->off_valid = false;
@@ -1667,8 +1679,8 @@ int cube_p3m_buffer_v(cube_p3m_ctx* ctx, float* vp, int64_t* pid, const int32_t*
       KScope k(&ctx->tm, "buffer_v", (double)n * 12);
       buffer_v(g, ctx->off.p, ctx->vp[0].p, pid ? ctx->pid[0].p : nullptr, ctx->s);
     }
-    CUBE_HIP(hipMemcpyAsync(vp, ctx->vp[0].p, sizeof(float) * 3 * n, hipMemcpyDeviceToHost, ctx->s));
-    if (pid) CUBE_HIP(hipMemcpyAsync(pid, ctx->pid[0].p, sizeof(int64_t) * n, hipMemcpyDeviceToHost, ctx->s));
+    ctx->transfers.out(vp, ctx->vp[0].p, sizeof(float) * 3 * n, ctx->s);
+    if (pid) ctx->transfers.out(pid, ctx->pid[0].p, sizeof(int64_t) * n, ctx->s);
     CUBE_HIP(hipStreamSynchronize(ctx->s));
     ctx->layout = 0;  // positions were not uploaded
     ctx->vmax_valid = false;
@@ -1695,12 +1707,12 @@ int cube_p3m_state_download(cube_p3m_ctx* ctx, void* xp, float* vp, int64_t* pid
     const int64_t n = ctx->np;
     if (np) *np = n;
     if (n > np_cap) throw Error(CUBE_ERR_ARG, "download capacity too small");
-    if (xp) CUBE_HIP(hipMemcpyAsync(xp, ctx->xpc(), (size_t)n * 3 * ctx->esz(), hipMemcpyDeviceToHost, ctx->s));
-    if (vp) CUBE_HIP(hipMemcpyAsync(vp, ctx->vpc(), sizeof(float) * 3 * n, hipMemcpyDeviceToHost, ctx->s));
+    if (xp) ctx->transfers.out(xp, ctx->xpc(), (size_t)n * 3 * ctx->esz(), ctx->s);
+    if (vp) ctx->transfers.out(vp, ctx->vpc(), sizeof(float) * 3 * n, ctx->s);
     if (pid && ctx->has_pid)
-      CUBE_HIP(hipMemcpyAsync(pid, ctx->pidc(), sizeof(int64_t) * n, hipMemcpyDeviceToHost, ctx->s));
+      ctx->transfers.out(pid, ctx->pidc(), sizeof(int64_t) * n, ctx->s);
     if (rhoc)
-      CUBE_HIP(hipMemcpyAsync(rhoc, ctx->rhocc(), sizeof(int32_t) * ctx->g.ncells_ext, hipMemcpyDeviceToHost, ctx->s));
+      ctx->transfers.out(rhoc, ctx->rhocc(), sizeof(int32_t) * ctx->g.ncells_ext, ctx->s);
     CUBE_HIP(hipStreamSynchronize(ctx->s));
   });
 }

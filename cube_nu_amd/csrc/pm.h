@@ -6,6 +6,7 @@
 #include <type_traits>
 
 #include "common.h"
+#include "transfer.h"
 
 namespace cube {
 
@@ -123,6 +124,7 @@ struct DepBins {
   unsigned long long* ents = nullptr;  // entries
   void* scan_tmp = nullptr;
   size_t scan_tmp_bytes = 0;
+  PinnedPage* page = nullptr;  // the total's way to the host
 };
 bool pm_deposit_binned_applies(const PMLevel& L);
 int64_t pm_dep_blocks(const PMLevel& L);  // blocks per box

@@ -1238,8 +1238,9 @@ int64_t pm_dep_bin_count(int izipx, const PMLevel& L, const PMBox* boxes, int nb
   CUBE_HIP(hipGetLastError());
   scan_counts(S.count, S.start, nblk, S.scan_tmp, S.scan_tmp_bytes, s);
   int64_t total = 0;
-  CUBE_HIP(hipMemcpyAsync(&total, S.start + nblk, sizeof(int64_t), hipMemcpyDeviceToHost, s));
-  CUBE_HIP(hipStreamSynchronize(s));
+  ReadBack rb(*S.page);
+  rb.get(&total, S.start + nblk, sizeof(total), s);
+  rb.wait();
   return total;
 }
 

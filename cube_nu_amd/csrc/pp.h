@@ -1,6 +1,7 @@
 // pp.h -- short-range particle-particle force (PP_Force, kick.f90:376-588).
 #pragma once
 #include "common.h"
+#include "transfer.h"
 
 namespace cube {
 
@@ -52,6 +53,7 @@ struct PPScratch {
   unsigned* claim = nullptr;  // kPPClaimCounters * kPPClaimStride words
   void* scan_tmp = nullptr;
   size_t scan_tmp_bytes = 0;
+  PinnedPage* page = nullptr;  // the total's way to the host
 };
 
 // Bin the particles of each sub-tile (plus its ghost ring) into its PP grid.

@@ -598,8 +598,9 @@ int64_t pp_bin_count(int izipx, const PPLevel& L, const PPBox* boxes, int nbox, 
   CUBE_HIP(hipGetLastError());
   scan_counts(S.count, S.start, ncell, S.scan_tmp, S.scan_tmp_bytes, s);
   int64_t total = 0;
-  CUBE_HIP(hipMemcpyAsync(&total, S.start + ncell, sizeof(int64_t), hipMemcpyDeviceToHost, s));
-  CUBE_HIP(hipStreamSynchronize(s));
+  ReadBack rb(*S.page);
+  rb.get(&total, S.start + ncell, sizeof(total), s);
+  rb.wait();
   return total;
 }
 

@@ -1,0 +1,64 @@
+// transfer.h -- copies between host programs' arrays and the device.
+//
+// Host programs hand over ordinary (pageable) arrays, which the copy engine
+// cannot read: their bytes pass through pinned memory.  The runtime's own staging
+// is one thread's copy; here kLanes threads each copy every kLanes-th chunk through
+// two pinned buffers of their own while the engine moves the other.  Pinned arrays,
+// and those below kStageFrom, take the runtime's path.
+#pragma once
+#include "common.h"
+
+namespace cube {
+
+class Transfers {
+ public:
+  ~Transfers();
+  // host -> device, queued on s; the host array may change when it returns
+  void in(void* dev, const void* host, size_t bytes, hipStream_t s);
+  // device -> host after what s holds; the array is complete once s is synchronised
+  void out(void* host, const void* dev, size_t bytes, hipStream_t s);
+
+ private:
+  static constexpr int kLanes = 8;
+  static constexpr size_t kChunk = (size_t)2 << 20;      // 32 MB of pinned memory a context, from its first use on
+  static constexpr size_t kStageFrom = (size_t)8 << 20;
+  struct Lane {
+    char* buf[2] = {nullptr, nullptr};
+    hipEvent_t ev[2] = {nullptr, nullptr};
+  } lane_[kLanes];
+  bool make();
+  template <class Fn>
+  void run(Fn&& fn);
+};
+
+// A page of pinned memory for small results.
+struct PinnedPage {
+  static constexpr size_t kBytes = (size_t)64 << 10;
+  char* p = nullptr;
+  char* get();
+  ~PinnedPage();
+};
+
+// Small results read back together: get() queues the copies into a pinned page,
+// wait() synchronises once and hands them out (a copy to pageable memory stops the
+// host each time: 20 us).  One at a time for a page.
+class ReadBack {
+ public:
+  explicit ReadBack(PinnedPage& page) : page_(page) {}
+  ~ReadBack();
+  void get(void* dst, const void* dev, size_t bytes, hipStream_t s);
+  void wait();
+
+ private:
+  struct Item {
+    void* dst;
+    size_t at, bytes;
+  };
+  PinnedPage& page_;
+  size_t used_ = 0;
+  std::vector<Item> items_;
+  hipStream_t s_ = nullptr;
+  bool pending_ = false;
+};
+
+}  // namespace cube
