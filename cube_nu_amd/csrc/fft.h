@@ -62,6 +62,8 @@ template <typename R>
 bool fft_convolve_plane(const FFTCube<R>& c, R* rho, typename Cplx<R>::T* work, const float* G, int64_t nbox,
                         R div3, R div1, hipStream_t s, KTimer* tm, const char* tag, const FFTWindow* win);
 bool fft_plane_size(int n);  // FP32
+bool fft_convolve_plane_even(const FFTCube<float>& c, float* rho, float2* work, const float* G, int64_t nbox,
+                             float div3, float div1, hipStream_t s, KTimer* tm, const char* tag);
 template <typename R>
 bool fft_convolve_lines(const FFTCube<R>& c, R* rho, typename Cplx<R>::T* work, const float* G, int64_t nbox,
                         R div3, R div1, hipStream_t s, KTimer* tm, const char* tag);

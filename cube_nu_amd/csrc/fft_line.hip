@@ -229,9 +229,12 @@ bool fft_convolve_lines(const FFTCube<R>& c, R* rho, typename Cplx<R>::T* work, 
       CUBE_FFT_SIZE(112)
       CUBE_FFT_SIZE(128)
       CUBE_FFT_SIZE(208)
+      CUBE_FFT_SIZE(210)
       CUBE_FFT_SIZE(216)
       CUBE_FFT_SIZE(224)
+      CUBE_FFT_SIZE(234)
       CUBE_FFT_SIZE(240)
+      CUBE_FFT_SIZE(252)
       CUBE_FFT_SIZE(256)
       CUBE_FFT_SIZE(288)
 #undef CUBE_FFT_SIZE

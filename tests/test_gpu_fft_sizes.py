@@ -14,12 +14,14 @@ from cube_nu_amd import pmdiff  # noqa: E402
 from oracle import pm_torch as ref  # noqa: E402
 
 PLANES = [16, 24, 32, 40, 48, 56, 64, 72, 80, 88, 96, 104, 112, 120, 128, 144, 160, 168, 176, 192]
-LINES = [208, 216, 224, 240, 256, 288]
-GENERIC = [18, 90, 126, 200]
+EVEN = [18, 20, 22, 26, 28, 30, 36, 42, 44, 50, 52, 54, 60, 66, 70, 78, 84, 90, 98, 100, 108, 110, 126, 130, 132, 140,
+        150, 154, 156, 162, 180, 182, 196, 198]  # the other even sizes of the plane form
+LINES = [208, 210, 216, 224, 234, 240, 252, 256, 288]
+GENERIC = [200, 220, 242, 250]
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("n", PLANES + LINES + GENERIC)
+@pytest.mark.parametrize("n", PLANES + EVEN + LINES + GENERIC)
 def test_gpu_force_meshes_every_fft_size(n):
     B = 2 if n <= 128 else 1
     pm = pmdiff.PMForce(n, B, 1.0)
