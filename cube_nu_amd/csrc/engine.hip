@@ -577,7 +577,9 @@ void cube_p3m_ctx::run_level(int level, int slot, const std::vector<PMBox>& bx_i
     // second stream's list building (128-point planes of 67.5 KB: 1.9 ms
     // against 0.34 for line passes)
     if (level == 1) fft_convolve<R>(fc, mesh, cplx, G, 1, (R)0, (R)(float)n, s, &tm, tag, true);
-    else fft_convolve<R>(fc, mesh, cplx, G, nmesh, n3, (R)0, s, &tm, tag, false, direct ? &win : nullptr);  // kick.f90:846
+    else  // kick.f90:846
+      fft_convolve<R>(fc, mesh, cplx, G, nmesh, n3, (R)0, s, &tm, tag, false, direct ? &win : nullptr,
+                      (int64_t)bx_in.size());
     const int ishape = interp_shape<R>(level, (int)n, L, boxes.p, nb, in, mesh, kph == 0);
     {
       KScope k(&tm, (t + "interp_kick").c_str(), cells * sizeof(R));

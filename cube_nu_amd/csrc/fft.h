@@ -48,20 +48,25 @@ struct FFTWindow {
 template <typename R>
 bool fft_reads_windows(int n);
 
-// Sizes with a specialised form take it: plane passes (fft_plane.hip) where a
-// z-plane fits in LDS, line passes (fft_line.hip) for larger ones; the others
-// take the generic line passes.  small_lds: no pass that needs more than about
-// 40 KB of LDS per workgroup (a launch beside another stream's kernels).
+// Sizes with a specialised form take it: one pass (fft_box.hip) where a small
+// cube fits in LDS and there are many, plane passes (fft_plane.h) where a z-plane
+// fits, line passes (fft_line.hip) for larger ones; the others take the generic
+// line passes.  small_lds: no pass that needs more than about 40 KB of LDS per
+// workgroup (a launch beside another stream's kernels).  total: the cubes of the
+// whole level, of which nbox are a batch (0: nbox); the form follows it, so that
+// the workspace's batches give the same bits.
 template <typename R>
 void fft_convolve(const FFTCube<R>& c, R* rho, typename Cplx<R>::T* work, const float* G, int64_t nbox, R div3,
                   R div1, hipStream_t s, KTimer* tm = nullptr, const char* tag = "", bool small_lds = false,
-                  const FFTWindow* win = nullptr);
+                  const FFTWindow* win = nullptr, int64_t total = 0);
 
 // The specialised forms; false when n has none.
 template <typename R>
 bool fft_convolve_plane(const FFTCube<R>& c, R* rho, typename Cplx<R>::T* work, const float* G, int64_t nbox,
                         R div3, R div1, hipStream_t s, KTimer* tm, const char* tag, const FFTWindow* win);
 bool fft_plane_size(int n);  // FP32
+bool fft_convolve_boxes(int n, float* rho, const float* G, int64_t nbox, int64_t total, float div3, float div1,
+                        hipStream_t s, KTimer* tm, const char* tag, const FFTWindow* win);
 bool fft_convolve_plane_even(const FFTCube<float>& c, float* rho, float2* work, const float* G, int64_t nbox,
                              float div3, float div1, hipStream_t s, KTimer* tm, const char* tag);
 template <typename R>

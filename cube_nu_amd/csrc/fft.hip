@@ -486,10 +486,15 @@ template bool fft_reads_windows<double>(int);
 
 template <typename R>
 void fft_convolve(const FFTCube<R>& c, R* rho, typename Cplx<R>::T* work, const float* G, int64_t nbox, R div3,
-                  R div1, hipStream_t s, KTimer* tm, const char* tag, bool small_lds, const FFTWindow* win) {
+                  R div1, hipStream_t s, KTimer* tm, const char* tag, bool small_lds, const FFTWindow* win,
+                  int64_t total) {
   using C = typename Cplx<R>::T;
   if (use_plane_path()) {
     KTimer* t = tm ? tm : &null_timer();
+    if constexpr (std::is_same<R, float>::value) {
+      if (!small_lds && fft_convolve_boxes(c.n, rho, G, nbox, total > 0 ? total : nbox, div3, div1, s, t, tag, win))
+        return;
+    }
     // a plane of 88 points is the largest below 40 KB
     if (!(small_lds && c.n > 88) && fft_convolve_plane<R>(c, rho, work, G, nbox, div3, div1, s, t, tag, win)) return;
     if (win) throw Error(1, "FFT of " + std::to_string(c.n) + " points does not read windows");
@@ -532,9 +537,9 @@ void fft_convolve(const FFTCube<R>& c, R* rho, typename Cplx<R>::T* work, const 
 template struct FFTCube<float>;
 template struct FFTCube<double>;
 template void fft_convolve<float>(const FFTCube<float>&, float*, float2*, const float*, int64_t, float, float,
-                                  hipStream_t, KTimer*, const char*, bool, const FFTWindow*);
+                                  hipStream_t, KTimer*, const char*, bool, const FFTWindow*, int64_t);
 template void fft_convolve<double>(const FFTCube<double>&, double*, double2*, const float*, int64_t, double, double,
-                                   hipStream_t, KTimer*, const char*, bool, const FFTWindow*);
+                                   hipStream_t, KTimer*, const char*, bool, const FFTWindow*, int64_t);
 template void fft_r2c3d<float>(const FFTCube<float>&, const float*, float2*, int64_t, hipStream_t);
 template void fft_r2c3d<double>(const FFTCube<double>&, const double*, double2*, int64_t, hipStream_t);
 template void fft_c2r3d<float>(const FFTCube<float>&, float2*, float*, int64_t, hipStream_t);

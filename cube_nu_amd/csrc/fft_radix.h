@@ -1,5 +1,5 @@
 // fft_radix.h -- register-resident R-point DFTs for the size-specialised FFT
-// passes (fft_plane.hip, fft_line.hip), R = 2..18.
+// passes (fft_plane.h, fft_line.hip: R = 2..18; fft_box.hip: 24 and 32).
 //
 // R = 2, 3, 4, 5, 8 and 16 have their own butterflies; 7, 11 and 13 pair the
 // inputs m and R-m (half the products of the plain DFT); the other R = A B are

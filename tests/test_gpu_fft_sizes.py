@@ -21,13 +21,14 @@ GENERIC = [200, 220, 242, 250]
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("n", PLANES + EVEN + LINES + GENERIC)
-def test_gpu_force_meshes_every_fft_size(n):
-    B = 2 if n <= 128 else 1
+@pytest.mark.parametrize("n,batch", [(n, 2 if n <= 128 else 1) for n in PLANES + EVEN + LINES + GENERIC]
+                         + [(n, 512) for n in (16, 24, 32)])  # many small cubes: one workgroup each
+def test_gpu_force_meshes_every_fft_size(n, batch):
+    B = batch
     pm = pmdiff.PMForce(n, B, 1.0)
     G = torch.from_numpy(pm.green().astype(np.float64)).cuda()
     gen = torch.Generator(device="cuda").manual_seed(n)
-    np_ = min(n ** 3 // 4, 100003)
+    np_ = min(n ** 3 // 4, 200006 // B)
     x = torch.rand((B * np_, 3), generator=gen, device="cuda") * n
     _, F = pm.force(x)
     want = ref.fd_force(ref.potential(ref.deposit(x.double(), B, n), G))
