@@ -183,7 +183,7 @@ struct cube_p3m_ctx {
   DevBuf<unsigned long long> ldepents[6];
   DevBuf<PPBox> lppboxes[6];
   DevBuf<int32_t> lppcount[6];
-  DevBuf<int64_t> lppstart[6];
+  DevBuf<uint32_t> lppstart[6];
   DevBuf<float4> lppent[6];
   DevBuf<PMOut> pmout;
   DevBuf<PPOut> ppout;

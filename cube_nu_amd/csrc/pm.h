@@ -148,6 +148,8 @@ void mesh_add(R* a, const R* b, int64_t n, hipStream_t s);
 
 // Exclusive scan of int32 counts into int64 offsets (n+1 outputs).
 void scan_counts(const int32_t* in, int64_t* out, int64_t n, void* tmp, size_t tmp_bytes, hipStream_t s);
+// 32-bit starts (of a total below 2^32: the caller reads the 64-bit total, in tmp, and checks it).
+const int64_t* scan_counts32(const int32_t* in, uint32_t* out, int64_t n, void* tmp, size_t tmp_bytes, hipStream_t s);
 size_t scan_tmp_bytes(int64_t n);
 
 }  // namespace cube

@@ -1041,68 +1041,100 @@ __global__ void k_classify(Geo g, int ires_fixed, const int32_t* __restrict__ rh
   }
 }
 
-// Three-phase exclusive scan (block sums, scan of sums, block scan + add).
-constexpr int kScanBlock = 1024;
+// Exclusive scan of counts in three passes: the sums of chunks, their scan, and
+// the chunks after the sums before them.  A thread holds eight values, in two loads,
+// and the threads' sums are scanned by wavefront shifts: the passes run at the
+// rate of their bytes (191 million sub-bins of 512^3: 0.13 + 0.09 + 0.25 ms; a step
+// of the scan per LDS round trip took 0.78 + 0.53 + 1.54, with 64-bit starts).
+constexpr int kScanThreads = 256, kScanBlock = 8 * kScanThreads;
 
-__global__ void k_scan_sums(const int32_t* __restrict__ in, int64_t n, int64_t* __restrict__ sums) {
-  __shared__ int64_t red[256];
-  const int64_t b0 = (int64_t)blockIdx.x * kScanBlock;
-  int64_t s = 0;
-  for (int q = threadIdx.x; q < kScanBlock; q += blockDim.x)
-    if (b0 + q < n) s += in[b0 + q];
-  red[threadIdx.x] = s;
-  __syncthreads();
-  for (int k = blockDim.x / 2; k > 0; k >>= 1) {
-    if ((int)threadIdx.x < k) red[threadIdx.x] += red[threadIdx.x + k];
-    __syncthreads();
+// The sum of v over the threads before this one, and over all.
+template <typename T, int NT>
+__device__ inline T scan_threads(T v, T& total) {
+  __shared__ T w[NT / 64];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  T s = v;
+  for (int o = 1; o < 64; o <<= 1) {
+    const T u = __shfl_up(s, o, 64);
+    if (lane >= o) s += u;
   }
-  if (threadIdx.x == 0) sums[blockIdx.x] = red[0];
+  __syncthreads();  // the last call's sums are read
+  if (lane == 63) w[wave] = s;
+  __syncthreads();
+  T before = 0;
+  total = 0;
+  for (int k = 0; k < NT / 64; ++k) {
+    before += k < wave ? w[k] : 0;
+    total += w[k];
+  }
+  return before + s - v;
 }
 
-__global__ void k_scan_top(int64_t* sums, int64_t nb) {
-  // single workgroup sequential-over-chunks scan of the block sums
-  __shared__ int64_t buf[1024];
-  __shared__ int64_t carry;
-  if (threadIdx.x == 0) carry = 0;
-  __syncthreads();
-  for (int64_t c0 = 0; c0 < nb; c0 += 1024) {
-    int64_t v = (c0 + threadIdx.x < nb) ? sums[c0 + threadIdx.x] : 0;
-    buf[threadIdx.x] = v;
-    __syncthreads();
-    for (int o = 1; o < 1024; o <<= 1) {
-      int64_t a = (threadIdx.x >= (unsigned)o) ? buf[threadIdx.x - o] : 0;
-      __syncthreads();
-      buf[threadIdx.x] += a;
-      __syncthreads();
+// Values i .. i+7 (zero from n on); the array is 16-byte aligned.
+__device__ inline void scan_load(const int32_t* __restrict__ in, int64_t i, int64_t n, int32_t v[8]) {
+  if (i + 8 <= n) {
+    const int4 a = *reinterpret_cast<const int4*>(in + i), b = *reinterpret_cast<const int4*>(in + i + 4);
+    v[0] = a.x, v[1] = a.y, v[2] = a.z, v[3] = a.w, v[4] = b.x, v[5] = b.y, v[6] = b.z, v[7] = b.w;
+  } else {
+    for (int k = 0; k < 8; ++k) v[k] = i + k < n ? in[i + k] : 0;
+  }
+}
+
+__global__ void __launch_bounds__(kScanThreads) k_scan_sums(const int32_t* __restrict__ in, int64_t n,
+                                                            int64_t* __restrict__ sums) {
+  int32_t v[8];
+  scan_load(in, (int64_t)blockIdx.x * kScanBlock + 8 * threadIdx.x, n, v);
+  int64_t s = 0, total;
+  for (int k = 0; k < 8; ++k) s += v[k];
+  scan_threads<int64_t, kScanThreads>(s, total);
+  if (threadIdx.x == 0) sums[blockIdx.x] = total;
+}
+
+__global__ void __launch_bounds__(1024) k_scan_top(int64_t* __restrict__ sums, int64_t nb) {
+  int64_t carry = 0;
+  for (int64_t c0 = 0; c0 < nb; c0 += 8192) {
+    const int64_t i = c0 + 8 * threadIdx.x;
+    int64_t v[8], s = 0, total;
+    for (int k = 0; k < 8; ++k) {
+      v[k] = i + k < nb ? sums[i + k] : 0;
+      s += v[k];
     }
-    if (c0 + threadIdx.x < nb) sums[c0 + threadIdx.x] = carry + buf[threadIdx.x] - v;
-    __syncthreads();
-    if (threadIdx.x == 1023) carry += buf[1023];
-    __syncthreads();
+    int64_t e = carry + scan_threads<int64_t, 1024>(s, total);
+    for (int k = 0; k < 8; ++k) {
+      if (i + k < nb) sums[i + k] = e;
+      e += v[k];
+    }
+    carry += total;
   }
   if (threadIdx.x == 0) sums[nb] = carry;
 }
 
-__global__ void k_scan_apply(const int32_t* __restrict__ in, int64_t n, const int64_t* __restrict__ sums,
-                             int64_t* __restrict__ out, int64_t nb) {
-  __shared__ int64_t buf[kScanBlock];
-  const int64_t b0 = (int64_t)blockIdx.x * kScanBlock;
-  for (int q = threadIdx.x; q < kScanBlock; q += blockDim.x) buf[q] = (b0 + q < n) ? in[b0 + q] : 0;
-  __syncthreads();
-  for (int o = 1; o < kScanBlock; o <<= 1) {
-    int64_t a[kScanBlock / 256];
-    for (int r = 0; r < kScanBlock / 256; ++r) {
-      int q = threadIdx.x + r * 256;
-      a[r] = q >= o ? buf[q - o] : 0;
-    }
-    __syncthreads();
-    for (int r = 0; r < kScanBlock / 256; ++r) buf[threadIdx.x + r * 256] += a[r];
-    __syncthreads();
+template <typename T>
+struct alignas(16) Scan8 {
+  T v[8];
+};
+template <typename T>
+__global__ void __launch_bounds__(kScanThreads) k_scan_apply(const int32_t* __restrict__ in, int64_t n,
+                                                             const int64_t* __restrict__ sums, T* __restrict__ out,
+                                                             int64_t nb) {
+  const int64_t i = (int64_t)blockIdx.x * kScanBlock + 8 * threadIdx.x;
+  int32_t v[8];
+  scan_load(in, i, n, v);
+  T s = 0, total;
+  for (int k = 0; k < 8; ++k) s += (T)v[k];
+  T e = (T)sums[blockIdx.x] + scan_threads<T, kScanThreads>(s, total);
+  Scan8<T> o;
+  for (int k = 0; k < 8; ++k) {
+    o.v[k] = e;
+    e += (T)v[k];
   }
-  const int64_t base = sums[blockIdx.x];
-  for (int q = threadIdx.x; q < kScanBlock; q += blockDim.x)
-    if (b0 + q < n) out[b0 + q] = base + buf[q] - in[b0 + q];
-  if (blockIdx.x == 0 && threadIdx.x == 0) out[n] = sums[nb];
+  if (i + 8 <= n) {
+    *reinterpret_cast<Scan8<T>*>(out + i) = o;
+  } else {
+    for (int k = 0; k < 8; ++k)
+      if (i + k < n) out[i + k] = o.v[k];
+  }
+  if (blockIdx.x == 0 && threadIdx.x == 0) out[n] = (T)sums[nb];
 }
 
 // Deposit block edge: 16 fine cells for the tile/sub-tile levels (FP32), 8
@@ -1407,18 +1439,28 @@ void classify_subtiles(const Geo& g, int ires_fixed, const int32_t* rhoc, int32_
 
 size_t scan_tmp_bytes(int64_t n) { return sizeof(int64_t) * (size_t)(ceil_div(n, kScanBlock) + 2); }
 
-void scan_counts(const int32_t* in, int64_t* out, int64_t n, void* tmp, size_t tmp_bytes, hipStream_t s) {
-  int64_t nb = ceil_div(n, kScanBlock);
+namespace {
+template <typename T>
+const int64_t* scan_any(const int32_t* in, T* out, int64_t n, void* tmp, size_t tmp_bytes, hipStream_t s) {
+  const int64_t nb = ceil_div(n, kScanBlock);
   if (tmp_bytes < scan_tmp_bytes(n)) throw Error(1, "scan scratch too small");
+  if ((((uintptr_t)in | (uintptr_t)out) & 15) != 0) throw Error(1, "scan of a misaligned array");
   int64_t* sums = (int64_t*)tmp;
-  if (nb == 0) {
-    zero_async(out, sizeof(int64_t), s);
-    return;
-  }
-  hipLaunchKernelGGL(k_scan_sums, dim3((unsigned)nb), dim3(256), 0, s, in, n, sums);
+  if (nb > 0) hipLaunchKernelGGL(k_scan_sums, dim3((unsigned)nb), dim3(kScanThreads), 0, s, in, n, sums);
   hipLaunchKernelGGL(k_scan_top, dim3(1), dim3(1024), 0, s, sums, nb);
-  hipLaunchKernelGGL(k_scan_apply, dim3((unsigned)nb), dim3(256), 0, s, in, n, sums, out, nb);
+  hipLaunchKernelGGL(k_scan_apply<T>, dim3((unsigned)std::max<int64_t>(nb, 1)), dim3(kScanThreads), 0, s, in, n, sums,
+                     out, nb);
   CUBE_HIP(hipGetLastError());
+  return sums + nb;
+}
+}  // namespace
+
+void scan_counts(const int32_t* in, int64_t* out, int64_t n, void* tmp, size_t tmp_bytes, hipStream_t s) {
+  scan_any(in, out, n, tmp, tmp_bytes, s);
+}
+
+const int64_t* scan_counts32(const int32_t* in, uint32_t* out, int64_t n, void* tmp, size_t tmp_bytes, hipStream_t s) {
+  return scan_any(in, out, n, tmp, tmp_bytes, s);
 }
 
 }  // namespace cube

@@ -47,7 +47,7 @@ constexpr int kPPClaimCounters = 8, kPPClaimStride = 32;
 // Scratch the caller provides for one level batch.
 struct PPScratch {
   int32_t* count = nullptr;   // nbox * m^3 * kSX sub-bins
-  int64_t* start = nullptr;   // nbox * m^3 * kSX + 1
+  uint32_t* start = nullptr;  // nbox * m^3 * kSX + 1
   float4* entries = nullptr;  // capacity entries + kPPPad readable padding
   int64_t capacity = 0;
   unsigned* claim = nullptr;  // kPPClaimCounters * kPPClaimStride words
