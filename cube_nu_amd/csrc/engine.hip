@@ -187,7 +187,7 @@ struct cube_p3m_ctx {
   DevBuf<float4> lppent[6];
   DevBuf<PMOut> pmout;
   DevBuf<PPOut> ppout;
-  DevBuf<int32_t> ires, napm, cmax;
+  DevBuf<int32_t> ires, cmax;
   DevBuf<unsigned> ppclaim;
   DevBuf<int32_t> dflags, drank, dtable, dnewcount;
   DevBuf<int64_t> dbase;
@@ -395,7 +395,6 @@ void cube_p3m_ctx::init() {
   tune_file_read(tune_picks);
   pmout.ensure(4);
   ppout.ensure(1);
-  napm.ensure(8);
   ires.ensure(g.ns3);
   cmax.ensure(g.ns3);
   dflags.ensure(8);
@@ -850,12 +849,13 @@ void cube_p3m_ctx::kick_pass(const cube_kick_in& in, cube_kick_out& out, float* 
   // classification (kick.f90:108-138); a compute-only pass reuses the sizing
   // pass's classes
   if ((mask & 12) && SZ && !classified) {
-    classify_subtiles(g, cfg.ires_fixed, rhocc(), ires.p, napm.p, cmax.p, s);
+    classify_subtiles(g, cfg.ires_fixed, rhocc(), ires.p, cmax.p, s);
     ReadBack rb(page);
     rb.get(ires_h.data(), ires.p, sizeof(int32_t) * g.ns3, s);
     rb.get(cmax_h.data(), cmax.p, sizeof(int32_t) * g.ns3, s);
-    rb.get(out.napm, napm.p, sizeof(int32_t) * 7, s);
     rb.wait();
+    std::fill(out.napm, out.napm + 7, 0);
+    for (int32_t r : ires_h) ++out.napm[r - 1];
   }
   // PM3 (kick.f90:203-239)
   if ((mask & 4) && cfg.pm3) {
@@ -897,12 +897,13 @@ template <typename R>
 bool cube_p3m_ctx::classify_and_reserve(cube_kick_out& out, std::vector<int32_t>& ires_h,
                                         std::vector<int32_t>& cmax_h) {
   using C = typename Cplx<R>::T;
-  classify_subtiles(g, cfg.ires_fixed, rhocc(), ires.p, napm.p, cmax.p, s);
+  classify_subtiles(g, cfg.ires_fixed, rhocc(), ires.p, cmax.p, s);
   ReadBack rb(page);
   rb.get(ires_h.data(), ires.p, sizeof(int32_t) * g.ns3, s);
   rb.get(cmax_h.data(), cmax.p, sizeof(int32_t) * g.ns3, s);
-  rb.get(out.napm, napm.p, sizeof(int32_t) * 7, s);
   rb.wait();
+  std::fill(out.napm, out.napm + 7, 0);
+  for (int32_t r : ires_h) ++out.napm[r - 1];
   classified = true;
   bool multi = false;  // a PM3 or PP level in several workspace batches
   {

@@ -720,7 +720,6 @@ __global__ void __launch_bounds__(256) k_interp(PMLevel L, const PMBox* __restri
   __syncthreads();
   // 3. particles whose floor(xpos) lies in this block
   constexpr double kRes = 1.0 / (double)(1u << XP<IZ>::B);
-  const bool unit = !L.xdiv && L.xmul == 1.0;  // one mesh cell per coarse cell (PM1)
   R vm[3] = {0, 0, 0};
   for (int i0 = threadIdx.x; i0 < total; i0 += 2 * 256) {
 #pragma unroll
@@ -750,20 +749,129 @@ __global__ void __launch_bounds__(256) k_interp(PMLevel L, const PMBox* __restri
       int f[3];
       bool mine = true;
       for (int d = 0; d < 3; ++d) {
-        if (unit) {
-          // xpos = (c-1) + (u + 1/2) 2^-B - s exactly: floor c-1-s, fraction
-          // (u + 1/2) 2^-B (exact in R), the FP64 path's values
-          f[d] = ijk[d] - 1 - B.ushift[d] - f0[d];
-          tsc_weights_frac<R>(((R)uu[d] + (R)0.5) * (R)kRes, w[d]);
-        } else {
-          const double xpos = pm_xpos(L, ijk[d], ((double)uu[d] + 0.5) * kRes, B.ushift[d]);
-          f[d] = tsc_weights<R>(xpos, w[d]) - f0[d];
-        }
+        const double xpos = pm_xpos(L, ijk[d], ((double)uu[d] + 0.5) * kRes, B.ushift[d]);
+        f[d] = tsc_weights<R>(xpos, w[d]) - f0[d];
         mine = mine && f[d] >= 0 && f[d] < BD;
       }
       if (!mine) continue;
       R dv[3];
       tsc_gather<R>(lds, FS * FS * FS, FS, FS * FS, (f[2] * FS + f[1]) * FS + f[0], w, dv);
+      for (int d = 0; d < 3; ++d) {
+        const float v = (float)kick_update((R)v0[d], dv[d], kc);
+        vp[3 * ip + d] = v;
+        vm[d] = max(vm[d], (R)fabsf(v));
+      }
+    }
+  }
+  raise_maxima<R>(f2, vm, out);
+}
+
+// The same for one mesh cell per coarse cell (PM1): every particle of a coarse cell
+// has the same 27 mesh cells, so a wavefront takes a coarse cell, one particle per
+// lane: its loads are contiguous, the next cell's are on their way meanwhile, and
+// the forces are read from LDS as broadcasts.  Blocks of 4^3 or 2^3 cells keep the
+// chip busy on small images (192^3 is 216 blocks of 8^3).  512^3 1.31 ms (4 GB, 3.1
+// TB/s; 1.35 with a search of its cell per particle), 192^3 0.09 (0.40), 128^3 0.04
+// (0.32), its FP64 form 0.06 (0.34).
+template <typename R, int IZ, int BD>
+__global__ void __launch_bounds__(256, 8) k_interp_unit(PMLevel L, const PMBox* __restrict__ boxes,
+                                                     const XT<IZ>* __restrict__ xp, float* __restrict__ vp,
+                                                     const int32_t* __restrict__ rhoc, const int64_t* __restrict__ off,
+                                                     const R* __restrict__ phi, double kc, PMOut* __restrict__ out) {
+  constexpr int FS = BD + 2, PS = BD + 6, FN = FS * FS * FS;
+  __shared__ R ps[PS * PS * PS], fs[3 * FN];
+  __shared__ int cnt[BD * BD * BD];
+  __shared__ int64_t gof[BD * BD * BD];
+  if (L.kdev) kc = *L.kdev;
+  const uint32_t nblk = (uint32_t)(L.nforce + BD - 1) / BD;
+  const uint32_t by_ = blockIdx.x / nblk, bz_ = by_ / nblk, ibox = bz_ / nblk;
+  const int f0[3] = {(int)(blockIdx.x - by_ * nblk) * BD, (int)(by_ - bz_ * nblk) * BD, (int)(bz_ - ibox * nblk) * BD};
+  const PMBox B = boxes[ibox];
+  // coarse cell i holds the particles with floor(xpos) = i - 1 - ushift
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  if (threadIdx.x < BD * BD * BD) {
+    const int l[3] = {lane % BD, (lane / BD) % BD, lane / (BD * BD)};
+    int c[3];
+    bool ok = true;
+    for (int d = 0; d < 3; ++d) {
+      c[d] = f0[d] + l[d] + 1 + B.ushift[d];
+      ok = ok && c[d] >= B.nc1[d] && c[d] <= B.nc2[d];
+    }
+    const int64_t cell = ok ? rc_index(c[0], c[1], c[2], B.T, L.nte, L.ncb) : 0;
+    cnt[lane] = ok ? rhoc[cell] : 0;
+    gof[lane] = ok ? off[cell] : 0;
+  }
+  for (int t = threadIdx.x; t < PS * PS * PS; t += 256) {
+    const int l[3] = {t % PS, (t / PS) % PS, t / (PS * PS)};
+    int a[3];
+    bool ok = true;
+    for (int d = 0; d < 3; ++d) {
+      a[d] = f0[d] - 2 + l[d] + B.org[d] - L.m0;
+      if (L.periodic) a[d] = a[d] < 0 ? a[d] + L.n : (a[d] >= L.n ? a[d] - L.n : a[d]);
+      ok = ok && a[d] >= 0 && a[d] < L.n;
+    }
+    ps[t] = ok ? phi[B.moff + ((int64_t)a[2] * L.n + a[1]) * L.n + a[0]] : (R)0;
+  }
+  __syncthreads();
+  // a cell's first 64 particles
+  constexpr R kRes = (R)1 / (R)(1u << XP<IZ>::B);
+  uint32_t un[3] = {0, 0, 0};
+  float vn[3] = {0, 0, 0};
+  auto load = [&](int c) {
+    if (lane < cnt[c]) {
+      const int64_t ip = gof[c] + lane;
+      for (int d = 0; d < 3; ++d) {
+        un[d] = XP<IZ>::raw(xp, ip, d);
+        vn[d] = vp[3 * ip + d];
+      }
+    }
+  };
+  load(wave);
+  const FDWeights<R> W;
+  R f2 = 0;
+  if (threadIdx.x < FN) {
+    const int lx = threadIdx.x % FS, ly = (threadIdx.x / FS) % FS, lz = threadIdx.x / (FS * FS);
+    const R* p = ps + ((lz + 2) * PS + ly + 2) * PS + lx + 2;
+    const int st[3] = {1, PS, PS * PS};
+    R f[3];
+    for (int d = 0; d < 3; ++d) {
+      R a = 0;
+      a = a + p[-2 * st[d]] * W.w0;
+      a = a + p[-st[d]] * W.w1;
+      a = a + p[st[d]] * W.w2;
+      a = a + p[2 * st[d]] * W.w3;
+      f[d] = a;
+      fs[d * FN + threadIdx.x] = a;
+    }
+    // f2max over force cells 1..nforce (kick.f90:717); cell f0+BD is the next
+    // block's first cell and counting it twice is harmless.
+    const int l[3] = {lx, ly, lz};
+    bool in = true;
+    for (int d = 0; d < 3; ++d) in = in && f0[d] + l[d] >= 1 && f0[d] + l[d] <= L.nforce && l[d] <= BD;
+    if (in) f2 = (f[0] * f[0] + f[1] * f[1]) + f[2] * f[2];
+  }
+  __syncthreads();
+  R vm[3] = {0, 0, 0};
+  for (int c = wave; c < BD * BD * BD; c += 4) {
+    uint32_t u[3] = {un[0], un[1], un[2]};
+    float v0[3] = {vn[0], vn[1], vn[2]};
+    const int n = cnt[c];
+    const int64_t base = gof[c];
+    if (c + 4 < BD * BD * BD) load(c + 4);
+    const int li = ((c / (BD * BD)) * FS + (c / BD) % BD) * FS + c % BD;
+    for (int l = lane; l < n; l += 64) {
+      const int64_t ip = base + l;
+      if (l != lane)
+        for (int d = 0; d < 3; ++d) {
+          u[d] = XP<IZ>::raw(xp, ip, d);
+          v0[d] = vp[3 * ip + d];
+        }
+      // xpos = (c-1) + (u + 1/2) 2^-B - s exactly: fraction (u + 1/2) 2^-B (exact in R)
+      R w[3][3], dv[3];
+      for (int d = 0; d < 3; ++d) tsc_weights_frac<R>(((R)u[d] + (R)0.5) * kRes, w[d]);
+      int lv = li;
+      asm volatile("" : "+v"(lv));  // the 81 forces are read as they are used, not held for the cell's next 64 particles
+      tsc_gather<R>(fs, FN, FS, FS * FS, lv, w, dv);
       for (int d = 0; d < 3; ++d) {
         const float v = (float)kick_update((R)v0[d], dv[d], kc);
         vp[3 * ip + d] = v;
@@ -1013,7 +1121,7 @@ __global__ void k_green(int n, float apm_soft, float apm_range, float gridsize, 
 
 // kick.f90:110-133: npc_max = maxval(rhoc(sub-tile))/64.
 __global__ void k_classify(Geo g, int ires_fixed, const int32_t* __restrict__ rhoc, int32_t* __restrict__ ires,
-                           int32_t* __restrict__ napm, int32_t* __restrict__ cmax) {
+                           int32_t* __restrict__ cmax) {
   __shared__ int32_t red[256];
   const uint32_t it = blockIdx.x;
   const uint32_t nns = (uint32_t)g.nns;
@@ -1037,7 +1145,6 @@ __global__ void k_classify(Geo g, int ires_fixed, const int32_t* __restrict__ rh
     if (ires_fixed >= 2) r = ires_fixed;  // kick.f90:131 (commented there)
     ires[it] = r;
     cmax[it] = red[0];
-    atomicAdd(&napm[r - 1], 1);
   }
 }
 
@@ -1176,6 +1283,19 @@ void launch_deposit(const PMLevel& L, const PMBox* boxes, int nbox, const void* 
 template <typename R, int IZ, int BD>
 void launch_interp_bd(const PMLevel& L, const PMBox* boxes, int nbox, const void* xp, float* vp, const int32_t* rhoc,
                       const int64_t* off, const R* phi, double kc, PMOut* out, hipStream_t s) {
+  if (!L.xdiv && L.xmul == 1.0 && L.w == 1) {
+    // blocks of 4^3 cells, or of 2^3 where those are few (us, 4^3 / 2^3): 64^3 60 / 20,
+    // 128^3 (512 blocks) 77 / 41, 192^3 (1728) 99 / 89, 512^3 (32768) 1310 / 1600
+    const int64_t n4 = (L.nforce + 3) / 4, n2 = (L.nforce + 1) / 2;
+    if (n4 * n4 * n4 * nbox < 4096)
+      hipLaunchKernelGGL((k_interp_unit<R, IZ, 2>), dim3((unsigned)(n2 * n2 * n2 * nbox)), dim3(256), 0, s, L, boxes,
+                         (const XT<IZ>*)xp, vp, rhoc, off, phi, kc, out);
+    else
+      hipLaunchKernelGGL((k_interp_unit<R, IZ, 4>), dim3((unsigned)(n4 * n4 * n4 * nbox)), dim3(256), 0, s, L, boxes,
+                         (const XT<IZ>*)xp, vp, rhoc, off, phi, kc, out);
+    CUBE_HIP(hipGetLastError());
+    return;
+  }
   const int nblk = (L.nforce + BD - 1) / BD;
   const int64_t grid = (int64_t)nblk * nblk * nblk * nbox;
   // a block reads at most (BD/w + 1)^3 coarse cells
@@ -1430,10 +1550,9 @@ void zero_async(void* p, size_t bytes, hipStream_t s) {
   CUBE_HIP(hipGetLastError());
 }
 
-void classify_subtiles(const Geo& g, int ires_fixed, const int32_t* rhoc, int32_t* ires, int32_t* napm,
-                       int32_t* cmax, hipStream_t s) {
-  zero_async(napm, sizeof(int32_t) * 7, s);
-  hipLaunchKernelGGL(k_classify, dim3((unsigned)g.ns3), dim3(256), 0, s, g, ires_fixed, rhoc, ires, napm, cmax);
+void classify_subtiles(const Geo& g, int ires_fixed, const int32_t* rhoc, int32_t* ires, int32_t* cmax,
+                       hipStream_t s) {
+  hipLaunchKernelGGL(k_classify, dim3((unsigned)g.ns3), dim3(256), 0, s, g, ires_fixed, rhoc, ires, cmax);
   CUBE_HIP(hipGetLastError());
 }
 
