@@ -76,11 +76,11 @@ void Transfers::in(void* dev, const void* host, size_t bytes, hipStream_t s) {
     CUBE_HIP(hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, s));
     return;
   }
-  const size_t n = (bytes + kChunk - 1) / kChunk;
+  const size_t step = chunk(bytes), n = (bytes + step - 1) / step;
   run([&](Lane& l, size_t i) {
     int k = 0;
     for (size_t c = i; c < n; c += kLanes, k ^= 1) {
-      const size_t at = c * kChunk, len = std::min(kChunk, bytes - at);
+      const size_t at = c * step, len = std::min(step, bytes - at);
       hipError_t e = hipEventSynchronize(l.ev[k]);  // the buffer's last copy (of an earlier call, too)
       if (e != hipSuccess) return e;
       std::memcpy(l.buf[k], (const char*)host + at, len);
@@ -97,10 +97,10 @@ void Transfers::out(void* host, const void* dev, size_t bytes, hipStream_t s) {
     CUBE_HIP(hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, s));
     return;
   }
-  const size_t n = (bytes + kChunk - 1) / kChunk;
+  const size_t step = chunk(bytes), n = (bytes + step - 1) / step;
   run([&](Lane& l, size_t i) {
     auto queue = [&](size_t c, int k) {
-      const size_t at = c * kChunk, len = std::min(kChunk, bytes - at);
+      const size_t at = c * step, len = std::min(step, bytes - at);
       hipError_t e = hipEventSynchronize(l.ev[k]);  // the buffer's last copy
       if (e == hipSuccess) e = hipMemcpyAsync(l.buf[k], (const char*)dev + at, len, hipMemcpyDeviceToHost, s);
       if (e == hipSuccess) e = hipEventRecord(l.ev[k], s);
@@ -113,7 +113,7 @@ void Transfers::out(void* host, const void* dev, size_t bytes, hipStream_t s) {
     for (size_t c = i; c < n && e == hipSuccess; c += kLanes, k ^= 1) {
       e = hipEventSynchronize(l.ev[k]);
       if (e != hipSuccess) break;
-      std::memcpy((char*)host + c * kChunk, l.buf[k], std::min(kChunk, bytes - c * kChunk));
+      std::memcpy((char*)host + c * step, l.buf[k], std::min(step, bytes - c * step));
       if (c + 2 * kLanes < n) e = queue(c + 2 * kLanes, k);
     }
     return e;
