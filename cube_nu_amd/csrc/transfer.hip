@@ -8,13 +8,12 @@
 namespace cube {
 
 namespace {
-bool pinned(const void* p) {
+// An ordinary pointer: none the runtime knows (pinned, managed or device memory goes its way).
+bool pageable(const void* p) {
   hipPointerAttribute_t a;
-  if (hipPointerGetAttributes(&a, p) != hipSuccess) {
-    (void)hipGetLastError();  // an ordinary pointer
-    return false;
-  }
-  return a.type == hipMemoryTypeHost;
+  if (hipPointerGetAttributes(&a, p) == hipSuccess) return a.type == hipMemoryTypeUnregistered;
+  (void)hipGetLastError();
+  return true;
 }
 }  // namespace
 
@@ -72,7 +71,7 @@ void Transfers::run(Fn&& fn) {
 }
 
 void Transfers::in(void* dev, const void* host, size_t bytes, hipStream_t s) {
-  if (bytes < kStageFrom || pinned(host) || !make()) {
+  if (bytes < kStageFrom || !pageable(host) || !make()) {
     CUBE_HIP(hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, s));
     return;
   }
@@ -93,7 +92,7 @@ void Transfers::in(void* dev, const void* host, size_t bytes, hipStream_t s) {
 }
 
 void Transfers::out(void* host, const void* dev, size_t bytes, hipStream_t s) {
-  if (bytes < kStageFrom || pinned(host) || !make()) {
+  if (bytes < kStageFrom || !pageable(host) || !make()) {
     CUBE_HIP(hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, s));
     return;
   }
