@@ -532,7 +532,7 @@ __device__ inline int row_of(const unsigned* pre, int rows, unsigned k) {
 // pipe (busy 98 %, with NC = 3 83 %, of the cycles): 16 x 8 x 8 cells are read by
 // 1.8 times their particles, 8^3 by 2.0 times.  Four meshes of 256^3 with 128^3
 // particles each: 0.24 ms, NC = 3 0.53 ms (lists by tile of 8^3: 0.46 and 1.12);
-// three of 90^3, 750 000 particles: 0.065 and 0.15 ms (global atomics with their
+// three of 90^3, 750 000 particles: 0.060 and 0.11 ms (global atomics with their
 // pass to floats: 0.5 and 1.4).  CIC: the density of cube_pm_cic (contribution
 // u32(W 2^31)); four meshes of 128^3 with as many particles: 0.07 ms, with the sort
 // 0.18 (global atomics 0.65).
@@ -591,8 +591,19 @@ __global__ void __launch_bounds__(256) k_pm_deposit(const float4* __restrict__ r
   };
   int row = 0, m = 0;
   float4 v{}, g{};
-  if (threadIdx.x < total) fetch(threadIdx.x, row, m, v, g);
-  for (unsigned k = threadIdx.x; k < total; k += NT) {
+  // Long lists (above a particle a cell) in 32 segments, eight to a wavefront and eight
+  // lanes to a segment: the 64 particles of a dense row would meet in the same few cells
+  // (three meshes of 90^3, 750 000 clustered particles, NC = 3: 151 us with consecutive
+  // lanes, 108 so; four of 256^3 with 225 entries a tile 529 and 584).
+  unsigned k = threadIdx.x, k1 = total, step = NT;
+  if (total > 8 * NT) {
+    const unsigned seg = (threadIdx.x >> 6) * 8 + (threadIdx.x & 7);
+    k1 = (unsigned)((uint64_t)total * (seg + 1) / 32);
+    k = (unsigned)((uint64_t)total * seg / 32) + ((threadIdx.x & 63) >> 3);
+    step = 8;
+  }
+  if (k < k1) fetch(k, row, m, v, g);
+  for (; k < k1; k += step) {
     const int lz = row / ry, cy = row - lz * ry - 1, cz = lz - 1;
     const int cx = m == 1 ? (int)(__float_as_uint(v.w) & 1023u) - t.o[0] : (m == 0 ? -1 : t.w[0]);
     float w[3][K], gs[3] = {0, 0, 0};
@@ -606,7 +617,7 @@ __global__ void __launch_bounds__(256) k_pm_deposit(const float4* __restrict__ r
       gs[1] = (float)(g.y * S);
       gs[2] = (float)(g.z * S);
     }
-    if (k + NT < total) fetch(k + NT, row, m, v, g);
+    if (k + step < k1) fetch(k + step, row, m, v, g);
 #pragma unroll
     for (int k3 = 0; k3 < K; ++k3) {
       const int z = cz - LO + k3;
