@@ -15,6 +15,7 @@
 // associative, so every output is independent of thread order.
 #include <algorithm>
 #include <cmath>
+#include <initializer_list>
 #include <mutex>
 #include <string>
 
@@ -22,6 +23,7 @@
 #include "../../include/cube_pm.h"
 #include "common.h"
 #include "fft.h"
+#include "growbuf.h"
 #include "pm.h"
 
 // The allocation-free CIC entry point's device scratch (sized and explained
@@ -31,29 +33,17 @@ static __device__ __align__(256) unsigned long long scratch[(int64_t)1 << 23];
 namespace cube {
 namespace {
 
-template <typename T>
-struct PMBuf {
-  T* p = nullptr;
-  size_t n = 0;
-  T* ensure(size_t m) {
-    if (m > n) {
-      release();
-      const hipError_t e = hipMalloc(&p, m * sizeof(T));
-      if (e != hipSuccess) {
-        p = nullptr;
-        throw Error(CUBE_ERR_HIP, "hipMalloc of " + std::to_string(m * sizeof(T)) + " bytes failed");
-      }
-      n = m;
-    }
+struct DeviceMem {
+  static void* alloc(size_t bytes) {
+    void* p = nullptr;
+    if (hipMalloc(&p, bytes) != hipSuccess)
+      throw Error(CUBE_ERR_HIP, "hipMalloc of " + std::to_string(bytes) + " bytes failed");
     return p;
   }
-  void release() {
-    if (p) (void)hipFree(p);
-    p = nullptr;
-    n = 0;
-  }
-  ~PMBuf() { release(); }
+  static void free(void* p) { (void)hipFree(p); }
 };
+template <typename T>
+using PMBuf = GrowBuf<T, DeviceMem>;
 
 constexpr double kFix = 4294967296.0;  // 2^32
 
@@ -1104,16 +1094,21 @@ struct cube_pm_ctx {
   PMBuf<float> G, mesh, Fs, Fbar;
   PMBuf<float2> work;
   PMBuf<unsigned long long> acc;   // B*3*n^3, kept zero between calls
-  PMBuf<unsigned long long> accw;  // B*nw^3 for the CIC density, kept zero
+  PMBuf<unsigned long long> accw;  // B*nw^3 of the largest CIC density so far, kept zero
   PMBuf<unsigned int> gmax;
   // the particles' order: bin counts (kept zero) and starts, chunk sums, places
   // in the bins, sorted records, particles and cotangents
   PMBuf<unsigned int> bcount, bstart, bsums, rank, part;
   PMBuf<float4> rec, grec;
-  int nw_alloc = 0;
   Lattice lat;
   std::string err;
 
+  // a captured call's graph holds the addresses of the order's buffers
+  void hold_order() {
+    for (PMBuf<unsigned int>* b : {&bcount, &bstart, &bsums, &rank, &part}) b->hold();
+    rec.hold();
+    grec.hold();
+  }
   int64_t nbins(int64_t m) const { return cfg.batch * m * m * ceil_div(m, TX) * kBins; }
   static bool capturing(hipStream_t s) {
     hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
@@ -1169,6 +1164,7 @@ struct cube_pm_ctx {
     hipLaunchKernelGGL(k_pm_sort<M>, dim3(nblk(ntot)), dim3(256), 0, s, x, g, (uint32_t)np, (uint32_t)ntot, m, scale,
                        lat, bstart.p, rank.p, rec.p, part.p, grec.p, gmax.p);
     CUBE_HIP(hipGetLastError());
+    if (capturing(s)) hold_order();
   }
   // the order of x, with the cotangents g and the slots of their maximum (g may be null)
   void sort(const float* x, const float* g, int64_t np, hipStream_t s) {
@@ -1410,12 +1406,9 @@ int cube_pm_cic(cube_pm_ctx* ctx, const float* x, int64_t np, int32_t nw, float 
       CUBE_HIP(hipGetLastError());
       return;
     }
-    if (ctx->nw_alloc != nw) {
-      ctx->accw.release();
-      ctx->accw.ensure((size_t)(B * nw3));
-      hipLaunchKernelGGL(k_zero_u64, dim3(nblk(B * nw3)), dim3(256), 0, s, ctx->accw.p, B * nw3);
-      ctx->nw_alloc = nw;
-    }
+    if ((size_t)(B * nw3) > ctx->accw.n)
+      hipLaunchKernelGGL(k_zero_u64, dim3(nblk(B * nw3)), dim3(256), 0, s, ctx->accw.ensure((size_t)(B * nw3)), B * nw3);
+    if (ctx->capturing(s)) ctx->accw.hold();
     hipLaunchKernelGGL(k_cic_deposit, dim3(nblk(ntot)), dim3(256), 0, s, x, (uint32_t)np, (uint32_t)ntot, nw, scale, ctx->lat,
                        ctx->accw.p);
     hipLaunchKernelGGL(k_fix_to_float, dim3(nblk(B * nw3)), dim3(256), 0, s, ctx->accw.p, B * nw3, 1.0 / 2147483648.0,

@@ -28,6 +28,12 @@
  * into meshes use integer (fixed-point) atomics, so every result is
  * independent of thread order.  Return codes are the CUBE_ERR_* of
  * cube_p3m.h.
+ *
+ * Capture.  A call with a stream may be recorded into a HIP graph
+ * (cube_pm_cic: after a call with the same nw), which may be replayed until
+ * cube_pm_destroy: context memory that a recorded call uses is kept until then,
+ * whatever later calls need.  The caller's own arrays, and the order of
+ * replays among the other calls on the context, are the caller's to keep.
  */
 #ifndef CUBE_PM_H
 #define CUBE_PM_H
