@@ -1397,7 +1397,13 @@ int cube_pm_cic(cube_pm_ctx* ctx, const float* x, int64_t np, int32_t nw, float 
     const hipStream_t s = (hipStream_t)stream;
     const int B = ctx->cfg.batch;
     const int64_t ntot = np * B, nw3 = (int64_t)nw * nw * nw;
-    if (nw >= 8 && ntot >= cube_pm_ctx::kCICSortFrom && ctx->can_sort(ntot, nw, SIZE_MAX, s)) {
+    const bool captured = ctx->capturing(s),
+               srt = nw >= 8 && ntot >= cube_pm_ctx::kCICSortFrom && ctx->can_sort(ntot, nw, SIZE_MAX, s);
+    // the accumulator of the form by atomics is made in either form: a call recorded
+    // later may have more particles than the order's buffers hold, and cannot allocate
+    if ((size_t)(B * nw3) > ctx->accw.n && !(captured && srt))
+      hipLaunchKernelGGL(k_zero_u64, dim3(nblk(B * nw3)), dim3(256), 0, s, ctx->accw.ensure((size_t)(B * nw3)), B * nw3);
+    if (srt) {
       const Tiles tiles(nw, B);
       ctx->bin<true>(x, np, nw, scale, s);
       ctx->place<Sort::kCIC>(x, nullptr, np, nw, scale, s);
@@ -1406,9 +1412,7 @@ int cube_pm_cic(cube_pm_ctx* ctx, const float* x, int64_t np, int32_t nw, float 
       CUBE_HIP(hipGetLastError());
       return;
     }
-    if ((size_t)(B * nw3) > ctx->accw.n)
-      hipLaunchKernelGGL(k_zero_u64, dim3(nblk(B * nw3)), dim3(256), 0, s, ctx->accw.ensure((size_t)(B * nw3)), B * nw3);
-    if (ctx->capturing(s)) ctx->accw.hold();
+    if (captured) ctx->accw.hold();
     hipLaunchKernelGGL(k_cic_deposit, dim3(nblk(ntot)), dim3(256), 0, s, x, (uint32_t)np, (uint32_t)ntot, nw, scale, ctx->lat,
                        ctx->accw.p);
     hipLaunchKernelGGL(k_fix_to_float, dim3(nblk(B * nw3)), dim3(256), 0, s, ctx->accw.p, B * nw3, 1.0 / 2147483648.0,

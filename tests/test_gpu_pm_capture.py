@@ -70,3 +70,23 @@ def test_recorded_density_after_larger_calls(m):
         assert torch.equal(rho, want), k
     pm.close()
     other.close()
+
+
+def test_recorded_density_of_more_particles_than_before():
+    """After one call with the mesh's size a recorded call takes any number of
+    particles: the form by atomics needs no memory that depends on it."""
+    pm, other = (pmdiff.PMForce(32, 1, 1.0) for _ in range(2))
+    pm.cic(_positions(70001, 32, 1), 40, 1.25)
+    x = _positions(150001, 32, 2)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        rho = pm.cic(x, 40, 1.25)
+    for k in range(3):
+        y = _positions(150001, 32, 10 + k)
+        want = other.cic(y, 40, 1.25)
+        x.copy_(y)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(rho, want), k
+    pm.close()
+    other.close()
