@@ -1123,17 +1123,40 @@ struct cube_pm_ctx {
   // Many particles are sorted first; below these numbers the launches of that form
   // cost more than the global atomics of the other (which also serves meshes
   // beyond 1024 points, and a stream under capture whose order buffers would have
-  // to grow).  Measured sorted / not, us: forces at 64^3 51 / 39 (8192 particles),
-  // 51 / 52 (16384), 53 / 75 (32768), at 128^3 87 / 62, 87 / 78, 88 / 106; adjoints
-  // at 64^3 58 / 52 (4096), 58 / 69 (8192), 59 / 102 (16384), at 128^3 104 / 92, 105
-  // / 110, 105 / 147.
+  // to grow).  Measured sorted / not, us, with phi: forces of 17000 particles on
+  // 48^3 39 / 50, 128^3 68 / 81, 256^3 302 / 317, 512^3 5480 / 5750; adjoints of 8192
+  // on 48^3 46 / 65, 128^3 83 / 114, 256^3 421 / 604, 512^3 6390 / 7700; where F is
+  // asked for, which the sorted form's gather does not read, it is up to 16 % slower on
+  // meshes of more than some 250 cells a particle (256^3, 25000: 374 / 337) and
+  // faster below (100000: 385 / 481).
   static constexpr int64_t kSortFrom = 16384, kSortFromG = 8192;
-  // CIC densities, eight atomics a particle (sorted / not, us): on 64^3 20 / 13
-  // (16384), 20 / 28 (65536), 34 / 94 (262144), on 256^3 54 / 50, 59 / 68, 72 / 137;
-  // meshes below 8 points are all halo.
-  static constexpr int64_t kCICSortFrom = 65536;
+  // A tile's particles are one workgroup's, so a mesh of a few tiles would wait for as
+  // few workgroups: the measure is the largest tile's share of the cells.  Sorted / not,
+  // us, 300000 particles: forces on 12^3 (a share of 1/2.3) 2350 / 790, 18^3 (1/5.7) 930 /
+  // 530, 22^3 (1/10) 541 / 470, 24^3 (1/14) 427 / 485; adjoints on 18^3 2000 / 1710,
+  // 20^3 (1/8) 1474 / 1473, 22^3 1135 / 1653; densities on 16^3 (1/4) 535 / 103, 24^3 174 /
+  // 126, 28^3 (1/21) 120 / 119 (130000 particles 61 / 56), 32^3 (1/32) 90 / 108 (47 / 51).
+  static constexpr int64_t kShare = 12, kShareG = 8, kShareCIC = 20, kShareCICFew = 32;
+  bool shared(int64_t m, int64_t among) const {
+    const int64_t largest = std::min<int64_t>(m, TX) * std::min<int64_t>(m, TY) * std::min<int64_t>(m, TZ);
+    return cfg.batch * m * m * m >= among * largest;
+  }
   bool sorted(int64_t ntot, bool with_g, hipStream_t s) const {
-    return ntot >= (with_g ? kSortFromG : kSortFrom) && can_sort(ntot, cfg.n, with_g ? grec.n : part.n, s);
+    return ntot >= (with_g ? kSortFromG : kSortFrom) && shared(cfg.n, with_g ? kShareG : kShare) &&
+           can_sort(ntot, cfg.n, with_g ? grec.n : part.n, s);
+  }
+  // CIC densities, eight atomics a particle, of 65536 particles anywhere (sorted / not,
+  // us: 32^3 33 / 31, 48^3 25 / 31, 256^3 59 / 68).  Sites of a lattice come in the order of
+  // the mesh, which suits the atomics as long as particles have moved little and cells
+  // hold several (rms of 0.6 and 2 spacings): 98304 particles on 8 cells each 23 / 22
+  // and 26 / 42, 110592 on one 28 / 18 and 35 / 29, 131072 on 3.4 24 / 22 and 28 / 41, 221184 on
+  // one 28 / 33 and 40 / 65, 65536 on 64 29 / 33 and 31 / 40.
+  bool cic_sorted(int64_t ntot, int64_t nw, hipStream_t s) const {
+    const int64_t cells = cfg.batch * nw * nw * nw;
+    int64_t from = lat.L == 0 ? 65536 : 60000 + 120000 * ntot / cells;
+    if (!shared(nw, kShareCICFew)) from = std::max<int64_t>(from, 262144);
+    // meshes below 8 points are all halo
+    return nw >= 8 && shared(nw, kShareCIC) && ntot >= from && can_sort(ntot, nw, SIZE_MAX, s);
   }
   // bin counts, starts and places of x on meshes of m^3 (and gmax cleared)
   template <bool CIC>
@@ -1397,8 +1420,7 @@ int cube_pm_cic(cube_pm_ctx* ctx, const float* x, int64_t np, int32_t nw, float 
     const hipStream_t s = (hipStream_t)stream;
     const int B = ctx->cfg.batch;
     const int64_t ntot = np * B, nw3 = (int64_t)nw * nw * nw;
-    const bool captured = ctx->capturing(s),
-               srt = nw >= 8 && ntot >= cube_pm_ctx::kCICSortFrom && ctx->can_sort(ntot, nw, SIZE_MAX, s);
+    const bool captured = ctx->capturing(s), srt = ctx->cic_sorted(ntot, nw, s);
     // the accumulator of the form by atomics is made in either form: a call recorded
     // later may have more particles than the order's buffers hold, and cannot allocate
     if ((size_t)(B * nw3) > ctx->accw.n && !(captured && srt))
