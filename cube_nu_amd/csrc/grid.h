@@ -1,0 +1,19 @@
+// grid.h -- blocks of a launch whose threads along x would pass 2^32.
+#pragma once
+#include <cstdint>
+
+namespace cube {
+
+// A launch dimension holds fewer than 2^32 threads, so blocks beyond 2^21 (of at
+// most 1024 threads) go on along y; block (x, y) is y * gridDim.x + x, and a kernel
+// drops those past its last.
+struct Blocks {
+  uint32_t x, y;
+};
+constexpr int64_t kBlocksX = (int64_t)1 << 21;
+constexpr Blocks blocks_xy(int64_t blocks) {
+  return blocks <= kBlocksX ? Blocks{(uint32_t)blocks, 1}
+                            : Blocks{(uint32_t)kBlocksX, (uint32_t)((blocks + kBlocksX - 1) / kBlocksX)};
+}
+
+}  // namespace cube

@@ -23,6 +23,7 @@
 #include "../../include/cube_pm.h"
 #include "common.h"
 #include "fft.h"
+#include "grid.h"
 #include "growbuf.h"
 #include "pm.h"
 
@@ -174,13 +175,18 @@ __device__ inline void point(const float* __restrict__ x, uint32_t p, uint32_t n
   else tsc_point(x, p, np, n, lt, b, i, d);
 }
 
+// Thread of a launch over the cells of meshes, whose blocks go on along y.
+__device__ inline int64_t cell_thread() {
+  return ((int64_t)blockIdx.y * gridDim.x + blockIdx.x) * blockDim.x + threadIdx.x;
+}
+
 __global__ void k_zero_u32(unsigned int* a, int64_t n) {
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const int64_t t = cell_thread();
   if (t < n) a[t] = 0;
 }
 
 __global__ void k_zero_u64(unsigned long long* a, int64_t n) {
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const int64_t t = cell_thread();
   if (t < n) a[t] = 0;
 }
 
@@ -226,14 +232,19 @@ __global__ void __launch_bounds__(1024) k_absmax(const float* __restrict__ g, in
 // one wavefront spread them over the chip).  NC = 1: rho += W (fixed point
 // 2^-32); NC = 3: Fbar[b][d] += W g_d at scale S.
 constexpr int kFew = 63;  // threads of a block that work: 21 particles
+// The particle (past the last one, none) of this thread; blocks go on along y.
+__device__ inline int64_t few_particle() {
+  return ((int64_t)blockIdx.y * gridDim.x + blockIdx.x) * (kFew / 3) + threadIdx.x / 3u;
+}
 template <int NC>
 __global__ void __launch_bounds__(64) k_tsc_deposit(const float* __restrict__ x, const float* __restrict__ g, uint32_t np, uint32_t ntot,
                               int n, Lattice lt, const unsigned int* __restrict__ gmax,
                               unsigned long long* __restrict__ acc) {
   const double S = NC == 3 ? fix_scale(gmax) : 1.0;
-  const uint32_t p = blockIdx.x * (kFew / 3) + threadIdx.x / 3u;
+  const int64_t q = few_particle();
   const int k3 = (int)(threadIdx.x % 3u);
-  if (threadIdx.x >= kFew || p >= ntot) return;
+  if (threadIdx.x >= kFew || q >= ntot) return;
+  const uint32_t p = (uint32_t)q;
   uint32_t b;
   int i[3];
   float d[3], w[3][3], gs[3] = {0, 0, 0};
@@ -266,7 +277,7 @@ __global__ void __launch_bounds__(64) k_tsc_deposit(const float* __restrict__ x,
 
 // out = acc * unit (as float), acc cleared for the next use.
 __global__ void k_fix_to_float(unsigned long long* __restrict__ acc, int64_t n, double unit, float* __restrict__ out) {
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const int64_t t = cell_thread();
   if (t >= n) return;
   out[t] = (float)((double)acc[t] * unit);
   acc[t] = 0;
@@ -276,7 +287,7 @@ __global__ void k_fix_to_float(unsigned long long* __restrict__ acc, int64_t n, 
 __global__ void k_sfix_to_float(unsigned long long* __restrict__ acc, int64_t n, const unsigned int* __restrict__ gmax,
                                 float* __restrict__ out) {
   const double S = fix_scale(gmax);
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const int64_t t = cell_thread();
   if (t >= n) return;
   out[t] = (float)((double)(long long)acc[t] / S);
   acc[t] = 0;
@@ -773,7 +784,7 @@ __device__ inline float add3(float v) {
 // acc_p = sum W F.
 __global__ void __launch_bounds__(64) k_tsc_interp(const float* __restrict__ x, uint32_t np, uint32_t ntot, int n,
                                                    Lattice lt, const float* __restrict__ F, float* __restrict__ acc) {
-  const int64_t q = (int64_t)blockIdx.x * (kFew / 3) + threadIdx.x / 3u;
+  const int64_t q = few_particle();
   const uint32_t p = (uint32_t)min(q, (int64_t)ntot - 1);
   const int k3 = (int)(threadIdx.x % 3u);
   uint32_t b;
@@ -806,7 +817,7 @@ __global__ void __launch_bounds__(64) k_tsc_interp(const float* __restrict__ x, 
 __global__ void __launch_bounds__(64) k_tsc_vjp(const float* __restrict__ x, uint32_t np, uint32_t ntot, int n,
                                                 Lattice lt, const float* __restrict__ F, const float* __restrict__ g,
                                                 const float* __restrict__ rhob, float* __restrict__ gx) {
-  const int64_t q = (int64_t)blockIdx.x * (kFew / 3) + threadIdx.x / 3u;
+  const int64_t q = few_particle();
   const uint32_t p = (uint32_t)min(q, (int64_t)ntot - 1);
   const int k3 = (int)(threadIdx.x % 3u);
   uint32_t b;
@@ -1080,6 +1091,11 @@ __global__ void k_cic_vjp(const float* __restrict__ x, uint32_t np, uint32_t nto
 }
 
 inline unsigned nblk(int64_t n, int t = 256) { return (unsigned)((n + t - 1) / t); }
+// Blocks of 256 threads over n cells (three meshes of 1126^3 are more than 2^32).
+inline dim3 cell_blocks(int64_t n) {
+  const Blocks b = blocks_xy(ceil_div(n, 256));
+  return dim3(b.x, b.y);
+}
 
 }  // namespace
 }  // namespace cube
@@ -1169,7 +1185,7 @@ struct cube_pm_ctx {
     rank.ensure((size_t)ntot);
     rec.ensure((size_t)ntot);
     if ((size_t)nb > bcount.n)
-      hipLaunchKernelGGL(k_zero_u32, dim3(nblk(nb)), dim3(256), 0, s, bcount.ensure((size_t)nb), nb);
+      hipLaunchKernelGGL(k_zero_u32, cell_blocks(nb), dim3(256), 0, s, bcount.ensure((size_t)nb), nb);
     const uint32_t untot = (uint32_t)ntot;
     hipLaunchKernelGGL(k_pm_count<CIC>, dim3(nblk(ntot)), dim3(256), 0, s, x, (uint32_t)np, untot, m, scale, lat,
                        bcount.p, rank.p);
@@ -1200,7 +1216,10 @@ struct cube_pm_ctx {
       place<Sort::kPart>(x, g, np, cfg.n, 1.0f, s);
     }
   }
-  static unsigned few_blocks(int64_t ntot) { return (unsigned)ceil_div(ntot, kFew / 3); }
+  static dim3 few_blocks(int64_t ntot) {
+    const Blocks b = blocks_xy(ceil_div(ntot, kFew / 3));
+    return dim3(b.x, b.y);
+  }
 
   void check_np(int64_t np) const {
     if (np <= 0) throw Error(CUBE_ERR_ARG, "np must be positive");
@@ -1212,6 +1231,7 @@ struct cube_pm_ctx {
   void fd(bool adjoint, const float* in, float* out, hipStream_t s) {
     const int n = cfg.n, v = quads(n, in, out) ? 4 : 1;
     const int64_t nthr = (int64_t)cfg.batch * n3 / v;
+    if (nthr > 0xffffff00ll) throw Error(CUBE_ERR_ARG, "more cells than threads in a launch");
     const dim3 grid(nblk(nthr));
     if (!adjoint && v == 4) hipLaunchKernelGGL(k_fd_force<4>, grid, dim3(256), 0, s, in, n, (uint32_t)nthr, out);
     else if (!adjoint) hipLaunchKernelGGL(k_fd_force<1>, grid, dim3(256), 0, s, in, n, (uint32_t)nthr, out);
@@ -1232,9 +1252,9 @@ struct cube_pm_ctx {
       hipLaunchKernelGGL((k_pm_deposit<1, false>), dim3(tiles.blocks()), dim3(256), 0, s, rec.p, nullptr, n, tiles,
                          bstart.p, nullptr, phi);
     } else {
-      hipLaunchKernelGGL(k_tsc_deposit<1>, dim3(few_blocks(ntot)), dim3(64), 0, s, x, nullptr, (uint32_t)np,
+      hipLaunchKernelGGL(k_tsc_deposit<1>, few_blocks(ntot), dim3(64), 0, s, x, nullptr, (uint32_t)np,
                          (uint32_t)ntot, n, lat, nullptr, acc.p);
-      hipLaunchKernelGGL(k_fix_to_float, dim3(nblk(B * n3)), dim3(256), 0, s, acc.p, B * n3, 1.0 / kFix, phi);
+      hipLaunchKernelGGL(k_fix_to_float, cell_blocks(B * n3), dim3(256), 0, s, acc.p, B * n3, 1.0 / kFix, phi);
     }
     fft_convolve<float>(fc, phi, work.p, G.p, B, (float)n3, 0.0f, s);
   }
@@ -1249,7 +1269,7 @@ struct cube_pm_ctx {
     if (!F && !srt) F = Fs.p;
     if (F) fd(false, phi, F, s);
     if (!srt)
-      hipLaunchKernelGGL(k_tsc_interp, dim3(few_blocks(ntot)), dim3(64), 0, s, x, (uint32_t)np, (uint32_t)ntot, n, lat,
+      hipLaunchKernelGGL(k_tsc_interp, few_blocks(ntot), dim3(64), 0, s, x, (uint32_t)np, (uint32_t)ntot, n, lat,
                          F, out);
     else if (quads(n, phi, nullptr))
       hipLaunchKernelGGL((k_pm_gather<false, 4>), dim3(tiles.blocks()), dim3(512), 0, s, rec.p, part.p, nullptr, n, tiles, bstart.p,
@@ -1282,14 +1302,14 @@ struct cube_pm_ctx {
       }
       hipLaunchKernelGGL(k_absmax, dim3((unsigned)std::min<int64_t>(ceil_div(3 * ntot, 4096), kSlots)), dim3(1024), 0,
                          s, g, 3 * ntot, gmax.p);
-      hipLaunchKernelGGL(k_tsc_deposit<3>, dim3(few_blocks(ntot)), dim3(64), 0, s, x, g, (uint32_t)np, (uint32_t)ntot,
+      hipLaunchKernelGGL(k_tsc_deposit<3>, few_blocks(ntot), dim3(64), 0, s, x, g, (uint32_t)np, (uint32_t)ntot,
                          n, lat, gmax.p, acc.p);
-      hipLaunchKernelGGL(k_sfix_to_float, dim3(nblk(3 * B * n3)), dim3(256), 0, s, acc.p, 3 * B * n3, gmax.p, Fbar.p);
+      hipLaunchKernelGGL(k_sfix_to_float, cell_blocks(3 * B * n3), dim3(256), 0, s, acc.p, 3 * B * n3, gmax.p, Fbar.p);
     }
     fd(true, Fbar.p, mesh.p, s);
     fft_convolve<float>(fc, mesh.p, work.p, G.p, B, (float)n3, 0.0f, s);
     if (!srt)
-      hipLaunchKernelGGL(k_tsc_vjp, dim3(few_blocks(ntot)), dim3(64), 0, s, x, (uint32_t)np, (uint32_t)ntot, n, lat, F,
+      hipLaunchKernelGGL(k_tsc_vjp, few_blocks(ntot), dim3(64), 0, s, x, (uint32_t)np, (uint32_t)ntot, n, lat, F,
                          g, mesh.p, gx);
     else if (quads(n, phi, mesh.p))
       hipLaunchKernelGGL((k_pm_gather<true, 4>), dim3(tiles.blocks()), dim3(512), 0, s, rec.p, nullptr, grec.p, n, tiles, bstart.p,
@@ -1348,7 +1368,7 @@ int cube_pm_create(const cube_pm_config* cfg, cube_pm_ctx** out) {
     c->work.ensure((size_t)(B * nk));
     c->acc.ensure((size_t)(3 * B * c->n3));
     c->gmax.ensure(kSlots * kSlotStride);
-    hipLaunchKernelGGL(k_zero_u64, dim3(nblk(3 * B * c->n3)), dim3(256), 0, nullptr, c->acc.p, 3 * B * c->n3);
+    hipLaunchKernelGGL(k_zero_u64, cell_blocks(3 * B * c->n3), dim3(256), 0, nullptr, c->acc.p, 3 * B * c->n3);
     CUBE_HIP(hipGetLastError());
     CUBE_HIP(hipDeviceSynchronize());
   });
@@ -1424,7 +1444,7 @@ int cube_pm_cic(cube_pm_ctx* ctx, const float* x, int64_t np, int32_t nw, float 
     // the accumulator of the form by atomics is made in either form: a call recorded
     // later may have more particles than the order's buffers hold, and cannot allocate
     if ((size_t)(B * nw3) > ctx->accw.n && !(captured && srt))
-      hipLaunchKernelGGL(k_zero_u64, dim3(nblk(B * nw3)), dim3(256), 0, s, ctx->accw.ensure((size_t)(B * nw3)), B * nw3);
+      hipLaunchKernelGGL(k_zero_u64, cell_blocks(B * nw3), dim3(256), 0, s, ctx->accw.ensure((size_t)(B * nw3)), B * nw3);
     if (srt) {
       const Tiles tiles(nw, B);
       ctx->bin<true>(x, np, nw, scale, s);
@@ -1437,7 +1457,7 @@ int cube_pm_cic(cube_pm_ctx* ctx, const float* x, int64_t np, int32_t nw, float 
     if (captured) ctx->accw.hold();
     hipLaunchKernelGGL(k_cic_deposit, dim3(nblk(ntot)), dim3(256), 0, s, x, (uint32_t)np, (uint32_t)ntot, nw, scale, ctx->lat,
                        ctx->accw.p);
-    hipLaunchKernelGGL(k_fix_to_float, dim3(nblk(B * nw3)), dim3(256), 0, s, ctx->accw.p, B * nw3, 1.0 / 2147483648.0,
+    hipLaunchKernelGGL(k_fix_to_float, cell_blocks(B * nw3), dim3(256), 0, s, ctx->accw.p, B * nw3, 1.0 / 2147483648.0,
                        rho);
     CUBE_HIP(hipGetLastError());
   });
@@ -1458,9 +1478,9 @@ int cube_pm_cic_noalloc(cube_pm_ctx* ctx, const float* x, int64_t np, int32_t nw
     const hipStream_t s = (hipStream_t)stream;
     const int64_t ntot = np * B;
     // the array keeps whatever the last call on this GPU left: clear it here
-    hipLaunchKernelGGL(k_zero_u64, dim3(nblk(B * nw3)), dim3(256), 0, s, acc, B * nw3);
+    hipLaunchKernelGGL(k_zero_u64, cell_blocks(B * nw3), dim3(256), 0, s, acc, B * nw3);
     hipLaunchKernelGGL(k_cic_deposit, dim3(nblk(ntot)), dim3(256), 0, s, x, (uint32_t)np, (uint32_t)ntot, nw, scale, ctx->lat, acc);
-    hipLaunchKernelGGL(k_fix_to_float, dim3(nblk(B * nw3)), dim3(256), 0, s, acc, B * nw3, 1.0 / 2147483648.0, rho);
+    hipLaunchKernelGGL(k_fix_to_float, cell_blocks(B * nw3), dim3(256), 0, s, acc, B * nw3, 1.0 / 2147483648.0, rho);
     CUBE_HIP(hipGetLastError());
   });
 }
