@@ -301,7 +301,7 @@ __global__ void k_sfix_to_float(unsigned long long* __restrict__ acc, int64_t n,
 // place in its bin (one atomic per run of lanes in the same bin; the order
 // within a bin is free, as everything summed over a bin is a sum of integers),
 // k_pm_sums and k_pm_scan the bins' starts, k_pm_sort the sorted records: the
-// fractions and the cell (10 bits per axis), and the particle.  Four meshes of
+// fractions and the cell along x (its row is the bin's), and the particle.  Four meshes of
 // 256^3 with 128^3 particles each: 60 + 10 + 28 + 72 us, where lists by tile, each
 // particle under the up to eight tiles its taps reach, by an atomic per listing
 // in two passes, took 1.6 ms.
@@ -443,8 +443,7 @@ __global__ void __launch_bounds__(256) k_pm_sort(const float* __restrict__ x, co
     float d[3];
     point<M == Sort::kCIC>(x, p, np, n, scale, lt, b, i, d);
     const uint32_t at = start[bin_of(b, i, n)] + rank[p];
-    rec[at] =
-        make_float4(d[0], d[1], d[2], __uint_as_float((uint32_t)i[0] | ((uint32_t)i[1] << 10) | ((uint32_t)i[2] << 20)));
+    rec[at] = make_float4(d[0], d[1], d[2], __uint_as_float((uint32_t)i[0]));
     if constexpr (M == Sort::kCotangent) {
       const float* gp = g + 3 * (int64_t)p;
       grec[at] = make_float4(gp[0], gp[1], gp[2], __uint_as_float(p));
@@ -606,7 +605,7 @@ __global__ void __launch_bounds__(256) k_pm_deposit(const float4* __restrict__ r
   if (k < k1) fetch(k, row, m, v, g);
   for (; k < k1; k += step) {
     const int lz = row / ry, cy = row - lz * ry - 1, cz = lz - 1;
-    const int cx = m == 1 ? (int)(__float_as_uint(v.w) & 1023u) - t.o[0] : (m == 0 ? -1 : t.w[0]);
+    const int cx = m == 1 ? (int)__float_as_uint(v.w) - t.o[0] : (m == 0 ? -1 : t.w[0]);
     float w[3][K], gs[3] = {0, 0, 0};
     const float d[3] = {v.x, v.y, v.z};
     for (int c = 0; c < 3; ++c) {
@@ -677,9 +676,12 @@ template <int V>
 __device__ inline Vec<V> ldv(const float* p) {
   return *reinterpret_cast<const Vec<V>*>(p);
 }
-template <int V>
-__device__ inline Vec<V> at_byte(const float* base, uint32_t off) {  // scalar base, 32-bit offset (meshes up to 1024^3)
-  return *reinterpret_cast<const Vec<V>*>(reinterpret_cast<const char*>(base) + off);
+// At a cell of a mesh of fewer than 2^32: a scalar base and a 32-bit offset of bytes up
+// to 1024^3 (!FAR), else of cells.
+template <int V, bool FAR>
+__device__ inline Vec<V> at_cell(const float* base, uint32_t cell) {
+  if constexpr (FAR) return ldv<V>(base + cell);
+  else return *reinterpret_cast<const Vec<V>*>(reinterpret_cast<const char*>(base) + 4u * cell);
 }
 // x-2 .. x+V+1 of a periodic row
 template <int V>
@@ -868,7 +870,7 @@ __global__ void __launch_bounds__(64) k_tsc_vjp(const float* __restrict__ x, uin
 // workgroups of 49 KB share a CU; the vector pipe is busy half of the time).
 // Four meshes of 256^3 with 128^3 particles each: 0.47 ms, VJP 0.56 ms, where
 // force meshes written and gathered from took 0.31 + 0.50 and 0.63 ms.
-template <bool VJP, int V>
+template <bool VJP, int V, bool FAR>
 __global__ void __launch_bounds__(512) k_pm_gather(const float4* __restrict__ rec,
                                                    const unsigned int* __restrict__ part,
                                                    const float4* __restrict__ grec, int n, Tiles ts,
@@ -900,7 +902,7 @@ __global__ void __launch_bounds__(512) k_pm_gather(const float4* __restrict__ re
       // (rows and columns of a ragged tile that no cell needs repeat the last one)
       const int z = wrap1(t.o[2] + min(pz, t.w[2] + 5) - 3, n), y = wrap1(t.o[1] + min(py, t.w[1] + 5) - 3, n),
                 gx = wrap1(min(t.o[0] + x - 4, V == 4 ? n : n + 2), n);
-      in[k] = at_byte<V>(pb, 4u * (((uint32_t)z * n + y) * n + gx));
+      in[k] = at_cell<V, FAR>(pb, ((uint32_t)z * n + y) * n + gx);
     }
   }
   if (threadIdx.x < 64) {  // at most 64 rows: the first wavefront's lanes
@@ -971,9 +973,9 @@ __global__ void __launch_bounds__(512) k_pm_gather(const float4* __restrict__ re
             ((uint32_t)wrap1(t.o[2] + min(fz, t.w[2] + 1) - 1, n) * n + wrap1(t.o[1] + min(fy, t.w[1] + 1) - 1, n)) * n;
         const int gx = t.o[0] + x;
         if (V == 4) {
-          r = at_byte<4>(rb, 4u * (row0 + wrap1(min(gx, n), n)));
+          r = at_cell<4, FAR>(rb, row0 + wrap1(min(gx, n), n));
         } else {
-          for (int k = 0; k < 4; ++k) r.v[k] = at_byte<1>(rb, 4u * (row0 + wrap1(min(gx + k, n), n))).v[0];
+          for (int k = 0; k < 4; ++k) r.v[k] = at_cell<1, FAR>(rb, row0 + wrap1(min(gx + k, n), n)).v[0];
         }
       }
       float4* dst = &fs[fz * FS + fy * FX + x + 1];
@@ -993,9 +995,9 @@ __global__ void __launch_bounds__(512) k_pm_gather(const float4* __restrict__ re
       }
       float r = 0;
       if (VJP)
-        r = at_byte<1>(rb, 4u * (((uint32_t)wrap1(t.o[2] + min(fz, t.w[2] + 1) - 1, n) * n +
-                                  wrap1(t.o[1] + min(fy, t.w[1] + 1) - 1, n)) * n +
-                                 wrap1(min(t.o[0] + x, n), n))).v[0];
+        r = at_cell<1, FAR>(rb, ((uint32_t)wrap1(t.o[2] + min(fz, t.w[2] + 1) - 1, n) * n +
+                                 wrap1(t.o[1] + min(fy, t.w[1] + 1) - 1, n)) * n +
+                                    wrap1(min(t.o[0] + x, n), n)).v[0];
       fs[fz * FS + fy * FX + x + 1] = make_float4(f[0], f[1], f[2], r);
     }
   } else {
@@ -1009,7 +1011,7 @@ __global__ void __launch_bounds__(512) k_pm_gather(const float4* __restrict__ re
   __syncthreads();
   for (unsigned k = threadIdx.x; k < total; k += NT) {
     const int64_t p = __float_as_uint(g.w);
-    const int lz = row / t.w[1], ly = row - lz * t.w[1], lx = (int)(__float_as_uint(v.w) & 1023u) - t.o[0];
+    const int lz = row / t.w[1], ly = row - lz * t.w[1], lx = (int)__float_as_uint(v.w) - t.o[0];
     float w[3][3], dw[3][3], a[3] = {0, 0, 0};
     const float d[3] = {v.x, v.y, v.z}, gx = g.x, gy = g.y, gz = g.z;
     for (int c = 0; c < 3; ++c) {
@@ -1130,15 +1132,16 @@ struct cube_pm_ctx {
     hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
     return hipStreamIsCapturing(s, &st) != hipSuccess || st != hipStreamCaptureStatusNone;
   }
-  // the buffers of an order of ntot particles on meshes of m^3 are there, or can be made
+  // the buffers of an order of ntot particles on meshes of m^3 (fewer than 2^32 cells) are
+  // there, or can be made
   bool can_sort(int64_t ntot, int64_t m, size_t have, hipStream_t s) const {
-    if (m > 1024 || nbins(m) >= ((int64_t)1 << 31)) return false;
+    if (m > 1625 || nbins(m) >= ((int64_t)1 << 31)) return false;
     return ((size_t)nbins(m) <= bcount.n && (size_t)ntot <= rank.n && (size_t)ntot <= rec.n && (size_t)ntot <= have) ||
            !capturing(s);
   }
   // Many particles are sorted first; below these numbers the launches of that form
   // cost more than the global atomics of the other (which also serves meshes
-  // beyond 1024 points, and a stream under capture whose order buffers would have
+  // beyond 1625 points, and a stream under capture whose order buffers would have
   // to grow).  Measured sorted / not, us, with phi: forces of 17000 particles on
   // 48^3 39 / 50, 128^3 68 / 81, 256^3 302 / 317, 512^3 5480 / 5750; adjoints of 8192
   // on 48^3 46 / 65, 128^3 83 / 114, 256^3 421 / 604, 512^3 6390 / 7700; where F is
@@ -1172,7 +1175,7 @@ struct cube_pm_ctx {
     int64_t from = lat.L == 0 ? 65536 : 60000 + 120000 * ntot / cells;
     if (!shared(nw, kShareCICFew)) from = std::max<int64_t>(from, 262144);
     // meshes below 8 points are all halo
-    return nw >= 8 && shared(nw, kShareCIC) && ntot >= from && can_sort(ntot, nw, SIZE_MAX, s);
+    return nw >= 8 && nw <= 1024 && shared(nw, kShareCIC) && ntot >= from && can_sort(ntot, nw, SIZE_MAX, s);
   }
   // bin counts, starts and places of x on meshes of m^3 (and gmax cleared)
   template <bool CIC>
@@ -1242,6 +1245,15 @@ struct cube_pm_ctx {
   static bool quads(int n, const void* a, const void* b) {
     return n % 4 == 0 && (((uintptr_t)a | (uintptr_t)b) & 15) == 0;
   }
+  // the gather of the order's particles, from quads of phi where it may
+  template <bool VJP>
+  void gather(bool quad, const float* phi, const float* F, const float* rhob, float* out, hipStream_t s) {
+    auto* const k = cfg.n <= 1024 ? (quad ? k_pm_gather<VJP, 4, false> : k_pm_gather<VJP, 1, false>)
+                                  : (quad ? k_pm_gather<VJP, 4, true> : k_pm_gather<VJP, 1, true>);
+    const Tiles tiles(cfg.n, cfg.batch);
+    hipLaunchKernelGGL(k, dim3(tiles.blocks()), dim3(512), 0, s, rec.p, part.p, grec.p, cfg.n, tiles, bstart.p, phi, F,
+                       rhob, out);
+  }
   // rho -> phi (B*n^3) at positions x; srt: through the sorted order (with g's)
   void potential(const float* x, const float* g, int64_t np, float* phi, bool srt, hipStream_t s) {
     const int n = cfg.n, B = cfg.batch;
@@ -1262,7 +1274,6 @@ struct cube_pm_ctx {
   void force(const float* x, int64_t np, float* F, float* phi, float* out, hipStream_t s) {
     const int n = cfg.n;
     const int64_t ntot = np * cfg.batch;
-    const Tiles tiles(n, cfg.batch);
     const bool srt = sorted(ntot, false, s);
     if (!phi) phi = mesh.p;
     potential(x, nullptr, np, phi, srt, s);
@@ -1271,12 +1282,8 @@ struct cube_pm_ctx {
     if (!srt)
       hipLaunchKernelGGL(k_tsc_interp, few_blocks(ntot), dim3(64), 0, s, x, (uint32_t)np, (uint32_t)ntot, n, lat,
                          F, out);
-    else if (quads(n, phi, nullptr))
-      hipLaunchKernelGGL((k_pm_gather<false, 4>), dim3(tiles.blocks()), dim3(512), 0, s, rec.p, part.p, nullptr, n, tiles, bstart.p,
-                         phi, nullptr, nullptr, out);
     else
-      hipLaunchKernelGGL((k_pm_gather<false, 1>), dim3(tiles.blocks()), dim3(512), 0, s, rec.p, part.p, nullptr, n, tiles, bstart.p,
-                         phi, nullptr, nullptr, out);
+      gather<false>(quads(n, phi, nullptr), phi, nullptr, nullptr, out, s);
     CUBE_HIP(hipGetLastError());
   }
   // its adjoint, with the F or the phi of the same x, or neither
@@ -1311,12 +1318,8 @@ struct cube_pm_ctx {
     if (!srt)
       hipLaunchKernelGGL(k_tsc_vjp, few_blocks(ntot), dim3(64), 0, s, x, (uint32_t)np, (uint32_t)ntot, n, lat, F,
                          g, mesh.p, gx);
-    else if (quads(n, phi, mesh.p))
-      hipLaunchKernelGGL((k_pm_gather<true, 4>), dim3(tiles.blocks()), dim3(512), 0, s, rec.p, nullptr, grec.p, n, tiles, bstart.p,
-                         phi, F, mesh.p, gx);
     else
-      hipLaunchKernelGGL((k_pm_gather<true, 1>), dim3(tiles.blocks()), dim3(512), 0, s, rec.p, nullptr, grec.p, n, tiles, bstart.p,
-                         phi, F, mesh.p, gx);
+      gather<true>(quads(n, phi, mesh.p), phi, F, mesh.p, gx, s);
     CUBE_HIP(hipGetLastError());
   }
 };
