@@ -1112,7 +1112,7 @@ struct cube_pm_ctx {
   PMBuf<float> G, mesh, Fs, Fbar;
   PMBuf<float2> work;
   PMBuf<unsigned long long> acc;   // B*3*n^3, kept zero between calls
-  PMBuf<unsigned long long> accw;  // B*nw^3 of the largest CIC density so far, kept zero
+  PMBuf<unsigned long long> accw;  // of the largest CIC density that acc cannot hold, kept zero
   PMBuf<unsigned int> gmax;
   // the particles' order: bin counts (kept zero) and starts, chunk sums, places
   // in the bins, sorted records, particles and cotangents
@@ -1444,10 +1444,13 @@ int cube_pm_cic(cube_pm_ctx* ctx, const float* x, int64_t np, int32_t nw, float 
     const int B = ctx->cfg.batch;
     const int64_t ntot = np * B, nw3 = (int64_t)nw * nw * nw;
     const bool captured = ctx->capturing(s), srt = ctx->cic_sorted(ntot, nw, s);
-    // the accumulator of the form by atomics is made in either form: a call recorded
-    // later may have more particles than the order's buffers hold, and cannot allocate
-    if ((size_t)(B * nw3) > ctx->accw.n && !(captured && srt))
-      hipLaunchKernelGGL(k_zero_u64, cell_blocks(B * nw3), dim3(256), 0, s, ctx->accw.ensure((size_t)(B * nw3)), B * nw3);
+    // The accumulator of the form by atomics: that of the forces, or a larger one, which
+    // is made in either form: a call recorded later may have more particles than
+    // the order's buffers hold, and cannot allocate.
+    const size_t cells = (size_t)(B * nw3);
+    const bool own = cells > ctx->acc.n;
+    if (own && cells > ctx->accw.n && !(captured && srt))
+      hipLaunchKernelGGL(k_zero_u64, cell_blocks(B * nw3), dim3(256), 0, s, ctx->accw.ensure(cells), B * nw3);
     if (srt) {
       const Tiles tiles(nw, B);
       ctx->bin<true>(x, np, nw, scale, s);
@@ -1457,11 +1460,11 @@ int cube_pm_cic(cube_pm_ctx* ctx, const float* x, int64_t np, int32_t nw, float 
       CUBE_HIP(hipGetLastError());
       return;
     }
-    if (captured) ctx->accw.hold();
+    if (own && captured) ctx->accw.hold();
+    unsigned long long* const acc = own ? ctx->accw.p : ctx->acc.p;
     hipLaunchKernelGGL(k_cic_deposit, dim3(nblk(ntot)), dim3(256), 0, s, x, (uint32_t)np, (uint32_t)ntot, nw, scale, ctx->lat,
-                       ctx->accw.p);
-    hipLaunchKernelGGL(k_fix_to_float, cell_blocks(B * nw3), dim3(256), 0, s, ctx->accw.p, B * nw3, 1.0 / 2147483648.0,
-                       rho);
+                       acc);
+    hipLaunchKernelGGL(k_fix_to_float, cell_blocks(B * nw3), dim3(256), 0, s, acc, B * nw3, 1.0 / 2147483648.0, rho);
     CUBE_HIP(hipGetLastError());
   });
 }

@@ -72,18 +72,19 @@ def test_recorded_density_after_larger_calls(m):
     other.close()
 
 
-def test_recorded_density_of_more_particles_than_before():
+@pytest.mark.parametrize("nw", [40, 72])  # within the forces' accumulator (three meshes of 32^3), and beyond it
+def test_recorded_density_of_more_particles_than_before(nw):
     """After one call with the mesh's size a recorded call takes any number of
     particles: the form by atomics needs no memory that depends on it."""
     pm, other = (pmdiff.PMForce(32, 1, 1.0) for _ in range(2))
-    pm.cic(_positions(70001, 32, 1), 40, 1.25)
+    pm.cic(_positions(70001, 32, 1), nw, nw / 32)
     x = _positions(150001, 32, 2)
     graph = torch.cuda.CUDAGraph()
     with torch.cuda.graph(graph):
-        rho = pm.cic(x, 40, 1.25)
+        rho = pm.cic(x, nw, nw / 32)
     for k in range(3):
         y = _positions(150001, 32, 10 + k)
-        want = other.cic(y, 40, 1.25)
+        want = other.cic(y, nw, nw / 32)
         x.copy_(y)
         graph.replay()
         torch.cuda.synchronize()
