@@ -1275,7 +1275,8 @@ struct cube_pm_ctx {
     const int n = cfg.n;
     const int64_t ntot = np * cfg.batch;
     const bool srt = sorted(ntot, false, s);
-    if (!phi) phi = mesh.p;
+    float* const to = phi;
+    if (!phi || ((uintptr_t)phi & 15) != 0) phi = mesh.p;  // the transform moves pairs of floats
     potential(x, nullptr, np, phi, srt, s);
     if (!F && !srt) F = Fs.p;
     if (F) fd(false, phi, F, s);
@@ -1284,6 +1285,8 @@ struct cube_pm_ctx {
                          F, out);
     else
       gather<false>(quads(n, phi, nullptr), phi, nullptr, nullptr, out, s);
+    if (to && to != phi)
+      CUBE_HIP(hipMemcpyAsync(to, phi, sizeof(float) * (size_t)(cfg.batch * n3), hipMemcpyDeviceToDevice, s));
     CUBE_HIP(hipGetLastError());
   }
   // its adjoint, with the F or the phi of the same x, or neither

@@ -121,6 +121,22 @@ class PMForce:
             raise ValueError("x must be (batch*np, 3)")
         return x.shape[0] // self.batch
 
+    def _cells(self, t: torch.Tensor | None, meshes: int, name: str):
+        """A mesh argument's pointer: the library reads or writes that many meshes of each batch."""
+        if t is None:
+            return None
+        want = self.batch * meshes * self.n ** 3
+        if t.numel() < want:
+            raise ValueError(f"{name} holds {t.numel()} values, not batch * {meshes} * n^3 = {want}")
+        return _ptr(t)
+
+    @staticmethod
+    def _like(t: torch.Tensor, x: torch.Tensor, name: str) -> C.c_void_p:
+        """The pointer of an argument with a value for each of x's."""
+        if t.numel() < x.numel():
+            raise ValueError(f"{name} must have the size of x, {tuple(x.shape)}, not {tuple(t.shape)}")
+        return _ptr(t)
+
     def mesh_tensor(self, device) -> torch.Tensor:
         return torch.empty((self.batch, 3, self.n, self.n, self.n), dtype=torch.float32, device=device)
 
@@ -129,28 +145,28 @@ class PMForce:
         np_ = self._np(x)
         F = self.mesh_tensor(x.device) if F is None else F
         acc = torch.empty_like(x)
-        self._check(self.lib.cube_pm_force(self.ctx, _ptr(x), np_, _ptr(F), _ptr(acc), _stream()))
+        self._check(self.lib.cube_pm_force(self.ctx, _ptr(x), np_, self._cells(F, 3, "F"), _ptr(acc), _stream()))
         return acc, F
 
     def force_vjp(self, x: torch.Tensor, F: torch.Tensor | None, g: torch.Tensor) -> torch.Tensor:
         """(d acc / d x)^T g; F = None recomputes the force meshes of x."""
-        gx = torch.empty_like(x)
-        self._check(self.lib.cube_pm_force_vjp(self.ctx, _ptr(x), self._np(x), None if F is None else _ptr(F),
-                                               _ptr(g.contiguous()), _ptr(gx), _stream()))
+        gx, g = torch.empty_like(x), g.contiguous()
+        self._check(self.lib.cube_pm_force_vjp(self.ctx, _ptr(x), self._np(x), self._cells(F, 3, "F"),
+                                               self._like(g, x, "g"), _ptr(gx), _stream()))
         return gx
 
     def force_phi(self, x: torch.Tensor, phi: torch.Tensor | None) -> torch.Tensor:
         """acc alone; the potential (batch, n, n, n) it came from goes to phi if given."""
         acc = torch.empty_like(x)
-        self._check(self.lib.cube_pm_force_phi(self.ctx, _ptr(x), self._np(x), None if phi is None else _ptr(phi),
-                                               _ptr(acc), _stream()))
+        self._check(self.lib.cube_pm_force_phi(self.ctx, _ptr(x), self._np(x), self._cells(phi, 1, "phi"), _ptr(acc),
+                                               _stream()))
         return acc
 
     def force_vjp_phi(self, x: torch.Tensor, phi: torch.Tensor, g: torch.Tensor) -> torch.Tensor:
         """force_vjp from the potential of x."""
-        gx = torch.empty_like(x)
-        self._check(self.lib.cube_pm_force_vjp_phi(self.ctx, _ptr(x), self._np(x), _ptr(phi), _ptr(g.contiguous()),
-                                                   _ptr(gx), _stream()))
+        gx, g = torch.empty_like(x), g.contiguous()
+        self._check(self.lib.cube_pm_force_vjp_phi(self.ctx, _ptr(x), self._np(x), self._cells(phi, 1, "phi"),
+                                                   self._like(g, x, "g"), _ptr(gx), _stream()))
         return gx
 
     def sites(self, dtype=torch.float64, device="cpu") -> torch.Tensor:

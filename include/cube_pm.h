@@ -84,7 +84,8 @@ int cube_pm_force_vjp(cube_pm_ctx* ctx, const float* x, int64_t np, const float*
 /* The same two with the potential phi (B*n^3 floats, [b][z][y][x]; a third of F)
  * in the place of F: cube_pm_force_phi writes it (phi may be NULL: context
  * scratch), cube_pm_force_vjp_phi reads it (or recomputes it: NULL).  The force
- * is formed from phi where it is interpolated. */
+ * is formed from phi where it is interpolated.  Arrays at multiples of 16 bytes
+ * are used where they are; a phi at another address is written as a copy. */
 int cube_pm_force_phi(cube_pm_ctx* ctx, const float* x, int64_t np, float* phi, float* acc, void* stream);
 int cube_pm_force_vjp_phi(cube_pm_ctx* ctx, const float* x, int64_t np, const float* phi, const float* g_acc,
                           float* g_x, void* stream);
