@@ -18,8 +18,12 @@ struct DriftParams {
   bool images;    // buffers are images of physical particles, velocities included
 };
 
+// Words of the flags, and of a slot's cache line.
+constexpr int kDriftFlags = 32, kRankedStride = 16;
+
 struct DriftScratch {
-  int32_t* flags = nullptr;     // [0] error bits, [1..3] max shift per axis
+  int32_t* flags = nullptr;     // kDriftFlags words: [0] error bits, [1..3] max shift per axis, [4] tile maximum
+  unsigned long long* ranked = nullptr;  // particles with a rank, in kSumSlots slots kRankedStride apart
   int32_t* rank = nullptr;      // per source particle
   int32_t* table = nullptr;     // per source cell (nt + 2 ring a side) per direction (count -> offset)
   int64_t table_cap = 0;        // int32 elements
@@ -44,7 +48,8 @@ void drift_shift(const DriftParams& P, const void* xp, const float* vp, const in
 // Passes 2-5 for tiles [t0, t1): rank, offsets, scatter (base scan done by caller
 // before the scatter).  count = true folds pass 1 into the rank pass (all tiles
 // at once; flags as pass 1, plus DRIFT_SHIFT_BOUND when a shift exceeds P.M, then an
-// upper bound given by the caller) and the destination counts into the offsets.
+// upper bound given by the caller) and the destination counts into the offsets; the
+// ranked particles are counted for the caller to compare with theirs.
 void drift_rank(const DriftParams& P, const void* xp, const float* vp, const int64_t* off, int t0, int t1,
                 DriftScratch& S, hipStream_t s, bool count = false);
 void drift_offsets(const DriftParams& P, int t0, int t1, DriftScratch& S, hipStream_t s, bool count = false);

@@ -177,7 +177,8 @@ template <int IZ, bool COUNT, bool LDS>
 __global__ void __launch_bounds__(256) k_drift_rank(DriftParams P, Runs R, const XT<IZ>* __restrict__ xp,
                                                     const float* __restrict__ vp, const int64_t* __restrict__ off,
                                                     int t0, int32_t* __restrict__ rank, int32_t* __restrict__ table,
-                                                    int32_t* __restrict__ flags) {
+                                                    int32_t* __restrict__ flags,
+                                                    unsigned long long* __restrict__ ranked) {
   extern __shared__ int32_t counts[];
   const uint32_t w = blockIdx.x * 4u + (threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
@@ -194,7 +195,7 @@ __global__ void __launch_bounds__(256) k_drift_rank(DriftParams P, Runs R, const
   if (LDS)
     for (int k = lane; k < o.cells * Dt; k += 64) mine[k] = 0;
   const int lo = 1 - 2 * P.ncb, hi = P.nt + 2 * P.ncb;
-  int err = 0, ms[3] = {0, 0, 0};
+  int err = 0, ms[3] = {0, 0, 0}, mine_ranked = 0;
   for (int p0 = 0; p0 < tot; p0 += 64) {
     const int pos = p0 + lane;
     const int ci = cell_at(starts, o.cells, pos);
@@ -225,6 +226,7 @@ __global__ void __launch_bounds__(256) k_drift_rank(DriftParams P, Runs R, const
       }
     }
     unsigned long long peers = __builtin_amdgcn_ballot_w64(key >= 0);
+    if (COUNT) mine_ranked += (int)__popcll(peers);
     for (int b = 0; b < bits; ++b) {
       const bool one = (key >> b) & 1;
       const unsigned long long m = __builtin_amdgcn_ballot_w64(one);
@@ -247,6 +249,7 @@ __global__ void __launch_bounds__(256) k_drift_rank(DriftParams P, Runs R, const
     if (lane == 0 && tot > 0) {
       if (err) atomicOr(&flags[0], err);
       for (int d = 0; d < 3; ++d) atomic_max_int(&flags[1 + d], ms[d]);
+      if (mine_ranked) atomicAdd(&ranked[blockIdx.x % kSumSlots * kRankedStride], (unsigned long long)mine_ranked);
     }
   }
 }
@@ -429,11 +432,11 @@ void rank_launch(const DriftParams& P, const void* xp, const float* vp, const in
   const int Dt = P.D[0] * P.D[1] * P.D[2];
   if (Dt <= kLdsDirs) {
     hipLaunchKernelGGL((k_drift_rank<IZ, COUNT, true>), grid, dim3(256), 4 * 8 * Dt * sizeof(int32_t), s, P, R,
-                       (const XT<IZ>*)xp, vp, off, t0, S.rank, S.table, S.flags);
+                       (const XT<IZ>*)xp, vp, off, t0, S.rank, S.table, S.flags, S.ranked);
   } else {
     zero_async(S.table, sizeof(int32_t) * (size_t)(t1 - t0) * R.na * R.na * R.na * Dt, s);
     hipLaunchKernelGGL((k_drift_rank<IZ, COUNT, false>), grid, dim3(256), 0, s, P, R, (const XT<IZ>*)xp, vp, off, t0,
-                       S.rank, S.table, S.flags);
+                       S.rank, S.table, S.flags, S.ranked);
   }
   CUBE_HIP(hipGetLastError());
 }

@@ -11,12 +11,14 @@
 #include <map>
 #include <memory>
 #include <mutex>
+#include <numeric>
 #include <string>
 
 #include "../../include/cube_p3m.h"
 #include "cic.h"
 #include "common.h"
 #include "drift.h"
+#include "drift_check.h"
 #include "fft.h"
 #include "ic.h"
 #include "pm.h"
@@ -171,6 +173,7 @@ struct cube_p3m_ctx {
   // (the buffer step), 0 not looked at yet (uploaded state), -1 they are not
   int images = 0;
   bool vimages = false;       // buffer velocities, too, are those of the physical particles
+  int64_t nphys = -1;         // physical particles of the buffered layout (-1: not counted)
   bool image_meshes = false;  // this kick's densities may be cut from whole-image meshes
   DevBuf<int32_t> dbad;
   DevBuf<char> stencil;  // coarse-level deposit: 27 tap sums per coarse cell
@@ -397,7 +400,7 @@ void cube_p3m_ctx::init() {
   ppout.ensure(1);
   ires.ensure(g.ns3);
   cmax.ensure(g.ns3);
-  dflags.ensure(8);
+  dflags.ensure(kDriftFlags + 2 * kSumSlots * kRankedStride);
   set_tf_default();
 }
 
@@ -1202,6 +1205,7 @@ void cube_p3m_ctx::drift(const cube_drift_in& in, cube_drift_out& out) {
   const int64_t nt3 = g.nt * g.nt * g.nt, nphys_cells = g.ntiles * nt3;
   DriftScratch S;
   S.flags = dflags.p;
+  S.ranked = (unsigned long long*)(dflags.p + kDriftFlags);
   S.newcount = dnewcount.ensure(nphys_cells);
   S.base = dbase.ensure(nphys_cells + 1);
   const int other = 1 - cur;
@@ -1212,7 +1216,7 @@ void cube_p3m_ctx::drift(const cube_drift_in& in, cube_drift_out& out) {
   // check runs on the device and is read back with the pass's flags (the
   // passes before the read write scratch arrays only)
   auto start_pass = [&]() {
-    zero_async(S.flags, sizeof(int32_t) * 8, s);
+    zero_async(S.flags, sizeof(int32_t) * (kDriftFlags + 2 * kSumSlots * kRankedStride), s);
     drift_tile_check(off.p, g.ncell_tile, (int)g.ntiles, g.np_tile_max, S.flags, s);
   };
   P.ring = (int)g.ncb;
@@ -1225,6 +1229,7 @@ void cube_p3m_ctx::drift(const cube_drift_in& in, cube_drift_out& out) {
     const int64_t tbudget = std::max<int64_t>(per_tile, ((int64_t)2 << 30) / 4);
     return (int)std::max<int64_t>(1, std::min<int64_t>(g.ntiles, tbudget / per_tile));
   };
+  std::vector<unsigned long long> ranked(kSumSlots * kRankedStride);
   auto count_scan = [&]() {  // flags and the scan of the destination counts
     {
       KScope k(&tm, "drift_scan", (double)nphys_cells * 12);
@@ -1233,6 +1238,7 @@ void cube_p3m_ctx::drift(const cube_drift_in& in, cube_drift_out& out) {
     ReadBack rb(page);
     rb.get(fl, S.flags, sizeof(fl), s);
     rb.get(&nplocal, S.base + nphys_cells, sizeof(nplocal), s);
+    rb.get(ranked.data(), S.ranked, sizeof(ranked[0]) * ranked.size(), s);
     rb.wait();
     if (fl[0] & DRIFT_TILE_OVERFLOW)
       throw Error(CUBE_ERR_TILE_OVERFLOW, "too many particles in this tile+buffer: " + std::to_string(fl[4]) + " > " +
@@ -1290,6 +1296,8 @@ void cube_p3m_ctx::drift(const cube_drift_in& in, cube_drift_out& out) {
     count_scan();
     if (fl[0] & DRIFT_SHIFT_BOUND) fused = false;
     else {
+      if (!drift_counts_agree((int64_t)std::accumulate(ranked.begin(), ranked.end(), 0ull), nplocal, P.images, nphys))
+        throw Error(CUBE_ERR_COUNT_MISMATCH, "warning: density different (rholocal /= rhoce)");
       ensure_set(other, nplocal);
       scatter(0, (int)g.ntiles);
     }
@@ -1371,6 +1379,7 @@ void cube_p3m_ctx::buffer(int64_t* np_ext) {
   layout = 1;
   images = 1;
   vimages = true;
+  nphys = np;
   np = n;
   off_valid = true;
   if (np_ext) *np_ext = n;
@@ -1430,6 +1439,19 @@ static int64_t host_sum(const int32_t* a, int64_t n) {
   return s;
 }
 
+// The physical cells' counts of rhoc (copied to `out` unless null), summed.
+static int64_t physical_counts(const Geo& g, const int32_t* rhoc, int32_t* out) {
+  int64_t n = 0;
+  for (int64_t T = 0; T < g.ntiles; ++T)
+    for (int64_t k = 1; k <= g.nt; ++k)
+      for (int64_t j = 1; j <= g.nt; ++j) {
+        const int64_t c = rc_index(1, j, k, T, g.nte, g.ncb);
+        n += host_sum(rhoc + c, g.nt);
+        if (out) std::copy(rhoc + c, rhoc + c + g.nt, out + c);
+      }
+  return n;
+}
+
 template <class F>
 static int guarded(cube_p3m_ctx* ctx, F&& f) {
   if (!ctx) return CUBE_ERR_ARG;
@@ -1465,6 +1487,7 @@ static void upload_ext(cube_p3m_ctx* c, const void* xp, const float* vp, const i
   c->vmax_valid = false;
   c->images = 0;
   c->vimages = false;
+  c->nphys = -1;
 }
 
 // The second species' outputs of a coupled kick: its PM1/PM2 maxima (its
@@ -1626,17 +1649,8 @@ int cube_p3m_buffer(cube_p3m_ctx* ctx, void* xp, float* vp, int64_t* pid, int32_
     if (!xp || !vp || !rhoc) throw Error(CUBE_ERR_ARG, "null argument");
     const Geo& g = ctx->g;
     // physical counts only: buffers are ignored (filled here)
-    std::vector<int32_t> rp(rhoc, rhoc + g.ncells_ext);
-    int64_t nphys = 0;
-    for (int64_t T = 0; T < g.ntiles; ++T)
-      for (int64_t k = 1 - g.ncb; k <= g.nt + g.ncb; ++k)
-        for (int64_t j = 1 - g.ncb; j <= g.nt + g.ncb; ++j)
-          for (int64_t i = 1 - g.ncb; i <= g.nt + g.ncb; ++i) {
-            const int64_t c = rc_index(i, j, k, T, g.nte, g.ncb);
-            const bool ph = i >= 1 && i <= g.nt && j >= 1 && j <= g.nt && k >= 1 && k <= g.nt;
-            if (!ph) rp[c] = 0;
-            else nphys += rp[c];
-          }
+    std::vector<int32_t> rp((size_t)g.ncells_ext, 0);
+    const int64_t nphys = physical_counts(g, rhoc, rp.data());
     if (nphys != nplocal) throw Error(CUBE_ERR_ARG, "nplocal differs from the physical sum of rhoc");
     ctx->ensure_set(0, std::max<int64_t>(nplocal, 1));
     ctx->cur = 0;
@@ -1699,6 +1713,7 @@ int cube_p3m_state_upload(cube_p3m_ctx* ctx, const void* xp, const float* vp, co
   return guarded(ctx, [&] {
     if (!xp || !vp || !rhoc) throw Error(CUBE_ERR_ARG, "null argument");
     upload_ext(ctx, xp, vp, pid, rhoc, np);
+    ctx->nphys = physical_counts(ctx->g, rhoc, nullptr);
     CUBE_HIP(hipStreamSynchronize(ctx->s));
   });
 }
