@@ -174,6 +174,7 @@ struct cube_p3m_ctx {
   int images = 0;
   bool vimages = false;       // buffer velocities, too, are those of the physical particles
   int64_t nphys = -1;         // physical particles of the buffered layout (-1: not counted)
+  int last_ring = 0;          // buffer cells around a tile whose particles the last drift read
   bool image_meshes = false;  // this kick's densities may be cut from whole-image meshes
   DevBuf<int32_t> dbad;
   DevBuf<char> stencil;  // coarse-level deposit: 27 tap sums per coarse cell
@@ -1331,6 +1332,7 @@ void cube_p3m_ctx::drift(const cube_drift_in& in, cube_drift_out& out) {
       scatter(t0, t1);
     }
   }
+  last_ring = P.ring;
   int32_t* rnew = rhoc[1 - rcur].p;
   drift_write_rhoc(P, S, rnew, s);
   ReadBack rb(page);
@@ -1885,6 +1887,8 @@ int cube_p3m_timing_report(cube_p3m_ctx* ctx, char* buf, int64_t len) {
     std::string r = ctx->tm.report();
     char extra[128];
     snprintf(extra, sizeof(extra), "pp_pairs_last %lld 0 0 0\n", (long long)ctx->last_pairs);
+    r += extra;
+    snprintf(extra, sizeof(extra), "drift_ring_last %d 0 0 0\n", ctx->last_ring);
     r += extra;
     snprintf(extra, sizeof(extra), "graph_captures %lld 0 0 0\ngraph_launches %lld 0 0 0\n",
              (long long)ctx->graph_captures, (long long)ctx->graph_launches);
