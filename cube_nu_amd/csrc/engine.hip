@@ -90,14 +90,17 @@ const std::vector<int> kTuneInterpShape = {0, 1, 2};
 // CUBE_AUTOTUNE_FILE, a context reads the picks recorded there (lines
 // "key pick") and appends every pick it makes, so later runs skip the trials.
 // A line whose key names no tuned choice, or whose pick is not one of that
-// choice's candidates (a file from another build, or edited), is ignored.
+// choice's candidates (a file from another build, or edited), is ignored; a choice
+// takes another name when its kernel is written anew, so that picks timed on the
+// one before are not taken (a load depth of 6, the first choice of an earlier pair
+// force, takes this one 27 ms instead of 23 at 512^3).
 std::mutex g_tune_file_mu;
 
 bool tune_pick_valid(const std::string& key, int pick) {
   static const std::pair<const char*, const std::vector<int>*> choices[] = {
-      {"pp_depth_l", &kTunePPDepth},
+      {"pp_depth_v2_l", &kTunePPDepth},
       {"dep_list_threads_l", &kTuneDepListThreads},
-      {"interp_shape_l", &kTuneInterpShape}};
+      {"interp_shape_v2_l", &kTuneInterpShape}};
   for (const auto& c : choices)
     if (key.compare(0, std::strlen(c.first), c.first) == 0)
       return std::find(c.second->begin(), c.second->end(), pick) != c.second->end();
@@ -770,7 +773,7 @@ template <typename R>
 int cube_p3m_ctx::interp_shape(int level, int n, const PMLevel& L, const PMBox* boxes, int nb, const cube_kick_in& in,
                                const R* phi, bool trials) {
   if (!std::is_same<R, float>::value || level < 2 || !pm_interp_cells_form(L)) return 0;
-  const std::string key = tune_key("interp_shape", level, n);
+  const std::string key = tune_key("interp_shape_v2", level, n);
   const auto it = tune_picks.find(key);
   if (it != tune_picks.end()) return it->second;
   if (!trials || no_trials) return 0;
@@ -796,7 +799,7 @@ int cube_p3m_ctx::tune_pp(int iapm, const PPLevel& L, const PPBox* boxes, int nb
   vtune.ensure((size_t)std::max<int64_t>(np, 1) * 3);
   otune.ensure(1);
   return autotune(
-      tune_key("pp_depth", iapm, L.npgrid), kTunePPDepth,
+      tune_key("pp_depth_v2", iapm, L.npgrid), kTunePPDepth,
       [&](int u) {
         CUBE_HIP(hipMemcpyAsync(vtune.p, vpc(), sizeof(float) * 3 * (size_t)np, hipMemcpyDeviceToDevice, s));
         zero_async(otune.p, sizeof(PPOut), s);
