@@ -21,6 +21,7 @@
 #include "drift_check.h"
 #include "fft.h"
 #include "ic.h"
+#include "plan.h"
 #include "pm.h"
 #include "pm_mesh.h"
 #include "pp.h"
@@ -170,7 +171,7 @@ struct cube_p3m_ctx {
   PinnedPage page;      // small read-backs
   Transfers transfers;  // host programs' arrays
   DevBuf<char> work;
-  DevBuf<float> gmesh, gfaces;  // whole-image mesh and window faces (pm_mesh.h)
+  DevBuf<float> gmesh;          // whole-image mesh (pm_mesh.h)
   DevBuf<int4> lorg[6];         // and the windows' origins, per slot as lboxes
   // buffer cells as periodic images of the physical ones: 1 by construction
   // (the buffer step), 0 not looked at yet (uploaded state), -1 they are not
@@ -178,7 +179,7 @@ struct cube_p3m_ctx {
   bool vimages = false;       // buffer velocities, too, are those of the physical particles
   int64_t nphys = -1;         // physical particles of the buffered layout (-1: not counted)
   int last_ring = 0;          // buffer cells around a tile whose particles the last drift read
-  bool image_meshes = false;  // this kick's densities may be cut from whole-image meshes
+  int64_t image_bytes = 0;    // the largest whole-image mesh this kick's densities may be cut from (0: none)
   DevBuf<int32_t> dbad;
   DevBuf<char> stencil;  // coarse-level deposit: 27 tap sums per coarse cell
   // per-slot box lists and binned lists (slot 0 PM1, 1 PM2, 2..5 PM3 at
@@ -360,8 +361,21 @@ struct cube_p3m_ctx {
     return L;
   }
   void check_images();
+  // A level's meshes in the workspace: held at once, from the image's mesh or
+  // deposited per window, bytes of all; work holds the meshes, their transforms and,
+  // of windows cut from the image's mesh, their faces.
+  struct LevelPlan {
+    bool image;
+    int64_t batch, bytes;
+  };
   template <typename R>
-  bool image_mesh_level(int level, const PMLevel& L, int64_t nbox, int64_t batch) const;
+  LevelPlan plan_level(int level, const PMLevel& L, int64_t nmesh) const;
+  template <typename R>
+  void plan_images(int mask);
+  int64_t image_mesh_bytes(const PMLevel& L) const {
+    const int64_t n = g.nc * L.w;
+    return 4 * n * n * n;
+  }
   void drift(const cube_drift_in& in, cube_drift_out& out);
   void buffer(int64_t* np_ext);
   void buffer_vel();
@@ -421,19 +435,40 @@ void cube_p3m_ctx::set_tf_default() {
   CUBE_HIP(hipStreamSynchronize(s));
 }
 
-// Whether a level's windows are cut from the whole image's mesh: the FP32
-// form, a level that most of the image takes (the tile level, and the
-// sub-tile level of at least half the sub-tiles: below that the boxes' own
-// particles are fewer than the image's), state whose buffer cells are the
-// periodic images they stand for, and meshes within half the workspace
-// budget.  Either form gives the same densities bit for bit.
+// A level's windows are cut from the whole image's mesh in the FP32 form, at a level
+// that most of the image takes (the tile level, and the sub-tile level of at
+// least half the sub-tiles: below that the boxes' own particles are fewer than
+// the image's), of state whose buffer cells are the periodic images they stand
+// for, and where the mesh has room.  Either form gives the same densities bit for bit.
 template <typename R>
-bool cube_p3m_ctx::image_mesh_level(int level, const PMLevel& L, int64_t nbox, int64_t batch) const {
-  if (!std::is_same<R, float>::value || level < 2 || !image_meshes || !pm_mesh_applies(g, L)) return false;
-  if (np > (int64_t)UINT32_MAX || (nu && nu->np > (int64_t)UINT32_MAX)) return false;  // 32-bit particle offsets
-  if (level >= 3 && 2 * nbox < g.ns3) return false;
-  const int64_t n = g.nc * L.w, bytes = 4 * (n * n * n + batch * 6 * (int64_t)L.n * L.n);
-  return bytes <= ws_budget() / 2;
+cube_p3m_ctx::LevelPlan cube_p3m_ctx::plan_level(int level, const PMLevel& L, int64_t nmesh) const {
+  LevelPlan P{};
+  P.image = std::is_same<R, float>::value && level >= 2 && image_bytes > 0 && pm_mesh_applies(g, L) &&
+            image_mesh_bytes(L) <= image_bytes && (level == 2 || 2 * nmesh >= g.ns3);
+  const int64_t per = mesh_bytes(L.n, sizeof(R)) + (P.image ? face_bytes(L.n) : 0);
+  P.batch = level_batch(ws_budget(), cfg.workspace_bytes > 0, image_bytes, per, nmesh);
+  P.bytes = P.batch * per;
+  return P;
+}
+
+// The whole-image meshes a kick of these phases may take.
+template <typename R>
+void cube_p3m_ctx::plan_images(int mask) {
+  image_bytes = 0;
+  if (!std::is_same<R, float>::value || !(mask & 6)) return;
+  check_images();
+  if (nu) nu->check_images();
+  if (images != 1 || (nu && nu->images != 1)) return;
+  if (np > (int64_t)UINT32_MAX || (nu && nu->np > (int64_t)UINT32_MAX)) return;  // 32-bit particle offsets
+  int64_t largest = 0;
+  for (int l = 1; l <= 6; ++l) largest = std::max(largest, mesh_bytes(tfn[l], sizeof(R)) + face_bytes(tfn[l]));
+  auto level = [&](const PMLevel& L) {
+    if (pm_mesh_applies(g, L) && image_fits(ws_budget(), cfg.workspace_bytes > 0, image_mesh_bytes(L), largest))
+      image_bytes = std::max(image_bytes, image_mesh_bytes(L));
+  };
+  if (mask & 2) level(level_pm2());
+  if ((mask & 4) && cfg.pm3)
+    for (int iapm = 2; iapm <= 5; ++iapm) level(level_pm3(iapm));
 }
 
 // One look at uploaded state (a read-back); state of the buffer step needs none.
@@ -456,23 +491,20 @@ void cube_p3m_ctx::run_level(int level, int slot, const std::vector<PMBox>& bx_i
   const bool SZ = kph != 2, CP = kph != 1;  // sizing and compute parts of this call
   const int64_t n = L0.n;
   const int64_t nreal = n * n * n, ncplx = n * n * (n / 2 + 1);
-  const int64_t per = nreal * (int64_t)sizeof(R) + ncplx * (int64_t)sizeof(C);
   std::string t(tag);
   // The coarse level is one periodic mesh shared by all tiles; tile and
   // sub-tile levels have one mesh per box, batched to fit the workspace.
-  const int64_t nmesh_total = (level == 1) ? 1 : (int64_t)bx_in.size();
-  const int64_t batch = (level == 1) ? 1 : std::max<int64_t>(1, std::min<int64_t>(nmesh_total, ws_budget() / per));
-  work.ensure((size_t)(batch * per));
+  const LevelPlan plan = plan_level<R>(level, L0, (level == 1) ? 1 : (int64_t)bx_in.size());
+  const int64_t batch = plan.batch;
+  const bool image = plan.image;
+  work.ensure((size_t)plan.bytes);
   R* mesh = (R*)work.p;
   C* cplx = (C*)(work.p + batch * nreal * sizeof(R));
+  float* faces = (float*)(cplx + batch * ncplx);  // (of windows of the image's mesh)
   const size_t bchunk = (level == 1) ? bx_in.size() : (size_t)batch;
   if (kph == 1 && bchunk < bx_in.size()) graph_ok = false;  // a captured kick holds one batch per level
-  const bool image = image_mesh_level<R>(level, L0, nmesh_total, batch);
   const MeshGeo M = mesh_geo(g, L0.w, (int)g.B);
-  if (image) {
-    gmesh.ensure((size_t)M.n * M.n * M.n);
-    gfaces.ensure((size_t)batch * 6 * n * n);
-  }
+  if (image) gmesh.ensure((size_t)M.n * M.n * M.n);
   DevBuf<PMBox>& boxes = lboxes[slot];
   boxes.ensure(std::max<size_t>(boxes.n, bchunk));
   for (size_t b0 = 0; b0 < bx_in.size(); b0 += bchunk) {
@@ -510,15 +542,15 @@ void cube_p3m_ctx::run_level(int level, int slot, const std::vector<PMBox>& bx_i
           pm1_deposit<R>((int)g.izipx, L, xpc(), rhocc(), off.p, st, mesh, in.mass_p_cdm, o, s);
       } else if (image) {
         if (SZ)
-          sig_add({(uint64_t)(uintptr_t)gmesh.p, (uint64_t)(uintptr_t)gfaces.p, (uint64_t)(uintptr_t)lorg[slot].p,
+          sig_add({(uint64_t)(uintptr_t)gmesh.p, (uint64_t)(uintptr_t)faces, (uint64_t)(uintptr_t)lorg[slot].p,
                    (uint64_t)direct});
         if constexpr (std::is_same<R, float>::value) {
           auto window = [&](cube_p3m_ctx* c, float m, float* out) {
             // the image's mesh holds every box of the level: once per level and species
             if (b0 == 0 || nu) pm_mesh_deposit((int)g.izipx, M, c->xpc(), c->rhocc(), c->off.p, gmesh.p, m, s);
-            pm_mesh_faces((int)g.izipx, M, L, boxes.p, nb, c->xpc(), c->rhocc(), c->off.p, gfaces.p, m, s);
-            if (direct) win = FFTWindow{gmesh.p, gfaces.p, lorg[slot].p, M.n};
-            else pm_mesh_window(M, (int)n, lorg[slot].p, nb, gmesh.p, gfaces.p, out, s);
+            pm_mesh_faces((int)g.izipx, M, L, boxes.p, nb, c->xpc(), c->rhocc(), c->off.p, faces, m, s);
+            if (direct) win = FFTWindow{gmesh.p, faces, lorg[slot].p, M.n};
+            else pm_mesh_window(M, (int)n, lorg[slot].p, nb, gmesh.p, faces, out, s);
           };
           if (CP) window(this, in.mass_p_cdm, mesh);
           if (CP && nu && level <= 2) {
@@ -903,7 +935,6 @@ void cube_p3m_ctx::kick_pass(const cube_kick_in& in, cube_kick_out& out, float* 
 template <typename R>
 bool cube_p3m_ctx::classify_and_reserve(cube_kick_out& out, std::vector<int32_t>& ires_h,
                                         std::vector<int32_t>& cmax_h) {
-  using C = typename Cplx<R>::T;
   classify_subtiles(g, cfg.ires_fixed, rhocc(), ires.p, cmax.p, s);
   ReadBack rb(page);
   rb.get(ires_h.data(), ires.p, sizeof(int32_t) * g.ns3, s);
@@ -914,44 +945,27 @@ bool cube_p3m_ctx::classify_and_reserve(cube_kick_out& out, std::vector<int32_t>
   classified = true;
   bool multi = false;  // a PM3 or PP level in several workspace batches
   {
-    int64_t need = 0;
-    auto level_ws = [&](int64_t n, int64_t nmesh, bool sub) {
+    int64_t need = 0, image = 0;
+    auto level_ws = [&](int level, const PMLevel& L, int64_t nmesh) {
       if (nmesh <= 0) return;
-      const int64_t per = n * n * n * (int64_t)sizeof(R) + n * n * (n / 2 + 1) * (int64_t)sizeof(C);
-      const int64_t batch = std::max<int64_t>(1, std::min<int64_t>(nmesh, ws_budget() / per));
-      need = std::max(need, batch * per);
-      if (sub && batch < nmesh) multi = true;
+      const LevelPlan P = plan_level<R>(level, L, nmesh);
+      need = std::max(need, P.bytes);
+      if (P.image) image = std::max(image, image_mesh_bytes(L));
+      if (level == 3 && P.batch < nmesh) multi = true;
     };
-    level_ws(g.nc, 1, false);
-    level_ws(g.ngt, g.ntiles, false);
+    PMLevel coarse{};
+    coarse.n = (int)g.nc;
+    level_ws(1, coarse, 1);
+    level_ws(2, level_pm2(), g.ntiles);
     for (int iapm = 2; iapm <= 5; ++iapm) {
       const int64_t nb = (int64_t)std::count(ires_h.begin(), ires_h.end(), iapm);
-      level_ws(g.nft[iapm], nb, true);
+      level_ws(3, level_pm3(iapm), nb);
       // the PP batch rule of pp_phase
       const int64_t m = (int64_t)g.ntt * kRatioSF[iapm] + 2, m3 = m * m * m * kSX;
       if (nb > 0 && std::max<int64_t>(1, ws_budget() / 4 / (m3 * 12)) < nb) multi = true;
     }
     work.ensure((size_t)need);
-    // the whole-image meshes of the levels that take them
-    int64_t cells = 0, faces = 0;
-    auto image_ws = [&](int level, const PMLevel& L, int64_t nmesh) {
-      if (nmesh <= 0) return;
-      const int64_t n = L.n;
-      const int64_t per = n * n * n * (int64_t)sizeof(R) + n * n * (n / 2 + 1) * (int64_t)sizeof(C);
-      const int64_t batch = std::max<int64_t>(1, std::min<int64_t>(nmesh, ws_budget() / per));
-      if (!image_mesh_level<R>(level, L, nmesh, batch)) return;
-      const int64_t m = g.nc * L.w;
-      cells = std::max(cells, m * m * m);
-      faces = std::max(faces, batch * 6 * n * n);
-    };
-    image_ws(2, level_pm2(), g.ntiles);
-    if (cfg.pm3)
-      for (int iapm = 2; iapm <= 5; ++iapm)
-        image_ws(3, level_pm3(iapm), (int64_t)std::count(ires_h.begin(), ires_h.end(), iapm));
-    if (cells > 0) {
-      gmesh.ensure((size_t)cells);
-      gfaces.ensure((size_t)faces);
-    }
+    if (image > 0) gmesh.ensure((size_t)(image / 4));
   }
   return multi;
 }
@@ -1128,14 +1142,7 @@ void cube_p3m_ctx::kick(const cube_kick_in& in, cube_kick_out& out, float* densi
   } hold{wsb};
   wsb = -1;
   wsb = ws_budget();
-  image_meshes = false;
-  if (std::is_same<R, float>::value && (mask & 6)) {
-    check_images();
-    if (nu && nu->images == 0) {
-      nu->check_images();
-    }
-    image_meshes = images == 1 && (!nu || nu->images == 1);
-  }
+  plan_images<R>(mask);
   const bool use_graph = graph_on && mask == 15 && !density_host && !nu;
   const bool overlap =
       !use_graph && overlap_on && mask == 15 && !density_host && !nu && cfg.pm3 && cfg.pp && kicks_done > 0;

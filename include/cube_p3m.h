@@ -68,7 +68,11 @@ typedef struct cube_p3m_config {
   double mass_nu;      /* sum of neutrino masses (eV)         parameters.f90:104 */
   float image_buffer;  /* parameters.f90:85 */
   float tile_buffer;   /* parameters.f90:86 */
-  int64_t workspace_bytes; /* device budget for batched tile meshes; 0 = auto */
+  int64_t workspace_bytes; /* device budget of a kick's meshes: the batched tile
+                          meshes and the whole-image mesh that they may be cut
+                          from (at least one tile mesh is held whatever it is).
+                          0 = auto: 35% of the free memory, at most 24 GiB, for
+                          the tile meshes, and half as much for the other */
   int32_t ires_fixed;  /* 0: sub-tile PM3/PP resolution from the occupancy
                           thresholds (kick.f90:116-130); 2..5: every sub-tile
                           at that ires (the commented ires(itile)=4, kick.f90:131) */
