@@ -547,7 +547,7 @@ void cube_p3m_ctx::run_level(int level, int slot, const std::vector<PMBox>& bx_i
         if constexpr (std::is_same<R, float>::value) {
           auto window = [&](cube_p3m_ctx* c, float m, float* out) {
             // the image's mesh holds every box of the level: once per level and species
-            if (b0 == 0 || nu) pm_mesh_deposit((int)g.izipx, M, c->xpc(), c->rhocc(), c->off.p, gmesh.p, m, s);
+            if (b0 == 0 || (nu && level <= 2)) pm_mesh_deposit((int)g.izipx, M, c->xpc(), c->rhocc(), c->off.p, gmesh.p, m, s);
             pm_mesh_faces((int)g.izipx, M, L, boxes.p, nb, c->xpc(), c->rhocc(), c->off.p, faces, m, s);
             if (direct) win = FFTWindow{gmesh.p, faces, lorg[slot].p, M.n};
             else pm_mesh_window(M, (int)n, lorg[slot].p, nb, gmesh.p, faces, out, s);
