@@ -26,6 +26,7 @@
 // particle moves by more than M cells, those beyond M have nothing to send: 192^3
 // in 64 tiles of 12^3 cells visits 14^3 of 24^3.
 #include "drift.h"
+#include "grid.h"
 
 namespace cube {
 namespace {
@@ -74,7 +75,7 @@ template <int IZ>
 __global__ void k_drift_shift(DriftParams P, const XT<IZ>* __restrict__ xp, const float* __restrict__ vp,
                               const int32_t* __restrict__ rhoc, const int64_t* __restrict__ off, int64_t ncells,
                               int32_t* __restrict__ flags, int32_t* __restrict__ newcount) {
-  const int64_t c = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
+  const int64_t c = ((int64_t)blockIdx.y * gridDim.x + blockIdx.x) * 4 + (threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
   if (c >= ncells) return;
   int T, ijk[3];
@@ -413,13 +414,13 @@ void drift_tile_check(const int64_t* off, int64_t ncell_tile, int ntiles, int64_
 
 void drift_shift(const DriftParams& P, const void* xp, const float* vp, const int32_t* rhoc, const int64_t* off,
                  int64_t ncells, DriftScratch& S, hipStream_t s) {
-  const int64_t nthr = ncells * 64;
+  const Blocks b = blocks_xy(ceil_div(ncells, 4));  // a wavefront per cell
   if (P.izipx == 2)
-    hipLaunchKernelGGL(k_drift_shift<2>, dim3((unsigned)ceil_div(nthr, 256)), dim3(256), 0, s, P,
-                       (const int16_t*)xp, vp, rhoc, off, ncells, S.flags, S.newcount);
+    hipLaunchKernelGGL(k_drift_shift<2>, dim3(b.x, b.y), dim3(256), 0, s, P, (const int16_t*)xp, vp, rhoc, off, ncells,
+                       S.flags, S.newcount);
   else
-    hipLaunchKernelGGL(k_drift_shift<1>, dim3((unsigned)ceil_div(nthr, 256)), dim3(256), 0, s, P, (const int8_t*)xp,
-                       vp, rhoc, off, ncells, S.flags, S.newcount);
+    hipLaunchKernelGGL(k_drift_shift<1>, dim3(b.x, b.y), dim3(256), 0, s, P, (const int8_t*)xp, vp, rhoc, off, ncells,
+                       S.flags, S.newcount);
   CUBE_HIP(hipGetLastError());
 }
 

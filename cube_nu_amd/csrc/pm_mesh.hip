@@ -14,6 +14,7 @@
 // k_mesh_window cuts the windows out.
 #include <algorithm>
 
+#include "grid.h"
 #include "pm_dev.h"
 #include "pm_mesh.h"
 
@@ -345,7 +346,7 @@ template <int IZ>
 __global__ void __launch_bounds__(256) k_mesh_images(Geo g, const XT<IZ>* __restrict__ xp,
                                                      const int32_t* __restrict__ rhoc,
                                                      const int64_t* __restrict__ off, int32_t* __restrict__ bad) {
-  const int64_t c = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
+  const int64_t c = ((int64_t)blockIdx.y * gridDim.x + blockIdx.x) * 4 + (threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
   if (c >= g.ncells_ext) return;
   const int64_t T = c / g.ncell_tile, e = c % g.ncell_tile;
@@ -441,7 +442,8 @@ void pm_mesh_window(const MeshGeo& M, int n, const int4* org, int nbox, const fl
 void mesh_check_images(int izipx, const Geo& g, const void* xp, const int32_t* rhoc, const int64_t* off, int32_t* bad,
                        hipStream_t s) {
   zero_async(bad, sizeof(int32_t), s);
-  const dim3 grid((unsigned)ceil_div(g.ncells_ext * 64, 256));
+  const Blocks b = blocks_xy(ceil_div(g.ncells_ext, 4));
+  const dim3 grid(b.x, b.y);
   if (izipx == 2)
     hipLaunchKernelGGL(k_mesh_images<2>, grid, dim3(256), 0, s, g, (const int16_t*)xp, rhoc, off, bad);
   else
