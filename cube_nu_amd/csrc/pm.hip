@@ -772,7 +772,10 @@ __global__ void __launch_bounds__(256) k_interp(PMLevel L, const PMBox* __restri
 // the forces are read from LDS as broadcasts.  Blocks of 4^3 or 2^3 cells keep the
 // chip busy on small images (192^3 is 216 blocks of 8^3).  512^3 1.31 ms (4 GB, 3.1
 // TB/s; 1.35 with a search of its cell per particle), 192^3 0.09 (0.40), 128^3 0.04
-// (0.32), its FP64 form 0.06 (0.34).
+// (0.32), its FP64 form 0.06 (0.34).  What a cell holds beyond its first kLong is the
+// whole workgroup's (64^3 with 30000 particles in one cell 0.17 ms; 0.55 with the cell a
+// wavefront's, 0.23 with a search per particle).
+constexpr int kLong = 512;
 template <typename R, int IZ, int BD>
 __global__ void __launch_bounds__(256, 8) k_interp_unit(PMLevel L, const PMBox* __restrict__ boxes,
                                                      const XT<IZ>* __restrict__ xp, float* __restrict__ vp,
@@ -782,6 +785,7 @@ __global__ void __launch_bounds__(256, 8) k_interp_unit(PMLevel L, const PMBox* 
   __shared__ R ps[PS * PS * PS], fs[3 * FN];
   __shared__ int cnt[BD * BD * BD];
   __shared__ int64_t gof[BD * BD * BD];
+  __shared__ unsigned long long long_cells;
   if (L.kdev) kc = *L.kdev;
   const uint32_t nblk = (uint32_t)(L.nforce + BD - 1) / BD;
   const uint32_t by_ = blockIdx.x / nblk, bz_ = by_ / nblk, ibox = bz_ / nblk;
@@ -798,8 +802,11 @@ __global__ void __launch_bounds__(256, 8) k_interp_unit(PMLevel L, const PMBox* 
       ok = ok && c[d] >= B.nc1[d] && c[d] <= B.nc2[d];
     }
     const int64_t cell = ok ? rc_index(c[0], c[1], c[2], B.T, L.nte, L.ncb) : 0;
-    cnt[lane] = ok ? rhoc[cell] : 0;
+    const int n = ok ? rhoc[cell] : 0;
+    cnt[lane] = n;
     gof[lane] = ok ? off[cell] : 0;
+    const unsigned long long m = __builtin_amdgcn_ballot_w64(n > kLong);
+    if (lane == 0) long_cells = m;
   }
   for (int t = threadIdx.x; t < PS * PS * PS; t += 256) {
     const int l[3] = {t % PS, (t / PS) % PS, t / (PS * PS)};
@@ -852,13 +859,25 @@ __global__ void __launch_bounds__(256, 8) k_interp_unit(PMLevel L, const PMBox* 
   }
   __syncthreads();
   R vm[3] = {0, 0, 0};
+  auto kick = [&](int c, int64_t ip, const uint32_t u[3], const float v0[3]) {
+    // xpos = (c-1) + (u + 1/2) 2^-B - s exactly: fraction (u + 1/2) 2^-B (exact in R)
+    R w[3][3], dv[3];
+    for (int d = 0; d < 3; ++d) tsc_weights_frac<R>(((R)u[d] + (R)0.5) * kRes, w[d]);
+    int lv = ((c / (BD * BD)) * FS + (c / BD) % BD) * FS + c % BD;
+    asm volatile("" : "+v"(lv));  // the 81 forces are read as they are used, not held for the cell's next 64 particles
+    tsc_gather<R>(fs, FN, FS, FS * FS, lv, w, dv);
+    for (int d = 0; d < 3; ++d) {
+      const float v = (float)kick_update((R)v0[d], dv[d], kc);
+      vp[3 * ip + d] = v;
+      vm[d] = max(vm[d], (R)fabsf(v));
+    }
+  };
   for (int c = wave; c < BD * BD * BD; c += 4) {
     uint32_t u[3] = {un[0], un[1], un[2]};
     float v0[3] = {vn[0], vn[1], vn[2]};
-    const int n = cnt[c];
+    const int n = min(cnt[c], kLong);
     const int64_t base = gof[c];
     if (c + 4 < BD * BD * BD) load(c + 4);
-    const int li = ((c / (BD * BD)) * FS + (c / BD) % BD) * FS + c % BD;
     for (int l = lane; l < n; l += 64) {
       const int64_t ip = base + l;
       if (l != lane)
@@ -866,17 +885,20 @@ __global__ void __launch_bounds__(256, 8) k_interp_unit(PMLevel L, const PMBox* 
           u[d] = XP<IZ>::raw(xp, ip, d);
           v0[d] = vp[3 * ip + d];
         }
-      // xpos = (c-1) + (u + 1/2) 2^-B - s exactly: fraction (u + 1/2) 2^-B (exact in R)
-      R w[3][3], dv[3];
-      for (int d = 0; d < 3; ++d) tsc_weights_frac<R>(((R)u[d] + (R)0.5) * kRes, w[d]);
-      int lv = li;
-      asm volatile("" : "+v"(lv));  // the 81 forces are read as they are used, not held for the cell's next 64 particles
-      tsc_gather<R>(fs, FN, FS, FS * FS, lv, w, dv);
+      kick(c, ip, u, v0);
+    }
+  }
+  for (unsigned long long m = long_cells; m; m &= m - 1) {
+    const int c = __ffsll((long long)m) - 1, n = cnt[c];
+    for (int l = kLong + (int)threadIdx.x; l < n; l += 256) {
+      const int64_t ip = gof[c] + l;
+      uint32_t u[3];
+      float v0[3];
       for (int d = 0; d < 3; ++d) {
-        const float v = (float)kick_update((R)v0[d], dv[d], kc);
-        vp[3 * ip + d] = v;
-        vm[d] = max(vm[d], (R)fabsf(v));
+        u[d] = XP<IZ>::raw(xp, ip, d);
+        v0[d] = vp[3 * ip + d];
       }
+      kick(c, ip, u, v0);
     }
   }
   raise_maxima<R>(f2, vm, out);
