@@ -1098,8 +1098,7 @@ void cube_p3m_ctx::kick_graph(const cube_kick_in& in, cube_kick_out& out, bool w
     CUBE_HIP(hipGraphLaunch(gexec[part], s));
   };
   tm.enabled = false;
-  // part 0: PM1 + PM2 (its sizing is box tables, stencil and, at first use,
-  // the PM2 FFT shape trials)
+  // part 0: PM1 + PM2 (its sizing is box tables, window origins and the stencil)
   kph = 1;
   gsig_acc.clear();
   kick_pass<R>(in, out, nullptr, 3, false, ires_h, cmax_h);

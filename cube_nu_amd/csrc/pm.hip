@@ -917,8 +917,9 @@ __global__ void __launch_bounds__(256, 8) k_interp_unit(PMLevel L, const PMBox* 
 // autotuner (every shape gives the same result): a larger block stages a
 // smaller share of halo (phi halo 4.2 -> 3.3 values per cell, FD force on 1.76
 // -> 1.58 cells per cell) with twice the threads.
-// Bound by LDS (85% busy at 512^3 PM3, half of it the bank conflicts of the
-// 81 random reads per particle) and VALU (85%) alike.  4096 boxes of 64^3
+// Bound by LDS (busy 86 % of the cycles at 512^3 PM3, nearly half of it with the bank
+// conflicts of the 81 random reads per particle; the vector pipe takes 42 % of its
+// issue slots, the texture data unit is busy 93 %).  4096 boxes of 64^3
 // cells, 1.34e8 particles: 9.9 -> 8.6 ms with quad loads of phi and the
 // separable gather, 6.6 with the FD reads free of bank conflicts (x along the
 // lanes, pairs along z) and the maxima compared before any reduction.

@@ -56,8 +56,9 @@ __device__ inline bool pp_cell(const PPLevel& L, const PPBox& B, int ci, int cj,
 // start + rank.  Sub-bins are numbered ((z*m + y)*m + x)*kSX + q: each (y, z)
 // row of the PP grid is one contiguous, x-ordered run of the CSR.  The count pass
 // needs no order: LDS adds take the ballots' place, and it writes every sub-bin, so
-// that none is cleared first.  Bound by the vector pipe and a chain of loads per
-// wavefront: 512^3 2.0 + 2.9 ms (2.5 + 2.9 with ballots in both; 3 GB of entries).
+// that none is cleared first.  Bound by a chain of loads per wavefront (the texture
+// data unit is busy 99 % of the cycles, the vector pipe 53 and 47 % of its issue
+// slots): 512^3 2.0 + 2.9 ms (2.5 + 2.9 with ballots in both; 3 GB of entries).
 template <int IZ, int FILL>
 __global__ void __launch_bounds__(256) k_pp_bin(PPLevel L, const PPBox* __restrict__ boxes, int nbox,
                                                 const XT<IZ>* __restrict__ xp, const int32_t* __restrict__ rhoc,

@@ -15,7 +15,9 @@ namespace cube {
 class Transfers {
  public:
   ~Transfers();
-  // host -> device, queued on s; the host array may change when it returns
+  // host -> device, queued on s.  An array that is staged may change when it returns;
+  // one the runtime copies itself (pinned, managed, small) only once s has come that
+  // far: the caller synchronises before it gives such an array back
   void in(void* dev, const void* host, size_t bytes, hipStream_t s);
   // device -> host after what s holds; the array is complete once s is synchronised
   void out(void* host, const void* dev, size_t bytes, hipStream_t s);
