@@ -222,12 +222,22 @@ bool fft_convolve_lines(const FFTCube<R>& c, R* rho, typename Cplx<R>::T* work, 
                         R div3, R div1, hipStream_t s, KTimer* tm, const char* tag) {
   if constexpr (std::is_same<R, float>::value) {
     const std::string t(tag);
+    // below 208 the plane form's sizes beyond 88 points, for coarse meshes beside another
+    // stream (with generic line passes: 104 0.042 / 0.096 ms alone, 144 0.063 / 0.122,
+    // 192 0.092 / 0.210); above, where no plane form is
     switch (c.n) {
 #define CUBE_FFT_SIZE(n) \
   case n: return run_lines<R, n>(c, rho, work, G, nbox, div3, div1, s, tm, t);
       CUBE_FFT_SIZE(96)
+      CUBE_FFT_SIZE(104)
       CUBE_FFT_SIZE(112)
+      CUBE_FFT_SIZE(120)
       CUBE_FFT_SIZE(128)
+      CUBE_FFT_SIZE(144)
+      CUBE_FFT_SIZE(160)
+      CUBE_FFT_SIZE(168)
+      CUBE_FFT_SIZE(176)
+      CUBE_FFT_SIZE(192)
       CUBE_FFT_SIZE(208)
       CUBE_FFT_SIZE(210)
       CUBE_FFT_SIZE(216)
