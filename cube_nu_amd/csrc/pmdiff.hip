@@ -530,9 +530,10 @@ __device__ inline int row_of(const unsigned* pre, int rows, unsigned k) {
 // (contribution int(W g S), out = sum / S).  The integers are those of
 // k_tsc_deposit: the outputs are the same bit for bit.  Bound by the latency of a
 // particle's chain of loads, weights and LDS adds, no pipe being full (four meshes
-// of 256^3: 37 % of the vector issue slots, LDS busy 41 % of the cycles, a third of
-// it with conflicts, the texture data unit 66 %; NC = 3 31, 51 and 63 %; CIC 45, 34 and
-// 72 %): 16 x 8 x 8 cells are read by 1.8 times their particles, 8^3 by 2.0 times.
+// of 256^3: 51 % of the vector issue slots, LDS busy 55 % of the cycles, a third of
+// it with conflicts, the texture data unit 84 %; NC = 3 39, 61 and 77 %; CIC, four of 128^3,
+// 56, 43 and 72 %): 16 x 8 x 8 cells are read by 1.8 times their particles, 8^3 by 2.0
+// times.  Few dense tiles (90^3) leave all of them below 60 %.
 // Four meshes of 256^3 with 128^3 particles each: 0.24 ms, NC = 3 0.53 ms (lists by
 // tile of 8^3: 0.46 and 1.12); three of 90^3, 750 000 particles: 0.060 and 0.11 ms
 // (global atomics with their pass to floats: 0.5 and 1.4).  CIC: the density of cube_pm_cic (contribution
@@ -869,9 +870,9 @@ __global__ void __launch_bounds__(64) k_tsc_vjp(const float* __restrict__ x, uin
 // part of phi: then no force mesh is read, or written, at all.  V = 4: quads
 // along x (n a multiple of 4, aligned meshes).  VJP: g_x = sum grad W (F.g +
 // rhobar); else acc = sum W F.  Bound by the latency of its three phases (three
-// workgroups of 49 KB share a CU; LDS is busy 63 % of the cycles, half of it with
-// conflicts, the vector pipe 27 % of its issue slots, the texture data unit 71 %; VJP 45, 27
-// and 86 %).
+// workgroups of 49 KB share a CU; LDS is busy 65 % of the cycles, half of it with
+// conflicts, the vector pipe 28 % of its issue slots, the texture data unit 71 %; VJP 47, 28
+// and 85 %).
 // Four meshes of 256^3 with 128^3 particles each: 0.47 ms, VJP 0.56 ms, where
 // force meshes written and gathered from took 0.31 + 0.50 and 0.63 ms.
 template <bool VJP, int V, bool FAR>
