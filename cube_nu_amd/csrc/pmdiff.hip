@@ -227,19 +227,16 @@ __global__ void __launch_bounds__(1024) k_absmax(const float* __restrict__ g, in
 // one wavefront spread them over the chip).  NC = 1: rho += W (fixed point
 // 2^-32); NC = 3: Fbar[b][d] += W g_d at scale S.
 constexpr int kFew = 63;  // threads of a block that work: 21 particles
-// The particle (past the last one, none) of this thread; blocks go on along y.
-__device__ inline int64_t few_particle() {
-  return ((int64_t)blockIdx.y * gridDim.x + blockIdx.x) * (kFew / 3) + threadIdx.x / 3u;
-}
+// This thread's particle of a launch from p0 on (past the last one, none; below 2^32 either way).
+__device__ inline uint32_t few_particle(uint32_t p0) { return p0 + blockIdx.x * (kFew / 3) + threadIdx.x / 3u; }
 template <int NC>
-__global__ void __launch_bounds__(64) k_tsc_deposit(const float* __restrict__ x, const float* __restrict__ g, uint32_t np, uint32_t ntot,
+__global__ void __launch_bounds__(64) k_tsc_deposit(const float* __restrict__ x, const float* __restrict__ g, uint32_t p0, uint32_t np, uint32_t ntot,
                               int n, Lattice lt, const unsigned int* __restrict__ gmax,
                               unsigned long long* __restrict__ acc) {
   const double S = NC == 3 ? fix_scale(gmax) : 1.0;
-  const int64_t q = few_particle();
+  const uint32_t p = few_particle(p0);
   const int k3 = (int)(threadIdx.x % 3u);
-  if (threadIdx.x >= kFew || q >= ntot) return;
-  const uint32_t p = (uint32_t)q;
+  if (threadIdx.x >= kFew || p >= ntot) return;
   uint32_t b;
   int i[3];
   float d[3], w[3][3], gs[3] = {0, 0, 0};
@@ -782,10 +779,9 @@ __device__ inline float add3(float v) {
 }
 
 // acc_p = sum W F.
-__global__ void __launch_bounds__(64) k_tsc_interp(const float* __restrict__ x, uint32_t np, uint32_t ntot, int n,
+__global__ void __launch_bounds__(64) k_tsc_interp(const float* __restrict__ x, uint32_t p0, uint32_t np, uint32_t ntot, int n,
                                                    Lattice lt, const float* __restrict__ F, float* __restrict__ acc) {
-  const int64_t q = few_particle();
-  const uint32_t p = (uint32_t)min(q, (int64_t)ntot - 1);
+  const uint32_t q = few_particle(p0), p = min(q, ntot - 1);
   const int k3 = (int)(threadIdx.x % 3u);
   uint32_t b;
   int i[3];
@@ -814,11 +810,10 @@ __global__ void __launch_bounds__(64) k_tsc_interp(const float* __restrict__ x, 
 }
 
 // g_x = sum grad W (F.g + rhobar).
-__global__ void __launch_bounds__(64) k_tsc_vjp(const float* __restrict__ x, uint32_t np, uint32_t ntot, int n,
+__global__ void __launch_bounds__(64) k_tsc_vjp(const float* __restrict__ x, uint32_t p0, uint32_t np, uint32_t ntot, int n,
                                                 Lattice lt, const float* __restrict__ F, const float* __restrict__ g,
                                                 const float* __restrict__ rhob, float* __restrict__ gx) {
-  const int64_t q = few_particle();
-  const uint32_t p = (uint32_t)min(q, (int64_t)ntot - 1);
+  const uint32_t q = few_particle(p0), p = min(q, ntot - 1);
   const int k3 = (int)(threadIdx.x % 3u);
   uint32_t b;
   int i[3];
@@ -1100,8 +1095,7 @@ inline unsigned nblk(int64_t n, int t = 256) { return (unsigned)((n + t - 1) / t
 // against 114).
 template <class Fn>
 inline void over_cells(int64_t n, Fn&& fn) {
-  constexpr int64_t kMost = (int64_t)1 << 30;
-  for (int64_t at = 0; at < n; at += kMost) fn(dim3(nblk(std::min(n - at, kMost))), at, std::min(n - at, kMost));
+  in_pieces(n, (int64_t)1 << 30, [&](int64_t at, int64_t m) { fn(dim3(nblk(m)), at, m); });
 }
 inline void zero_cells(unsigned long long* a, int64_t n, hipStream_t s) {
   over_cells(n, [&](dim3 grid, int64_t at, int64_t m) {
@@ -1235,9 +1229,12 @@ struct cube_pm_ctx {
       place<Sort::kPart>(x, g, np, cfg.n, 1.0f, s);
     }
   }
-  static dim3 few_blocks(int64_t ntot) {
-    const Blocks b = blocks_xy(ceil_div(ntot, kFew / 3));
-    return dim3(b.x, b.y);
+  // Launches of the forms for few particles, fn(blocks, first particle): one, but for more
+  // particles than fit the threads of a launch dimension.
+  template <class Fn>
+  static void over_few(int64_t ntot, Fn&& fn) {
+    in_pieces(ntot, ((int64_t)1 << 25) * (kFew / 3),
+              [&](int64_t p0, int64_t m) { fn(dim3((unsigned)ceil_div(m, kFew / 3)), (uint32_t)p0); });
   }
 
   void check_np(int64_t np) const {
@@ -1280,8 +1277,10 @@ struct cube_pm_ctx {
       hipLaunchKernelGGL((k_pm_deposit<1, false>), dim3(tiles.blocks()), dim3(256), 0, s, rec.p, nullptr, n, tiles,
                          bstart.p, nullptr, phi);
     } else {
-      hipLaunchKernelGGL(k_tsc_deposit<1>, few_blocks(ntot), dim3(64), 0, s, x, nullptr, (uint32_t)np,
-                         (uint32_t)ntot, n, lat, nullptr, acc.p);
+      over_few(ntot, [&](dim3 grid, uint32_t p0) {
+        hipLaunchKernelGGL(k_tsc_deposit<1>, grid, dim3(64), 0, s, x, nullptr, p0, (uint32_t)np, (uint32_t)ntot, n, lat,
+                           nullptr, acc.p);
+      });
       fix_to_float(acc.p, B * n3, 1.0 / kFix, phi, s);
     }
     fft_convolve<float>(fc, phi, work.p, G.p, B, (float)n3, 0.0f, s);
@@ -1297,8 +1296,9 @@ struct cube_pm_ctx {
     if (!F && !srt) F = Fs.p;
     if (F) fd(false, phi, F, s);
     if (!srt)
-      hipLaunchKernelGGL(k_tsc_interp, few_blocks(ntot), dim3(64), 0, s, x, (uint32_t)np, (uint32_t)ntot, n, lat,
-                         F, out);
+      over_few(ntot, [&](dim3 grid, uint32_t p0) {
+        hipLaunchKernelGGL(k_tsc_interp, grid, dim3(64), 0, s, x, p0, (uint32_t)np, (uint32_t)ntot, n, lat, F, out);
+      });
     else
       gather<false>(quads(n, phi, nullptr), phi, nullptr, nullptr, out, s);
     if (to && to != phi)
@@ -1328,8 +1328,10 @@ struct cube_pm_ctx {
       }
       hipLaunchKernelGGL(k_absmax, dim3((unsigned)std::min<int64_t>(ceil_div(3 * ntot, 4096), kSlots)), dim3(1024), 0,
                          s, g, 3 * ntot, gmax.p);
-      hipLaunchKernelGGL(k_tsc_deposit<3>, few_blocks(ntot), dim3(64), 0, s, x, g, (uint32_t)np, (uint32_t)ntot,
-                         n, lat, gmax.p, acc.p);
+      over_few(ntot, [&](dim3 grid, uint32_t p0) {
+        hipLaunchKernelGGL(k_tsc_deposit<3>, grid, dim3(64), 0, s, x, g, p0, (uint32_t)np, (uint32_t)ntot, n, lat,
+                           gmax.p, acc.p);
+      });
       over_cells(3 * B * n3, [&](dim3 grid, int64_t at, int64_t m) {
         hipLaunchKernelGGL(k_sfix_to_float, grid, dim3(256), 0, s, acc.p + at, m, gmax.p, Fbar.p + at);
       });
@@ -1337,8 +1339,9 @@ struct cube_pm_ctx {
     fd(true, Fbar.p, mesh.p, s);
     fft_convolve<float>(fc, mesh.p, work.p, G.p, B, (float)n3, 0.0f, s);
     if (!srt)
-      hipLaunchKernelGGL(k_tsc_vjp, few_blocks(ntot), dim3(64), 0, s, x, (uint32_t)np, (uint32_t)ntot, n, lat, F,
-                         g, mesh.p, gx);
+      over_few(ntot, [&](dim3 grid, uint32_t p0) {
+        hipLaunchKernelGGL(k_tsc_vjp, grid, dim3(64), 0, s, x, p0, (uint32_t)np, (uint32_t)ntot, n, lat, F, g, mesh.p, gx);
+      });
     else
       gather<true>(quads(n, phi, mesh.p), phi, F, mesh.p, gx, s);
     CUBE_HIP(hipGetLastError());
@@ -1464,12 +1467,12 @@ int cube_pm_cic(cube_pm_ctx* ctx, const float* x, int64_t np, int32_t nw, float 
     const hipStream_t s = (hipStream_t)stream;
     const int B = ctx->cfg.batch;
     const int64_t ntot = np * B, nw3 = (int64_t)nw * nw * nw;
-    const bool captured = ctx->capturing(s), srt = ctx->cic_sorted(ntot, nw, s);
+    const bool srt = ctx->cic_sorted(ntot, nw, s);
     // The accumulator of the form by atomics: that of the forces, or a larger one, which
     // is made in either form: a call recorded later may have more particles than
     // the order's buffers hold, and cannot allocate.
     const size_t cells = (size_t)(B * nw3);
-    const bool own = cells > ctx->acc.n;
+    const bool own = cells > ctx->acc.n, captured = own && ctx->capturing(s);
     if (own && cells > ctx->accw.n && !(captured && srt))
       zero_cells(ctx->accw.ensure(cells), B * nw3, s);
     if (srt) {
@@ -1481,7 +1484,7 @@ int cube_pm_cic(cube_pm_ctx* ctx, const float* x, int64_t np, int32_t nw, float 
       CUBE_HIP(hipGetLastError());
       return;
     }
-    if (own && captured) ctx->accw.hold();
+    if (captured) ctx->accw.hold();
     unsigned long long* const acc = own ? ctx->accw.p : ctx->acc.p;
     hipLaunchKernelGGL(k_cic_deposit, dim3(nblk(ntot)), dim3(256), 0, s, x, (uint32_t)np, (uint32_t)ntot, nw, scale, ctx->lat,
                        acc);

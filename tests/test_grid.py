@@ -1,8 +1,8 @@
 """Launches of more blocks than a dimension's threads allow (cube_nu_amd/csrc/grid.h):
-every block has its place, and no dimension reaches 2^32 threads.  The forms for
-few particles have 21 particles to a block of 64 threads, and take up to 2^32 - 257
-particles (a recorded call, or meshes beyond 1024 points); along x alone they
-would end at 1.41e9.
+every block has its place, and no dimension reaches 2^32 threads; or, in pieces, every
+item has one, and no piece is larger than it may be.  The forms for few particles have
+21 particles to a block of 64 threads, and take up to 2^32 - 257 particles (a recorded
+call, or meshes of few tiles); in one launch they would end at 1.41e9.
 """
 import os
 import shutil
@@ -35,6 +35,37 @@ int main() {
 def test_every_block_has_a_place(tmp_path):
     src = tmp_path / "t.cpp"
     src.write_text(PROGRAM)
+    subprocess.run(["g++", "-std=c++17", "-I", CSRC, str(src), "-o", str(tmp_path / "t")], check=True)
+    r = subprocess.run([str(tmp_path / "t")], capture_output=True, text=True)
+    assert r.returncode == 0 and r.stdout == "ok\n", r.stdout
+
+
+PIECES = r"""
+#include <cstdio>
+#include "grid.h"
+int main() {
+  const int64_t cells = (int64_t)1 << 30, few = ((int64_t)1 << 25) * 21;
+  const int64_t n[] = {1, 21, cells - 1, cells, cells + 1, 3ll * 1152 * 1152 * 1152, few, few + 1, 0xffffff00ll};
+  for (int64_t most : {cells, few})
+    for (int64_t k : n) {
+      int64_t next = 0;
+      bool ok = true;
+      cube::in_pieces(k, most, [&](int64_t at, int64_t m) {
+        ok = ok && at == next && m > 0 && m <= most;
+        next = at + m;
+      });
+      if (!ok || next != k) { std::printf("%lld\n", (long long)k); return 1; }
+    }
+  std::puts(cells < 0xffffffffll && few / 21 * 64 < 0xffffffffll ? "ok" : "too large");
+  return 0;
+}
+"""
+
+
+@pytest.mark.skipif(shutil.which("g++") is None, reason="no host compiler")
+def test_pieces_hold_every_item_once(tmp_path):
+    src = tmp_path / "t.cpp"
+    src.write_text(PIECES)
     subprocess.run(["g++", "-std=c++17", "-I", CSRC, str(src), "-o", str(tmp_path / "t")], check=True)
     r = subprocess.run([str(tmp_path / "t")], capture_output=True, text=True)
     assert r.returncode == 0 and r.stdout == "ok\n", r.stdout
