@@ -168,7 +168,7 @@ __device__ inline int cell_at(int starts, int cells, int pos) {
 // caller redoes the drift with the measured bound.  P.images: the ring is cut to
 // the bound, so every particle that moves as far as it, wherever it goes, sets that
 // flag (by a margin beyond the rounding of the positions, which differ between a
-// particle and its images).  The run's counts are kept in LDS up to kLdsDirs
+// particle and its images; along an axis at rest, M = 0, any that moves does).  The run's counts are kept in LDS up to kLdsDirs
 // directions and written once, else in the (cleared) table.  A wave per cell with
 // a loop over its directions, their counts in memory and every cell of the
 // extended tiles took 0.353 ms at 192^3 (64 tiles of 12^3 cells, 57 million
@@ -211,7 +211,7 @@ __global__ void __launch_bounds__(256) k_drift_rank(DriftParams P, Runs R, const
           if (g[d] < lo || g[d] > hi) err |= DRIFT_OUT_OF_RANGE;
         if (P.images)
           for (int d = 0; d < 3; ++d)
-            if (!(fabs(P.dt_mid * (double)vp[3 * ip + d] * P.inv_rcs) <= P.M[d] - 1e-6)) err |= DRIFT_SHIFT_BOUND;
+            if (!(fabs(P.dt_mid * (double)vp[3 * ip + d] * P.inv_rcs) <= fmax(P.M[d] - 1e-6, 0.0))) err |= DRIFT_SHIFT_BOUND;
       }
       if (physical(P, g)) {
         bool fits = true;

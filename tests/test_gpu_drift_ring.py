@@ -49,3 +49,32 @@ def test_ring_and_restart(izipx, nnt, cells, follow, ring, again):
     assert st == 0 and d["nlayer"] == oo["nlayer"] and d["nplocal"] == oo["nplocal"]
     assert np.array_equal(rg, ro)
     assert np.array_equal(xg, xo) and np.array_equal(vg, vo) and np.array_equal(pg, po)
+
+
+@pytest.mark.parametrize("rest", [(0, 0, 1), (1, 0, 1), (1, 1, 1)])
+def test_axes_at_rest(rest):
+    """Where nothing moves along an axis its bound is 0, and no particle is beyond it."""
+    geo = Geometry(64, nnt=4, nns=2)
+    xp, vp, pid, rhoc = buffered_set(geo, seed=8, mean=5.0)
+    vp = vp * np.float32(3.0 / np.abs(vp).max()) * np.array([1 - r for r in rest], np.float32)
+    p = P3M(64, nnt=4, nns=2)
+    try:
+        p.upload(xp, np.ascontiguousarray(vp), pid, rhoc)
+        k = p.kick_resident(a_mid=0.5, dt=0.0)
+        p.buffer_v_resident()
+        xe, ve, pe, re = p.download()
+        p.timing(True)
+        p.timing_reset()
+        dt = 0.4 * geo.ratio_cs / 3.0
+        d = p.drift_resident(dt_old=dt, dt=dt, vz_max=k["vz_max"])
+        rep = p.timing_report()
+        xg, vg, pg, rg = p.download()
+    finally:
+        p.close()
+    assert list(np.abs(ve).max(0) == 0) == [bool(r) for r in rest]
+    assert rep["drift_ring_last"]["calls"] == (0 if all(rest) else 1)
+    assert rep["drift_rank"]["calls"] == 1 and "drift_shift" not in rep
+    st, xo, vo, po, ro, oo = orc.drift(oparams(geo), xe, ve, pe, re, dt, dt, k["vz_max"])
+    assert st == 0 and d["nlayer"] == oo["nlayer"] and d["nplocal"] == oo["nplocal"]
+    assert np.array_equal(rg, ro)
+    assert np.array_equal(xg, xo) and np.array_equal(vg, vo) and np.array_equal(pg, po)
