@@ -495,9 +495,9 @@ void fft_convolve(const FFTCube<R>& c, R* rho, typename Cplx<R>::T* work, const 
       if (!small_lds && fft_convolve_boxes(c.n, rho, G, nbox, total > 0 ? total : nbox, div3, div1, s, t, tag, win))
         return;
     }
-    // planes of 88 points hold 32 KB, in FP64 of 64 34 KB; beyond (96 have line passes) it is 38
-    // KB and more, and the FP64 coarse meshes of 72 to 88 take as long by lines (kicks of
-    // 320^3 89.5 / 89.6 ms, 352^3 99.7 / 99.5)
+    // planes of 88 points hold 32 KB, in FP64 of 64 34 KB; beyond it is 38 KB and more: FP32
+    // has register lines there, and the FP64 coarse meshes of 72 to 88 take as long by
+    // generic ones (kicks of 320^3 89.5 / 89.6 ms, 352^3 99.7 / 99.5)
     const int small = sizeof(R) == 8 ? 64 : 88;
     if (!(small_lds && c.n > small) && fft_convolve_plane<R>(c, rho, work, G, nbox, div3, div1, s, t, tag, win)) return;
     if (win) throw Error(1, "FFT of " + std::to_string(c.n) + " points does not read windows");
